@@ -84,7 +84,8 @@ void freeAll(mfcl_ctx* c) {
   freePtr(c->ws_arena.p);
   freePtr(c->ws_io.p);
   freePtr(c->ws_arm.p);
-  c->ws_convex = c->ws_arena = c->ws_io = c->ws_arm = DevBuf();
+  freePtr(c->ws_cand.p);
+  c->ws_convex = c->ws_arena = c->ws_io = c->ws_arm = c->ws_cand = DevBuf();
   c->ws_convex_pairs = c->ws_arm_configs = 0;
   c->mesh_ws_waves = c->mesh_ws_cap = 0;
   c->d_counters = nullptr;
@@ -97,7 +98,7 @@ int reserveConvex(mfcl_ctx* ctx, uint64_t n) {
   // the counters of the last query live in this buffer
   ctx->d_counters = nullptr;
   ctx->d_qcounts = nullptr;
-  const size_t arena = epaArenaBytes(kReservedArenaSlices, 256);
+  const size_t arena = epaArenaBytes(kReservedArenaSlices);
   if (int rc = ensure(ctx, ctx->ws_convex, convexWsBytes(n, arena))) return rc;
   ctx->ws_convex_pairs = convexWsMaxPairs(ctx->ws_convex.bytes, arena);
   return MFCL_OK;
@@ -264,7 +265,7 @@ int mfcl_tune(mfcl_ctx* ctx, int32_t knob, int32_t value) {
   MFCL_NOT_WHILE_CAPTURING(ctx);
   switch (knob) {
     case MFCL_TUNE_GJK_GROUP:
-      if (value != 1 && value != 16 && value != 32 && value != 64) break;
+      if (value != 0 && value != 1 && value != 16 && value != 32 && value != 64) break;
       ctx->tune.gjk_group = value;
       return MFCL_OK;
     case MFCL_TUNE_EPA_THREADS:
@@ -570,7 +571,7 @@ int mfcl_convex_collide_contacts_dev(mfcl_ctx* ctx, const uint32_t* pa, const ui
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
   ctx->counters[0] = n;
   ConvexWs ws;
-  if (!carveConvexWs(ctx->ws_convex.p, ctx->ws_convex.bytes, n, epaArenaBytes(kReservedArenaSlices, 256), ws)) {
+  if (!carveConvexWs(ctx->ws_convex.p, ctx->ws_convex.bytes, n, epaArenaBytes(kReservedArenaSlices), ws)) {
     ctx->err = "convex workspace layout exceeds its allocation";
     return MFCL_E_STATE;
   }
@@ -603,7 +604,7 @@ int mfcl_convex_query_static_dev(mfcl_ctx* ctx, const uint32_t* pa, const uint32
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
   ctx->counters[0] = n;
   ConvexWs ws;
-  if (!carveConvexWs(ctx->d_static_scratch, kStaticScratchBytes, n, epaArenaBytes(kStaticArenaSlices, 256), ws)) {
+  if (!carveConvexWs(ctx->d_static_scratch, kStaticScratchBytes, n, epaArenaBytes(kStaticArenaSlices), ws)) {
     ctx->err = "static workspace layout exceeds its size";
     return MFCL_E_STATE;
   }

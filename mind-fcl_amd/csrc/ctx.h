@@ -101,10 +101,10 @@ struct mfcl_ctx {
   int n_cu{256};                 // compute units
   // launch-shape knobs (set by mfcl_tune / the autotuner)
   struct {
-    int gjk_group{1};           // lanes per pair in the GJK stage (1, 16, 32, 64)
-    int epa_threads{131072};    // persistent EPA lanes (multiple of 256): 64 per wavefront
+    int gjk_group{0};           // 0 by batch size; 1 a lane per pair; 16, 32, 64 a wavefront per pair
+    int epa_threads{196608};    // persistent EPA lanes (multiple of 256): 64 per wavefront
     int guess_policy{1};        // warm start: 0 MLP direction for every pair, 1 not for predicted penetration
-    int epa_lds_faces{64};      // face capacity of the LDS polytope (overflow continues or reruns at full size)
+    int epa_lds_faces{42};      // face capacity of the LDS polytope (overflow continues or reruns at full size)
     int epa_spill{1};           // overflow continues in a device-memory polytope (1) or reruns (0)
     int epa_overflow_waves{512};   // persistent wavefronts (one per block) for overflow pairs
     int mesh_blocks_per_cu{3};  // persistent mesh-traversal blocks (4 waves, one query each) per CU
@@ -162,6 +162,7 @@ struct mfcl_ctx {
   // upload (query entry points never grow them) and, for the host-pointer
   // wrappers, ws_io
   mfcl::DevBuf ws_convex, ws_arena, ws_io, ws_arm;
+  mfcl::DevBuf ws_cand;         // mesh-shape candidates
   uint64_t ws_convex_pairs{0};  // pairs ws_convex holds
   uint64_t ws_arm_configs{0};   // configurations ws_arm holds (for ws_arm_key's arm)
   uint64_t ws_arm_key[4]{};     // links, broadphase cap, max pairs per config, pair capacity
@@ -229,12 +230,13 @@ struct ConvexWs {
   void* queue;         // EPA queue
   void* oflow;         // EPA overflow queue
   double* lane_dirs;   // lane kernel direction slots
-  void* arena;         // EPA continuation polytopes (device memory), one per wavefront that may need one
+  void* arena;         // EPA dumps: pairs that continue at full capacity
   size_t arena_bytes;
 };
-// EPA continuation arena of the reserved workspace (2048 polytopes of 256
-// faces) and of the static one (256 such polytopes).
-size_t epaArenaBytes(int slices, int max_faces);
+// Bytes for the EPA dumps of the reserved workspace and of the static one,
+// in slices (about five dumps of the default LDS polytope each).
+size_t epaArenaBytes(int slices);
+constexpr size_t kEpaArenaSlice = 61696;
 constexpr int kReservedArenaSlices = 2048, kStaticArenaSlices = 256;
 size_t convexWsBytes(uint64_t n, size_t arena_bytes);
 uint64_t convexWsMaxPairs(size_t bytes, size_t arena_bytes);

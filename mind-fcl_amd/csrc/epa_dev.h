@@ -3,13 +3,17 @@
 //
 // GPU representation: one wavefront per pair; the polytope lives in that
 // wavefront's LDS slice as slot arrays of vertices, edges and faces (16-bit
-// indices, FP64 geometry) that the 64 lanes scan in parallel; creation
+// indices, FP64 geometry), visited by the 64 lanes in parallel; creation
 // stamps stand in for the reference's newest-first element lists.
+//
+// The loop is bound by the latency of one pair's chain of dependent steps.
+// What a step keeps between its phases lives in LDS, the support search is
+// one out-of-line function (wave_dev.h), and nothing spills.
 #pragma once
 
 #include <type_traits>
 
-#include "narrow_dev.h"
+#include "wave_dev.h"
 
 namespace mfcl {
 
@@ -20,27 +24,88 @@ constexpr int16_t kNil = -1;
 // as a scalar so that the branch on it is a scalar branch.
 MFCL_D bool ub(bool c) { return __builtin_amdgcn_readfirstlane(c ? 1 : 0) != 0; }
 
-struct EVert {
+struct EVertCore {
   double vx, vy, vz;  // vertex on the Minkowski difference
   double dx, dy, dz;  // direction that produced it
+  int32_t h0, h1;     // the support vertices of the two hulls (-1: primitive or unknown)
   int32_t stamp;      // creation order; < 0: free slot
   int16_t new_edge;
-  uint8_t remove, pad;
-  int32_t h0, h1;     // the support vertices of the two hulls (-1: primitive or unknown)
+  uint8_t remove, pad0;
 };
-struct EEdge {
+struct EEdgeCore {
   double d2, wx, wy, wz;  // squared distance to origin, witness
   int32_t stamp;
   int16_t v0, v1, f0, f1;
   uint8_t in, vis;
-  uint16_t pad;
+  uint16_t pad0;
 };
-struct EFace {
+struct EFaceCore {
   double d2, wx, wy, wz;
   int32_t stamp;
   int16_t e0, e1, e2;
   uint8_t in, vis;
+  int16_t a;     // the first edge's first vertex
+  uint8_t cls;   // NormalClass (kNormals polytopes)
+  uint8_t pad0;
 };
+// A face with its outward unit normal, which does not change while the face
+// lives -- unless the origin lies close to its plane: then n is the plane's
+// normal of either sign, and the side is decided by the vertices of the
+// moment.
+enum NormalClass : uint8_t { kNormalOut = 0, kNormalClose = 1, kNormalNone = 2 };
+struct EFaceNormal : EFaceCore {
+  double nx, ny, nz;
+};
+// PAD: records of an odd number of 8-byte words, so that the 64 lanes'
+// accesses to one field of consecutive slots spread over the LDS banks
+// (64- and 48-byte records put every fourth slot on the same bank).
+template <class R, bool PAD>
+struct Rec : R {};
+template <class R>
+struct Rec<R, true> : R {
+  int32_t spread[2];
+};
+static_assert(sizeof(Rec<EVertCore, true>) == 72 && sizeof(Rec<EEdgeCore, true>) == 56 &&
+                  sizeof(Rec<EVertCore, false>) == 64 && sizeof(EFaceCore) == 48 && sizeof(EFaceNormal) == 72,
+              "record sizes");
+
+// Where a polytope's slot arrays live and how an expansion marks its faces:
+// kWords 64-bit masks (64 kWords faces at most, kWords faces per lane; the
+// faces keep their normals), or, with 0, marks in the records.  Small: the
+// wavefront's share of a block's LDS.  Mid and Large: LDS at the request's
+// full capacity, up to 256 faces and beyond.  Global: device memory, a
+// capacity beyond the LDS.  sync() orders one lane's writes
+// before other lanes' reads of the same wavefront: LDS executes a
+// wavefront's operations in order, so a compiler barrier suffices there;
+// device memory needs a workgroup-scope fence.
+template <int WORDS>
+struct MaskMem {
+  static constexpr int kWords = WORDS;
+  static constexpr bool kPad = true;
+  using Face = EFaceNormal;
+  template <class T>
+  using P = MFCL_LDS T*;
+  static MFCL_D void sync() { __builtin_amdgcn_wave_barrier(); }
+};
+using SmallMem = MaskMem<1>;
+using MidMem = MaskMem<4>;
+struct LargeMem {
+  static constexpr int kWords = 0;
+  static constexpr bool kPad = false;
+  using Face = EFaceCore;
+  template <class T>
+  using P = MFCL_LDS T*;
+  static MFCL_D void sync() { __builtin_amdgcn_wave_barrier(); }
+};
+struct GlobalMem {
+  static constexpr int kWords = 0;
+  static constexpr bool kPad = false;
+  using Face = EFaceCore;
+  template <class T>
+  using P = T*;
+  static MFCL_D void sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); }
+};
+constexpr int kSmallFaces = 64, kMidFaces = 256;
 
 // Arena sizing for a given face capacity: vertices = edges = floor(1.51 F)
 // (epa_polytope.hpp:90-95).
@@ -53,16 +118,22 @@ __host__ __device__ inline ArenaDims arenaDims(int max_faces) {
   d.nf = max_faces;
   return d;
 }
-// Scratch record per border edge of one expansion (see Poly::expand).
+// Scratch record per border edge of one expansion (see coverBorder).
 struct BorderRec {
-  int32_t pre;     // elements (edges and faces) created before this edge's face
+  int16_t pre;     // elements (edges and faces) created before this edge's face
   int16_t e, rank; // edge slot, rank in descending stamp order
   int16_t fe, ff;  // the list of free edge / face slots (entry k: the k-th free slot)
   int8_t t0, t1;   // lower-ranked border edges sharing endpoint v0 / v1
 };
-__host__ __device__ inline size_t arenaBytes(int max_faces) {
+template <class M>
+__host__ __device__ inline size_t polyBytes(int max_faces) {
   const ArenaDims d = arenaDims(max_faces);
-  size_t b = sizeof(EVert) * d.nv + sizeof(EEdge) * d.nv + sizeof(EFace) * d.nf + sizeof(BorderRec) * d.nv;
+  return (sizeof(Rec<EVertCore, M::kPad>) + sizeof(Rec<EEdgeCore, M::kPad>)) * d.nv +
+         sizeof(typename M::Face) * d.nf;
+}
+template <class M>
+__host__ __device__ inline size_t arenaBytes(int max_faces) {
+  const size_t b = polyBytes<M>(max_faces) + sizeof(BorderRec) * arenaDims(max_faces).nv;
   return (b + 255) & ~static_cast<size_t>(255);
 }
 
@@ -144,23 +215,6 @@ MFCL_D void triDist0(d3 a, d3 b, d3 c, MinD& o) {
   o.w = best.w;
 }
 
-// Where a polytope's slot arrays live: the wavefront's LDS slice (the
-// normal case) or a device-memory arena (a polytope that outgrew the LDS
-// slice and continues at full capacity).  sync() orders one lane's writes
-// before other lanes' reads of the same wavefront: LDS executes a
-// wavefront's operations in order, so a compiler barrier suffices there;
-// device memory needs a workgroup-scope fence.
-struct LdsMem {
-  template <class T>
-  using P = MFCL_LDS T*;
-  static MFCL_D void sync() { __builtin_amdgcn_wave_barrier(); }
-};
-struct GlbMem {
-  template <class T>
-  using P = T*;
-  static MFCL_D void sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); }
-};
-
 // The polytope, processed by the 64 lanes of one wavefront together.
 // Elements live in fixed slot arrays (slot s is visited by lane s % 64);
 // a slot is free when its stamp is negative.  Every element gets a creation
@@ -173,6 +227,10 @@ struct GlbMem {
 // with identical arguments.
 template <class M>
 struct PolyT {
+  using EVert = Rec<EVertCore, M::kPad>;
+  using EEdge = Rec<EEdgeCore, M::kPad>;
+  using EFace = typename M::Face;
+  using Base = typename M::template P<char>;
   typename M::template P<EVert> V;
   typename M::template P<EEdge> E;
   typename M::template P<EFace> F;
@@ -180,34 +238,219 @@ struct PolyT {
   int nv, nf;   // slot capacities: vertices and edges nv, faces nf
   int stamp;    // creation counter
 
-  MFCL_D d3 vloc(int16_t i) const { return {V[i].vx, V[i].vy, V[i].vz}; }
-  MFCL_D d3 vdir(int16_t i) const { return {V[i].dx, V[i].dy, V[i].dz}; }
-
-  // epa_polytope.hpp:77-125: everything free
-  MFCL_D void reset() {
-    const int l = __lane_id();
-    for (int s = l; s < nv; s += 64) {
-      V[s].stamp = -1;
-      E[s].stamp = -1;
-    }
-    for (int s = l; s < nf; s += 64) F[s].stamp = -1;
+  MFCL_D PolyT(Base base, int cap_faces) {
+    const ArenaDims d = arenaDims(cap_faces);
+    V = (typename M::template P<EVert>)(base);
+    E = (typename M::template P<EEdge>)(base + sizeof(EVert) * d.nv);
+    F = (typename M::template P<EFace>)(base + (sizeof(EVert) + sizeof(EEdge)) * d.nv);
+    BL = (typename M::template P<BorderRec>)(base + (sizeof(EVert) + sizeof(EEdge)) * d.nv + sizeof(EFace) * d.nf);
+    nv = d.nv;
+    nf = d.nf;
     stamp = 0;
-    M::sync();
   }
-  // lowest free slot (the reference pops its free list; which slot is used
-  // does not matter, only the capacity does)
-  template <class A>
-  MFCL_D int16_t allocSlot(A arr, int cap) const {
+  MFCL_D d3 vloc(int i) const { return {V[i].vx, V[i].vy, V[i].vz}; }
+
+  // the initial polytope: vertices V[0 .. n_v) (written by the caller),
+  // edges and faces from 4-bit tables (entry k at bits 4 k); stamps in the
+  // order vertices, edges, faces; an edge's first face is its f0, the second
+  // its f1.  false: it does not fit.
+  MFCL_D bool build(int n_v, int n_e, int n_f, uint64_t v0, uint64_t v1, uint64_t e0, uint64_t e1, uint64_t e2) {
     const int l = __lane_id();
-    for (int base = 0; base < cap; base += 64) {
-      const int s = base + l;
-      const unsigned long long m = __ballot(s < cap && arr[s].stamp < 0);
-      if (m) return static_cast<int16_t>(base + __ffsll(m) - 1);
+    if (n_v > nv || n_e > nv || n_f > nf) return false;
+    for (int s = l; s < nv; s += 64) {
+      V[s].stamp = s < n_v ? s : -1;
+      if (s >= n_e) E[s].stamp = -1;
     }
-    return kNil;
+    for (int s = l + n_f; s < nf; s += 64) F[s].stamp = -1;
+    auto nib = [](uint64_t t, int k) { return static_cast<int16_t>((t >> (4 * k)) & 15u); };
+    if (l < n_e) {
+      auto& e = E[l];
+      e.v0 = nib(v0, l);
+      e.v1 = nib(v1, l);
+      int16_t f0 = kNil, f1 = kNil;
+      for (int k = 0; k < n_f; ++k)
+        if (nib(e0, k) == l || nib(e1, k) == l || nib(e2, k) == l) {
+          if (f0 == kNil) f0 = static_cast<int16_t>(k);
+          else f1 = static_cast<int16_t>(k);
+        }
+      e.f0 = f0;
+      e.f1 = f1;
+      MinD m;
+      segDist(d3{0, 0, 0}, vloc(e.v0), vloc(e.v1), m);
+      e.in = m.in; e.d2 = m.d2; e.wx = m.w.x; e.wy = m.w.y; e.wz = m.w.z;
+      e.stamp = n_v + l;
+    }
+    M::sync();
+    if (l < n_f) {
+      auto& f = F[l];
+      f.e0 = nib(e0, l); f.e1 = nib(e1, l); f.e2 = nib(e2, l);
+      int16_t a, b, c;
+      faceVerts(l, a, b, c);
+      setFace(f, a, vloc(a), vloc(b), vloc(c));
+      f.stamp = n_v + n_e + l;
+    }
+    stamp = n_v + n_e + n_f;
+    M::sync();
+    return true;
   }
-  MFCL_D int16_t addVertex(d3 v, d3 d, int h0 = -1, int h1 = -1) {
-    const int16_t i = allocSlot(V, nv);
+  MFCL_D void faceVerts(int fi, int16_t& a, int16_t& b, int16_t& c) const {
+    const auto& f = F[fi];
+    a = E[f.e0].v0;
+    b = E[f.e0].v1;
+    const int16_t p = E[f.e1].v0, q = E[f.e1].v1;
+    c = (p != a && p != b) ? p : q;
+  }
+
+  // A new face's distance record and, where faces keep it, its normal
+  // (epa_polytope.hpp:347-405: outward when the origin is at least 1e-4 from
+  // the plane).  a, b, c in faceVerts' order.
+  template <class FR>
+  MFCL_D void setFace(FR& f, int ia, d3 a, d3 b, d3 c) const {
+    MinD m;
+    triDist0(a, b, c, m);
+    f.in = m.in; f.d2 = m.d2; f.wx = m.w.x; f.wy = m.w.y; f.wz = m.w.z;
+    f.a = static_cast<int16_t>(ia);
+    if constexpr (M::kWords > 0) {
+      const d3 n = cross(a - b, b - c);
+      const double nn = norm(n);
+      const d3 dir = n / nn;
+      const double od = dot(a, dir);
+      const bool close = !(fabs(od) >= 1e-4);
+      const d3 out = close || od > 0 ? dir : -dir;
+      f.cls = nn <= 0.0 ? kNormalNone : (close ? kNormalClose : kNormalOut);
+      f.nx = out.x; f.ny = out.y; f.nz = out.z;
+    }
+  }
+  // Whether a plane near the origin has its outward side against dir (the
+  // same in all lanes): away from the farther vertices.  max / min over the
+  // vertices: order-free, so a parallel pass.
+  MFCL_D bool closeFlips(d3 dir) const {
+    double maxp = 0.0, minn = 0.0;
+    for (int s = __lane_id(); s < nv; s += 64) {
+      if (V[s].stamp < 0) continue;
+      const double dv = dot(vloc(s), dir);
+      if (dv > maxp) maxp = dv;
+      if (dv < minn) minn = dv;
+    }
+#pragma nounroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double om = __shfl_xor(maxp, off), on = __shfl_xor(minn, off);
+      if (om > maxp) maxp = om;
+      if (on < minn) minn = on;
+    }
+    return ub(fabs(maxp) > fabs(minn));
+  }
+
+  // Better in the order (d2, kind, newest first) -- the first element of
+  // the reference's vertex, edge, face scans with strict '<'.  rank: kind
+  // and age, smaller first.
+  MFCL_D static bool better(double d2, uint32_t rank, double bd, uint32_t br) {
+    return d2 < bd || (d2 == bd && rank < br);
+  }
+  MFCL_D static uint32_t rankOf(int kind, int st) {
+    return (static_cast<uint32_t>(kind) << 28) | (0x0FFFFFFFu - static_cast<uint32_t>(st));
+  }
+  // epa_polytope.hpp:292-345; kind: 0 none, 1 vertex, 2 edge, 3 face
+  MFCL_D void minToOrigin(bool excl_vertex, int& kind, int& idx) const {
+    const int l = __lane_id();
+    double bd = INFINITY;
+    uint32_t br = 0xFFFFFFFFu;
+    int bi = kNil;
+#pragma nounroll
+    for (int s = l; s < nv; s += 64) {
+      const auto& e = E[s];
+      const int st = e.stamp, sv = V[s].stamp;
+      const double ed = e.d2;
+      const bool ein = e.in;
+      const d3 v = vloc(s);
+      if (!excl_vertex && sv >= 0) {
+        const double d2 = sqnorm(v);
+        const uint32_t r = rankOf(1, sv);
+        if (better(d2, r, bd, br)) { bd = d2; br = r; bi = s; }
+      }
+      if (st >= 0 && (excl_vertex || ein)) {
+        const uint32_t r = rankOf(2, st);
+        if (better(ed, r, bd, br)) { bd = ed; br = r; bi = s; }
+      }
+    }
+#pragma nounroll
+    for (int s = l; s < nf; s += 64) {
+      const auto& f = F[s];
+      const int st = f.stamp;
+      const double fd = f.d2;
+      if (st >= 0 && f.in) {
+        const uint32_t r = rankOf(3, st);
+        if (better(fd, r, bd, br)) { bd = fd; br = r; bi = s; }
+      }
+    }
+    // the smallest d2 over the wavefront, then the first rank among the
+    // lanes that hold it (usually one)
+    double m = -max8(-bd);
+    m = fmin(m, dppD<kDppMirror>(m));
+    m = fmin(fmin(readLaneF64(m, 0), readLaneF64(m, 16)), fmin(readLaneF64(m, 32), readLaneF64(m, 48)));
+    unsigned long long who = __ballot(bd == m && br != 0xFFFFFFFFu);
+    // only finite candidates beat the reference's initial INFINITY
+    if (who == 0ull || !ub(m < INFINITY)) {
+      kind = 0;
+      idx = kNil;
+      return;
+    }
+    int w = __builtin_ctzll(who);
+    uint32_t r = __builtin_amdgcn_readlane(br, w);
+    for (who &= who - 1; who; who &= who - 1) {
+      const int o = __builtin_ctzll(who);
+      const uint32_t ro = __builtin_amdgcn_readlane(br, o);
+      if (ro < r) {
+        r = ro;
+        w = o;
+      }
+    }
+    kind = static_cast<int>(r >> 28);
+    idx = __builtin_amdgcn_readlane(bi, w);
+  }
+
+  // epa_polytope.hpp:347-405: a face's outward normal; ok: the face is not
+  // degenerate (area > 0).
+  struct Normal {
+    d3 n;
+    bool ok;
+  };
+  MFCL_D Normal normalOut(int fi) const {
+    Normal r;
+    int cls;
+    if constexpr (M::kWords > 0) {
+      const auto& f = F[fi];
+      r.n = d3{f.nx, f.ny, f.nz};
+      cls = f.cls;
+    } else {
+      int16_t ia, ib, ic;
+      faceVerts(fi, ia, ib, ic);
+      const d3 a = vloc(ia), b = vloc(ib), c = vloc(ic);
+      const d3 n = cross(a - b, b - c);
+      const double nn = norm(n);
+      const d3 dir = n / nn;
+      const double od = dot(a, dir);
+      const bool close = !(fabs(od) >= 1e-4);
+      r.n = close || od > 0 ? dir : -dir;
+      cls = nn <= 0.0 ? kNormalNone : (close ? kNormalClose : kNormalOut);
+    }
+    cls = __builtin_amdgcn_readfirstlane(cls);
+    r.ok = cls != kNormalNone;
+    if (cls == kNormalClose && closeFlips(r.n)) r.n = -r.n;
+    return r;
+  }
+  MFCL_D d3 faceAnchor(int fi) const { return vloc(F[fi].a); }
+  MFCL_D bool anyLane(bool b) const { return __ballot(b) != 0ull; }
+
+  // Slot of the new vertex (the lowest free one), kNil when there is none.
+  MFCL_D int addVertex(d3 v, d3 d, int h0, int h1) {
+    const int l = __lane_id();
+    int i = kNil;
+    for (int base = 0; base < nv && i == kNil; base += 64) {
+      const int s = base + l;
+      const unsigned long long m = __ballot(s < nv && V[s].stamp < 0);
+      if (m) i = base + __builtin_ctzll(m);
+    }
     if (i == kNil) return kNil;
     auto& x = V[i];
     x.vx = v.x; x.vy = v.y; x.vz = v.z;
@@ -217,151 +460,35 @@ struct PolyT {
     M::sync();
     return i;
   }
-  MFCL_D int16_t addEdge(int16_t a, int16_t b) {
-    if (a == kNil || b == kNil) return kNil;
-    const int16_t i = allocSlot(E, nv);
-    if (i == kNil) return kNil;
-    auto& e = E[i];
-    e.v0 = a;
-    e.v1 = b;
-    e.f0 = e.f1 = kNil;
-    e.vis = kUnknown;
-    MinD m;
-    segDist(d3{0, 0, 0}, vloc(a), vloc(b), m);
-    e.in = m.in; e.d2 = m.d2; e.wx = m.w.x; e.wy = m.w.y; e.wz = m.w.z;
-    e.stamp = stamp++;
-    M::sync();
-    return i;
-  }
-  MFCL_D int16_t addFace(int16_t e1, int16_t e2, int16_t e3) {
-    if (e1 == kNil || e2 == kNil || e3 == kNil) return kNil;
-    const int16_t i = allocSlot(F, nf);
-    if (i == kNil) return kNil;
-    auto& f = F[i];
-    f.e0 = e1; f.e1 = e2; f.e2 = e3;
-    f.vis = kFUnknown;
-    const int16_t a = E[e1].v0, b = E[e1].v1;
-    const int16_t c = (E[e2].v0 != a && E[e2].v0 != b) ? E[e2].v0 : E[e2].v1;
-    MinD m;
-    triDist0(vloc(a), vloc(b), vloc(c), m);
-    f.in = m.in; f.d2 = m.d2; f.wx = m.w.x; f.wy = m.w.y; f.wz = m.w.z;
-    f.stamp = stamp++;
-    M::sync();
-    // the face stays in the polytope even when an edge already has two faces
-    const int16_t es[3] = {e1, e2, e3};
-    for (int k = 0; k < 3; ++k) {
-      auto& ek = E[es[k]];
-      if (ub(ek.f0 == kNil)) {
-        ek.f0 = i;
-      } else {
-        if (ub(ek.f1 != kNil)) return kNil;
-        ek.f1 = i;
-      }
-      M::sync();
-    }
-    return i;
-  }
-  MFCL_D void faceVerts(int16_t fi, int16_t& a, int16_t& b, int16_t& c) const {
-    const auto& f = F[fi];
-    a = E[f.e0].v0;
-    b = E[f.e0].v1;
-    c = (E[f.e1].v0 != a && E[f.e1].v0 != b) ? E[f.e1].v0 : E[f.e1].v1;
-  }
 
-  // Wavefront argmin of (d2, kind, newest first) -- the first element of
-  // the reference's vertex, edge, face scans with strict '<'.
-  MFCL_D static bool better(double d2, int kind, int st, double bd, int bk, int bs) {
-    if (d2 < bd) return true;
-    if (!(d2 == bd)) return false;
-    if (kind != bk) return kind < bk;
-    return st > bs;
-  }
-  // epa_polytope.hpp:292-345; kind: 0 none, 1 vertex, 2 edge, 3 face
-  MFCL_D void minToOrigin(bool excl_vertex, int& kind, int16_t& idx) const {
-    const int l = __lane_id();
-    double bd = INFINITY;
-    int bk = 4, bs = -1, bi = kNil;
-    if (!excl_vertex)
-      for (int s = l; s < nv; s += 64) {
-        const int st = V[s].stamp;
-        if (st < 0) continue;
-        const double d2 = sqnorm(vloc(static_cast<int16_t>(s)));
-        if (better(d2, 1, st, bd, bk, bs)) { bd = d2; bk = 1; bs = st; bi = s; }
-      }
-    for (int s = l; s < nv; s += 64) {
-      const auto& e = E[s];
-      const int st = e.stamp;
-      if (st < 0) continue;
-      if (!excl_vertex && !e.in) continue;
-      if (better(e.d2, 2, st, bd, bk, bs)) { bd = e.d2; bk = 2; bs = st; bi = s; }
-    }
-    for (int s = l; s < nf; s += 64) {
-      const auto& f = F[s];
-      const int st = f.stamp;
-      if (st < 0 || !f.in) continue;
-      if (better(f.d2, 3, st, bd, bk, bs)) { bd = f.d2; bk = 3; bs = st; bi = s; }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const double od = __shfl_xor(bd, off);
-      const int ok = __shfl_xor(bk, off), os = __shfl_xor(bs, off), oi = __shfl_xor(bi, off);
-      if (better(od, ok, os, bd, bk, bs)) { bd = od; bk = ok; bs = os; bi = oi; }
-    }
-    // identical in every lane after the butterfly: taken as scalars, so
-    // the callers branch on them with scalar branches
-    const int ubk = __builtin_amdgcn_readfirstlane(bk);
-    const int ubi = __builtin_amdgcn_readfirstlane(bi);
-    const int fin = __builtin_amdgcn_readfirstlane(bd < INFINITY ? 1 : 0);
-    // only finite candidates beat the reference's initial INFINITY
-    if (ubk == 4 || !fin) {
-      kind = 0;
-      idx = kNil;
-    } else {
-      kind = ubk;
-      idx = static_cast<int16_t>(ubi);
-    }
-  }
-  // epa_polytope.hpp:347-405
-  MFCL_D bool faceNormalOut(int16_t fi, d3& normal, double* area) const {
+  // Whether face fi sees p (epa_polytope_expand.hpp:12-30), evaluated by
+  // one lane for its own face; the vertex fallback of the normal is scanned
+  // by that lane alone.
+  MFCL_D bool outsideLane(int fi, d3 p) const {
     int16_t ia, ib, ic;
     faceVerts(fi, ia, ib, ic);
     const d3 a = vloc(ia), b = vloc(ib), c = vloc(ic);
     const d3 n = cross(a - b, b - c);
     const double nn = norm(n);
-    if (area) *area = 0.5 * nn;
-    if (ub(nn <= 0.0)) return false;
+    if (nn <= 0.0) return true;
     const d3 dir = n / nn;
     const double od = dot(a, dir);
-    if (ub(fabs(od) >= 1e-4)) {
+    d3 normal;
+    if (fabs(od) >= 1e-4) {
       normal = od > 0 ? dir : -dir;
-      return true;
+    } else {
+      double maxp = 0.0, minn = 0.0;
+#pragma nounroll
+      for (int s = 0; s < nv; ++s) {
+        if (V[s].stamp < 0) continue;
+        const double dv = dot(vloc(s), dir);
+        if (dv > maxp) maxp = dv;
+        if (dv < minn) minn = dv;
+      }
+      normal = fabs(maxp) > fabs(minn) ? -dir : dir;
     }
-    // max / min over the vertices: order-free, so a parallel pass
-    double maxp = 0.0, minn = 0.0;
-    for (int s = __lane_id(); s < nv; s += 64) {
-      if (V[s].stamp < 0) continue;
-      const double dv = dot(vloc(static_cast<int16_t>(s)), dir);
-      if (dv > maxp) maxp = dv;
-      if (dv < minn) minn = dv;
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const double om = __shfl_xor(maxp, off), on = __shfl_xor(minn, off);
-      if (om > maxp) maxp = om;
-      if (on < minn) minn = on;
-    }
-    normal = fabs(maxp) > fabs(minn) ? -dir : dir;
-    return true;
+    return dot(normal, p - a) >= 0.0;
   }
-  MFCL_D d3 faceAnchor(int16_t fi) const { return vloc(E[F[fi].e0].v0); }
-  // epa_polytope_expand.hpp:12-30
-  MFCL_D bool outside(int16_t fi, d3 p) const {
-    d3 n;
-    double area = 0;
-    if (!faceNormalOut(fi, n, &area)) return ub(area <= 0.0);
-    return ub(dot(n, p - faceAnchor(fi)) >= 0.0);
-  }
-  MFCL_D bool anyLane(bool b) const { return __ballot(b) != 0ull; }
 
   // epa_polytope_expand.hpp:32-281. 0 ok, 1 failed, 2 malloc failed,
   // 3 (only when may_spill) this polytope's capacity might not hold the
@@ -369,16 +496,246 @@ struct PolyT {
   // in a polytope of the full capacity.
   // The reference's depth-first flood fill marks the faces reachable from
   // `start` through faces that see nv; that set, and the border / internal
-  // edge marks, do not depend on the visiting order, so it runs here as
-  // rounds of a parallel breadth-first fill.
-  MFCL_D int expand(d3 nv_, d3 nd, int nh0, int nh1, int16_t start, bool may_spill) {
+  // edge marks, do not depend on the visiting order.  kWords faces per lane,
+  // the visible set as bit masks: every face's test of nv runs first, all at
+  // once (with the normals that the faces keep, a dot product); the fill's
+  // rounds are then a few scalar instructions each.
+  struct Mask {
+    unsigned long long w[M::kWords > 0 ? M::kWords : 1];
+    MFCL_D bool has(int k) const {
+      if (k == kNil) return false;
+      unsigned long long m = w[0];
+#pragma unroll
+      for (int i = 1; i < M::kWords; ++i) m = (k >> 6) == i ? w[i] : m;
+      return ((m >> (k & 63)) & 1ull) != 0;
+    }
+  };
+  MFCL_D int expandMask(d3 nv_, d3 nd, int nh0, int nh1, int start, bool may_spill) {
+    constexpr int W = M::kWords;
+    const int l = __lane_id();
+    const unsigned long long below = (1ull << l) - 1;
+    bool live[W], out[W], open[W];
+    int g[W][3];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int s = 64 * i + l;
+      live[i] = s < nf && F[s < nf ? s : 0].stamp >= 0;
+      out[i] = open[i] = false;
+      g[i][0] = g[i][1] = g[i][2] = kNil;
+      int cls = kNormalOut;
+      d3 n = {0, 0, 0}, a = {0, 0, 0};
+      if (live[i]) {
+        const auto& f = F[s];
+        const int es[3] = {f.e0, f.e1, f.e2};
+        n = d3{f.nx, f.ny, f.nz};
+        cls = f.cls;
+        a = vloc(f.a);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int x = E[es[k]].f0, y = E[es[k]].f1;
+          g[i][k] = x == s ? y : x;
+          open[i] = open[i] || g[i][k] == kNil;
+        }
+      }
+      for (unsigned long long m = __ballot(live[i] && cls == kNormalClose); m; m &= m - 1) {
+        const int w = __builtin_ctzll(m);
+        const bool flip = closeFlips(d3{readLaneF64(n.x, w), readLaneF64(n.y, w), readLaneF64(n.z, w)});
+        if (l == w && flip) n = -n;
+      }
+      // epa_polytope_expand.hpp:12-30
+      out[i] = live[i] && (cls == kNormalNone || dot(n, nv_ - a) >= 0.0);
+    }
+    Mask vis;
+#pragma unroll
+    for (int i = 0; i < W; ++i) vis.w[i] = (start >> 6) == i ? 1ull << (start & 63) : 0ull;
+    while (true) {
+      unsigned long long any = 0;
+      Mask more;
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        more.w[i] = __ballot(out[i] && (vis.has(g[i][0]) || vis.has(g[i][1]) || vis.has(g[i][2]))) & ~vis.w[i];
+        any |= more.w[i];
+      }
+      if (!any) break;
+#pragma unroll
+      for (int i = 0; i < W; ++i) vis.w[i] |= more.w[i];
+    }
+    bool bad = false;
+    int free_f = 0;
+    bool mine[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      mine[i] = live[i] && ((vis.w[i] >> l) & 1ull) != 0;
+      bad = bad || (mine[i] && open[i]);
+      free_f += __popcll(__ballot(64 * i + l < nf && (!live[i] || mine[i])));
+    }
+    // an open edge on a visible face is a malformed polytope
+    if (anyLane(bad)) return 1;
+    // edge marks from the face classes; border edges compacted into BL
+    int nb = 0, free_e = 0, free_v = 0;
+    for (int base = 0; base < nv; base += 64) {
+      const int s = base + l;
+      bool border = false, fr = false, fv = false;
+      if (s < nv) {
+        auto& e = E[s];
+        const bool alive = e.stamp >= 0;
+        const bool a = vis.has(e.f0), b = vis.has(e.f1);
+        border = alive && a != b;
+        fr = !alive || (a && b);
+        fv = V[s].stamp < 0;
+        e.vis = border ? kBorder : (alive && a ? kInternal : kUnknown);
+        V[s].remove = 1;
+        V[s].new_edge = kNil;
+      }
+      const unsigned long long m = __ballot(border);
+      if (border) BL[nb + __popcll(m & below)].e = static_cast<int16_t>(s);
+      nb += __popcll(m);
+      free_e += __popcll(__ballot(fr));
+      free_v += __popcll(__ballot(fv));
+    }
+    // Whether the expansion certainly fits: one vertex, at most two new
+    // edges per border edge and one face per border edge must find slots.
+    // Vertices that the expansion removes are not counted as free.
+    if (may_spill && !(free_v >= 1 && free_e >= 2 * nb && free_f >= nb)) return 3;
+    M::sync();
+    // drop the visible faces (detaching them from their border edges), the
+    // internal edges and the vertices left without a non-internal edge
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+      if (mine[i]) F[64 * i + l].stamp = -1;
+    for (int s = l; s < nv; s += 64) {
+      auto& e = E[s];
+      if (e.stamp < 0) continue;
+      if (e.vis == kInternal) {
+        e.stamp = -1;
+        continue;
+      }
+      V[e.v0].remove = 0;
+      V[e.v1].remove = 0;
+      if (e.vis == kBorder) {
+        if (vis.has(e.f0)) e.f0 = e.f1;
+        e.f1 = kNil;
+      }
+    }
+    M::sync();
+    for (int s = l; s < nv; s += 64)
+      if (V[s].stamp >= 0 && V[s].remove) V[s].stamp = -1;
+    M::sync();
+    const int nvi = addVertex(nv_, nd, nh0, nh1);
+    if (nvi == kNil) return 2;
+    if (W > 1 && nb > 64) return coverBorder(static_cast<int16_t>(nvi));
+    // New faces over the border edges, one border edge per lane (with at
+    // most 64 faces there are at most 49: k connected visible faces have at
+    // most k + 2 border edges, the others at most 3 (64 - k)); see
+    // coverBorder for the order.
+    int be = 0, bst = -1, ba = 0, bb = 0;
+    if (l < nb) {
+      be = BL[l].e;
+      const auto& e = E[be];
+      bst = e.stamp;
+      ba = e.v0;
+      bb = e.v1;
+    }
+    int rank = 0, t0 = 0, t1 = 0;
+    for (int k = 0; k < nb; ++k) {
+      const int sk = __builtin_amdgcn_readlane(bst, k);
+      const int ak = __builtin_amdgcn_readlane(ba, k), bk = __builtin_amdgcn_readlane(bb, k);
+      if (sk > bst) {
+        ++rank;
+        t0 += ak == ba || bk == ba;
+        t1 += ak == bb || bk == bb;
+      }
+    }
+    if (anyLane(l < nb && (t0 > 1 || t1 > 1))) return 2;  // a third face on a new edge
+    const int made = 1 + (t0 == 0) + (t1 == 0);
+    int pre = 0, total = 0;
+    for (int k = 0; k < nb; ++k) {
+      const int sk = __builtin_amdgcn_readlane(bst, k), mk = __builtin_amdgcn_readlane(made, k);
+      total += mk;
+      if (sk > bst) pre += mk;
+    }
+    const int new_edges = total - nb;
+    if (new_edges > free_e || nb > free_f) return 2;
+    // the free slot lists (before any slot is taken)
+    for (int base = 0, c = 0; base < nv && c < new_edges; base += 64) {
+      const int s = base + l;
+      const bool fr = s < nv && E[s].stamp < 0;
+      const unsigned long long m = __ballot(fr);
+      const int pos = c + __popcll(m & below);
+      if (fr && pos < new_edges) BL[pos].fe = static_cast<int16_t>(s);
+      c += __popcll(m);
+    }
+    {
+      int c = 0;
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const bool fr = 64 * i + l < nf && (!live[i] || mine[i]);
+        const unsigned long long m = __ballot(fr);
+        const int pos = c + __popcll(m & below);
+        if (fr && pos < nb) BL[pos].ff = static_cast<int16_t>(64 * i + l);
+        c += __popcll(m);
+      }
+    }
+    M::sync();
+    // new edges: the k-th created edge takes the k-th free edge slot
+    const d3 va = vloc(ba), vb = vloc(bb);
+    if (l < nb) {
+      int q = 0;
+#pragma nounroll
+      for (int side = 0; side < 2; ++side) {
+        if ((side ? t1 : t0) != 0) continue;
+        const int vq = side ? bb : ba;
+        const int16_t slot = BL[pre - rank + q].fe;
+        auto& x = E[slot];
+        x.v0 = static_cast<int16_t>(nvi);
+        x.v1 = static_cast<int16_t>(vq);
+        x.f0 = x.f1 = kNil;
+        MinD m;
+        segDist(d3{0, 0, 0}, nv_, d3{side ? vb.x : va.x, side ? vb.y : va.y, side ? vb.z : va.z}, m);
+        x.in = m.in; x.d2 = m.d2; x.wx = m.w.x; x.wy = m.w.y; x.wz = m.w.z;
+        x.stamp = stamp + pre + q;
+        V[vq].new_edge = slot;
+        ++q;
+      }
+    }
+    M::sync();
+    // faces: the face of rank r takes the r-th free face slot; the border
+    // edge keeps its hidden face as f0; each new edge gets its lower-ranked
+    // face as f0 and the other as f1
+    bool clash = false;
+    if (l < nb) {
+      const int16_t slot = BL[rank].ff;
+      const int ne0 = V[ba].new_edge, ne1 = V[bb].new_edge;
+      auto& f = F[slot];
+      f.e0 = static_cast<int16_t>(be);
+      f.e1 = static_cast<int16_t>(ne0);
+      f.e2 = static_cast<int16_t>(ne1);
+      setFace(f, ba, va, vb, nv_);
+      f.stamp = stamp + pre + (t0 == 0) + (t1 == 0);
+      auto& ej = E[be];
+      if (ej.f0 == kNil) ej.f0 = slot;
+      else if (ej.f1 != kNil) clash = true;
+      else ej.f1 = slot;
+      if (t0 == 0) E[ne0].f0 = slot; else E[ne0].f1 = slot;
+      if (t1 == 0) E[ne1].f0 = slot; else E[ne1].f1 = slot;
+    }
+    stamp += total;
+    M::sync();
+    return anyLane(clash) ? 2 : 0;
+  }
+
+  // The same for any capacity, the face classes marked in LDS and the
+  // border edges in BL (polytopes beyond kSmallFaces).
+  MFCL_D int expandLarge(d3 nv_, d3 nd, int nh0, int nh1, int start) {
     const int l = __lane_id();
     for (int s = l; s < nv; s += 64) {
       V[s].remove = 1;
       V[s].new_edge = kNil;
       E[s].vis = kUnknown;
     }
-    for (int s = l; s < nf; s += 64) F[s].vis = kFUnknown;
+    // a face that does not see the new vertex is never visible, unless the
+    // fill starts from it
+    for (int s = l; s < nf; s += 64) F[s].vis = F[s].stamp >= 0 && outsideLane(s, nv_) ? kFUnknown : kHidden;
     M::sync();
     F[start].vis = kVisible;
     M::sync();
@@ -390,14 +747,12 @@ struct PolyT {
         const int16_t es[3] = {f.e0, f.e1, f.e2};
         bool near_visible = false;
         for (int k = 0; k < 3; ++k) {
-          if (es[k] == kNil) continue;
           const auto& e = E[es[k]];
           const int16_t g = e.f0 == s ? e.f1 : e.f0;
           if (g != kNil && F[g].vis == kVisible) near_visible = true;
         }
         if (!near_visible) continue;
-        const bool out = outsideLane(static_cast<int16_t>(s), nv_);
-        F[s].vis = out ? kVisible : kHidden;
+        F[s].vis = kVisible;
         changed = true;
       }
       M::sync();
@@ -410,22 +765,25 @@ struct PolyT {
       if (f.stamp < 0 || f.vis != kVisible) continue;
       const int16_t es[3] = {f.e0, f.e1, f.e2};
       for (int k = 0; k < 3; ++k) {
-        if (es[k] == kNil) { bad = true; continue; }
         const auto& e = E[es[k]];
         const int16_t g = e.f0 == s ? e.f1 : e.f0;
         if (g == kNil) bad = true;
       }
     }
     if (anyLane(bad)) return 1;
-    if (may_spill && !fits()) return 3;
     // edge marks from the final face classes
     for (int s = l; s < nv; s += 64) {
       auto& e = E[s];
       if (e.stamp < 0) continue;
       const bool v0 = e.f0 != kNil && F[e.f0].vis == kVisible;
       const bool v1 = e.f1 != kNil && F[e.f1].vis == kVisible;
-      if (v0 && v1) e.vis = kInternal;
-      else if (v0 || v1) e.vis = kBorder;
+      if (v0 && v1) {
+        e.vis = kInternal;
+      } else if (v0 || v1) {
+        e.vis = kBorder;
+        if (v0) e.f0 = e.f1;
+        e.f1 = kNil;
+      }
     }
     M::sync();
     for (int s = l; s < nv; s += 64) {
@@ -435,33 +793,18 @@ struct PolyT {
       V[e.v1].remove = 0;
     }
     M::sync();
-    // drop the visible faces (detaching them from their border edges), the
-    // internal edges and the vertices left without a non-internal edge
-    for (int s = l; s < nf; s += 64) {
-      auto& f = F[s];
-      if (f.stamp < 0 || f.vis != kVisible) continue;
-      const int16_t es[3] = {f.e0, f.e1, f.e2};
-      for (int k = 0; k < 3; ++k) {
-        if (es[k] == kNil) continue;
-        auto& ek = E[es[k]];
-        if (ek.vis == kInternal) continue;  // removed below
-        if (ek.f0 == s) ek.f0 = ek.f1;
-        ek.f1 = kNil;
-      }
-      f.stamp = -1;
-    }
+    // drop the visible faces, the internal edges and the vertices left
+    // without a non-internal edge
+    for (int s = l; s < nf; s += 64)
+      if (F[s].stamp >= 0 && F[s].vis == kVisible) F[s].stamp = -1;
     for (int s = l; s < nv; s += 64) {
-      auto& e = E[s];
-      if (e.stamp >= 0 && e.vis == kInternal) e.stamp = -1;
-    }
-    for (int s = l; s < nv; s += 64) {
-      auto& v = V[s];
-      if (v.stamp >= 0 && v.remove) v.stamp = -1;
+      if (E[s].stamp >= 0 && E[s].vis == kInternal) E[s].stamp = -1;
+      if (V[s].stamp >= 0 && V[s].remove) V[s].stamp = -1;
     }
     M::sync();
-    const int16_t nvi = addVertex(nv_, nd, nh0, nh1);
+    const int nvi = addVertex(nv_, nd, nh0, nh1);
     if (nvi == kNil) return 2;
-    return coverBorder(nvi);
+    return coverBorder(static_cast<int16_t>(nvi));
   }
 
   // New faces over the border edges (epa_polytope_expand.hpp:233-281).  The
@@ -517,7 +860,7 @@ struct PolyT {
       int pre = 0;
       for (int k = 0; k < nb; ++k)
         if (BL[k].rank < r) pre += 1 + (BL[k].t0 == 0) + (BL[k].t1 == 0);
-      BL[j].pre = pre;
+      BL[j].pre = static_cast<int16_t>(pre);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) new_edges += __shfl_xor(new_edges, off);
@@ -583,9 +926,7 @@ struct PolyT {
       auto& f = F[slot];
       f.e0 = ei; f.e1 = ne0; f.e2 = ne1;
       f.vis = kFUnknown;
-      MinD m;
-      triDist0(vloc(a), vloc(b), vloc(nvi), m);
-      f.in = m.in; f.d2 = m.d2; f.wx = m.w.x; f.wy = m.w.y; f.wz = m.w.z;
+      setFace(f, a, vloc(a), vloc(b), vloc(nvi));
       f.stamp = stamp + bj.pre + (bj.t0 == 0) + (bj.t1 == 0);
     }
     M::sync();
@@ -609,560 +950,509 @@ struct PolyT {
     return anyLane(clash) ? 2 : 0;
   }
 
-  // Whether the expansion whose visible faces are marked certainly fits:
-  // after the visible faces, the internal edges and the vertices left
-  // without a non-internal edge are freed, one vertex, at most two new
-  // edges per border edge and one face per border edge must find slots.
-  // Marks only; nothing is changed.
-  MFCL_D bool fits() const {
-    const int l = __lane_id();
-    int free_v = 0, free_e = 0, free_f = 0, nb = 0;
-    for (int base = 0; base < nf; base += 64) {
-      const int s = base + l;
-      bool fr = false;
-      if (s < nf) fr = F[s].stamp < 0 || F[s].vis == kVisible;
-      free_f += __popcll(__ballot(fr));
-    }
-    for (int base = 0; base < nv; base += 64) {
-      const int s = base + l;
-      bool fe = false, bd = false, fv = false;
-      if (s < nv) {
-        const auto& e = E[s];
-        if (e.stamp < 0) {
-          fe = true;
-        } else {
-          const bool v0 = e.f0 != kNil && F[e.f0].vis == kVisible;
-          const bool v1 = e.f1 != kNil && F[e.f1].vis == kVisible;
-          fe = v0 && v1;
-          bd = v0 != v1;
-        }
-        // a vertex stays when some edge of the polytope that is not internal
-        // touches it; counted below as free only when it has no such edge
-        fv = V[s].stamp < 0;
-      }
-      free_e += __popcll(__ballot(fe));
-      nb += __popcll(__ballot(bd));
-      free_v += __popcll(__ballot(fv));
-    }
-    // the vertices removed by the expansion are not counted as free: the
-    // test only needs one vertex slot, so a free one must exist already
-    return free_v >= 1 && free_e >= 2 * nb && free_f >= nb;
-  }
-
- private:
-  // outside() evaluated by one lane for its own face (no cross-lane work:
-  // the vertex fallback of faceNormalOut is scanned by that lane alone)
-  MFCL_D bool outsideLane(int16_t fi, d3 p) const {
-    int16_t ia, ib, ic;
-    faceVerts(fi, ia, ib, ic);
-    const d3 a = vloc(ia), b = vloc(ib), c = vloc(ic);
-    const d3 n = cross(a - b, b - c);
-    const double nn = norm(n);
-    if (nn <= 0.0) return 0.5 * nn <= 0.0;
-    const d3 dir = n / nn;
-    const double od = dot(a, dir);
-    d3 normal;
-    if (fabs(od) >= 1e-4) {
-      normal = od > 0 ? dir : -dir;
-    } else {
-      double maxp = 0.0, minn = 0.0;
-      for (int s = 0; s < nv; ++s) {
-        if (V[s].stamp < 0) continue;
-        const double dv = dot(vloc(static_cast<int16_t>(s)), dir);
-        if (dv > maxp) maxp = dv;
-        if (dv < minn) minn = dv;
-      }
-      normal = fabs(maxp) > fabs(minn) ? -dir : dir;
-    }
-    return dot(normal, p - faceAnchor(fi)) >= 0.0;
-  }
 };
 
-using Poly = PolyT<LdsMem>;
-using PolyG = PolyT<GlbMem>;
-
-// Result of the EPA stage in shape-0 frame.
+// The closest feature of one iteration: what the witness points are formed
+// from.
+struct RawF {
+  double m[4];     // d2, then the witness
+  double v[3][6];  // vertex and direction of a, b, c
+  int h[3][2];     // support vertices of a, b, c (-1: primitive or unknown)
+  int kind, pad;
+};
+// Where a pair that outgrows its polytope continues: the expansion it is at.
+struct EpaResume {
+  d3 nv, nd;
+  int it, stamp, nh0, nh1, start, item;
+};
+// The result in shape-0 frame (status: EpaStatus, or kEpaSpill).
 struct EpaOut {
-  int status;
   double depth;
   d3 p0, p1;
-  int iters;
-  int scanned_extra;  // hull vertices scanned by the out-of-line helpers
-  int spilled;        // 1: continued in the device-memory polytope
+  int iters, scanned;
 };
-
-// The out-of-line helpers take the Minkowski difference by value (a
-// reference would keep the caller's copy in private memory for the whole
-// EPA loop); this adds the vertices they scan to the pair's tally on exit.
-template <class MK>
-struct ScanTally {
-  MK& md;
-  EpaOut& o;
-  int start;
-  MFCL_D ScanTally(MK& m, EpaOut& out) : md(m), o(out), start(m.scanned) {}
-  MFCL_D ~ScanTally() { o.scanned_extra += md.scanned - start; }
+// A wavefront's LDS slice: the pair's configuration and simplex, the records
+// above, then the polytope arena at kEpaHeadBytes.
+struct EpaLds {
+  WaveCfg cfg;
+  SmpD s;
+  RawF raw;
+  EpaResume res;
+  EpaOut out;
 };
+constexpr int kEpaSpill = 5;
+constexpr size_t kEpaHeadBytes = (sizeof(EpaLds) + 15) & ~static_cast<size_t>(15);
+template <class M>
+__host__ __device__ inline size_t epaSliceBytes(int cap_faces) {
+  return kEpaHeadBytes + arenaBytes<M>(cap_faces);
+}
+// A spilled pair in device memory: RawF, EpaResume and the slot arrays.
+constexpr size_t kEpaDumpHead = sizeof(RawF) + sizeof(EpaResume);
+__host__ __device__ inline size_t epaDumpBytes(int cap_faces) {
+  return (kEpaDumpHead + polyBytes<SmallMem>(cap_faces) + 255) & ~static_cast<size_t>(255);
+}
+static_assert(sizeof(RawF) % 8 == 0 && sizeof(EpaResume) % 8 == 0, "dumped as 8-byte words");
 
-template <class MK>
-MFCL_D void touchingPoint(MK& md, d3 d, EpaOut& o) {
-  const d3 mid = (md.support0(d) + md.support1(-d)) / 2;
-  o.p0 = mid;
-  o.p1 = mid;
+MFCL_D d3 ldsGet(const MFCL_LDS d3& o) { return d3{o.x, o.y, o.z}; }
+MFCL_D d3 ldsGet(const MFCL_LDS double* o) { return d3{o[0], o[1], o[2]}; }
+MFCL_D void ldsSet(MFCL_LDS d3& o, d3 v) { o.x = v.x; o.y = v.y; o.z = v.z; }
+MFCL_D const MFCL_LDS MVD& smpVert(const MFCL_LDS SmpD& s, int k) {
+  return k == 0 ? s.a : (k == 1 ? s.b : (k == 2 ? s.c : s.e));
+}
+MFCL_D void ldsSync() { __builtin_amdgcn_wave_barrier(); }
+MFCL_D MFCL_LDS char* ldsArena(MFCL_LDS EpaLds* L) { return (MFCL_LDS char*)(L) + kEpaHeadBytes; }
+
+// Vertex i of an initial polytope (every lane writes the same).
+template <class M>
+MFCL_D void putVertex(PolyT<M>& P, int i, d3 v, d3 d) {
+  auto& x = P.V[i];
+  x.vx = v.x; x.vy = v.y; x.vz = v.z;
+  x.dx = d.x; x.dy = d.y; x.dz = d.z;
+  x.h0 = x.h1 = -1;
+}
+template <class M>
+MFCL_D void putVertex(PolyT<M>& P, int i, const MFCL_LDS MVD& m) { putVertex(P, i, ldsGet(m.v), ldsGet(m.d)); }
+// epa_simplex2polytope.hpp:184-217 (a capacity of 4 faces, the least there
+// is, holds it)
+template <class M>
+MFCL_D bool buildTetra(PolyT<M>& P) {
+  M::sync();
+  return P.build(4, 6, 4, 0x333210ull, 0x210021ull, 0x5430ull, 0x3541ull, 0x2102ull);
 }
 
-// epa_simplex2polytope.hpp:184-217; returns 0 ok, 2 failed
-__device__ __attribute__((noinline)) int tetra(Poly& P, const MVD& a, const MVD& b, const MVD& c, const MVD& d) {
-  P.reset();
-  int16_t v[4], e[6], f[4];
-  v[0] = P.addVertex(a.v, a.d);
-  v[1] = P.addVertex(b.v, b.d);
-  v[2] = P.addVertex(c.v, c.d);
-  v[3] = P.addVertex(d.v, d.d);
-  e[0] = P.addEdge(v[0], v[1]);
-  e[1] = P.addEdge(v[1], v[2]);
-  e[2] = P.addEdge(v[2], v[0]);
-  e[3] = P.addEdge(v[3], v[0]);
-  e[4] = P.addEdge(v[3], v[1]);
-  e[5] = P.addEdge(v[3], v[2]);
-  f[0] = P.addFace(e[0], e[1], e[2]);
-  f[1] = P.addFace(e[3], e[4], e[0]);
-  f[2] = P.addFace(e[4], e[5], e[1]);
-  f[3] = P.addFace(e[5], e[3], e[2]);
-  for (int i = 0; i < 4; ++i)
-    if (f[i] == kNil) return 2;
-  return 0;
+// simplexToPolytope's status: a negative value is a failure, kS2pTouching
+// leaves the points in out, any other is the polytope's creation counter.
+constexpr int kS2pFailed = -1, kS2pTouching = 0;
+
+MFCL_D int touchingPoint(MinkW& md, d3 d, MFCL_LDS EpaLds* L) {
+  const WaveSup a = md.sup(d);
+  const d3 mid = (a.p0 + a.p1) / 2;
+  ldsSet(L->out.p0, mid);
+  ldsSet(L->out.p1, mid);
+  return kS2pTouching;
 }
 
-// s2p status: 0 OK, 1 touching, 2 failed
-template <class MK>
-__device__ __attribute__((noinline)) int s2p3(Poly& P, MK md, const MVD& a, const MVD& b, const MVD& c, double thr, EpaOut& o) {
-  ScanTally tally(md, o);
-  d3 n = cross(b.v - a.v, c.v - a.v);
-  if (sqnorm(n) <= 0.0) return 2;
-  n = normalized(n);
-  const d3 d0 = md.support(n);
-  const double t0 = planeDist(d0, a.v, b.v, c.v);
-  const d3 dir1 = -n;
-  const d3 d1 = md.support(dir1);
-  const double t1 = planeDist(d1, a.v, b.v, c.v);
-  if (t0 <= thr) { touchingPoint(md, n, o); return 1; }
-  if (t1 <= thr) { touchingPoint(md, dir1, o); return 1; }
-  if (t0 > t1) return tetra(P, a, b, c, MVD{d0, n});
-  return tetra(P, a, b, c, MVD{d1, dir1});
+// Out of line: few pairs start from a triangle or a segment.  tri: the
+// simplex vertices that form the triangle, (a, b, c), (a, c, e), (a, b, e)
+// or (b, c, e).
+template <class M>
+__device__ __attribute__((noinline)) int s2p3(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int cap_faces,
+                                              int tri, double thr) {
+  PolyT<M> P(arena, cap_faces);
+  MinkW md{&L->cfg, 0};
+  const MFCL_LDS MVD& va = smpVert(L->s, tri == 3 ? 1 : 0);
+  const MFCL_LDS MVD& vb = smpVert(L->s, tri == 1 || tri == 3 ? 2 : 1);
+  const MFCL_LDS MVD& vc = smpVert(L->s, tri == 0 ? 2 : 3);
+  const d3 a = ldsGet(va.v), b = ldsGet(vb.v), c = ldsGet(vc.v);
+  int r = kS2pFailed;
+  d3 n = cross(b - a, c - a);
+  if (!ub(sqnorm(n) <= 0.0)) {
+    n = normalized(n);
+    const d3 d0 = md.support(n);
+    const double t0 = planeDist(d0, a, b, c);
+    const d3 dir1 = -n;
+    const d3 d1 = md.support(dir1);
+    const double t1 = planeDist(d1, a, b, c);
+    if (ub(t0 <= thr)) {
+      r = touchingPoint(md, n, L);
+    } else if (ub(t1 <= thr)) {
+      r = touchingPoint(md, dir1, L);
+    } else {
+      const bool up = ub(t0 > t1);
+      putVertex(P, 0, va);
+      putVertex(P, 1, vb);
+      putVertex(P, 2, vc);
+      putVertex(P, 3, up ? d0 : d1, up ? n : dir1);
+      if (buildTetra(P)) r = P.stamp;
+    }
+  }
+  L->out.scanned += md.scanned;
+  return r;
 }
 
-template <class MK>
-__device__ __attribute__((noinline)) int s2p2(Poly& P, MK md, const MVD& a, const MVD& b, double thr, EpaOut& o) {
-  ScanTally tally(md, o);
+template <class M>
+MFCL_D int s2p2Run(PolyT<M>& P, MinkW& md, MFCL_LDS EpaLds* L, double thr) {
   const double thr2 = thr * thr;
-  const d3 ab = b.v - a.v;
-  if (sqnorm(ab) < thr2) return 2;
+  const d3 a = ldsGet(L->s.a.v), b = ldsGet(L->s.b.v);
+  const d3 ab = b - a;
+  if (ub(sqnorm(ab) < thr2)) return kS2pFailed;
   const d3 abu = normalized(ab);
   d3 dinit = {abu.y, -abu.x, 0};
   bool valid = sqnorm(dinit) > thr2;
   if (!valid) { dinit = d3{abu.z, 0, -abu.x}; valid = sqnorm(dinit) > thr2; }
   if (!valid) { dinit = d3{0, abu.z, -abu.y}; valid = sqnorm(dinit) > thr2; }
-  if (!valid) return 2;
+  if (ub(!valid)) return kS2pFailed;
   dinit = normalized(dinit);
-  d3 dcur = dinit, dfound = {0, 0, 0}, vfound = {0, 0, 0};
+  d3 d = dinit, v = {0, 0, 0};
   bool found = false;
+#pragma nounroll
   for (int i = 0; i < 72; ++i) {
-    const d3 vcur = md.support(dcur);
-    if (lineDist(vcur, a.v, b.v) > thr) {
-      vfound = vcur;
-      dfound = dcur;
+    v = md.support(d);
+    if (ub(lineDist(v, a, b) > thr)) {
       found = true;
       break;
     }
     const double step = 2.0 * 3.145926 / 72;  // the reference's pi constant (sic)
-    dcur = normalized(dcur + step * cross(abu, vcur));
+    d = normalized(d + step * cross(abu, v));
   }
-  if (!found) { touchingPoint(md, dinit, o); return 1; }
-  const MVD v0 = {vfound, dfound};
-  MVD v1;
-  v1.d = -v0.d;
-  v1.v = md.support(v1.d);
-  if (lineDist(v1.v, a.v, b.v) < thr) { touchingPoint(md, v1.d, o); return 1; }
-  const d3 n = cross(v0.v - a.v, v1.v - a.v);
-  if (sqnorm(n) < thr2) return 2;
-  MVD v2;
-  v2.d = normalized(n);
-  v2.v = md.support(v2.d);
-  if (lineDist(v2.v, a.v, b.v) < thr) { touchingPoint(md, v2.d, o); return 1; }
-  MVD v3;
-  v3.d = -v2.d;
-  v3.v = md.support(v3.d);
-  if (lineDist(v3.v, a.v, b.v) < thr) { touchingPoint(md, v3.d, o); return 1; }
-  P.reset();
-  int16_t v[6], e[12], f[8];
-  v[0] = P.addVertex(a.v, a.d);
-  v[1] = P.addVertex(v0.v, v0.d);
-  v[2] = P.addVertex(b.v, b.d);
-  v[3] = P.addVertex(v1.v, v1.d);
-  v[4] = P.addVertex(v2.v, v2.d);
-  v[5] = P.addVertex(v3.v, v3.d);
-  e[0] = P.addEdge(v[0], v[1]);
-  e[1] = P.addEdge(v[1], v[2]);
-  e[2] = P.addEdge(v[2], v[3]);
-  e[3] = P.addEdge(v[3], v[0]);
-  e[4] = P.addEdge(v[4], v[0]);
-  e[5] = P.addEdge(v[4], v[1]);
-  e[6] = P.addEdge(v[4], v[2]);
-  e[7] = P.addEdge(v[4], v[3]);
-  e[8] = P.addEdge(v[5], v[0]);
-  e[9] = P.addEdge(v[5], v[1]);
-  e[10] = P.addEdge(v[5], v[2]);
-  e[11] = P.addEdge(v[5], v[3]);
-  f[0] = P.addFace(e[4], e[5], e[0]);
-  f[1] = P.addFace(e[5], e[6], e[1]);
-  f[2] = P.addFace(e[6], e[7], e[2]);
-  f[3] = P.addFace(e[7], e[4], e[3]);
-  f[4] = P.addFace(e[8], e[9], e[0]);
-  f[5] = P.addFace(e[9], e[10], e[1]);
-  f[6] = P.addFace(e[10], e[11], e[2]);
-  f[7] = P.addFace(e[11], e[8], e[3]);
-  for (int i = 0; i < 8; ++i)
-    if (f[i] == kNil) return 2;
-  return 0;
+  if (!found) return touchingPoint(md, dinit, L);
+  // the octahedron a, v0, b, v1, v2, v3: v1 opposite v0, v2 and v3 along
+  // the normal of (a, v0, v1).  Too small a capacity fails as the
+  // reference's allocation does, after the searches.
+  const bool room = P.nv >= 12 && P.nf >= 8;
+  if (room) {
+    putVertex(P, 0, L->s.a);
+    putVertex(P, 2, L->s.b);
+  }
+  d3 v0 = v;
+#pragma nounroll
+  for (int k = 0; k < 4; ++k) {
+    if (k == 2) {
+      const d3 n = cross(v0 - a, v - a);
+      if (ub(sqnorm(n) < thr2)) return kS2pFailed;
+      d = normalized(n);
+    } else if (k > 0) {
+      d = -d;
+    }
+    if (k > 0) {
+      v = md.support(d);
+      if (ub(lineDist(v, a, b) < thr)) return touchingPoint(md, d, L);
+    }
+    if (room) putVertex(P, k == 0 ? 1 : k + 2, v, d);
+  }
+  if (!room) return kS2pFailed;
+  M::sync();
+  P.build(6, 12, 8, 0x555544443210ull, 0x321032100321ull, 0xBA987654ull, 0x8BA94765ull, 0x32103210ull);
+  return P.stamp;
+}
+template <class M>
+__device__ __attribute__((noinline)) int s2p2(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int cap_faces,
+                                              double thr) {
+  PolyT<M> P(arena, cap_faces);
+  MinkW md{&L->cfg, 0};
+  const int r = s2p2Run(P, md, L, thr);
+  L->out.scanned += md.scanned;
+  return r;
 }
 
-// epa_simplex2polytope.hpp:46-110
-template <class MK>
-MFCL_D int simplexToPolytope(Poly& P, MK& md, const SmpD& s, double thr, EpaOut& o) {
+// epa_simplex2polytope.hpp:46-110 on the simplex in LDS.
+template <class M>
+MFCL_D int simplexToPolytope(PolyT<M>& P, MinkW& md, MFCL_LDS EpaLds* L, typename M::template P<char> arena,
+                             int cap_faces, double thr) {
+  const MFCL_LDS SmpD& s = L->s;
   const double thr2 = thr * thr;
-  if (s.rank > 0 && sqnorm(s.a.v) <= thr2) { touchingPoint(md, s.a.d, o); return 1; }
-  if (s.rank > 1 && sqnorm(s.b.v) <= thr2) { touchingPoint(md, s.b.d, o); return 1; }
-  if (s.rank > 2 && sqnorm(s.c.v) <= thr2) { touchingPoint(md, s.c.d, o); return 1; }
-  if (s.rank > 3 && sqnorm(s.e.v) <= thr2) { touchingPoint(md, s.e.d, o); return 1; }
-  if (s.rank == 4) {
-    const d3 z = {0, 0, 0};
-    if (planeDist(z, s.a.v, s.b.v, s.c.v) < thr) return s2p3(P, md, s.a, s.b, s.c, thr, o);
-    if (planeDist(z, s.a.v, s.c.v, s.e.v) < thr) return s2p3(P, md, s.a, s.c, s.e, thr, o);
-    if (planeDist(z, s.a.v, s.b.v, s.e.v) < thr) return s2p3(P, md, s.a, s.b, s.e, thr, o);
-    if (planeDist(z, s.b.v, s.c.v, s.e.v) < thr) return s2p3(P, md, s.b, s.c, s.e, thr, o);
-    return tetra(P, s.a, s.b, s.c, s.e);
+  const int rank = __builtin_amdgcn_readfirstlane(s.rank);
+  const int q = __lane_id() & 3;
+  // a simplex vertex at the origin, one vertex per lane
+  const unsigned long long at = __ballot(q < rank && sqnorm(ldsGet(smpVert(s, q).v)) <= thr2) & 15ull;
+  if (at) return touchingPoint(md, ldsGet(smpVert(s, __builtin_ctzll(at)).d), L);
+  if (rank <= 1) {
+    const WaveSup a = md.sup(ldsGet(s.a.d));
+    ldsSet(L->out.p0, a.p0);
+    ldsSet(L->out.p1, a.p1);
+    return kS2pTouching;
   }
-  if (s.rank == 3) return s2p3(P, md, s.a, s.b, s.c, thr, o);
-  if (s.rank == 2) return s2p2(P, md, s.a, s.b, thr, o);
-  o.p0 = md.support0(s.a.d);
-  o.p1 = md.support1(-s.a.d);
-  return 1;
+  if (rank == 2) return s2p2<M>(L, arena, cap_faces, thr);
+  if (rank == 3) return s2p3<M>(L, arena, cap_faces, 0, thr);
+  // the distances of the faces (a, b, c), (a, c, e), (a, b, e), (b, c, e)
+  // from the origin, one per lane
+  const d3 x = ldsGet(smpVert(s, q == 3 ? 1 : 0).v), y = ldsGet(smpVert(s, q & 1 ? 2 : 1).v),
+           w = ldsGet(smpVert(s, q == 0 ? 2 : 3).v);
+  const unsigned long long flat = __ballot(planeDist(d3{0, 0, 0}, x, y, w) < thr) & 15ull;
+  if (flat) return s2p3<M>(L, arena, cap_faces, __builtin_ctzll(flat), thr);
+  putVertex(P, 0, s.a);
+  putVertex(P, 1, s.b);
+  putVertex(P, 2, s.c);
+  putVertex(P, 3, s.e);
+  return buildTetra(P) ? P.stamp : kS2pFailed;
 }
 
-struct RawF {
-  int kind;
-  MinD m;
-  MVD a, b, c;
-  int h[3][2];  // support vertices of a, b, c (-1: primitive or unknown)
-};
-
-MFCL_D void ldsSet(MFCL_LDS d3& o, d3 v) {
-  o.x = v.x;
-  o.y = v.y;
-  o.z = v.z;
-}
-MFCL_D d3 ldsGet(const MFCL_LDS d3& o) { return d3{o.x, o.y, o.z}; }
-
-template <class PT>
-MFCL_D void toRaw(const PT& P, int kind, int16_t i, MFCL_LDS RawF& r) {
-  r.kind = kind;
-  auto rec = [&](int k, int16_t v) {
-    r.h[k][0] = P.V[v].h0;
-    r.h[k][1] = P.V[v].h1;
-  };
-  if (kind == 1) {
-    const d3 v = P.vloc(i);
-    r.m.in = true; r.m.d2 = sqnorm(v); ldsSet(r.m.w, v);
-    ldsSet(r.a.v, v); ldsSet(r.a.d, P.vdir(i));
-    rec(0, i);
-  } else if (kind == 2) {
-    const auto& e = P.E[i];
-    r.m.in = e.in; r.m.d2 = e.d2; ldsSet(r.m.w, d3{e.wx, e.wy, e.wz});
-    ldsSet(r.a.v, P.vloc(e.v0)); ldsSet(r.a.d, P.vdir(e.v0));
-    ldsSet(r.b.v, P.vloc(e.v1)); ldsSet(r.b.d, P.vdir(e.v1));
-    rec(0, e.v0);
-    rec(1, e.v1);
-  } else {
-    const auto& f = P.F[i];
-    r.m.in = f.in; r.m.d2 = f.d2; ldsSet(r.m.w, d3{f.wx, f.wy, f.wz});
-    int16_t ia, ib, ic;
-    P.faceVerts(i, ia, ib, ic);
-    ldsSet(r.a.v, P.vloc(ia)); ldsSet(r.a.d, P.vdir(ia));
-    ldsSet(r.b.v, P.vloc(ib)); ldsSet(r.b.d, P.vdir(ib));
-    ldsSet(r.c.v, P.vloc(ic)); ldsSet(r.c.d, P.vdir(ic));
-    rec(0, ia);
-    rec(1, ib);
-    rec(2, ic);
-  }
-}
-
-// epa.hpp:11-113; returns 0 ok, 1 failed, 2 converge
-// nh0 / nh1 receive the support vertices of the last support point.
-template <class PT, class MK>
-MFCL_D int nextDir(const PT& P, MK& md, int kind, int16_t fi, double tol, d3& nd, d3& nv, int16_t& start, int& nh0,
-                   int& nh1) {
-  constexpr double kOuter = 1e-3 * 1e-3;
-  auto face_cand = [&](int16_t f, bool try_w) -> int {
-    d3 fn;
-    if (!P.faceNormalOut(f, fn, nullptr)) return 1;
-    const d3 on = P.faceAnchor(f);
-    const auto& F = P.F[f];
-    if (try_w && ub(F.d2 > kOuter)) {
-      nd = normalized(d3{F.wx, F.wy, F.wz});
-      nv = md.supportFrom(nd, -1, -1, nh0, nh1);
-      if (ub(dot(fn, nv - on) >= 0.0)) { start = f; return 0; }
-    }
-    nd = fn;
-    nv = md.supportFrom(nd, -1, -1, nh0, nh1);
-    if (ub(dot(fn, nv - on) > tol)) { start = f; return 0; }
-    return 2;
-  };
-  if (kind == 3) return face_cand(fi, true);
+// The closest feature's record, one word or double per lane.
+template <class M>
+MFCL_D void toRaw(const PolyT<M>& P, int kind, int i, MFCL_LDS RawF& r) {
+  using D = typename M::template P<const double>;
+  const int l = __lane_id();
+  int16_t ia, ib, ic;
+  D rec;
   if (kind == 2) {
-    const auto& e = P.E[fi];
-    const int16_t f0 = e.f0, f1 = e.f1;
-    if (ub(f0 == kNil || f1 == kNil)) return 1;  // open edge: malformed polytope
-    if (ub(e.d2 > kOuter)) {
-      nd = normalized(d3{e.wx, e.wy, e.wz});
-      nv = md.supportFrom(nd, -1, -1, nh0, nh1);
-      if (P.outside(f0, nv)) { start = f0; return 0; }
-      if (P.outside(f1, nv)) { start = f1; return 0; }
-    }
-    const int s0 = face_cand(f0, false);
-    if (s0 == 0) return 0;
-    return face_cand(f1, false);
-  }
-  return 1;
-}
-
-// epa.hpp:269-299 (edge case: squared norm of the segment projection, as in the reference)
-MFCL_D bool epaTerminate(const MFCL_LDS RawF& f, d3 nv, double tol) {
-  double d2;
-  if (f.kind == 2) {
-    MinD m;
-    segDist(nv, ldsGet(f.a.v), ldsGet(f.b.v), m);
-    d2 = m.d2;
+    ia = P.E[i].v0;
+    ib = ic = P.E[i].v1;
+    rec = (D)(&P.E[i]);
   } else {
-    const double t = planeDist(nv, ldsGet(f.a.v), ldsGet(f.b.v), ldsGet(f.c.v));
-    d2 = t * t;
+    P.faceVerts(i, ia, ib, ic);
+    rec = (D)(&P.F[i]);
   }
-  return d2 < tol * tol;
+  const int k = l < 18 ? l / 6 : (l - 22) >> 1;
+  const int v = k == 0 ? ia : (k == 1 ? ib : ic);
+  if (l < 18) ((MFCL_LDS double*)r.v)[l] = ((D)(&P.V[v]))[l - 6 * k];
+  else if (l < 22) r.m[l - 18] = rec[l - 18];
+  else if (l < 28) r.h[k][l & 1] = l & 1 ? P.V[v].h1 : P.V[v].h0;
+  else if (l == 28) r.kind = kind;
+  ldsSync();
 }
 
-// epa.hpp:341-498
+// epa.hpp:341-498: depth and witness points into L->out.
 // support0 / support1 of a recorded direction come from the recorded
 // support vertices when there are (the same points the support searches
 // returned when the polytope vertex was created).
-template <class MK>
-__device__ __attribute__((noinline)) void assignPair(MK md, d3 cand_d, int ch0, int ch1, const MFCL_LDS RawF& f,
-                                                     EpaOut& o) {
-  ScanTally tally(md, o);
-  auto p0 = [&](int k, const MFCL_LDS MVD& m) { return md.point0At(f.h[k][0], ldsGet(m.d)); };
-  auto p1 = [&](int k, const MFCL_LDS MVD& m) { return md.point1At(f.h[k][1], ldsGet(m.d)); };
-  if (f.kind == 1) {
-    o.p0 = p0(0, f.a);
-    o.p1 = p1(0, f.a);
-    o.depth = norm(ldsGet(f.a.v));
-    return;
-  }
-  if (f.kind == 2) {
-    o.depth = sqrt(f.m.d2);
-    const d3 p = ldsGet(f.m.w), a = ldsGet(f.a.v), b = ldsGet(f.b.v);
+__device__ __attribute__((noinline)) static void assignPair(MFCL_LDS EpaLds* L, double cx, double cy, double cz, int ch0,
+                                                            int ch1) {
+  MinkW md{&L->cfg, 0};
+  const MFCL_LDS RawF& f = L->raw;
+  MFCL_LDS EpaOut& o = L->out;
+  const int kind = __builtin_amdgcn_readfirstlane(f.kind);
+  const d3 a = ldsGet(f.v[0]), b = ldsGet(f.v[1]), p = ldsGet(f.m + 1);
+  double w[3] = {1, 0, 0};
+  int n = 0;         // blended vertices
+  bool one = false;  // the first vertex's points as they are
+  double depth = sqrt(f.m[0]);
+  if (kind == 2) {
     const d3 ab = b - a;
     int ax = 0;
     double mx = fabs(ab.x);
     if (fabs(ab.y) > mx) { ax = 1; mx = fabs(ab.y); }
     if (fabs(ab.z) > mx) { ax = 2; mx = fabs(ab.z); }
-    if (mx <= 1e-10) {
-      o.p0 = p0(0, f.a);
-      o.p1 = p1(0, f.a);
-      return;
+    if (ub(mx <= 1e-10)) {
+      one = true;
+    } else {
+      const double s = (comp(p, ax) - comp(a, ax)) / (comp(b, ax) - comp(a, ax));
+      if (ub(!(s < 0 || s > 1.0))) {
+        w[0] = 1.0 - s;
+        w[1] = s;
+        n = 2;
+      }
     }
-    const double s = (comp(p, ax) - comp(a, ax)) / (comp(b, ax) - comp(a, ax));
-    if (!(s < 0 || s > 1.0)) {
-      const double wa = 1.0 - s, wb = s;
-      o.p0 = wa * p0(0, f.a) + wb * p0(1, f.b);
-      o.p1 = wa * p1(0, f.a) + wb * p1(1, f.b);
-      return;
-    }
-  } else if (f.kind == 3) {
-    o.depth = sqrt(f.m.d2);
-    const d3 a = ldsGet(f.a.v), b = ldsGet(f.b.v), c = ldsGet(f.c.v), p = ldsGet(f.m.w);
+  } else {
+    const d3 c = ldsGet(f.v[2]);
     const d3 dl0 = a - b, dl1 = b - c, dl2 = c - a;
     const double area = sqrt(sqnorm(cross(dl0, dl1)));
-    const double w0 = norm(cross(dl1, b - p)) / area;
-    const double w1 = norm(cross(dl2, c - p)) / area;
+    w[0] = norm(cross(dl1, b - p)) / area;
+    w[1] = norm(cross(dl2, c - p)) / area;
     const double chk = norm(cross(dl0, a - p)) / area;
-    const double w2 = 1.0 - w0 - w1;
-    if (!(fabs(chk - w2) > 0.01)) {
-      o.p0 = w0 * p0(0, f.a) + w1 * p0(1, f.b) + w2 * p0(2, f.c);
-      o.p1 = w0 * p1(0, f.a) + w1 * p1(1, f.b) + w2 * p1(2, f.c);
-      return;
-    }
+    w[2] = 1.0 - w[0] - w[1];
+    if (ub(!(fabs(chk - w[2]) > 0.01))) n = 3;
   }
-  const d3 q0 = md.point0At(ch0, cand_d);
-  const d3 q1 = md.point1At(ch1, cand_d);
-  o.p0 = q0;
-  o.p1 = q1;
-  o.depth = norm(q0 - q1);
-}
-
-// Copies an LDS polytope into a device-memory one of larger capacity: the
-// same slot numbers, the extra slots free.  Slot numbers never influence a
-// result, so continuing there equals a run at the larger capacity from the
-// start.
-template <class R>
-MFCL_D void copyRecord(R* dst, const MFCL_LDS R* src) {
-  static_assert(sizeof(R) % 4 == 0, "records copy as words");
-  const MFCL_LDS uint32_t* a = reinterpret_cast<const MFCL_LDS uint32_t*>(src);
-  uint32_t* b = reinterpret_cast<uint32_t*>(dst);
-#pragma unroll
-  for (int k = 0; k < static_cast<int>(sizeof(R) / 4); ++k) b[k] = a[k];
-}
-MFCL_D void spillPoly(const Poly& L, PolyG& G) {
-  const int l = __lane_id();
-  for (int s = l; s < G.nv; s += 64) {
-    if (s < L.nv) {
-      copyRecord(&G.V[s], &L.V[s]);
-      copyRecord(&G.E[s], &L.E[s]);
+  d3 q0 = {0, 0, 0}, q1 = q0;
+  const bool cand = n == 0 && !one;
+#pragma nounroll
+  for (int k = 0; k < (n ? n : 1); ++k) {
+    const int h0 = cand ? ch0 : f.h[k][0], h1 = cand ? ch1 : f.h[k][1];
+    const d3 d = cand ? d3{cx, cy, cz} : ldsGet(f.v[k] + 3);
+    d3 a0, a1;
+    md.pointsAt(h0, h1, d, a0, a1);
+    if (n == 0) {
+      q0 = a0;
+      q1 = a1;
     } else {
-      G.V[s].stamp = -1;
-      G.E[s].stamp = -1;
+      const double wk = k == 0 ? w[0] : (k == 1 ? w[1] : w[2]);
+      q0 = k == 0 ? wk * a0 : q0 + wk * a0;
+      q1 = k == 0 ? wk * a1 : q1 + wk * a1;
     }
   }
-  for (int s = l; s < G.nf; s += 64) {
-    if (s < L.nf) copyRecord(&G.F[s], &L.F[s]);
-    else G.F[s].stamp = -1;
-  }
-  G.stamp = L.stamp;
-  GlbMem::sync();
+  if (cand) depth = norm(q0 - q1);
+  ldsSet(o.p0, q0);
+  ldsSet(o.p1, q1);
+  o.depth = depth;
+  o.scanned += md.scanned;
 }
 
-// Where a pair continues when its LDS polytope might not hold an
-// expansion: a device-memory polytope arena (null: nowhere) of capacity
-// `faces` faces.
-struct SpillTarget {
-  char* base;
-  int faces;
-};
-
-template <class MK>
-__device__ __attribute__((noinline)) EpaOut epaContinue(Poly& P, MK md, double tol, int max_iter, EpaOut o,
-                                                        MFCL_LDS RawF& raw, int it, d3 nv, d3 nd, int nh0, int nh1,
-                                                        int16_t start, SpillTarget st);
-
-// The EPA iterations (epa.hpp:137-237) from iteration `it`; with `pending`
-// the iteration's expansion (nv, nd, start) is still to run.  A polytope in
-// LDS whose expansion may not fit (expand() == 3, only with a spill target)
-// continues in a device-memory polytope of full capacity (epaContinue, out
-// of line: it runs for few pairs and keeps its registers out of this loop).
-template <bool SPILL, class PT, class MK>
-MFCL_D void epaLoop(PT& P, MK& md, double tol, int max_iter, EpaOut& o, MFCL_LDS RawF& raw, int it, bool pending,
-                    d3 nv, d3 nd, int nh0, int nh1, int16_t start, SpillTarget st) {
+// epa.hpp:137-257 on the pair and simplex in L (resume: from the expansion
+// in L->res, the polytope in L already).  Returns the status; depth, points,
+// iterations and vertices scanned in L->out.  may_spill: the request's
+// capacity is larger than this polytope's; a pair whose expansion might not
+// fit stops before it (kEpaSpill, L->res filled in).
+template <class M>
+__device__ __attribute__((noinline)) int epaRun(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int cap_faces,
+                                                double tol, int max_iter, bool may_spill, bool resume) {
+  constexpr double kOuter = 1e-3 * 1e-3;
+  constexpr double kRatio = 1.0 - 1e-3;
+  PolyT<M> P(arena, cap_faces);
+  MinkW md{&L->cfg, 0};
+  MFCL_LDS EpaOut& o = L->out;
+  o.iters = 0;
+  o.scanned = 0;
+  o.depth = 0;
+  ldsSet(o.p0, d3{0, 0, 0});
+  ldsSet(o.p1, d3{0, 0, 0});
+  int it = 0, start = kNil, nh0 = -1, nh1 = -1, status = kEpaFailed;
+  d3 nd = {0, 0, 0}, nv = {0, 0, 0};
+  if (resume) {
+    it = __builtin_amdgcn_readfirstlane(L->res.it);
+    start = __builtin_amdgcn_readfirstlane(L->res.start);
+    nh0 = __builtin_amdgcn_readfirstlane(L->res.nh0);
+    nh1 = __builtin_amdgcn_readfirstlane(L->res.nh1);
+    P.stamp = __builtin_amdgcn_readfirstlane(L->res.stamp);
+    nv = ldsGet(L->res.nv);
+    nd = ldsGet(L->res.nd);
+  } else {
+    const int s2p = __builtin_amdgcn_readfirstlane(simplexToPolytope(P, md, L, arena, cap_faces, tol));
+    o.scanned += md.scanned;
+    md.scanned = 0;
+    if (s2p < 0) return kEpaFailed;
+    if (s2p == kS2pTouching) return kEpaTouching;
+    P.stamp = s2p;
+  }
+  bool pending = resume;
   while (true) {
     if (!pending) {
-      int kind;
-      int16_t fi;
+      int kind, fi;
       P.minToOrigin(false, kind, fi);
-      if (kind == 0) { o.status = kEpaFailed; return; }
       if (kind == 1) {
         const double vd2 = sqnorm(P.vloc(fi));
-        constexpr double kRatio = 1.0 - 1e-3;
-        int k2;
-        int16_t i2;
+        int k2, i2;
         P.minToOrigin(true, k2, i2);
-        if (k2 == 0) { o.status = kEpaFailed; return; }
-        if (k2 == 2) {
-          if (ub(kRatio * P.E[i2].d2 < vd2)) { kind = 2; fi = i2; }
-        } else if (k2 == 3) {
-          if (ub(kRatio * P.F[i2].d2 < vd2)) { kind = 3; fi = i2; }
-        }
+        if (k2 == 0) break;
+        const double d2 = k2 == 2 ? P.E[i2].d2 : P.F[i2].d2;
+        if (ub(kRatio * d2 < vd2)) { kind = k2; fi = i2; }
       }
-      if (kind != 2 && kind != 3) { o.status = kEpaFailed; return; }
-      toRaw(P, kind, fi, raw);
-      nd = d3{0, 0, 0};
-      nv = d3{0, 0, 0};
+      if (kind != 2 && kind != 3) break;
+      toRaw(P, kind, fi, L->raw);
+      // epa.hpp:11-113: candidate directions -- the witness's (phase 0,
+      // when it is far enough from the origin), then the normal of the face
+      // or of the edge's first and second face (phases 1, 2) -- until a
+      // support point lies beyond its face
+      int fa = fi, fb = fi;
+      if (kind == 2) {
+        fa = __builtin_amdgcn_readfirstlane(P.E[fi].f0);
+        fb = __builtin_amdgcn_readfirstlane(P.E[fi].f1);
+        if (fa == kNil || fb == kNil) break;  // open edge: malformed polytope
+      }
+      const typename PolyT<M>::Normal na = P.normalOut(fa), nb = kind == 2 ? P.normalOut(fb) : na;
+      if (kind == 3 && !na.ok) break;
+      int ph = ub(L->raw.m[0] > kOuter) ? 0 : 1, ds = -1;
+      double ba = 0;
       start = kNil;
       nh0 = nh1 = -1;
-      // statuses and the start face are the same in every lane: scalars
-      const int ds = __builtin_amdgcn_readfirstlane(nextDir(P, md, kind, fi, tol, nd, nv, start, nh0, nh1));
-      start = static_cast<int16_t>(__builtin_amdgcn_readfirstlane(start));
-      if (ds == 1) { o.status = kEpaFailed; return; }
-      if (ds == 2) {
-        assignPair(md, nd, nh0, nh1, raw, o);
-        o.iters = it;
-        o.status = kEpaOK;
-        return;
+      while (ds < 0) {
+        if (ph == 1 && !na.ok) ph = 2;  // an edge's degenerate first face
+        if (ph == 2 && !nb.ok) {
+          ds = 1;
+          break;
+        }
+        nd = ph == 0 ? normalized(ldsGet(L->raw.m + 1)) : (ph == 1 ? na.n : nb.n);
+        const WaveSup s = md.sup(nd);
+        nv = s.p0 - s.p1;
+        nh0 = s.i0;
+        nh1 = s.i1;
+        ba = dot(na.n, nv - P.faceAnchor(fa));
+        const double bb = kind == 2 ? dot(nb.n, nv - P.faceAnchor(fb)) : 0.0;
+        if (ph == 0) {
+          // a degenerate face counts as seen (its area is not positive)
+          if (ub(!na.ok || ba >= 0.0)) { start = fa; ds = 0; }
+          else if (kind == 2 && ub(!nb.ok || bb >= 0.0)) { start = fb; ds = 0; }
+          else ph = 1;
+        } else if (ub((ph == 1 ? ba : bb) > tol)) {
+          start = ph == 1 ? fa : fb;
+          ds = 0;
+        } else if (kind == 3 || ph == 2) {
+          ds = 2;
+        } else {
+          ph = 2;
+        }
       }
-      if (start == kNil) { o.status = kEpaFailed; return; }
-      if (ub(epaTerminate(raw, nv, tol))) {
-        assignPair(md, nd, nh0, nh1, raw, o);
-        o.iters = it;
-        o.status = kEpaOK;
-        return;
+      if (ds == 1) break;
+      // epa.hpp:269-299: converged when the support point is within tol of
+      // the closest feature -- a face's plane (ba is that distance, signed;
+      // the face is not degenerate here), or a segment (the squared norm of
+      // the projection, as in the reference)
+      double d2 = ba * ba;
+      if (kind == 2) {
+        MinD m;
+        segDist(nv, ldsGet(L->raw.v[0]), ldsGet(L->raw.v[1]), m);
+        d2 = m.d2;
+      }
+      if (ds == 2 || ub(d2 < tol * tol)) {
+        status = kEpaOK;
+        break;
       }
     }
     pending = false;
-    const int ex = __builtin_amdgcn_readfirstlane(P.expand(nv, nd, nh0, nh1, start, SPILL && st.base != nullptr));
-    if constexpr (SPILL && std::is_same<PT, Poly>::value) {
-      if (ex == 3) {
-        o = epaContinue(P, md, tol, max_iter, o, raw, it, nv, nd, nh0, nh1, start, st);
-        return;
-      }
+    int ex;
+    if constexpr (M::kWords > 0) ex = P.expandMask(nv, nd, nh0, nh1, start, may_spill);
+    else ex = P.expandLarge(nv, nd, nh0, nh1, start);
+    ex = __builtin_amdgcn_readfirstlane(ex);
+    if (M::kWords > 0 && ex == 3) {
+      ldsSet(L->res.nv, nv);
+      ldsSet(L->res.nd, nd);
+      L->res.it = it;
+      L->res.stamp = P.stamp;
+      L->res.nh0 = nh0;
+      L->res.nh1 = nh1;
+      L->res.start = start;
+      o.scanned += md.scanned;
+      return kEpaSpill;
     }
-    if (ex == 1) { o.status = kEpaFailed; return; }
+    if (ex == 1) break;
     if (ex == 2) {
-      assignPair(md, nd, nh0, nh1, raw, o);
-      o.iters = it;
-      o.status = kEpaMallocFailed;
-      return;
+      status = kEpaMallocFailed;
+      break;
     }
     ++it;
     if (it >= max_iter) {
-      assignPair(md, nd, nh0, nh1, raw, o);
-      o.iters = it;
-      o.status = kEpaIterLimit;
-      return;
+      status = kEpaIterLimit;
+      break;
     }
   }
+  o.scanned += md.scanned;
+  if (status != kEpaFailed) {
+    o.iters = it;
+    assignPair(L, nd.x, nd.y, nd.z, nh0, nh1);
+  }
+  return status;
 }
 
-template <class MK>
-__device__ __attribute__((noinline)) EpaOut epaContinue(Poly& P, MK md, double tol, int max_iter, EpaOut o,
-                                                        MFCL_LDS RawF& raw, int it, d3 nv, d3 nd, int nh0, int nh1,
-                                                        int16_t start, SpillTarget st) {
-  const ArenaDims fd = arenaDims(st.faces);
-  PolyG G;
-  G.V = reinterpret_cast<EVert*>(st.base);
-  G.E = reinterpret_cast<EEdge*>(st.base + sizeof(EVert) * fd.nv);
-  G.F = reinterpret_cast<EFace*>(st.base + sizeof(EVert) * fd.nv + sizeof(EEdge) * fd.nv);
-  G.BL = reinterpret_cast<BorderRec*>(st.base + sizeof(EVert) * fd.nv + sizeof(EEdge) * fd.nv +
-                                      sizeof(EFace) * fd.nf);
-  G.nv = fd.nv;
-  G.nf = fd.nf;
-  spillPoly(P, G);
-  o.spilled = 1;
-  const int scanned0 = md.scanned;
-  epaLoop<false>(G, md, tol, max_iter, o, raw, it, true, nv, nd, nh0, nh1, start, SpillTarget{nullptr, 0});
-  o.scanned_extra += md.scanned - scanned0;
-  return o;
+// A spilled pair to / from device memory: the records keep their slot
+// numbers, the larger polytope's extra slots are free.  Slot numbers never
+// influence a result, so continuing there equals a run at the larger
+// capacity from the start.
+MFCL_D void copyOut(char* dst, const MFCL_LDS char* src, size_t bytes) {
+  uint64_t* d = reinterpret_cast<uint64_t*>(dst);
+  const MFCL_LDS uint64_t* s = (const MFCL_LDS uint64_t*)(src);
+  for (uint32_t k = __lane_id(); k < bytes / 8; k += 64) d[k] = s[k];
 }
-
-// epa.hpp:137-257.  st: where the pair continues if P (of smaller capacity
-// than the request's) might not hold an expansion.
-template <bool SPILL, class MK>
-MFCL_D void epaEvaluate(Poly& P, MK& md, const SmpD& s, double tol, int max_iter, EpaOut& o,
-                        MFCL_LDS RawF& raw, SpillTarget st) {
-  o.iters = 0;
-  o.scanned_extra = 0;
-  o.spilled = 0;
-  o.depth = 0;
-  o.p0 = d3{0, 0, 0};
-  o.p1 = d3{0, 0, 0};
-  const int s2p = simplexToPolytope(P, md, s, tol, o);
-  if (s2p == 2) { o.status = kEpaFailed; return; }
-  if (s2p == 1) { o.depth = 0.0; o.status = kEpaTouching; return; }
-  epaLoop<SPILL>(P, md, tol, max_iter, o, raw, 0, false, d3{0, 0, 0}, d3{0, 0, 0}, -1, -1, kNil, st);
+MFCL_D void epaDump(char* dst, MFCL_LDS EpaLds* L, int cap_faces, int item) {
+  L->res.item = item;
+  ldsSync();
+  copyOut(dst, (const MFCL_LDS char*)(&L->raw), sizeof(RawF));
+  copyOut(dst + sizeof(RawF), (const MFCL_LDS char*)(&L->res), sizeof(EpaResume));
+  copyOut(dst + kEpaDumpHead, ldsArena(L), polyBytes<SmallMem>(cap_faces));
+}
+MFCL_D int epaDumpItem(const char* src) {
+  return reinterpret_cast<const EpaResume*>(src + sizeof(RawF))->item;
+}
+// n records of type FROM into records that are FROM or a prefix of it
+template <class FROM, class P>
+MFCL_D void copyRecs(P dst, const char* src, int n) {
+  using To = std::remove_reference_t<decltype(*dst)>;
+  constexpr int kWords = sizeof(To) / 8, kFrom = sizeof(FROM) / 8;
+  static_assert(kWords <= kFrom, "a prefix");
+  using Wp = std::conditional_t<std::is_same<P, To*>::value && std::is_pointer<P>::value && sizeof(P) == 8, uint64_t*,
+                                MFCL_LDS uint64_t*>;
+  Wp d = (Wp)(dst);
+  const uint64_t* s = reinterpret_cast<const uint64_t*>(src);
+  for (int k = static_cast<int>(__lane_id()); k < n * kWords; k += 64) d[k] = s[k / kWords * kFrom + k % kWords];
+}
+template <class M>
+MFCL_D void epaLoad(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int cap_faces, const char* src,
+                    int small_faces) {
+  const ArenaDims sd = arenaDims(small_faces);
+  PolyT<M> P(arena, cap_faces);
+  const uint64_t* w = reinterpret_cast<const uint64_t*>(src);
+  for (uint32_t k = __lane_id(); k < kEpaDumpHead / 8; k += 64) {
+    if (k < sizeof(RawF) / 8) ((MFCL_LDS uint64_t*)(&L->raw))[k] = w[k];
+    else ((MFCL_LDS uint64_t*)(&L->res))[k - sizeof(RawF) / 8] = w[k];
+  }
+  src += kEpaDumpHead;
+  using S = PolyT<SmallMem>;
+  copyRecs<S::EVert>(P.V, src, sd.nv);
+  src += sizeof(S::EVert) * sd.nv;
+  copyRecs<S::EEdge>(P.E, src, sd.nv);
+  src += sizeof(S::EEdge) * sd.nv;
+  copyRecs<S::EFace>(P.F, src, sd.nf);
+  for (int s = sd.nv + static_cast<int>(__lane_id()); s < P.nv; s += 64) P.V[s].stamp = P.E[s].stamp = -1;
+  for (int s = sd.nf + static_cast<int>(__lane_id()); s < P.nf; s += 64) P.F[s].stamp = -1;
+  M::sync();
+  ldsSync();
 }
 
 }  // namespace mfcl

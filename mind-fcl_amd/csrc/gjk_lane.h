@@ -230,13 +230,9 @@ MFCL_D void coopScanBatch(uint64_t& m, uint64_t vp, int nv, float rb, d3 d, int 
                         (fabsf(static_cast<float>(dx[j])) + fabsf(static_cast<float>(dy[j])) +
                          fabsf(static_cast<float>(dz[j])));
     int idx;
-    if (best[j] - second[j] > bound) {
-      idx = bi[j] < pn[j] ? bi[j] : 0;
-      scanned += static_cast<uint64_t>(pn[j]);
-    } else {
-      idx = waveRescan64(pv[j], pn[j], dx[j], dy[j], dz[j], lane);
-      scanned += static_cast<uint64_t>(2 * pn[j]);
-    }
+    if (best[j] - second[j] > bound) idx = bi[j] < pn[j] ? bi[j] : 0;
+    else idx = waveRescan64(pv[j], pn[j], dx[j], dy[j], dz[j], lane);
+    scanned += static_cast<uint64_t>(pn[j]);
     if (lane == p[j]) res = idx;
   }
 }

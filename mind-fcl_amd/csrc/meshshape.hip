@@ -10,10 +10,11 @@
 // Three launches: (1) one wavefront per query walks the mesh's OBB tree
 // against the shape's box (its frame, FP32 test with the conservative
 // margin of the mesh-mesh traversal), 64 nodes per step off an LDS stack,
-// and appends every reached leaf as a (query, triangle) candidate; (2) 16
-// lanes per candidate run the leaf test in FP64 exactly as the reference
-// orders it, counting and recording colliding triangles; (3) one lane per
-// query writes the result and sorts its kept triangle ids.  The set of
+// and appends every reached leaf as a (query, triangle) candidate; (2) the
+// leaf tests in FP64 exactly as the reference orders them, closed forms one
+// per lane and searches one per wavefront, counting and recording colliding
+// triangles; (3) one wavefront per query writes the result and its kept
+// triangles in ascending order.  The set of
 // colliding triangles does not depend on the tree, so booleans and complete
 // sets equal the reference's; which ones are kept when more than
 // max_contacts collide follows the traversal here, not the reference's
@@ -32,7 +33,6 @@
 namespace mfcl {
 
 constexpr int kMsStack = 2048;  // node ids per wavefront (LDS)
-constexpr int kMsGroup = 16;    // lanes per leaf test
 
 struct MeshShapeArgs {
   ShapeTables T;
@@ -54,6 +54,7 @@ struct MeshShapeArgs {
   uint32_t* bv_tests;  // per query: OBB tests
   uint32_t* overflow;  // per query: 1 when the LDS stack would overflow
   int max_contacts;
+  int32_t* tri_tmp;    // colliding triangles in the order of arrival
   int32_t* tri_out;
   int gjk_max_it;
   double gjk_tol;
@@ -278,226 +279,250 @@ MFCL_D bool boxTriHit(double s0, double s1, double s2, const tf3& ts, const tf3&
   return dot(n, d3{pmin[0], pmin[1], pmin[2]}) <= 0 && dot(n, d3{pmax[0], pmax[1], pmax[2]}) >= 0;
 }
 
-__global__ void __launch_bounds__(256) msLeafKernel(MeshShapeArgs A, uint64_t ncand) {
-  __shared__ MinkCfg cfgs[256 / kMsGroup];
-  const uint64_t k = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kMsGroup;
-  const int lg = static_cast<int>(threadIdx.x % kMsGroup);
-  if (k >= ncand) return;  // uniform across a group
+// A candidate's query, triangle and poses.
+struct MsItem {
+  uint64_t q;
+  uint32_t t, shp;
+  tf3 tm, ts;
+  const float4* tri;
+  d3 P1, P2, P3;
+};
+MFCL_D MsItem msItem(const MeshShapeArgs& A, uint64_t k) {
+  MsItem m;
   const uint64_t c = A.cand[k];
-  const uint64_t q = c >> 32;
-  const uint32_t t = static_cast<uint32_t>(c & 0xFFFFFFFFull);
-  const uint32_t mesh = A.mesh_ids[q], shp = A.shape_ids[q];
-  const tf3 tm = poseFromQuat(A.pose_m + 7 * q), ts = poseFromQuat(A.pose_s + 7 * q);
-  const float4* tri = A.tris + 3 * (static_cast<uint64_t>(A.tri_base[mesh]) + t);
-  const d3 P1 = {tri[0].x, tri[0].y, tri[0].z}, P2 = {tri[1].x, tri[1].y, tri[1].z},
-           P3 = {tri[2].x, tri[2].y, tri[2].z};
-  const DevShape S = loadShape(A.T, shp);
-  bool hit;
-  if (S.type == kSphere) {
-    hit = sphereTriHit(S.p0, ts.t, apply(tm, P1), apply(tm, P2), apply(tm, P3));
-  } else if (S.type == kBox) {
-    hit = boxTriHit(S.p0, S.p1, S.p2, ts, tm, P1, P2, P3);
-  } else {
-    DevShape B;
-    B.type = kTriangle;
-    B.p0 = B.p1 = B.p2 = 0;
-    B.verts = tri;
-    B.nv = 3;
-    B.rbound = 0.f;
-    B.lv = nullptr;
-    B.ls = 0;
-    B.nbr = nullptr;
-    B.seed = nullptr;
-    B.wblk = nullptr;
-    d3 int0 = {0, 0, 0};
-    if (S.type == kConvex) {
-      const double4 ci = A.interior[shp];
-      int0 = d3{ci.x, ci.y, ci.z};
-    }
-    const d3 int1 = (P1 + P2 + P3) / 3.0;
-    MFCL_LDS MinkCfg* cfg = (MFCL_LDS MinkCfg*)(&cfgs[threadIdx.x / kMsGroup]);
-    writeCfg(cfg, S, ts, B, tm, int0, int1);
-    MinkL<kMsGroup> md{cfg, lg, 0};
-    hit = mprIntersect(md, A.gjk_max_it, A.gjk_tol) == kMprIntersect;
-  }
-  if (lg != 0 || !hit) return;
+  m.q = c >> 32;
+  m.t = static_cast<uint32_t>(c & 0xFFFFFFFFull);
+  m.shp = A.shape_ids[m.q];
+  m.tm = poseFromQuat(A.pose_m + 7 * m.q);
+  m.ts = poseFromQuat(A.pose_s + 7 * m.q);
+  m.tri = A.tris + 3 * (static_cast<uint64_t>(A.tri_base[A.mesh_ids[m.q]]) + m.t);
+  m.P1 = d3{m.tri[0].x, m.tri[0].y, m.tri[0].z};
+  m.P2 = d3{m.tri[1].x, m.tri[1].y, m.tri[1].z};
+  m.P3 = d3{m.tri[2].x, m.tri[2].y, m.tri[2].z};
+  return m;
+}
+// The wavefront's Minkowski difference of (shape, triangle).
+MFCL_D void msCfg(const MeshShapeArgs& A, const MsItem& m, MFCL_LDS WaveCfg* cfg, d3 int0, d3 int1) {
+  DevShape B;
+  B.type = kTriangle;
+  B.p0 = B.p1 = B.p2 = 0;
+  B.verts = m.tri;
+  B.nv = 3;
+  B.rbound = 0.f;
+  B.lv = nullptr;
+  B.ls = 0;
+  B.nbr = nullptr;
+  B.seed = nullptr;
+  B.wblk = nullptr;
+  waveCfgSet(cfg, loadShape(A.T, m.shp), m.ts, B, m.tm, int0, int1);
+}
+
+// Leaf tests: each wavefront takes `chunk` consecutive candidates; its lanes
+// run the spheres' and boxes' closed forms together, then the wavefront the
+// others' MPR one after the other.
+MFCL_D void msHit(const MeshShapeArgs& A, uint64_t q, uint32_t t) {
   const uint32_t slot = atomicAdd(&A.counts[q], 1u);
   if (static_cast<int>(slot) < A.max_contacts)
-    A.tri_out[q * static_cast<uint64_t>(A.max_contacts) + slot] = static_cast<int32_t>(t);
+    A.tri_tmp[q * static_cast<uint64_t>(A.max_contacts) + slot] = static_cast<int32_t>(t);
+}
+__global__ void __launch_bounds__(256) msLeafKernel(MeshShapeArgs A, uint64_t ncand, int chunk) {
+  __shared__ WaveCfg cfgs[4];
+  MFCL_LDS WaveCfg* cfg = (MFCL_LDS WaveCfg*)(&cfgs[threadIdx.x >> 6]);
+  const int lane = threadIdx.x & 63;
+  const uint64_t base = ((static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6) * chunk;
+  bool search = false;
+  if (lane < chunk && base + lane < ncand) {
+    const MsItem m = msItem(A, base + lane);
+    const DevShape S = loadShape(A.T, m.shp);
+    if (S.type == kSphere) {
+      if (sphereTriHit(S.p0, m.ts.t, apply(m.tm, m.P1), apply(m.tm, m.P2), apply(m.tm, m.P3))) msHit(A, m.q, m.t);
+    } else if (S.type == kBox) {
+      if (boxTriHit(S.p0, S.p1, S.p2, m.ts, m.tm, m.P1, m.P2, m.P3)) msHit(A, m.q, m.t);
+    } else {
+      search = true;
+    }
+  }
+  for (unsigned long long todo = __ballot(search); todo; todo &= todo - 1) {
+    const MsItem m = msItem(A, base + __builtin_ctzll(todo));
+    d3 int0 = {0, 0, 0};
+    if (A.T.type[m.shp] == kConvex) {
+      const double4 ci = A.interior[m.shp];
+      int0 = d3{ci.x, ci.y, ci.z};
+    }
+    msCfg(A, m, cfg, int0, (m.P1 + m.P2 + m.P3) / 3.0);
+    MinkW md{cfg, 0};
+    const bool hit = mprIntersect(md, A.gjk_max_it, A.gjk_tol) == kMprIntersect;
+    if (hit && lane == 0) msHit(A, m.q, m.t);
+  }
 }
 
 // Penetration enabled (shapeTriangleIntersect with contact outputs,
-// gjk_solver-inl.h:545-563): one wavefront per candidate, taken from a
-// shared counter.  Spheres take sphereTriContact; every other shape runs
-// GJK from -UnitX and EPA on (shape, triangle) (gjk_solver-inl.h:452-527),
-// the EPA polytope in the wavefront's LDS slice (cap_faces faces) and,
-// when it might outgrow it, in the wavefront's device-memory polytope of the
-// request's capacity.  A hit records the contact with the traversal's
-// normal reversal (bvh_solver-inl.h:55-65, shape_pair_intersect-inl.h:
-// 19-26): b1 = the triangle, b2 = -1.
-constexpr size_t kMsCfgBytes = (sizeof(MinkCfg) + 15) & ~static_cast<size_t>(15);
-constexpr size_t kMsRawBytes = (sizeof(RawF) + 15) & ~static_cast<size_t>(15);
-constexpr size_t kMsPolyBytes = (sizeof(Poly) + 15) & ~static_cast<size_t>(15);
-inline size_t msSliceBytes(int cap_faces) { return kMsCfgBytes + kMsRawBytes + kMsPolyBytes + arenaBytes(cap_faces); }
-
+// gjk_solver-inl.h:545-563).  Spheres take sphereTriContact, one per lane;
+// every other shape runs GJK from -UnitX and EPA on (shape, triangle)
+// (gjk_solver-inl.h:452-527), one per wavefront, the EPA polytope in the
+// wavefront's LDS slice (cap_faces faces); pairs that might outgrow it
+// continue (or, out of dump slots, restart) at the request's capacity in a
+// second launch.  A hit records the contact with the traversal's normal
+// reversal (bvh_solver-inl.h:55-65, shape_pair_intersect-inl.h:19-26): b1 =
+// the triangle, b2 = -1.
 struct MsPen {
-  mfcl_mesh_contact* contacts;  // n * max_contacts
-  int cap_faces;                // LDS polytope capacity
-  size_t slice_bytes;           // LDS bytes per wavefront
-  char* arena;                  // device-memory polytopes, one per wavefront of the grid
+  mfcl_mesh_contact* tmp;  // n * max_contacts, in the order of arrival
+  int cap_faces;           // LDS polytope capacity
+  size_t slice_bytes;      // LDS bytes per wavefront
+  char* dumps;             // pairs to continue
+  uint32_t n_dumps;
+  size_t dump_bytes;
+  uint32_t* redo;          // pairs to restart
+  uint32_t* cnt;           // MsCount
+  char* arena;             // device-memory polytopes, one per block of the full-capacity pass (null: in LDS)
   size_t arena_slice;
   int epa_max_faces, epa_max_it;
   double epa_tol;
-  uint32_t* next;               // candidate cursor
 };
+enum MsCount : int { kMsNext = 0, kMsDumps = 1, kMsRedo = 2, kMsFullNext = 3, kMsCounts = 8 };
 
-__global__ void __launch_bounds__(256, 2) msPenKernel(MeshShapeArgs A, MsPen E, uint64_t ncand) {
+MFCL_D void msContact(const MeshShapeArgs& A, const MsPen& E, uint64_t q, uint32_t t, d3 pos, d3 nrm, double depth) {
+  const uint32_t slot = atomicAdd(&A.counts[q], 1u);
+  if (static_cast<int>(slot) >= A.max_contacts) return;
+  mfcl_mesh_contact& o = E.tmp[q * static_cast<uint64_t>(A.max_contacts) + slot];
+  o.b1 = static_cast<int32_t>(t);
+  o.b2 = -1;
+  o.pos[0] = pos.x; o.pos[1] = pos.y; o.pos[2] = pos.z;
+  o.normal[0] = -nrm.x; o.normal[1] = -nrm.y; o.normal[2] = -nrm.z;
+  o.depth = depth;
+}
+// The contact of a pair whose EPA ended with `status` (lane 0 writes).
+MFCL_D void msEpaContact(const MeshShapeArgs& A, const MsPen& E, const MsItem& m, const MFCL_LDS EpaLds* L, int status) {
+  if (status == kEpaFailed || __lane_id() != 0) return;
+  const d3 p0 = ldsGet(L->out.p0), p1 = ldsGet(L->out.p1);
+  d3 n1 = p0 - p1;
+  n1 = sqnorm(n1) <= 0 ? d3{0, 0, 1} : normalized(n1);
+  msContact(A, E, m.q, m.t, apply(m.ts, 0.5 * (p0 + p1)), mul(m.ts.R, n1), L->out.depth);
+}
+// GJK of the configuration in L; the simplex into L->s when it intersects.
+MFCL_D bool msGjk(const MeshShapeArgs& A, MFCL_LDS EpaLds* L) {
+  MinkW md{&L->cfg, 0};
+  Smp s;
+  smpInit(s);
+  GjkOut g;
+  gjkEvaluate(md, s, d3{-1, 0, 0}, A.gjk_tol, A.gjk_max_it, false, g);
+  if (__builtin_amdgcn_readfirstlane(g.status) != kGjkIntersect) return false;
+  L->s.rank = s.rank;
+  ldsSet(L->s.a.v, s.a.v); ldsSet(L->s.a.d, md.dirOf(static_cast<int>(s.a.id)));
+  ldsSet(L->s.b.v, s.b.v); ldsSet(L->s.b.d, md.dirOf(static_cast<int>(s.b.id)));
+  ldsSet(L->s.c.v, s.c.v); ldsSet(L->s.c.d, md.dirOf(static_cast<int>(s.c.id)));
+  ldsSet(L->s.e.v, s.e.v); ldsSet(L->s.e.d, md.dirOf(static_cast<int>(s.e.id)));
+  return true;
+}
+
+__global__ void __launch_bounds__(256, 3) msPenKernel(MeshShapeArgs A, MsPen E, uint64_t ncand, int chunk) {
   extern __shared__ __align__(16) char ms_lds[];
+  MFCL_LDS EpaLds* L = (MFCL_LDS EpaLds*)((MFCL_LDS char*)(ms_lds) + (threadIdx.x >> 6) * E.slice_bytes);
   const int lane = threadIdx.x & 63;
-  const ArenaDims dims = arenaDims(E.cap_faces);
-  MFCL_LDS char* slice = (MFCL_LDS char*)(ms_lds) + static_cast<size_t>(threadIdx.x >> 6) * E.slice_bytes;
-  MFCL_LDS MinkCfg* cfg = (MFCL_LDS MinkCfg*)(slice);
-  MFCL_LDS RawF* raw = (MFCL_LDS RawF*)(slice + kMsCfgBytes);
-  MFCL_LDS char* base = slice + kMsCfgBytes + kMsRawBytes + kMsPolyBytes;
-  Poly& poly = *reinterpret_cast<Poly*>(ms_lds + static_cast<size_t>(threadIdx.x >> 6) * E.slice_bytes +
-                                        kMsCfgBytes + kMsRawBytes);
-  poly.V = (MFCL_LDS EVert*)(base);
-  poly.E = (MFCL_LDS EEdge*)(base + sizeof(EVert) * dims.nv);
-  poly.F = (MFCL_LDS EFace*)(base + sizeof(EVert) * dims.nv + sizeof(EEdge) * dims.nv);
-  poly.BL = (MFCL_LDS BorderRec*)(base + sizeof(EVert) * dims.nv + sizeof(EEdge) * dims.nv +
-                                  sizeof(EFace) * dims.nf);
-  poly.nv = dims.nv;
-  poly.nf = dims.nf;
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  const SpillTarget st{E.cap_faces < E.epa_max_faces ? E.arena + wave * E.arena_slice : nullptr, E.epa_max_faces};
-  for (;;) {
-    uint32_t k = 0;
-    if (lane == 0) k = atomicAdd(E.next, 1u);
-    k = __shfl(k, 0);
-    if (k >= ncand) break;
-    const uint64_t c = A.cand[k];
-    const uint64_t q = c >> 32;
-    const uint32_t t = static_cast<uint32_t>(c & 0xFFFFFFFFull);
-    const uint32_t mesh = A.mesh_ids[q], shp = A.shape_ids[q];
-    const tf3 tm = poseFromQuat(A.pose_m + 7 * q), ts = poseFromQuat(A.pose_s + 7 * q);
-    const float4* tri = A.tris + 3 * (static_cast<uint64_t>(A.tri_base[mesh]) + t);
-    const d3 P1 = {tri[0].x, tri[0].y, tri[0].z}, P2 = {tri[1].x, tri[1].y, tri[1].z},
-             P3 = {tri[2].x, tri[2].y, tri[2].z};
-    const DevShape S = loadShape(A.T, shp);
-    bool hit = false;
-    d3 pos = {0, 0, 0}, nrm = {0, 0, 0};
-    double depth = 0;
-    if (S.type == kSphere) {
+  const uint64_t base = ((static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6) * chunk;
+  bool search = false;
+  if (lane < chunk && base + lane < ncand) {
+    const MsItem m = msItem(A, base + lane);
+    if (A.T.type[m.shp] == kSphere) {
       SphereTriContact sc;
-      hit = sphereTriContact(S.p0, ts.t, apply(tm, P1), apply(tm, P2), apply(tm, P3), &sc);
-      pos = sc.pos;
-      nrm = sc.normal;
-      depth = sc.depth;
+      if (sphereTriContact(A.T.param[m.shp].x, m.ts.t, apply(m.tm, m.P1), apply(m.tm, m.P2), apply(m.tm, m.P3), &sc))
+        msContact(A, E, m.q, m.t, sc.pos, sc.normal, sc.depth);
     } else {
-      DevShape B;
-      B.type = kTriangle;
-      B.p0 = B.p1 = B.p2 = 0;
-      B.verts = tri;
-      B.nv = 3;
-      B.rbound = 0.f;
-      B.lv = nullptr;
-      B.ls = 0;
-      B.nbr = nullptr;
-      B.seed = nullptr;
-      B.wblk = nullptr;
-      writeCfg(cfg, S, ts, B, tm, d3{0, 0, 0}, d3{0, 0, 0});
-      MinkL<64> md{cfg, lane, 0};
-      Smp smp;
-      GjkOut g;
-      gjkEvaluate(md, smp, d3{-1, 0, 0}, A.gjk_tol, A.gjk_max_it, false, g);
-      if (g.status == kGjkIntersect) {
-        SmpD sd;
-        sd.rank = smp.rank;
-        storeMVD(sd.a, smp.a.v, slotDir(cfg, smp.a.id));
-        storeMVD(sd.b, smp.b.v, slotDir(cfg, smp.b.id));
-        storeMVD(sd.c, smp.c.v, slotDir(cfg, smp.c.id));
-        storeMVD(sd.e, smp.e.v, slotDir(cfg, smp.e.id));
-        EpaOut eo;
-        if (st.base) epaEvaluate<true>(poly, md, sd, E.epa_tol, E.epa_max_it, eo, *raw, st);
-        else epaEvaluate<false>(poly, md, sd, E.epa_tol, E.epa_max_it, eo, *raw, st);
-        if (eo.status != kEpaFailed) {
-          hit = true;
-          d3 n1 = eo.p0 - eo.p1;
-          n1 = sqnorm(n1) <= 0 ? d3{0, 0, 1} : normalized(n1);
-          pos = apply(ts, 0.5 * (eo.p0 + eo.p1));
-          nrm = mul(ts.R, n1);
-          depth = eo.depth;
-        }
-      }
+      search = true;
     }
-    if (lane != 0 || !hit) continue;
-    const uint32_t slot = atomicAdd(&A.counts[q], 1u);
-    if (static_cast<int>(slot) < A.max_contacts) {
-      mfcl_mesh_contact& o = E.contacts[q * static_cast<uint64_t>(A.max_contacts) + slot];
-      o.b1 = static_cast<int32_t>(t);
-      o.b2 = -1;
-      o.pos[0] = pos.x; o.pos[1] = pos.y; o.pos[2] = pos.z;
-      o.normal[0] = -nrm.x; o.normal[1] = -nrm.y; o.normal[2] = -nrm.z;
-      o.depth = depth;
+  }
+  for (unsigned long long todo = __ballot(search); todo; todo &= todo - 1) {
+    const uint64_t k = base + __builtin_ctzll(todo);
+    msCfg(A, msItem(A, k), &L->cfg, d3{0, 0, 0}, d3{0, 0, 0});
+    if (!msGjk(A, L)) continue;
+    const int st = epaRun<SmallMem>(L, ldsArena(L), E.cap_faces, E.epa_tol, E.epa_max_it, E.cap_faces < E.epa_max_faces,
+                                    false);
+    if (st != kEpaSpill) {
+      msEpaContact(A, E, msItem(A, k), L, st);
+      continue;
     }
+    uint32_t slot = 0;
+    if (lane == 0) slot = atomicAdd(E.cnt + kMsDumps, 1u);
+    slot = __builtin_amdgcn_readfirstlane(slot);
+    if (slot < E.n_dumps) epaDump(E.dumps + slot * E.dump_bytes, L, E.cap_faces, static_cast<int>(k));
+    else if (lane == 0) E.redo[atomicAdd(E.cnt + kMsRedo, 1u)] = static_cast<uint32_t>(k);
   }
 }
 
-// Result headers of a penetration-enabled query; the kept contacts sorted
-// by triangle id.
-__global__ void msFinishPenKernel(MeshShapeArgs A, mfcl_mesh_contact* contacts, mfcl_mesh_result* out) {
-  const uint64_t q = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= A.n) return;
+template <class M>
+__global__ void __launch_bounds__(64) msPenFullKernel(MeshShapeArgs A, MsPen E) {
+  extern __shared__ __align__(16) char ms_lds[];
+  MFCL_LDS EpaLds* L = (MFCL_LDS EpaLds*)((MFCL_LDS char*)(ms_lds));
+  typename M::template P<char> arena;
+  if constexpr (std::is_same<M, GlobalMem>::value) arena = E.arena + blockIdx.x * E.arena_slice;
+  else arena = ldsArena(L);
+  const uint32_t asked = E.cnt[kMsDumps];
+  const uint32_t dumps = asked < E.n_dumps ? asked : E.n_dumps, count = dumps + E.cnt[kMsRedo];
+  for (;;) {
+    uint32_t i = 0;
+    if (threadIdx.x == 0) i = atomicAdd(E.cnt + kMsFullNext, 1u);
+    i = __builtin_amdgcn_readfirstlane(i);
+    if (i >= count) break;
+    const bool resume = i < dumps;
+    const char* dump = E.dumps + i * E.dump_bytes;
+    const uint32_t k = __builtin_amdgcn_readfirstlane(resume ? static_cast<uint32_t>(epaDumpItem(dump)) : E.redo[i - dumps]);
+    const MsItem m = msItem(A, k);
+    msCfg(A, m, &L->cfg, d3{0, 0, 0}, d3{0, 0, 0});
+    if (resume) epaLoad<M>(L, arena, E.epa_max_faces, dump, E.cap_faces);
+    else if (!msGjk(A, L)) continue;
+    const int st = epaRun<M>(L, arena, E.epa_max_faces, E.epa_tol, E.epa_max_it, false, resume);
+    msEpaContact(A, E, msItem(A, k), L, st);
+  }
+}
+
+// Result headers, one wavefront per query.  Kept triangles (contacts) move
+// from the order of arrival to ascending triangle ids: a triangle's place is
+// the number of smaller ids (each triangle is a candidate once).
+MFCL_D int msHeader(const MeshShapeArgs& A, uint64_t q, mfcl_mesh_result* out) {
   const uint32_t cnt = A.counts[q];
   const int kept = static_cast<int>(cnt) < A.max_contacts ? static_cast<int>(cnt) : A.max_contacts;
-  mfcl_mesh_result r;
-  r.hit = A.overflow[q] ? -1 : (cnt > 0 ? 1 : 0);
-  r.n_contacts = kept;
-  r.bv_tests = static_cast<int32_t>(A.bv_tests[q]);
-  r.leaf_tests = static_cast<int32_t>(A.leaves[q]);
-  out[q] = r;
+  if (threadIdx.x == 0) {
+    mfcl_mesh_result r;
+    r.hit = A.overflow[q] ? -1 : (cnt > 0 ? 1 : 0);
+    r.n_contacts = kept;
+    r.bv_tests = static_cast<int32_t>(A.bv_tests[q]);
+    r.leaf_tests = static_cast<int32_t>(A.leaves[q]);
+    out[q] = r;
+  }
+  return kept;
+}
+constexpr int kMsMaxContacts = 1024;
+MFCL_D int msPlace(const int32_t* ids, int kept, int32_t id) {
+  int r = 0;
+  for (int j = 0; j < kept; ++j) r += ids[j] < id;
+  return r;
+}
+__global__ void __launch_bounds__(64) msFinishPenKernel(MeshShapeArgs A, const mfcl_mesh_contact* tmp,
+                                                        mfcl_mesh_contact* contacts, mfcl_mesh_result* out) {
+  __shared__ int32_t ids[kMsMaxContacts];
+  const uint64_t q = blockIdx.x;
+  const int kept = msHeader(A, q, out), l = threadIdx.x;
+  const mfcl_mesh_contact* in = tmp + q * static_cast<uint64_t>(A.max_contacts);
   mfcl_mesh_contact* o = contacts + q * static_cast<uint64_t>(A.max_contacts);
-  for (int i = 1; i < kept; ++i) {
-    const mfcl_mesh_contact key = o[i];
-    int j = i - 1;
-    while (j >= 0 && o[j].b1 > key.b1) {
-      o[j + 1] = o[j];
-      --j;
-    }
-    o[j + 1] = key;
-  }
-  for (int i = kept; i < A.max_contacts; ++i) {
-    mfcl_mesh_contact z;
-    z.b1 = z.b2 = -1;
-    z.pos[0] = z.pos[1] = z.pos[2] = 0;
-    z.normal[0] = z.normal[1] = z.normal[2] = 0;
-    z.depth = 0;
-    o[i] = z;
-  }
+  for (int i = l; i < kept; i += 64) ids[i] = in[i].b1;
+  __syncthreads();
+  for (int i = l; i < kept; i += 64) o[msPlace(ids, kept, ids[i])] = in[i];
+  // the others: b1 = b2 = -1, zeros (eight 8-byte words a record)
+  uint64_t* w = reinterpret_cast<uint64_t*>(o);
+  static_assert(sizeof(mfcl_mesh_contact) == 64, "eight words");
+  for (int i = 8 * kept + l; i < 8 * A.max_contacts; i += 64) w[i] = i % 8 == 0 ? ~0ull : 0ull;
 }
 
-__global__ void msFinishKernel(MeshShapeArgs A, mfcl_mesh_result* out) {
-  const uint64_t q = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= A.n) return;
-  const uint32_t cnt = A.counts[q];
-  const int kept = static_cast<int>(cnt) < A.max_contacts ? static_cast<int>(cnt) : A.max_contacts;
-  mfcl_mesh_result r;
-  r.hit = A.overflow[q] ? -1 : (cnt > 0 ? 1 : 0);
-  r.n_contacts = kept;
-  r.bv_tests = static_cast<int32_t>(A.bv_tests[q]);
-  r.leaf_tests = static_cast<int32_t>(A.leaves[q]);
-  out[q] = r;
+__global__ void __launch_bounds__(64) msFinishKernel(MeshShapeArgs A, mfcl_mesh_result* out) {
+  __shared__ int32_t ids[kMsMaxContacts];
+  const uint64_t q = blockIdx.x;
+  const int kept = msHeader(A, q, out), l = threadIdx.x;
+  const int32_t* in = A.tri_tmp + q * static_cast<uint64_t>(A.max_contacts);
   int32_t* o = A.tri_out + q * static_cast<uint64_t>(A.max_contacts);
-  for (int i = 1; i < kept; ++i) {
-    const int32_t key = o[i];
-    int j = i - 1;
-    while (j >= 0 && o[j] > key) {
-      o[j + 1] = o[j];
-      --j;
-    }
-    o[j + 1] = key;
-  }
-  for (int i = kept; i < A.max_contacts; ++i) o[i] = -1;
+  for (int i = l; i < kept; i += 64) ids[i] = in[i];
+  __syncthreads();
+  for (int i = l; i < kept; i += 64) o[msPlace(ids, kept, ids[i])] = ids[i];
+  for (int i = kept + l; i < A.max_contacts; i += 64) o[i] = -1;
 }
 
 __global__ void msZeroKernel(uint32_t* p, uint64_t n) {
@@ -505,23 +530,8 @@ __global__ void msZeroKernel(uint32_t* p, uint64_t n) {
   if (i < n) p[i] = 0;
 }
 
-namespace {
-struct DevAllocs {
-  std::vector<void*> p;
-  ~DevAllocs() {
-    for (void* q : p) (void)hipFree(q);
-  }
-  void* get(size_t bytes) {
-    void* q = nullptr;
-    if (hipMalloc(&q, bytes ? bytes : 8) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    p.push_back(q);
-    return q;
-  }
-};
-}  // namespace
+// Dump slots and blocks of the full-capacity pass.
+constexpr uint32_t kMsDumpSlots = 2048, kMsFullBlocks = 512;
 
 int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* shape_ids, const float* pose_m7,
                      const float* pose_s7, uint64_t n, const mfcl_request* req, mfcl_mesh_result* out,
@@ -552,19 +562,41 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
     }
   }
   const hipStream_t s = ctx->stream;
-  DevAllocs m;
-  auto* dm = static_cast<uint32_t*>(m.get(4 * n));
-  auto* ds = static_cast<uint32_t*>(m.get(4 * n));
-  auto* dpm = static_cast<float*>(m.get(28 * n));
-  auto* dps = static_cast<float*>(m.get(28 * n));
-  auto* dcnt = static_cast<uint32_t*>(m.get(4 * 4 * n));  // counts, leaves, bv tests, overflow
-  auto* dcc = static_cast<unsigned long long*>(m.get(16));  // candidate count, EPA cursor
-  auto* dout = static_cast<mfcl_mesh_result*>(m.get(sizeof(mfcl_mesh_result) * n));
-  auto* dtri = static_cast<int32_t*>(m.get(4 * n * static_cast<uint64_t>(maxc)));
-  if (!dm || !ds || !dpm || !dps || !dcnt || !dcc || !dout || !dtri) {
-    ctx->err = "out of device memory for the mesh-shape query";
-    return MFCL_E_NOMEM;
+  // the call's buffers, carved from the context's host-call workspace; the
+  // candidates, whose number is known only after the tree walk, from a
+  // workspace of their own (64 per query, grown to the exact count and rerun)
+  const uint64_t slots = n * static_cast<uint64_t>(maxc);
+  int lds_faces = std::min(std::min(req->epa_max_faces, 42), kSmallFaces);
+  while (lds_faces > 4 && 4 * epaSliceBytes<SmallMem>(lds_faces) > static_cast<size_t>(ctx->max_lds_per_block))
+    lds_faces /= 2;
+  const bool spills = pen && lds_faces < req->epa_max_faces;
+  const bool mid = req->epa_max_faces <= kMidFaces;
+  const size_t full_slice =
+      mid ? epaSliceBytes<MidMem>(req->epa_max_faces) : epaSliceBytes<LargeMem>(req->epa_max_faces);
+  const bool full_lds = full_slice <= static_cast<size_t>(ctx->max_lds_per_block);
+  const size_t arena_slice = full_lds ? 0 : arenaBytes<GlobalMem>(req->epa_max_faces);
+  const size_t b_out = pen ? sizeof(mfcl_mesh_contact) * slots : 4 * slots;
+  const size_t sizes[] = {4 * n, 4 * n, 28 * n, 28 * n, 16 * n, 64, sizeof(mfcl_mesh_result) * n, b_out, b_out,
+                          spills ? kMsDumpSlots * epaDumpBytes(lds_faces) : 0, spills ? arena_slice * kMsFullBlocks : 0};
+  constexpr int kPieces = sizeof(sizes) / sizeof(sizes[0]);
+  size_t total = 0;
+  for (size_t b : sizes) total += (b + 255) & ~static_cast<size_t>(255);
+  if (int rc = ensure(ctx, ctx->ws_io, total)) return rc;
+  char* piece[kPieces];
+  {
+    char* p = static_cast<char*>(ctx->ws_io.p);
+    for (int k = 0; k < kPieces; ++k) {
+      piece[k] = p;
+      p += (sizes[k] + 255) & ~static_cast<size_t>(255);
+    }
   }
+  auto* dm = reinterpret_cast<uint32_t*>(piece[0]);
+  auto* ds = reinterpret_cast<uint32_t*>(piece[1]);
+  auto* dpm = reinterpret_cast<float*>(piece[2]);
+  auto* dps = reinterpret_cast<float*>(piece[3]);
+  auto* dcnt = reinterpret_cast<uint32_t*>(piece[4]);            // counts, leaves, bv tests, overflow
+  auto* dcc = reinterpret_cast<unsigned long long*>(piece[5]);   // candidate count, MsCount
+  auto* dout = reinterpret_cast<mfcl_mesh_result*>(piece[6]);
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(dm, mesh_ids, 4 * n, hipMemcpyHostToDevice, s));
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(ds, shape_ids, 4 * n, hipMemcpyHostToDevice, s));
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(dpm, pose_m7, 28 * n, hipMemcpyHostToDevice, s));
@@ -588,21 +620,20 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
   A.overflow = dcnt + 3 * n;
   A.cand_count = dcc;
   A.max_contacts = maxc;
-  A.tri_out = dtri;
+  A.tri_tmp = reinterpret_cast<int32_t*>(piece[7]);
+  A.tri_out = reinterpret_cast<int32_t*>(piece[8]);
   A.gjk_max_it = req->gjk_max_iterations;
   A.gjk_tol = req->gjk_tolerance;
-  // candidates: sized for 64 per query, grown to the exact count and rerun
   uint64_t cap = std::max<uint64_t>(64 * n, 1 << 16);
   unsigned long long ncand = 0;
   for (int attempt = 0; attempt < 2; ++attempt) {
-    A.cand = static_cast<uint64_t*>(m.get(8 * cap));
-    if (!A.cand) {
-      ctx->err = "out of device memory for the mesh-shape candidates";
-      return MFCL_E_NOMEM;
-    }
+    // 8 bytes per candidate, then 4 for the restart list
+    if (int rc = ensure(ctx, ctx->ws_cand, 12 * cap)) return rc;
+    cap = std::max<uint64_t>(cap, ctx->ws_cand.bytes / 12);
+    A.cand = static_cast<uint64_t*>(ctx->ws_cand.p);
     A.cand_cap = cap;
     msZeroKernel<<<static_cast<unsigned>((4 * n + 255) / 256), 256, 0, s>>>(dcnt, 4 * n);
-    msZeroKernel<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(dcc), 2);
+    msZeroKernel<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(dcc), 16);
     msCandKernel<<<static_cast<unsigned>(n), 64, 0, s>>>(A);
     MFCL_HIP_TRY(ctx, hipGetLastError());
     MFCL_HIP_TRY(ctx, hipMemcpyAsync(&ncand, dcc, 8, hipMemcpyDeviceToHost, s));
@@ -614,54 +645,49 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
     ctx->err = "mesh-shape candidate count changed between runs";
     return MFCL_E_STATE;
   }
-  if (!pen) {
-    if (ncand)
-      msLeafKernel<<<static_cast<unsigned>((ncand * kMsGroup + 255) / 256), 256, 0, s>>>(A, ncand);
-    msFinishKernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(A, dout);
-    MFCL_HIP_TRY(ctx, hipGetLastError());
-    MFCL_HIP_TRY(ctx, hipMemcpyAsync(out, dout, sizeof(mfcl_mesh_result) * n, hipMemcpyDeviceToHost, s));
-    if (tri_ids)
-      MFCL_HIP_TRY(ctx, hipMemcpyAsync(tri_ids, dtri, 4 * n * static_cast<uint64_t>(maxc), hipMemcpyDeviceToHost, s));
-    MFCL_HIP_TRY(ctx, hipStreamSynchronize(s));
-    return MFCL_OK;
-  }
-  // penetration enabled: GJK + EPA per candidate, 4 wavefronts per block
-  if (ncand > 0xF0000000ull) {
+  if (pen && ncand > 0xF0000000ull) {
     ctx->err = "too many mesh-shape candidates for one penetration-enabled call";
     return MFCL_E_INVALID;
+  }
+  // as many candidates per wavefront as leave the chip filled a few times
+  const uint64_t waves = 64ull * static_cast<uint64_t>(ctx->n_cu);
+  const int chunk = static_cast<int>(std::min<uint64_t>(64, (ncand + waves - 1) / waves));
+  const unsigned blocks = chunk ? static_cast<unsigned>((ncand + 4ull * chunk - 1) / (4ull * chunk)) : 0;
+  if (!pen) {
+    if (ncand) msLeafKernel<<<blocks, 256, 0, s>>>(A, ncand, chunk);
+    msFinishKernel<<<static_cast<unsigned>(n), 64, 0, s>>>(A, dout);
+    MFCL_HIP_TRY(ctx, hipGetLastError());
+    MFCL_HIP_TRY(ctx, hipMemcpyAsync(out, dout, sizeof(mfcl_mesh_result) * n, hipMemcpyDeviceToHost, s));
+    if (tri_ids) MFCL_HIP_TRY(ctx, hipMemcpyAsync(tri_ids, A.tri_out, 4 * slots, hipMemcpyDeviceToHost, s));
+    MFCL_HIP_TRY(ctx, hipStreamSynchronize(s));
+    return MFCL_OK;
   }
   MsPen E;
   E.epa_max_faces = req->epa_max_faces;
   E.epa_max_it = req->epa_max_iterations;
   E.epa_tol = req->epa_tolerance;
-  int lds_faces = std::min(E.epa_max_faces, 64);
-  while (lds_faces > 4 && 4 * msSliceBytes(lds_faces) > static_cast<size_t>(ctx->max_lds_per_block)) lds_faces /= 2;
   E.cap_faces = lds_faces;
-  E.slice_bytes = msSliceBytes(lds_faces);
-  const uint64_t blocks64 = std::min<uint64_t>((ncand + 3) / 4, 2ull * static_cast<uint64_t>(ctx->n_cu));
-  const unsigned blocks = static_cast<unsigned>(std::max<uint64_t>(blocks64, 1));
-  E.arena = nullptr;
-  E.arena_slice = arenaBytes(E.epa_max_faces);
-  if (lds_faces < E.epa_max_faces) {
-    E.arena = static_cast<char*>(m.get(E.arena_slice * 4 * blocks));
-    if (!E.arena) {
-      ctx->err = "out of device memory for the mesh-shape EPA polytopes";
-      return MFCL_E_NOMEM;
-    }
+  E.slice_bytes = epaSliceBytes<SmallMem>(lds_faces);
+  E.tmp = reinterpret_cast<mfcl_mesh_contact*>(piece[7]);
+  auto* dcon = reinterpret_cast<mfcl_mesh_contact*>(piece[8]);
+  E.dumps = piece[9];
+  E.n_dumps = spills ? kMsDumpSlots : 0;
+  E.dump_bytes = epaDumpBytes(lds_faces);
+  E.redo = reinterpret_cast<uint32_t*>(A.cand + cap);
+  E.cnt = reinterpret_cast<uint32_t*>(dcc) + 2;
+  E.arena = piece[10];
+  E.arena_slice = arena_slice;
+  if (ncand) {
+    msPenKernel<<<blocks, 256, 4 * E.slice_bytes, s>>>(A, E, ncand, chunk);
+    const unsigned fb = static_cast<unsigned>(std::min<uint64_t>(kMsFullBlocks, ncand));
+    if (spills && full_lds && mid) msPenFullKernel<MidMem><<<fb, 64, full_slice, s>>>(A, E);
+    else if (spills && full_lds) msPenFullKernel<LargeMem><<<fb, 64, full_slice, s>>>(A, E);
+    else if (spills) msPenFullKernel<GlobalMem><<<fb, 64, kEpaHeadBytes, s>>>(A, E);
   }
-  E.contacts = static_cast<mfcl_mesh_contact*>(m.get(sizeof(mfcl_mesh_contact) * n * static_cast<uint64_t>(maxc)));
-  E.next = reinterpret_cast<uint32_t*>(dcc) + 2;  // the candidate counter's third word
-  if (!E.contacts) {
-    ctx->err = "out of device memory for the mesh-shape contacts";
-    return MFCL_E_NOMEM;
-  }
-  msZeroKernel<<<1, 64, 0, s>>>(E.next, 1);
-  if (ncand) msPenKernel<<<blocks, 256, 4 * E.slice_bytes, s>>>(A, E, ncand);
-  msFinishPenKernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(A, E.contacts, dout);
+  msFinishPenKernel<<<static_cast<unsigned>(n), 64, 0, s>>>(A, E.tmp, dcon, dout);
   MFCL_HIP_TRY(ctx, hipGetLastError());
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(out, dout, sizeof(mfcl_mesh_result) * n, hipMemcpyDeviceToHost, s));
-  MFCL_HIP_TRY(ctx, hipMemcpyAsync(contacts, E.contacts, sizeof(mfcl_mesh_contact) * n * static_cast<uint64_t>(maxc),
-                                   hipMemcpyDeviceToHost, s));
+  MFCL_HIP_TRY(ctx, hipMemcpyAsync(contacts, dcon, sizeof(mfcl_mesh_contact) * slots, hipMemcpyDeviceToHost, s));
   MFCL_HIP_TRY(ctx, hipStreamSynchronize(s));
   return MFCL_OK;
 }
