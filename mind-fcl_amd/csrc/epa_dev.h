@@ -236,6 +236,9 @@ struct PolyT {
   typename M::template P<EFace> F;
   typename M::template P<BorderRec> BL;  // nv records
   int nv, nf;   // slot capacities: vertices and edges nv, faces nf
+  // slots in use lie below these (the lowest free ones are taken first);
+  // those beyond are free and not initialised
+  int hv, he, hf;
   int stamp;    // creation counter
 
   MFCL_D PolyT(Base base, int cap_faces) {
@@ -246,7 +249,7 @@ struct PolyT {
     BL = (typename M::template P<BorderRec>)(base + (sizeof(EVert) + sizeof(EEdge)) * d.nv + sizeof(EFace) * d.nf);
     nv = d.nv;
     nf = d.nf;
-    stamp = 0;
+    hv = he = hf = stamp = 0;
   }
   MFCL_D d3 vloc(int i) const { return {V[i].vx, V[i].vy, V[i].vz}; }
 
@@ -257,11 +260,10 @@ struct PolyT {
   MFCL_D bool build(int n_v, int n_e, int n_f, uint64_t v0, uint64_t v1, uint64_t e0, uint64_t e1, uint64_t e2) {
     const int l = __lane_id();
     if (n_v > nv || n_e > nv || n_f > nf) return false;
-    for (int s = l; s < nv; s += 64) {
-      V[s].stamp = s < n_v ? s : -1;
-      if (s >= n_e) E[s].stamp = -1;
-    }
-    for (int s = l + n_f; s < nf; s += 64) F[s].stamp = -1;
+    if (l < n_v) V[l].stamp = l;
+    hv = n_v;
+    he = n_e;
+    hf = n_f;
     auto nib = [](uint64_t t, int k) { return static_cast<int16_t>((t >> (4 * k)) & 15u); };
     if (l < n_e) {
       auto& e = E[l];
@@ -326,7 +328,7 @@ struct PolyT {
   // vertices: order-free, so a parallel pass.
   MFCL_D bool closeFlips(d3 dir) const {
     double maxp = 0.0, minn = 0.0;
-    for (int s = __lane_id(); s < nv; s += 64) {
+    for (int s = __lane_id(); s < hv; s += 64) {
       if (V[s].stamp < 0) continue;
       const double dv = dot(vloc(s), dir);
       if (dv > maxp) maxp = dv;
@@ -356,32 +358,29 @@ struct PolyT {
     double bd = INFINITY;
     uint32_t br = 0xFFFFFFFFu;
     int bi = kNil;
+    if (!excl_vertex)
 #pragma nounroll
-    for (int s = l; s < nv; s += 64) {
+      for (int s = l; s < hv; s += 64) {
+        const int st = V[s].stamp;
+        const double d2 = sqnorm(vloc(s));
+        const uint32_t r = rankOf(1, st);
+        if (st >= 0 && better(d2, r, bd, br)) { bd = d2; br = r; bi = s; }
+      }
+#pragma nounroll
+    for (int s = l; s < he; s += 64) {
       const auto& e = E[s];
-      const int st = e.stamp, sv = V[s].stamp;
-      const double ed = e.d2;
-      const bool ein = e.in;
-      const d3 v = vloc(s);
-      if (!excl_vertex && sv >= 0) {
-        const double d2 = sqnorm(v);
-        const uint32_t r = rankOf(1, sv);
-        if (better(d2, r, bd, br)) { bd = d2; br = r; bi = s; }
-      }
-      if (st >= 0 && (excl_vertex || ein)) {
-        const uint32_t r = rankOf(2, st);
-        if (better(ed, r, bd, br)) { bd = ed; br = r; bi = s; }
-      }
+      const int st = e.stamp;
+      const double d2 = e.d2;
+      const uint32_t r = rankOf(2, st);
+      if (st >= 0 && (excl_vertex || e.in) && better(d2, r, bd, br)) { bd = d2; br = r; bi = s; }
     }
 #pragma nounroll
-    for (int s = l; s < nf; s += 64) {
+    for (int s = l; s < hf; s += 64) {
       const auto& f = F[s];
       const int st = f.stamp;
-      const double fd = f.d2;
-      if (st >= 0 && f.in) {
-        const uint32_t r = rankOf(3, st);
-        if (better(fd, r, bd, br)) { bd = fd; br = r; bi = s; }
-      }
+      const double d2 = f.d2;
+      const uint32_t r = rankOf(3, st);
+      if (st >= 0 && f.in && better(d2, r, bd, br)) { bd = d2; br = r; bi = s; }
     }
     // the smallest d2 over the wavefront, then the first rank among the
     // lanes that hold it (usually one)
@@ -446,12 +445,15 @@ struct PolyT {
   MFCL_D int addVertex(d3 v, d3 d, int h0, int h1) {
     const int l = __lane_id();
     int i = kNil;
-    for (int base = 0; base < nv && i == kNil; base += 64) {
+    for (int base = 0; base < hv && i == kNil; base += 64) {
       const int s = base + l;
-      const unsigned long long m = __ballot(s < nv && V[s].stamp < 0);
+      const unsigned long long m = __ballot(s < hv && V[s].stamp < 0);
       if (m) i = base + __builtin_ctzll(m);
     }
-    if (i == kNil) return kNil;
+    if (i == kNil) {
+      if (hv >= nv) return kNil;
+      i = hv++;
+    }
     auto& x = V[i];
     x.vx = v.x; x.vy = v.y; x.vz = v.z;
     x.dx = d.x; x.dy = d.y; x.dz = d.z;
@@ -479,7 +481,7 @@ struct PolyT {
     } else {
       double maxp = 0.0, minn = 0.0;
 #pragma nounroll
-      for (int s = 0; s < nv; ++s) {
+      for (int s = 0; s < hv; ++s) {
         if (V[s].stamp < 0) continue;
         const double dv = dot(vloc(s), dir);
         if (dv > maxp) maxp = dv;
@@ -500,16 +502,13 @@ struct PolyT {
   // the visible set as bit masks: every face's test of nv runs first, all at
   // once (with the normals that the faces keep, a dot product); the fill's
   // rounds are then a few scalar instructions each.
-  struct Mask {
-    unsigned long long w[M::kWords > 0 ? M::kWords : 1];
-    MFCL_D bool has(int k) const {
-      if (k == kNil) return false;
-      unsigned long long m = w[0];
-#pragma unroll
-      for (int i = 1; i < M::kWords; ++i) m = (k >> 6) == i ? w[i] : m;
-      return ((m >> (k & 63)) & 1ull) != 0;
-    }
-  };
+  // One word: the mask itself; more: a flag per face (a lookup in several
+  // words costs more instructions than the LDS read).
+  MFCL_D bool isVisible(unsigned long long mask, int k) const {
+    if (k == kNil) return false;
+    if constexpr (M::kWords == 1) return ((mask >> (k & 63)) & 1ull) != 0;
+    else return F[k].vis == kVisible;
+  }
   MFCL_D int expandMask(d3 nv_, d3 nd, int nh0, int nh1, int start, bool may_spill) {
     constexpr int W = M::kWords;
     const int l = __lane_id();
@@ -519,17 +518,19 @@ struct PolyT {
 #pragma unroll
     for (int i = 0; i < W; ++i) {
       const int s = 64 * i + l;
-      live[i] = s < nf && F[s < nf ? s : 0].stamp >= 0;
-      out[i] = open[i] = false;
+      live[i] = out[i] = open[i] = false;
       g[i][0] = g[i][1] = g[i][2] = kNil;
+      if (64 * i >= hf) continue;
+      live[i] = s < hf && F[s < hf ? s : 0].stamp >= 0;
       int cls = kNormalOut;
       d3 n = {0, 0, 0}, a = {0, 0, 0};
       if (live[i]) {
-        const auto& f = F[s];
+        auto& f = F[s];
         const int es[3] = {f.e0, f.e1, f.e2};
         n = d3{f.nx, f.ny, f.nz};
         cls = f.cls;
         a = vloc(f.a);
+        if (W > 1) f.vis = kFUnknown;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
           const int x = E[es[k]].f0, y = E[es[k]].f1;
@@ -545,54 +546,69 @@ struct PolyT {
       // epa_polytope_expand.hpp:12-30
       out[i] = live[i] && (cls == kNormalNone || dot(n, nv_ - a) >= 0.0);
     }
-    Mask vis;
-#pragma unroll
-    for (int i = 0; i < W; ++i) vis.w[i] = (start >> 6) == i ? 1ull << (start & 63) : 0ull;
-    while (true) {
-      unsigned long long any = 0;
-      Mask more;
-#pragma unroll
-      for (int i = 0; i < W; ++i) {
-        more.w[i] = __ballot(out[i] && (vis.has(g[i][0]) || vis.has(g[i][1]) || vis.has(g[i][2]))) & ~vis.w[i];
-        any |= more.w[i];
+    unsigned long long vis = 1ull << (start & 63);
+    bool mine[W];
+    if constexpr (W == 1) {
+      while (true) {
+        const unsigned long long more =
+            __ballot(out[0] && (isVisible(vis, g[0][0]) || isVisible(vis, g[0][1]) || isVisible(vis, g[0][2]))) & ~vis;
+        if (!more) break;
+        vis |= more;
       }
-      if (!any) break;
+      mine[0] = live[0] && ((vis >> l) & 1ull) != 0;
+    } else {
+      M::sync();
+      F[start].vis = kVisible;
+      M::sync();
 #pragma unroll
-      for (int i = 0; i < W; ++i) vis.w[i] |= more.w[i];
+      for (int i = 0; i < W; ++i) mine[i] = 64 * i + l == start;
+      while (true) {
+        bool grew = false;
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          if (64 * i >= hf) continue;
+          if (out[i] && !mine[i] && (isVisible(0, g[i][0]) || isVisible(0, g[i][1]) || isVisible(0, g[i][2]))) {
+            mine[i] = grew = true;
+            F[64 * i + l].vis = kVisible;
+          }
+        }
+        M::sync();
+        if (!anyLane(grew)) break;
+      }
     }
     bool bad = false;
-    int free_f = 0;
-    bool mine[W];
+    int below_f = 0;  // free face slots below hf, those of the visible faces included
 #pragma unroll
     for (int i = 0; i < W; ++i) {
-      mine[i] = live[i] && ((vis.w[i] >> l) & 1ull) != 0;
       bad = bad || (mine[i] && open[i]);
-      free_f += __popcll(__ballot(64 * i + l < nf && (!live[i] || mine[i])));
+      if (64 * i < hf) below_f += __popcll(__ballot(64 * i + l < hf && (!live[i] || mine[i])));
     }
     // an open edge on a visible face is a malformed polytope
     if (anyLane(bad)) return 1;
     // edge marks from the face classes; border edges compacted into BL
-    int nb = 0, free_e = 0, free_v = 0;
-    for (int base = 0; base < nv; base += 64) {
+    int nb = 0, below_e = 0, free_v = nv - hv;
+    for (int base = 0; base < he; base += 64) {
       const int s = base + l;
-      bool border = false, fr = false, fv = false;
-      if (s < nv) {
+      bool border = false, fr = false;
+      if (s < he) {
         auto& e = E[s];
         const bool alive = e.stamp >= 0;
-        const bool a = vis.has(e.f0), b = vis.has(e.f1);
-        border = alive && a != b;
+        const bool a = alive && isVisible(vis, e.f0), b = alive && isVisible(vis, e.f1);
+        border = a != b;
         fr = !alive || (a && b);
-        fv = V[s].stamp < 0;
-        e.vis = border ? kBorder : (alive && a ? kInternal : kUnknown);
-        V[s].remove = 1;
-        V[s].new_edge = kNil;
+        e.vis = border ? kBorder : (a ? kInternal : kUnknown);
       }
       const unsigned long long m = __ballot(border);
       if (border) BL[nb + __popcll(m & below)].e = static_cast<int16_t>(s);
       nb += __popcll(m);
-      free_e += __popcll(__ballot(fr));
-      free_v += __popcll(__ballot(fv));
+      below_e += __popcll(__ballot(fr));
     }
+    for (int base = 0; base < hv; base += 64) {
+      const int s = base + l;
+      if (s < hv) V[s].remove = 1;
+      free_v += __popcll(__ballot(s < hv && V[s < hv ? s : 0].stamp < 0));
+    }
+    const int free_e = below_e + nv - he, free_f = below_f + nf - hf;
     // Whether the expansion certainly fits: one vertex, at most two new
     // edges per border edge and one face per border edge must find slots.
     // Vertices that the expansion removes are not counted as free.
@@ -603,7 +619,7 @@ struct PolyT {
 #pragma unroll
     for (int i = 0; i < W; ++i)
       if (mine[i]) F[64 * i + l].stamp = -1;
-    for (int s = l; s < nv; s += 64) {
+    for (int s = l; s < he; s += 64) {
       auto& e = E[s];
       if (e.stamp < 0) continue;
       if (e.vis == kInternal) {
@@ -613,13 +629,13 @@ struct PolyT {
       V[e.v0].remove = 0;
       V[e.v1].remove = 0;
       if (e.vis == kBorder) {
-        if (vis.has(e.f0)) e.f0 = e.f1;
+        if (isVisible(vis, e.f0)) e.f0 = e.f1;
         e.f1 = kNil;
       }
     }
     M::sync();
-    for (int s = l; s < nv; s += 64)
-      if (V[s].stamp >= 0 && V[s].remove) V[s].stamp = -1;
+    for (int s = l; s < hv; s += 64)
+      if (V[s].remove) V[s].stamp = -1;
     M::sync();
     const int nvi = addVertex(nv_, nd, nh0, nh1);
     if (nvi == kNil) return 2;
@@ -657,9 +673,11 @@ struct PolyT {
     const int new_edges = total - nb;
     if (new_edges > free_e || nb > free_f) return 2;
     // the free slot lists (before any slot is taken)
-    for (int base = 0, c = 0; base < nv && c < new_edges; base += 64) {
+    for (int k = below_e + l; k < new_edges; k += 64) BL[k].fe = static_cast<int16_t>(he + k - below_e);
+    for (int k = below_f + l; k < nb; k += 64) BL[k].ff = static_cast<int16_t>(hf + k - below_f);
+    for (int base = 0, c = 0; base < he && c < new_edges; base += 64) {
       const int s = base + l;
-      const bool fr = s < nv && E[s].stamp < 0;
+      const bool fr = s < he && E[s < he ? s : 0].stamp < 0;
       const unsigned long long m = __ballot(fr);
       const int pos = c + __popcll(m & below);
       if (fr && pos < new_edges) BL[pos].fe = static_cast<int16_t>(s);
@@ -669,7 +687,8 @@ struct PolyT {
       int c = 0;
 #pragma unroll
       for (int i = 0; i < W; ++i) {
-        const bool fr = 64 * i + l < nf && (!live[i] || mine[i]);
+        if (64 * i >= hf) continue;
+        const bool fr = 64 * i + l < hf && (!live[i] || mine[i]);
         const unsigned long long m = __ballot(fr);
         const int pos = c + __popcll(m & below);
         if (fr && pos < nb) BL[pos].ff = static_cast<int16_t>(64 * i + l);
@@ -720,6 +739,8 @@ struct PolyT {
       if (t1 == 0) E[ne1].f0 = slot; else E[ne1].f1 = slot;
     }
     stamp += total;
+    he += max(0, new_edges - below_e);
+    hf += max(0, nb - below_f);
     M::sync();
     return anyLane(clash) ? 2 : 0;
   }
@@ -728,20 +749,17 @@ struct PolyT {
   // border edges in BL (polytopes beyond kSmallFaces).
   MFCL_D int expandLarge(d3 nv_, d3 nd, int nh0, int nh1, int start) {
     const int l = __lane_id();
-    for (int s = l; s < nv; s += 64) {
-      V[s].remove = 1;
-      V[s].new_edge = kNil;
-      E[s].vis = kUnknown;
-    }
+    for (int s = l; s < hv; s += 64) V[s].remove = 1;
+    for (int s = l; s < he; s += 64) E[s].vis = kUnknown;
     // a face that does not see the new vertex is never visible, unless the
     // fill starts from it
-    for (int s = l; s < nf; s += 64) F[s].vis = F[s].stamp >= 0 && outsideLane(s, nv_) ? kFUnknown : kHidden;
+    for (int s = l; s < hf; s += 64) F[s].vis = F[s].stamp >= 0 && outsideLane(s, nv_) ? kFUnknown : kHidden;
     M::sync();
     F[start].vis = kVisible;
     M::sync();
     while (true) {
       bool changed = false;
-      for (int s = l; s < nf; s += 64) {
+      for (int s = l; s < hf; s += 64) {
         const auto& f = F[s];
         if (f.stamp < 0 || f.vis != kFUnknown) continue;
         const int16_t es[3] = {f.e0, f.e1, f.e2};
@@ -760,7 +778,7 @@ struct PolyT {
     }
     // an open edge on a visible face is a malformed polytope
     bool bad = false;
-    for (int s = l; s < nf; s += 64) {
+    for (int s = l; s < hf; s += 64) {
       const auto& f = F[s];
       if (f.stamp < 0 || f.vis != kVisible) continue;
       const int16_t es[3] = {f.e0, f.e1, f.e2};
@@ -772,7 +790,7 @@ struct PolyT {
     }
     if (anyLane(bad)) return 1;
     // edge marks from the final face classes
-    for (int s = l; s < nv; s += 64) {
+    for (int s = l; s < he; s += 64) {
       auto& e = E[s];
       if (e.stamp < 0) continue;
       const bool v0 = e.f0 != kNil && F[e.f0].vis == kVisible;
@@ -786,7 +804,7 @@ struct PolyT {
       }
     }
     M::sync();
-    for (int s = l; s < nv; s += 64) {
+    for (int s = l; s < he; s += 64) {
       const auto& e = E[s];
       if (e.stamp < 0 || e.vis == kInternal) continue;
       V[e.v0].remove = 0;
@@ -795,12 +813,12 @@ struct PolyT {
     M::sync();
     // drop the visible faces, the internal edges and the vertices left
     // without a non-internal edge
-    for (int s = l; s < nf; s += 64)
+    for (int s = l; s < hf; s += 64)
       if (F[s].stamp >= 0 && F[s].vis == kVisible) F[s].stamp = -1;
-    for (int s = l; s < nv; s += 64) {
-      if (E[s].stamp >= 0 && E[s].vis == kInternal) E[s].stamp = -1;
-      if (V[s].stamp >= 0 && V[s].remove) V[s].stamp = -1;
-    }
+    for (int s = l; s < he; s += 64)
+      if (E[s].vis == kInternal) E[s].stamp = -1;
+    for (int s = l; s < hv; s += 64)
+      if (V[s].remove) V[s].stamp = -1;
     M::sync();
     const int nvi = addVertex(nv_, nd, nh0, nh1);
     if (nvi == kNil) return 2;
@@ -821,9 +839,9 @@ struct PolyT {
     const int l = __lane_id();
     const unsigned long long below = (1ull << l) - 1;
     int nb = 0;
-    for (int base = 0; base < nv; base += 64) {
+    for (int base = 0; base < he; base += 64) {
       const int s = base + l;
-      const bool isb = s < nv && E[s].stamp >= 0 && E[s].vis == kBorder;
+      const bool isb = s < he && E[s].stamp >= 0 && E[s].vis == kBorder;
       const unsigned long long m = __ballot(isb);
       if (isb) BL[nb + __popcll(m & below)].e = static_cast<int16_t>(s);
       nb += __popcll(m);
@@ -865,25 +883,27 @@ struct PolyT {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) new_edges += __shfl_xor(new_edges, off);
     // capacity
-    int free_e = 0, free_f = 0;
-    for (int base = 0; base < nv; base += 64) free_e += __popcll(__ballot(base + l < nv && E[base + l].stamp < 0));
-    for (int base = 0; base < nf; base += 64) free_f += __popcll(__ballot(base + l < nf && F[base + l].stamp < 0));
+    int below_e = 0, below_f = 0;
+    for (int base = 0; base < he; base += 64) below_e += __popcll(__ballot(base + l < he && E[base + l].stamp < 0));
+    for (int base = 0; base < hf; base += 64) below_f += __popcll(__ballot(base + l < hf && F[base + l].stamp < 0));
     new_edges = __builtin_amdgcn_readfirstlane(new_edges);
-    if (new_edges > free_e || nb > free_f) return 2;
+    if (new_edges > below_e + nv - he || nb > below_f + nf - hf) return 2;
     // the free slot lists (before any slot is taken)
     {
+      for (int k = below_e + l; k < new_edges; k += 64) BL[k].fe = static_cast<int16_t>(he + k - below_e);
+      for (int k = below_f + l; k < nb; k += 64) BL[k].ff = static_cast<int16_t>(hf + k - below_f);
       int ce = 0, cf = 0;
-      for (int base = 0; base < nv; base += 64) {
+      for (int base = 0; base < he; base += 64) {
         const int s = base + l;
-        const bool fr = s < nv && E[s].stamp < 0;
+        const bool fr = s < he && E[s].stamp < 0;
         const unsigned long long m = __ballot(fr);
         const int pos = ce + __popcll(m & below);
         if (fr && pos < new_edges) BL[pos].fe = static_cast<int16_t>(s);
         ce += __popcll(m);
       }
-      for (int base = 0; base < nf; base += 64) {
+      for (int base = 0; base < hf; base += 64) {
         const int s = base + l;
-        const bool fr = s < nf && F[s].stamp < 0;
+        const bool fr = s < hf && F[s].stamp < 0;
         const unsigned long long m = __ballot(fr);
         const int pos = cf + __popcll(m & below);
         if (fr && pos < nb) BL[pos].ff = static_cast<int16_t>(s);
@@ -946,6 +966,8 @@ struct PolyT {
       if (bj.t1 == 0) x1.f0 = slot; else x1.f1 = slot;
     }
     stamp += new_edges + nb;
+    he += max(0, new_edges - below_e);
+    hf += max(0, nb - below_f);
     M::sync();
     return anyLane(clash) ? 2 : 0;
   }
@@ -963,7 +985,7 @@ struct RawF {
 // Where a pair that outgrows its polytope continues: the expansion it is at.
 struct EpaResume {
   d3 nv, nd;
-  int it, stamp, nh0, nh1, start, item;
+  int it, stamp, nh0, nh1, start, item, hv, he, hf, pad;
 };
 // The result in shape-0 frame (status: EpaStatus, or kEpaSpill).
 struct EpaOut {
@@ -1020,9 +1042,9 @@ MFCL_D bool buildTetra(PolyT<M>& P) {
   return P.build(4, 6, 4, 0x333210ull, 0x210021ull, 0x5430ull, 0x3541ull, 0x2102ull);
 }
 
-// simplexToPolytope's status: a negative value is a failure, kS2pTouching
-// leaves the points in out, any other is the polytope's creation counter.
-constexpr int kS2pFailed = -1, kS2pTouching = 0;
+// simplexToPolytope's status: failed, touching (the points in out), or the
+// initial polytope that was built.
+constexpr int kS2pFailed = -1, kS2pTouching = 0, kS2pTetra = 4, kS2pOcta = 6;
 
 MFCL_D int touchingPoint(MinkW& md, d3 d, MFCL_LDS EpaLds* L) {
   const WaveSup a = md.sup(d);
@@ -1063,7 +1085,7 @@ __device__ __attribute__((noinline)) int s2p3(MFCL_LDS EpaLds* L, typename M::te
       putVertex(P, 1, vb);
       putVertex(P, 2, vc);
       putVertex(P, 3, up ? d0 : d1, up ? n : dir1);
-      if (buildTetra(P)) r = P.stamp;
+      if (buildTetra(P)) r = kS2pTetra;
     }
   }
   L->out.scanned += md.scanned;
@@ -1123,7 +1145,7 @@ MFCL_D int s2p2Run(PolyT<M>& P, MinkW& md, MFCL_LDS EpaLds* L, double thr) {
   if (!room) return kS2pFailed;
   M::sync();
   P.build(6, 12, 8, 0x555544443210ull, 0x321032100321ull, 0xBA987654ull, 0x8BA94765ull, 0x32103210ull);
-  return P.stamp;
+  return kS2pOcta;
 }
 template <class M>
 __device__ __attribute__((noinline)) int s2p2(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int cap_faces,
@@ -1164,7 +1186,7 @@ MFCL_D int simplexToPolytope(PolyT<M>& P, MinkW& md, MFCL_LDS EpaLds* L, typenam
   putVertex(P, 1, s.b);
   putVertex(P, 2, s.c);
   putVertex(P, 3, s.e);
-  return buildTetra(P) ? P.stamp : kS2pFailed;
+  return buildTetra(P) ? kS2pTetra : kS2pFailed;
 }
 
 // The closest feature's record, one word or double per lane.
@@ -1282,6 +1304,9 @@ __device__ __attribute__((noinline)) int epaRun(MFCL_LDS EpaLds* L, typename M::
     nh0 = __builtin_amdgcn_readfirstlane(L->res.nh0);
     nh1 = __builtin_amdgcn_readfirstlane(L->res.nh1);
     P.stamp = __builtin_amdgcn_readfirstlane(L->res.stamp);
+    P.hv = __builtin_amdgcn_readfirstlane(L->res.hv);
+    P.he = __builtin_amdgcn_readfirstlane(L->res.he);
+    P.hf = __builtin_amdgcn_readfirstlane(L->res.hf);
     nv = ldsGet(L->res.nv);
     nd = ldsGet(L->res.nd);
   } else {
@@ -1290,7 +1315,11 @@ __device__ __attribute__((noinline)) int epaRun(MFCL_LDS EpaLds* L, typename M::
     md.scanned = 0;
     if (s2p < 0) return kEpaFailed;
     if (s2p == kS2pTouching) return kEpaTouching;
-    P.stamp = s2p;
+    // (the octahedron's and the triangle's builders work on copies of P)
+    P.hv = s2p;
+    P.he = s2p == kS2pTetra ? 6 : 12;
+    P.hf = s2p == kS2pTetra ? 4 : 8;
+    P.stamp = P.hv + P.he + P.hf;
   }
   bool pending = resume;
   while (true) {
@@ -1376,6 +1405,9 @@ __device__ __attribute__((noinline)) int epaRun(MFCL_LDS EpaLds* L, typename M::
       ldsSet(L->res.nd, nd);
       L->res.it = it;
       L->res.stamp = P.stamp;
+      L->res.hv = P.hv;
+      L->res.he = P.he;
+      L->res.hf = P.hf;
       L->res.nh0 = nh0;
       L->res.nh1 = nh1;
       L->res.start = start;
@@ -1449,8 +1481,6 @@ MFCL_D void epaLoad(MFCL_LDS EpaLds* L, typename M::template P<char> arena, int 
   copyRecs<S::EEdge>(P.E, src, sd.nv);
   src += sizeof(S::EEdge) * sd.nv;
   copyRecs<S::EFace>(P.F, src, sd.nf);
-  for (int s = sd.nv + static_cast<int>(__lane_id()); s < P.nv; s += 64) P.V[s].stamp = P.E[s].stamp = -1;
-  for (int s = sd.nf + static_cast<int>(__lane_id()); s < P.nf; s += 64) P.F[s].stamp = -1;
   M::sync();
   ldsSync();
 }
