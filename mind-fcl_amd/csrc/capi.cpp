@@ -293,7 +293,7 @@ int mfcl_tune(mfcl_ctx* ctx, int32_t knob, int32_t value) {
       ctx->tune.lane_refill = value;
       return MFCL_OK;
     case MFCL_TUNE_MLP_WAVES:
-      if (value != 4 && value != 8 && value != 16) break;
+      if (value != 0 && value != 4 && value != 8 && value != 16) break;
       ctx->tune.mlp_waves = value;
       return MFCL_OK;
     case MFCL_TUNE_MESH_STACK:

@@ -44,11 +44,9 @@ struct MlpState {
   float* m{nullptr};
   float* v{nullptr};
   float* loss{nullptr};
-  void* wbuf{nullptr};     // BF16 copies of W (forward) and W^T (backward)
-  __bf16 *w1{nullptr}, *w2{nullptr}, *w3{nullptr}, *w4{nullptr};
-  __bf16 *w1t{nullptr}, *w2t{nullptr}, *w3t{nullptr}, *w4t{nullptr};
-  DevBuf ws;               // activations
-  void* pack{nullptr};     // fused-inference weight image (BF16, K-permuted) + biases
+  DevBuf ws;               // a training step's partial gradients, one set per block
+  uint64_t ws_rows{0};     // rows the workspace was reserved for
+  void* pack{nullptr};     // BF16 weight images in the products' order (forward, transposed), then the biases
   int step{0};
 };
 
@@ -109,7 +107,7 @@ struct mfcl_ctx {
     int epa_overflow_waves{512};   // persistent wavefronts (one per block) for overflow pairs
     int mesh_blocks_per_cu{3};  // persistent mesh-traversal blocks (4 waves, one query each) per CU
     int mesh_stack{16384};      // node-pair stack entries per wavefront
-    int mlp_waves{8};           // wavefronts per block of the fused warm-start inference
+    int mlp_waves{0};           // wavefronts per block of the fused warm-start inference (0: by batch size)
     int lane_refill{48};        // lane kernel: 0 one pair per lane; k > 0 refill lanes when <= k run
   } tune;
   std::string err;

@@ -7,15 +7,15 @@
 // (GJKSolver::gjk_guess, include/fcl/narrowphase/detail/gjk_solver.h:140-163);
 // the exact algorithm still decides every result.
 //
-// Every product runs on the MFMA units as BF16 x BF16 -> FP32 through one
-// hand-written kernel, C[M][N] = A[M][K] . B[N][K]^T with both operands
-// K-contiguous (v_mfma_f32_32x32x16_bf16: one 32x32 tile per wavefront,
-// split-K with FP32 atomics for the weight gradients).  Activations are
-// sample-major; the epilogues also write the transposed copies that the
-// weight-gradient products read.  Training keeps FP32 master weights with
-// Adam; BF16 copies of W and W^T feed the forward and backward products.
+// Every product runs on the MFMA units as BF16 x BF16 -> FP32
+// (v_mfma_f32_32x32x16_bf16), each wavefront carrying 32 rows through the
+// whole network with its activations in registers: inference and training
+// write no activation to memory.  Training keeps FP32 master weights with
+// Adam; BF16 images of the weights, in the order the products read them,
+// are refreshed after each update.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -32,105 +32,61 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBlk = 256;
 
-// ------------------------------------------------------------------ GEMM
-enum Epi : int {
-  kEpiStore = 0,     // C (FP32, row-major ldc); atomic add when split over K
-  kEpiBiasGelu = 1,  // Z = C + b (FP32), H = gelu(Z) (BF16), H^T (BF16)
-  kEpiBias = 2,      // Y = C + b (FP32)
-  kEpiGeluGrad = 3,  // dZ = C * gelu'(Z) -> BF16 and its transpose
-  kEpiGelu = 4,      // H = gelu(C + b) (BF16 only: inference)
-};
-
-struct EpiArgs {
-  float* c;          // kEpiStore / kEpiBias / kEpiBiasGelu(Z)
-  int ldc;
-  const float* bias;
-  const float* z;    // kEpiGeluGrad: saved pre-activations, row-major ldc
-  __bf16* h;         // BF16 output, row-major ldc
-  __bf16* ht;        // BF16 transposed output, row-major ldt
-  int ldt;
-  int atomic;        // kEpiStore: accumulate with atomics
-};
-
-__device__ __forceinline__ float geluF(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float geluGradF(float x) {
-  const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-  const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
-  return cdf + x * pdf;
+// GELU from the normal distribution's tail q(t) = Phi(-t), t = |x|: log2 q is
+// smooth, and takes a polynomial of degree 10 (least squares, reweighted
+// towards the largest error in q).  No branch: erff's two ranges both ran for
+// every value (the lanes differ), and took most of the inference kernel.
+// Largest error over [-12, 12] against 64 bits: GELU 1.2e-7 (with erff
+// 2.4e-7), its derivative 1.3e-7 (1.4e-7).
+__device__ __forceinline__ float normalTail(float x) {
+  const float t = fabsf(x);
+  float p = -1.339073474e-08f;
+  p = __builtin_fmaf(p, t, 5.026773238e-07f);
+  p = __builtin_fmaf(p, t, -7.691206520e-06f);
+  p = __builtin_fmaf(p, t, 6.081214087e-05f);
+  p = __builtin_fmaf(p, t, -2.368241694e-04f);
+  p = __builtin_fmaf(p, t, -6.996445154e-05f);
+  p = __builtin_fmaf(p, t, 7.014930714e-03f);
+  p = __builtin_fmaf(p, t, -5.247886106e-02f);
+  p = __builtin_fmaf(p, t, -4.592103362e-01f);
+  p = __builtin_fmaf(p, t, -1.151105285e+00f);
+  p = __builtin_fmaf(p, t, -1.0f);
+  return __builtin_amdgcn_exp2f(p);
 }
-
-// One wavefront per 32x32 output tile; blockIdx.y selects the K chunk.
-// Register layout of the 32x32 accumulator (16 FP32 per lane):
-//   acc[r] = C[m0 + 8 (r / 4) + 4 (lane / 32) + r % 4][n0 + lane % 32].
-template <int EPI>
-__global__ void __launch_bounds__(kBlk) gemmNT(const __bf16* __restrict__ A, int lda, const __bf16* __restrict__ B,
-                                               int ldb, int M, int N, int K, int kchunk, EpiArgs e) {
-  const int lane = threadIdx.x & 63;
-  const int tiles_n = N / 32;
-  const int tile = blockIdx.x * (kBlk / 64) + threadIdx.x / 64;
-  if (tile >= (M / 32) * tiles_n) return;
-  const int m0 = (tile / tiles_n) * 32, n0 = (tile % tiles_n) * 32;
-  const int kb = blockIdx.y * kchunk;
-  const int ke = kb + kchunk < K ? kb + kchunk : K;
-  const int h = lane >> 5, r32 = lane & 31;
-  const __bf16* pa = A + static_cast<size_t>(m0 + r32) * lda + h * 8;
-  const __bf16* pb = B + static_cast<size_t>(n0 + r32) * ldb + h * 8;
-  f32x16 acc = {};
-  for (int k = kb; k < ke; k += 16) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + k);
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(pb + k);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  const int n = n0 + r32;
+// x Phi(x) = max(x, 0) - |x| q
+__device__ __forceinline__ float geluF(float x, float q) { return __builtin_fmaf(-fabsf(x), q, fmaxf(x, 0.f)); }
+__device__ __forceinline__ float geluF(float x) { return geluF(x, normalTail(x)); }
+// GELU's derivative Phi(x) + x phi(x)
+__device__ __forceinline__ float geluGradF(float x, float q) {
+  return __builtin_fmaf(x * 0.39894228040143268f, __builtin_amdgcn_exp2f(x * x * -0.72134752044448170f),
+                        x > 0.f ? 1.f - q : q);
+}
+// The 16 accumulators of unit tile t start from the units' biases.
+__device__ __forceinline__ f32x16 biasTile(const float* bias, int t, int h) {
+  f32x16 acc;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + 8 * (r / 4) + 4 * h + (r % 4);
-    const float c = acc[r];
-    const size_t o = static_cast<size_t>(m) * e.ldc + n;
-    if constexpr (EPI == kEpiStore) {
-      if (e.atomic) atomicAdd(&e.c[o], c);
-      else e.c[o] = c;
-    } else if constexpr (EPI == kEpiBias) {
-      e.c[o] = c + e.bias[n];
-    } else if constexpr (EPI == kEpiBiasGelu) {
-      const float z = c + e.bias[n];
-      e.c[o] = z;
-      const __bf16 hv = static_cast<__bf16>(geluF(z));
-      e.h[o] = hv;
-      e.ht[static_cast<size_t>(n) * e.ldt + m] = hv;
-    } else if constexpr (EPI == kEpiGelu) {
-      e.h[o] = static_cast<__bf16>(geluF(c + e.bias[n]));
-    } else {  // kEpiGeluGrad
-      const __bf16 g = static_cast<__bf16>(c * geluGradF(e.z[o]));
-      e.h[o] = g;
-      e.ht[static_cast<size_t>(n) * e.ldt + m] = g;
-    }
+  for (int q = 0; q < 4; ++q) {
+    const float4 b = *reinterpret_cast<const float4*>(bias + 32 * t + 8 * q + 4 * h);
+    acc[4 * q] = b.x;
+    acc[4 * q + 1] = b.y;
+    acc[4 * q + 2] = b.z;
+    acc[4 * q + 3] = b.w;
   }
-}
-
-template <int EPI>
-static void launchGemm(const __bf16* A, int lda, const __bf16* B, int ldb, int M, int N, int K, int ksplit,
-                       const EpiArgs& e, hipStream_t s) {
-  const int tiles = (M / 32) * (N / 32);
-  const int kchunk = ((K / ksplit + 15) / 16) * 16;
-  const int kz = (K + kchunk - 1) / kchunk;
-  dim3 grid((tiles + kBlk / 64 - 1) / (kBlk / 64), kz);
-  gemmNT<EPI><<<grid, kBlk, 0, s>>>(A, lda, B, ldb, M, N, K, kchunk, e);
+  return acc;
 }
 
 // ---------------------------------------------------------------- features
 // Per pair: relative translation of b in a's frame (3), relative rotation
 // quaternion (4, w >= 0), descriptors of a and b (16 + 16); columns 39..63
-// are zero.  Written as BF16 rows of 64 (and optionally the transpose).
+// are zero.
 __global__ void __launch_bounds__(kBlk) featureKernel(const uint32_t* pa, const uint32_t* pb, const float* posea,
                                                       const float* poseb, const float* desc, uint32_t n_shapes,
-                                                      uint64_t n, uint64_t n_pad, __bf16* X, __bf16* XT,
-                                                      float* xf) {
+                                                      uint64_t n, float* xf) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n_pad) return;
+  if (i >= n) return;
   float f[kMlpInPad];
   for (int k = 0; k < kMlpInPad; ++k) f[k] = 0.f;
-  if (i < n && pa[i] < n_shapes && pb[i] < n_shapes) {
+  if (pa[i] < n_shapes && pb[i] < n_shapes) {
     const float* A = posea + 7 * i;
     const float* B = poseb + 7 * i;
     float qa[4] = {A[3], A[4], A[5], A[6]}, qb[4] = {B[3], B[4], B[5], B[6]};
@@ -155,71 +111,7 @@ __global__ void __launch_bounds__(kBlk) featureKernel(const uint32_t* pa, const 
     const float* db = desc + 16 * static_cast<size_t>(pb[i]);
     for (int k = 0; k < 16; ++k) { f[7 + k] = da[k]; f[23 + k] = db[k]; }
   }
-  for (int k = 0; k < kMlpInPad; ++k) {
-    const __bf16 v = static_cast<__bf16>(f[k]);
-    if (X) X[i * kMlpInPad + k] = v;
-    if (XT) XT[static_cast<size_t>(k) * n_pad + i] = v;
-    if (xf) xf[i * kMlpInPad + k] = f[k];
-  }
-}
-
-// ------------------------------------------------------------------ loss
-// L = mean over valid rows of (1 - cos(y[0:3], t[0:3])) + wd (y3 - t3)^2;
-// rows with t = 0 direction are masked.  Writes dY (BF16, rows of 32; only
-// the first 4 columns non-zero) and its transpose.
-__global__ void __launch_bounds__(kBlk) lossKernel(const float* Y, const float* T, uint64_t n, uint64_t n_pad,
-                                                   float inv_count, float wd, __bf16* dY, __bf16* dYT,
-                                                   float* loss_sum) {
-  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  float g[4] = {0, 0, 0, 0};
-  float l = 0.f;
-  if (i < n) {
-    const float* y = Y + i * kMlpOutPad;
-    const float* t = T + 4 * i;
-    const float tn = sqrtf(t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
-    if (tn > 0.f) {
-      const float yn = fmaxf(sqrtf(y[0] * y[0] + y[1] * y[1] + y[2] * y[2]), 1e-12f);
-      const float c = (y[0] * t[0] + y[1] * t[1] + y[2] * t[2]) / (yn * tn);
-      l = 1.f - c;
-      for (int k = 0; k < 3; ++k) g[k] = -(t[k] / tn - c * y[k] / yn) / yn * inv_count;
-      const float e = y[3] - t[3];
-      l += wd * e * e;
-      g[3] = 2.f * wd * e * inv_count;
-    }
-  }
-  if (i < n_pad) {
-    for (int k = 0; k < kMlpOutPad; ++k) {
-      const __bf16 v = static_cast<__bf16>(k < 4 ? g[k] : 0.f);
-      dY[i * kMlpOutPad + k] = v;
-      dYT[static_cast<size_t>(k) * n_pad + i] = v;
-    }
-  }
-  // block reduction of the loss, one atomic per block
-  __shared__ float red[kBlk / 64];
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int w = 0; w < kBlk / 64; ++w) s += red[w];
-    atomicAdd(loss_sum, s * inv_count);
-  }
-}
-
-// Row sums of a BF16 matrix [rows][n] (bias gradients from dZ^T).
-__global__ void __launch_bounds__(kBlk) rowSumKernel(const __bf16* AT, uint64_t n, float* out) {
-  const int row = blockIdx.x;
-  float s = 0.f;
-  for (uint64_t k = threadIdx.x; k < n; k += blockDim.x) s += static_cast<float>(AT[row * n + k]);
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  __shared__ float red[kBlk / 64];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float t = 0.f;
-    for (int w = 0; w < kBlk / 64; ++w) t += red[w];
-    out[row] += t;
-  }
+  for (int k = 0; k < kMlpInPad; ++k) xf[i * kMlpInPad + k] = f[k];
 }
 
 __global__ void fillKernel(float* p, uint64_t n, float v) {
@@ -227,52 +119,9 @@ __global__ void fillKernel(float* p, uint64_t n, float v) {
   if (i < n) p[i] = v;
 }
 
-// Adam on the FP32 master parameters; padding entries have zero gradients
-// and stay zero.
-__global__ void adamKernel(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2,
-                           float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-// BF16 copies of the weights: W (forward operand) and W^T (backward operand).
-__global__ void castKernel(const float* W, int rows, int cols, __bf16* Wb, __bf16* WTb) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * cols) return;
-  const int r = i / cols, c = i % cols;
-  const __bf16 v = static_cast<__bf16>(W[i]);
-  Wb[i] = v;
-  if (WTb) WTb[c * rows + r] = v;
-}
-
-// Output -> unit guess direction (shape a frame) and distance estimate.
-// policy 1: pairs predicted to penetrate keep the solver's default guess
-// (UnitX, gjk_solver-inl.h:77-78), whose final GJK simplex seeds EPA.
-__global__ void guessKernel(const float* Y, uint64_t n, int policy, float* guess3, float* dist) {
-  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float* y = Y + i * kMlpOutPad;
-  float nn = sqrtf(y[0] * y[0] + y[1] * y[1] + y[2] * y[2]);
-  float g0 = 1.f, g1 = 0.f, g2 = 0.f;
-  if (nn > 1e-20f && !(policy == 1 && y[3] < 0.f)) { g0 = y[0] / nn; g1 = y[1] / nn; g2 = y[2] / nn; }
-  guess3[3 * i] = g0;
-  guess3[3 * i + 1] = g1;
-  guess3[3 * i + 2] = g2;
-  if (dist) dist[i] = y[3];
-}
-
-// ------------------------------------------------------- fused inference
-// Features, the four layers and the normalisation in one kernel: weights
-// live in LDS (copied once per block from a packed image), and each
-// wavefront carries 32 pairs through the network with the activations kept
-// in registers.  Formulation: C = W . X^T (rows = units, columns = pairs),
-// so a layer's accumulator tile holds, in lane l, pair l % 32 and the 16
+// --------------------------------------------------------- weight images
+// Formulation: C = W . X^T (rows = units, columns = rows of the batch), so a
+// layer's accumulator tile holds, in lane l, batch row l % 32 and the 16
 // units 8 (r / 4) + 4 (l / 32) + r % 4 of the tile; the next layer takes
 // those registers directly as its B operand (8 per K step) by contracting
 // over the units in that order -- the packed weights are laid out with the
@@ -281,9 +130,15 @@ __global__ void guessKernel(const float* Y, uint64_t n, int policy, float* guess
 // Packed image (bf16x8 per lane): [layer][out tile][K step][lane], with
 //   element i of lane l = W[32 t + l % 32][k(j, l / 32, i)],
 //   layer 1: k = 16 j + 8 h + i (features in natural order),
-//   layers 2-4: k = 32 (j / 2) + 16 (j % 2) + 8 (i / 4) + 4 h + i % 4.
+//   layers 2-4: k = 32 (j / 2) + 16 (j % 2) + 8 (i / 4) + 4 h + i % 4;
+// then, for the backward products (C = W^T . dZ), the same of the
+// transposed layers 4 (one K step: four output units), 3 and 2:
+//   element i of lane l = W[k(j, l / 32, i)][32 t + l % 32].
 constexpr int kPackL1 = 4 * 4, kPackL2 = 4 * 8, kPackL3 = 4 * 8, kPackL4 = 1 * 8;  // (tile, K step) blocks
-constexpr int kPackBlocks = kPackL1 + kPackL2 + kPackL3 + kPackL4;
+constexpr int kPackFwd = kPackL1 + kPackL2 + kPackL3 + kPackL4;
+constexpr int kPackT4 = 4 * 1, kPackT3 = 4 * 8, kPackT2 = 4 * 8;
+constexpr int kPackBlocks = kPackFwd + kPackT4 + kPackT3 + kPackT2;
+constexpr int kPackFwdBytes = kPackFwd * 64 * 16;
 constexpr int kPackBytes = kPackBlocks * 64 * 16;
 constexpr int kPackBiasFloats = 3 * kHid + kMlpOutPad;
 
@@ -304,9 +159,18 @@ __global__ void packKernel(const float* P, __bf16* pack, float* bias) {
     } else if (b < kPackL1 + kPackL2 + kPackL3) {
       const int q = b - kPackL1 - kPackL2, t = q / 8, j = q % 8;
       v = P[kOffW3 + (32 * t + m) * kHid + permK(j, h, e)];
-    } else {
+    } else if (b < kPackFwd) {
       const int j = b - kPackL1 - kPackL2 - kPackL3;
       v = P[kOffW4 + m * kHid + permK(j, h, e)];
+    } else if (b < kPackFwd + kPackT4) {
+      const int t = b - kPackFwd;
+      v = P[kOffW4 + permK(0, h, e) * kHid + 32 * t + m];
+    } else if (b < kPackFwd + kPackT4 + kPackT3) {
+      const int q = b - kPackFwd - kPackT4, t = q / 8, j = q % 8;
+      v = P[kOffW3 + permK(j, h, e) * kHid + 32 * t + m];
+    } else {
+      const int q = b - kPackFwd - kPackT4 - kPackT3, t = q / 8, j = q % 8;
+      v = P[kOffW2 + permK(j, h, e) * kHid + 32 * t + m];
     }
     pack[idx] = static_cast<__bf16>(v);
   }
@@ -318,6 +182,15 @@ __global__ void packKernel(const float* P, __bf16* pack, float* bias) {
   }
 }
 
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// ------------------------------------------------------- fused inference
+// Features, the four layers and the normalisation in one kernel: weights
+// live in LDS (copied once per block from the packed image), and each
+// wavefront carries 32 pairs through the network.
+
 // one hidden layer: 4 output tiles, KS K steps, B operands in x[KS]
 template <int KS>
 __device__ __forceinline__ void denseGelu(const MFCL_LDS bf16x8* W, const bf16x8* x, const float* bias, int lane,
@@ -325,22 +198,81 @@ __device__ __forceinline__ void denseGelu(const MFCL_LDS bf16x8* W, const bf16x8
   const int h = lane >> 5;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    f32x16 acc = {};
+    f32x16 acc = biasTile(bias, t, h);
 #pragma unroll
-    for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(W[(t * KS + j) * 64 + lane], x[j], acc, 0, 0, 0);
+    for (int j = 0; j < KS; ++j) acc = mfma(W[(t * KS + j) * 64 + lane], x[j], acc);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       bf16x8 o;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = 8 * s + i;
-        const int unit = 32 * t + 8 * (r / 4) + 4 * h + (r % 4);
-        o[i] = static_cast<__bf16>(geluF(acc[r] + bias[unit]));
-      }
+      for (int i = 0; i < 8; ++i) o[i] = static_cast<__bf16>(geluF(acc[8 * s + i]));
       out[2 * t + s] = o;
     }
     // keep the scheduler from overlapping the tiles (register pressure)
     __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// Layers 1-4 on the feature operands x0: outputs 0..3 of row lane % 32 are
+// registers 0..3 of the lanes below 32 (bias not added).
+__device__ __forceinline__ f32x16 network(const MFCL_LDS bf16x8* W, const float* bias, const bf16x8* x0, int lane) {
+  const MFCL_LDS bf16x8* W2 = W + kPackL1 * 64;
+  const MFCL_LDS bf16x8* W3 = W2 + kPackL2 * 64;
+  const MFCL_LDS bf16x8* W4 = W3 + kPackL3 * 64;
+  bf16x8 a1[8], a2[8];
+  denseGelu<4>(W, x0, bias, lane, a1);
+  denseGelu<8>(W2, a1, bias + kHid, lane, a2);
+  denseGelu<8>(W3, a2, bias + 2 * kHid, lane, a1);
+  f32x16 acc = {};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc = mfma(W4[j * 64 + lane], a1[j], acc);
+  return acc;
+}
+// The weights into the block's LDS (dynamic, kPackFwdBytes + biases).
+__device__ __forceinline__ void loadWeights(uint4* lds, const uint4* pack, const float* bias_g, const float*& bias) {
+  for (int k = threadIdx.x; k < kPackFwdBytes / 16; k += blockDim.x) lds[k] = pack[k];
+  float* b = reinterpret_cast<float*>(lds + kPackFwdBytes / 16);
+  for (int k = threadIdx.x; k < kPackBiasFloats; k += blockDim.x) b[k] = bias_g[k];
+  bias = b;
+  __syncthreads();
+}
+// Feature row i (zeros from n on) as B operands: lanes h = 0 / 1 hold
+// columns 16 j + 0..7 / 16 j + 8..15.
+__device__ __forceinline__ void featureOperands(const float* xf, uint64_t i, uint64_t n, int h, bf16x8* x0) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float4 u = make_float4(0, 0, 0, 0), w = u;
+    if (i < n) {
+      const float4* f = reinterpret_cast<const float4*>(xf + i * kMlpInPad + 16 * j + 8 * h);
+      u = f[0];
+      w = f[1];
+    }
+    const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x0[j][e] = static_cast<__bf16>(v[e]);
+  }
+}
+
+// The forward pass on feature rows.
+__global__ void __launch_bounds__(512) mlpForwardFused(const float* xf, uint64_t n, const uint4* pack_g,
+                                                       const float* bias_g, float* y4) {
+  extern __shared__ __align__(16) uint4 lds_pack[];
+  const float* bias;
+  loadWeights(lds_pack, pack_g, bias_g, bias);
+  const MFCL_LDS bf16x8* W = (const MFCL_LDS bf16x8*)(lds_pack);
+  const int lane = threadIdx.x & 63, h = lane >> 5;
+  const uint64_t ntiles = (n + 31) / 32;
+  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t nwaves = (static_cast<uint64_t>(gridDim.x) * blockDim.x) >> 6;
+  for (uint64_t tile = wave; tile < ntiles; tile += nwaves) {
+    const uint64_t i = tile * 32 + (lane & 31);
+    bf16x8 x0[4];
+    featureOperands(xf, i, n, h, x0);
+    const f32x16 acc = network(W, bias, x0, lane);
+    if (h == 0 && i < n) {
+      const float* b4 = bias + 3 * kHid;
+      // rows of 4 floats; the caller's pointer need not be 16-byte aligned
+      for (int k = 0; k < 4; ++k) y4[4 * i + k] = acc[k] + b4[k];
+    }
   }
 }
 
@@ -353,15 +285,9 @@ __global__ void __launch_bounds__(BLK) mlpGuessFused(const uint32_t* pa, const u
                                                       uint64_t n, const uint4* pack_g, const float* bias_g, int policy,
                                                       float* guess3, float* dist) {
   extern __shared__ __align__(16) uint4 lds_pack[];
-  for (int k = threadIdx.x; k < kPackBytes / 16; k += blockDim.x) lds_pack[k] = pack_g[k];
-  float* bias = reinterpret_cast<float*>(lds_pack + kPackBytes / 16);
-  for (int k = threadIdx.x; k < kPackBiasFloats; k += blockDim.x) bias[k] = bias_g[k];
-  __syncthreads();
+  const float* bias;
+  loadWeights(lds_pack, pack_g, bias_g, bias);
   const MFCL_LDS bf16x8* W = (const MFCL_LDS bf16x8*)(lds_pack);
-  const MFCL_LDS bf16x8* W1 = W;
-  const MFCL_LDS bf16x8* W2 = W1 + kPackL1 * 64;
-  const MFCL_LDS bf16x8* W3 = W2 + kPackL2 * 64;
-  const MFCL_LDS bf16x8* W4 = W3 + kPackL3 * 64;
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const uint64_t ntiles = (n + 31) / 32;
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
@@ -409,13 +335,7 @@ __global__ void __launch_bounds__(BLK) mlpGuessFused(const uint32_t* pa, const u
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e = 0; e < 8; ++e) x0[j][e] = static_cast<__bf16>(h ? feat(16 * j + 8 + e) : feat(16 * j + e));
-    bf16x8 a1[8], a2[8];
-    denseGelu<4>(W1, x0, bias, lane, a1);
-    denseGelu<8>(W2, a1, bias + kHid, lane, a2);
-    denseGelu<8>(W3, a2, bias + 2 * kHid, lane, a1);
-    f32x16 acc = {};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(W4[j * 64 + lane], a1[j], acc, 0, 0, 0);
+    const f32x16 acc = network(W, bias, x0, lane);
     // outputs 0..3 of pair lane % 32 are rows 0..3: registers 0..3 of the lanes with h = 0
     if (h == 0 && i < n) {
       const float* b4 = bias + 3 * kHid;
@@ -431,10 +351,325 @@ __global__ void __launch_bounds__(BLK) mlpGuessFused(const uint32_t* pa, const u
   }
 }
 
+// ------------------------------------------------------- fused training
+// Forward, loss, backward and the weight gradients of 128 rows per block
+// and step, 32 rows per wavefront, in one persistent kernel (one block of
+// four wavefronts per CU).  The layered kernels this replaces wrote and read
+// every activation, its transpose and its pre-activation (5.4 KB a row) and
+// took 0.86 ms of a 65,536-row step's 0.92 ms, against 17 GFLOP of products
+// (7 us of the MFMA units).
+//
+// Forward as in inference, GELU's derivative kept in FP32.  A
+// weight gradient dW = dZ . H^T contracts over the rows, so its operands
+// need the rows of one unit in one lane: the transpose of an activation tile
+// is a product with the identity (exact: one term per sum), whose
+// accumulators, rounded back to the BF16 values they are, go to LDS as
+// operands.  All four wavefronts' operands (128 rows) are then contracted by
+// the wavefront that owns the output tiles: wavefront w keeps the gradient
+// rows 32 w .. 32 w + 31 of layers 1-3 and the columns 32 w .. of layer 4 in
+// FP32 accumulators (176 registers) until the block's last step; the blocks'
+// sums are added by reduceAdamKernel.
+constexpr int kPartFloats = kMlpParams + 32;  // a block's gradients, then its loss
+constexpr size_t kGradFloat4 = 3 * 16 * kBlk;  // a block's GELU derivatives
+
+struct TrainLds {
+  bf16x8 x0t[4][2][2][64];      // [wavefront][feature tile][K step][lane]
+  bf16x8 ht[3][4][4][2][64];    // [layer][wavefront][unit tile][K step][lane]
+  bf16x8 dzt[4][4][2][64];      // [wavefront][unit tile][K step][lane]
+  float db[4][3][kHid];         // bias gradients by wavefront
+  float db4[4][32];
+  float loss[4];
+};
+
+// The transposed operands of one 32-unit tile held as K steps a0, a1.
+__device__ __forceinline__ f32x16 transposeTile(bf16x8 a0, bf16x8 a1, const bf16x8* ident) {
+  f32x16 c = {};
+  c = mfma(a0, ident[0], c);
+  return mfma(a1, ident[1], c);
+}
+__device__ __forceinline__ void putOperands(MFCL_LDS bf16x8* o, const f32x16& c, int lane) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    bf16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = static_cast<__bf16>(c[8 * s + i]);
+    o[64 * s + lane] = v;
+  }
+}
+
+// GELU's derivatives of a layer, 64 per lane in FP32, in the block's stretch
+// of the workspace (196 KB a block, which stays in its XCD's L2), 16 bytes per
+// lane and step.  In registers beside the gradients' accumulators they spilled
+// (2 KB a lane: 233 us a step's kernel; layer 3 alone in registers 167 us).
+struct GradMem {
+  float4* p;  // this thread's first entry
+  __device__ __forceinline__ void put(int t, const float* g) const {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[(4 * t + q) * kBlk] = make_float4(g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]);
+  }
+  __device__ __forceinline__ void get(int t, float* g) const {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 v = p[(4 * t + q) * kBlk];
+      g[4 * q] = v.x;
+      g[4 * q + 1] = v.y;
+      g[4 * q + 2] = v.z;
+      g[4 * q + 3] = v.w;
+    }
+  }
+};
+// A hidden layer with GELU's derivative: activations to out, their
+// transposes to LDS.
+template <int KS>
+__device__ __forceinline__ void trainDense(const bf16x8* W, const bf16x8* x, const float* bias, int lane, bf16x8* out,
+                                           const GradMem& grad, const bf16x8* ident, MFCL_LDS bf16x8* ht) {
+  const int h = lane >> 5;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    f32x16 acc = biasTile(bias, t, h);
+#pragma unroll
+    for (int j = 0; j < KS; ++j) acc = mfma(W[(t * KS + j) * 64 + lane], x[j], acc);
+    float g[16];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float z = acc[8 * s + i], q = normalTail(z);
+        o[i] = static_cast<__bf16>(geluF(z, q));
+        g[8 * s + i] = geluGradF(z, q);
+      }
+      out[2 * t + s] = o;
+    }
+    grad.put(t, g);
+    putOperands(ht + 128 * t, transposeTile(out[2 * t], out[2 * t + 1], ident), lane);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// dZ of the layer below: dz_out = (W^T dz) * gelu'.
+template <int KS>
+__device__ __forceinline__ void trainBack(const bf16x8* WT, const bf16x8* dz, const GradMem& grad, int lane, bf16x8* out) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float g[16];
+    grad.get(t, g);
+    f32x16 acc = {};
+#pragma unroll
+    for (int j = 0; j < KS; ++j) acc = mfma(WT[(t * KS + j) * 64 + lane], dz[j], acc);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = static_cast<__bf16>(acc[8 * s + i] * g[8 * s + i]);
+      out[2 * t + s] = o;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// dZ's transposed operands to LDS and its row sums to the bias gradients.
+__device__ __forceinline__ void putDz(const bf16x8* dz, const bf16x8* ident, MFCL_LDS bf16x8* dzt, int lane, float* db) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const f32x16 c = transposeTile(dz[2 * t], dz[2 * t + 1], ident);
+    putOperands(dzt + 128 * t, c, lane);
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s += c[r];
+    db[t] += s;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// acc[n] += dZ tile (all four wavefronts' rows) . H tile n
+template <int NT>
+__device__ __forceinline__ void weightGrad(const MFCL_LDS bf16x8* dzt, int mt, const MFCL_LDS bf16x8* ht, int wave_stride,
+                                           f32x16* acc, int lane) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bf16x8 a = dzt[((w * 4 + mt) * 2 + s) * 64 + lane];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = mfma(a, ht[w * wave_stride + (t * 2 + s) * 64 + lane], acc[t]);
+    }
+}
+template <int NT>
+__device__ __forceinline__ void storeGrad(float* W, int ld, int m0, int n0, const f32x16* acc, int lane) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      W[(m0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4)) * ld + n0 + 32 * t + (lane & 31)] = acc[t][r];
+}
+
+__global__ void __launch_bounds__(kBlk, 1) mlpTrainFused(const float* xf, const float* target, uint64_t n,
+                                                         const bf16x8* pack, const float* bias, float inv_count,
+                                                         float wd, float* part, float4* gelu_grad) {
+  extern __shared__ __align__(16) char lds_raw[];
+  MFCL_LDS TrainLds* L = (MFCL_LDS TrainLds*)((MFCL_LDS char*)(lds_raw));
+  const int lane = threadIdx.x & 63, h = lane >> 5, wv = threadIdx.x >> 6;
+  // identity operands for activations (units in the accumulators' order) and
+  // for features (natural order)
+  bf16x8 ident[2], ident0[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      ident[s][i] = static_cast<__bf16>((lane & 31) == 16 * s + 8 * (i / 4) + 4 * h + (i % 4) ? 1.f : 0.f);
+      ident0[s][i] = static_cast<__bf16>((lane & 31) == 16 * s + 8 * h + i ? 1.f : 0.f);
+    }
+  f32x16 gw1[2] = {}, gw2[4] = {}, gw3[4] = {}, gw4[1] = {};
+  float db1[4] = {0, 0, 0, 0}, db2[4] = {0, 0, 0, 0}, db3[4] = {0, 0, 0, 0}, db4 = 0.f, loss = 0.f;
+  const GradMem g1{gelu_grad + blockIdx.x * kGradFloat4 + threadIdx.x};
+  const GradMem g2{g1.p + 16 * kBlk}, g3{g2.p + 16 * kBlk};
+  MFCL_LDS bf16x8* dzt = &L->dzt[wv][0][0][0];
+  const MFCL_LDS bf16x8* dz_all = &L->dzt[0][0][0][0];
+  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * 128; base < n; base += static_cast<uint64_t>(gridDim.x) * 128) {
+    // opaque, so that the weights and biases are read again for each step:
+    // hoisted out of the loop they would fill the registers several times over
+    asm volatile("" : "+s"(pack), "+s"(bias));
+    const bf16x8* W1 = pack;
+    const bf16x8* W2 = W1 + kPackL1 * 64;
+    const bf16x8* W3 = W2 + kPackL2 * 64;
+    const bf16x8* W4 = W3 + kPackL3 * 64;
+    const bf16x8* T4 = W4 + kPackL4 * 64;
+    const bf16x8* T3 = T4 + kPackT4 * 64;
+    const bf16x8* T2 = T3 + kPackT3 * 64;
+    const uint64_t i = base + 32 * wv + (lane & 31);
+    bf16x8 a[8], b[8];
+    {
+      bf16x8 x0[4];
+      featureOperands(xf, i, n, h, x0);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        putOperands(&L->x0t[wv][t][0][0], transposeTile(x0[2 * t], x0[2 * t + 1], ident0), lane);
+      trainDense<4>(W1, x0, bias, lane, a, g1, ident, &L->ht[0][wv][0][0][0]);
+    }
+    trainDense<8>(W2, a, bias + kHid, lane, b, g2, ident, &L->ht[1][wv][0][0][0]);
+    trainDense<8>(W3, b, bias + 2 * kHid, lane, a, g3, ident, &L->ht[2][wv][0][0][0]);
+    // outputs and loss: mean over valid rows of (1 - cos(y[0:3], t[0:3])) +
+    // wd (y3 - t3)^2; rows with a zero target direction are masked.  Row
+    // lane % 32 is in the lanes below 32.
+    f32x16 y = {};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y = mfma(W4[j * 64 + lane], a[j], y);
+    bf16x8 dy[2] = {};
+    if (h == 0 && i < n) {
+      const float* t = target + 4 * i;
+      const float* b4 = bias + 3 * kHid;
+      const float y0 = y[0] + b4[0], y1 = y[1] + b4[1], y2 = y[2] + b4[2], y3 = y[3] + b4[3];
+      const float tn = sqrtf(t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
+      if (tn > 0.f) {
+        const float yn = fmaxf(sqrtf(y0 * y0 + y1 * y1 + y2 * y2), 1e-12f);
+        const float c = (y0 * t[0] + y1 * t[1] + y2 * t[2]) / (yn * tn);
+        const float e = y3 - t[3];
+        loss += (1.f - c + wd * e * e) * inv_count;
+        dy[0][0] = static_cast<__bf16>(-(t[0] / tn - c * y0 / yn) / yn * inv_count);
+        dy[0][1] = static_cast<__bf16>(-(t[1] / tn - c * y1 / yn) / yn * inv_count);
+        dy[0][2] = static_cast<__bf16>(-(t[2] / tn - c * y2 / yn) / yn * inv_count);
+        dy[0][3] = static_cast<__bf16>(2.f * wd * e * inv_count);
+      }
+    }
+    // layer 4
+    {
+      const f32x16 c = transposeTile(dy[0], dy[1], ident);
+      putOperands(dzt, c, lane);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) db4 += c[r];
+    }
+    trainBack<1>(T4, dy, g3, lane, b);
+    __syncthreads();
+    weightGrad<1>(dz_all, 0, &L->ht[2][0][wv][0][0], 512, gw4, lane);
+    __syncthreads();
+    // layer 3
+    putDz(b, ident, dzt, lane, db3);
+    trainBack<8>(T3, b, g2, lane, a);
+    __syncthreads();
+    weightGrad<4>(dz_all, wv, &L->ht[1][0][0][0][0], 512, gw3, lane);
+    __syncthreads();
+    // layer 2
+    putDz(a, ident, dzt, lane, db2);
+    trainBack<8>(T2, a, g1, lane, b);
+    __syncthreads();
+    weightGrad<4>(dz_all, wv, &L->ht[0][0][0][0][0], 512, gw2, lane);
+    __syncthreads();
+    // layer 1
+    putDz(b, ident, dzt, lane, db1);
+    __syncthreads();
+    weightGrad<2>(dz_all, wv, &L->x0t[0][0][0][0], 256, gw1, lane);
+    __syncthreads();
+  }
+  float* P = part + static_cast<size_t>(blockIdx.x) * kPartFloats;
+  storeGrad<2>(P + kOffW1, kMlpInPad, 32 * wv, 0, gw1, lane);
+  storeGrad<4>(P + kOffW2, kHid, 32 * wv, 0, gw2, lane);
+  storeGrad<4>(P + kOffW3, kHid, 32 * wv, 0, gw3, lane);
+  storeGrad<1>(P + kOffW4, kHid, 0, 32 * wv, gw4, lane);
+  // bias gradients and loss: lanes l and l + 32 hold the same unit's halves
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const float s1 = db1[t] + __shfl_xor(db1[t], 32), s2 = db2[t] + __shfl_xor(db2[t], 32),
+                s3 = db3[t] + __shfl_xor(db3[t], 32);
+    if (h == 0) {
+      L->db[wv][0][32 * t + lane] = s1;
+      L->db[wv][1][32 * t + lane] = s2;
+      L->db[wv][2][32 * t + lane] = s3;
+    }
+  }
+  const float s4 = db4 + __shfl_xor(db4, 32);
+  if (h == 0) L->db4[wv][lane] = s4;
+  for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+  if (lane == 0) L->loss[wv] = loss;
+  __syncthreads();
+  auto sum4 = [](const MFCL_LDS float* p, int stride) { return (p[0] + p[stride]) + (p[2 * stride] + p[3 * stride]); };
+  for (int k = threadIdx.x; k < 3 * kHid; k += kBlk) {
+    const int off = k < kHid ? kOffB1 : (k < 2 * kHid ? kOffB2 : kOffB3);
+    P[off + k % kHid] = sum4(&L->db[0][0][0] + k, 3 * kHid);
+  }
+  if (threadIdx.x < 32) {
+    P[kOffB4 + threadIdx.x] = sum4(&L->db4[0][0] + threadIdx.x, 32);
+    P[kMlpParams + threadIdx.x] = threadIdx.x == 0 ? sum4(&L->loss[0], 1) : 0.f;
+  }
+}
+
+// Sums the blocks' partial gradients (and losses), 64 parameters per block
+// of 256 threads, each parameter's partials split over four of them and
+// added in a fixed order; then Adam on the FP32 master parameters.  Padding
+// entries have zero gradients and stay zero.
+struct AdamArgs {
+  float* p;
+  float* m;
+  float* v;
+  float lr, b1, b2, eps, c1, c2;
+  int apply;
+};
+__global__ void __launch_bounds__(kBlk) reduceAdamKernel(const float* part, int n_part, float* grad, float* loss,
+                                                         AdamArgs a) {
+  __shared__ float red[4][64];
+  const int g = threadIdx.x >> 6, k = threadIdx.x & 63;
+  const int i = blockIdx.x * 64 + k;
+  float s = 0.f;
+  if (i < kPartFloats)
+#pragma unroll 8
+    for (int b = g; b < n_part; b += 4) s += part[static_cast<size_t>(b) * kPartFloats + i];
+  red[g][k] = s;
+  __syncthreads();
+  if (g != 0 || i >= kPartFloats) return;
+  s = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  if (i >= kMlpParams) {
+    if (i == kMlpParams) *loss = s;
+    return;
+  }
+  grad[i] = s;
+  if (!a.apply) return;
+  const float mi = a.b1 * a.m[i] + (1.f - a.b1) * s;
+  const float vi = a.b2 * a.v[i] + (1.f - a.b2) * s * s;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  a.p[i] -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+}
+
 // ------------------------------------------------------------- host side
 namespace {
-
-uint64_t pad32(uint64_t n) { return (n + 31) / 32 * 32; }
 
 int ensureMlp(mfcl_ctx* ctx) {
   if (ctx->mlp.params) return MFCL_OK;
@@ -442,138 +677,32 @@ int ensureMlp(mfcl_ctx* ctx) {
   return MFCL_E_STATE;
 }
 
-// Refreshes the BF16 weight copies from the FP32 master parameters.
+const uint4* packOf(const mfcl_ctx* ctx) { return static_cast<const uint4*>(ctx->mlp.pack); }
+const float* packBias(const mfcl_ctx* ctx) {
+  return reinterpret_cast<const float*>(static_cast<const char*>(ctx->mlp.pack) + kPackBytes);
+}
+
+// Refreshes the BF16 weight images from the FP32 master parameters.
 void castWeights(mfcl_ctx* ctx, hipStream_t s) {
   auto& M = ctx->mlp;
   const int T = 256;
   packKernel<<<(kPackBlocks * 64 * 8 + T - 1) / T, T, 0, s>>>(M.params, reinterpret_cast<__bf16*>(M.pack),
-                                                               reinterpret_cast<float*>(static_cast<char*>(M.pack) +
-                                                                                        kPackBytes));
-  castKernel<<<(kHid * kMlpInPad + T - 1) / T, T, 0, s>>>(M.params + kOffW1, kHid, kMlpInPad, M.w1, M.w1t);
-  castKernel<<<(kHid * kHid + T - 1) / T, T, 0, s>>>(M.params + kOffW2, kHid, kHid, M.w2, M.w2t);
-  castKernel<<<(kHid * kHid + T - 1) / T, T, 0, s>>>(M.params + kOffW3, kHid, kHid, M.w3, M.w3t);
-  castKernel<<<(kMlpOutPad * kHid + T - 1) / T, T, 0, s>>>(M.params + kOffW4, kMlpOutPad, kHid, M.w4, M.w4t);
+                                                               const_cast<float*>(packBias(ctx)));
 }
 
-struct Acts {
-  __bf16 *x, *xt, *h1, *h1t, *h2, *h2t, *h3, *h3t, *dy, *dyt, *dz3, *dz3t, *dz2, *dz2t, *dz1, *dz1t;
-  float *z1, *z2, *z3, *y, *xf;
-};
-
-// Carves the activation workspace for n_pad rows (training needs all of it,
-// inference only x, h1..h3 and y).
-size_t actsBytes(uint64_t np, bool train) {
-  const size_t bf_in = np * kMlpInPad * 2, bf_h = np * kHid * 2, bf_o = np * kMlpOutPad * 2;
-  const size_t f_h = np * kHid * 4, f_o = np * kMlpOutPad * 4, f_in = np * kMlpInPad * 4;
-  size_t total = bf_in + 3 * bf_h + f_o + 256 * 8;
-  if (train) total += bf_in + 3 * bf_h + 2 * bf_o + 6 * bf_h + 3 * f_h + f_in + 256 * 16;
-  return total;
+// Blocks of a training step: one per CU, at most one per 128 rows.
+unsigned trainBlocks(const mfcl_ctx* ctx, uint64_t rows) {
+  return static_cast<unsigned>(std::min<uint64_t>((rows + 127) / 128, static_cast<uint64_t>(ctx->n_cu)));
 }
 
-int carveActs(mfcl_ctx* ctx, uint64_t np, bool train, Acts& a) {
-  const size_t bf_in = np * kMlpInPad * 2, bf_h = np * kHid * 2, bf_o = np * kMlpOutPad * 2;
-  const size_t f_h = np * kHid * 4, f_o = np * kMlpOutPad * 4, f_in = np * kMlpInPad * 4;
-  if (actsBytes(np, train) > ctx->mlp.ws.bytes) {
-    ctx->err = "MLP workspace too small for " + std::to_string(np) +
-               " rows: call mfcl_reserve(ctx, MFCL_WS_MLP, rows) first";
-    return MFCL_E_STATE;
-  }
-  char* p = static_cast<char*>(ctx->mlp.ws.p);
-  auto take = [&](size_t b) {
-    char* q = p;
-    p += (b + 255) & ~static_cast<size_t>(255);
-    return q;
-  };
-  std::memset(&a, 0, sizeof(a));
-  a.x = reinterpret_cast<__bf16*>(take(bf_in));
-  a.h1 = reinterpret_cast<__bf16*>(take(bf_h));
-  a.h2 = reinterpret_cast<__bf16*>(take(bf_h));
-  a.h3 = reinterpret_cast<__bf16*>(take(bf_h));
-  a.y = reinterpret_cast<float*>(take(f_o));
-  if (train) {
-    a.xt = reinterpret_cast<__bf16*>(take(bf_in));
-    a.h1t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.h2t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.h3t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dy = reinterpret_cast<__bf16*>(take(bf_o));
-    a.dyt = reinterpret_cast<__bf16*>(take(bf_o));
-    a.dz3 = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dz3t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dz2 = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dz2t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dz1 = reinterpret_cast<__bf16*>(take(bf_h));
-    a.dz1t = reinterpret_cast<__bf16*>(take(bf_h));
-    a.z1 = reinterpret_cast<float*>(take(f_h));
-    a.z2 = reinterpret_cast<float*>(take(f_h));
-    a.z3 = reinterpret_cast<float*>(take(f_h));
-    a.xf = reinterpret_cast<float*>(take(f_in));
-  }
-  return MFCL_OK;
-}
+// Workspace of a block: its partial gradients and GELU derivatives.
+constexpr size_t kBlockBytes = sizeof(float) * kPartFloats + sizeof(float4) * kGradFloat4;
 
-void forward(mfcl_ctx* ctx, const Acts& a, uint64_t np, bool train, hipStream_t s) {
-  auto& M = ctx->mlp;
-  const int N = static_cast<int>(np);
-  EpiArgs e{};
-  if (train) {
-    e = EpiArgs{a.z1, kHid, M.params + kOffB1, nullptr, a.h1, a.h1t, N, 0};
-    launchGemm<kEpiBiasGelu>(a.x, kMlpInPad, M.w1, kMlpInPad, N, kHid, kMlpInPad, 1, e, s);
-    e = EpiArgs{a.z2, kHid, M.params + kOffB2, nullptr, a.h2, a.h2t, N, 0};
-    launchGemm<kEpiBiasGelu>(a.h1, kHid, M.w2, kHid, N, kHid, kHid, 1, e, s);
-    e = EpiArgs{a.z3, kHid, M.params + kOffB3, nullptr, a.h3, a.h3t, N, 0};
-    launchGemm<kEpiBiasGelu>(a.h2, kHid, M.w3, kHid, N, kHid, kHid, 1, e, s);
-  } else {
-    e = EpiArgs{nullptr, kHid, M.params + kOffB1, nullptr, a.h1, nullptr, 0, 0};
-    launchGemm<kEpiGelu>(a.x, kMlpInPad, M.w1, kMlpInPad, N, kHid, kMlpInPad, 1, e, s);
-    e.bias = M.params + kOffB2; e.h = a.h2;
-    launchGemm<kEpiGelu>(a.h1, kHid, M.w2, kHid, N, kHid, kHid, 1, e, s);
-    e.bias = M.params + kOffB3; e.h = a.h3;
-    launchGemm<kEpiGelu>(a.h2, kHid, M.w3, kHid, N, kHid, kHid, 1, e, s);
-  }
-  e = EpiArgs{a.y, kMlpOutPad, M.params + kOffB4, nullptr, nullptr, nullptr, 0, 0};
-  launchGemm<kEpiBias>(a.h3, kHid, M.w4, kHid, N, kMlpOutPad, kHid, 1, e, s);
-}
-
-// Gradients of the mean loss into M.grad (zeroed here).
-void backward(mfcl_ctx* ctx, const Acts& a, uint64_t np, hipStream_t s) {
-  auto& M = ctx->mlp;
-  const int N = static_cast<int>(np);
-  fillKernel<<<(kMlpParams + 255) / 256, 256, 0, s>>>(M.grad, kMlpParams, 0.f);
-  const int ks = N >= 4096 ? N / 2048 : 1;  // split the batch dimension of the weight gradients
-  EpiArgs e{};
-  // layer 4
-  e = EpiArgs{M.grad + kOffW4, kHid, nullptr, nullptr, nullptr, nullptr, 0, 1};
-  launchGemm<kEpiStore>(a.dyt, N, a.h3t, N, kMlpOutPad, kHid, N, ks, e, s);
-  rowSumKernel<<<kMlpOutPad, kBlk, 0, s>>>(a.dyt, np, M.grad + kOffB4);
-  e = EpiArgs{nullptr, kHid, nullptr, a.z3, a.dz3, a.dz3t, N, 0};
-  launchGemm<kEpiGeluGrad>(a.dy, kMlpOutPad, M.w4t, kMlpOutPad, N, kHid, kMlpOutPad, 1, e, s);
-  // layer 3
-  e = EpiArgs{M.grad + kOffW3, kHid, nullptr, nullptr, nullptr, nullptr, 0, 1};
-  launchGemm<kEpiStore>(a.dz3t, N, a.h2t, N, kHid, kHid, N, ks, e, s);
-  rowSumKernel<<<kHid, kBlk, 0, s>>>(a.dz3t, np, M.grad + kOffB3);
-  e = EpiArgs{nullptr, kHid, nullptr, a.z2, a.dz2, a.dz2t, N, 0};
-  launchGemm<kEpiGeluGrad>(a.dz3, kHid, M.w3t, kHid, N, kHid, kHid, 1, e, s);
-  // layer 2
-  e = EpiArgs{M.grad + kOffW2, kHid, nullptr, nullptr, nullptr, nullptr, 0, 1};
-  launchGemm<kEpiStore>(a.dz2t, N, a.h1t, N, kHid, kHid, N, ks, e, s);
-  rowSumKernel<<<kHid, kBlk, 0, s>>>(a.dz2t, np, M.grad + kOffB2);
-  e = EpiArgs{nullptr, kHid, nullptr, a.z1, a.dz1, a.dz1t, N, 0};
-  launchGemm<kEpiGeluGrad>(a.dz2, kHid, M.w2t, kHid, N, kHid, kHid, 1, e, s);
-  // layer 1
-  e = EpiArgs{M.grad + kOffW1, kMlpInPad, nullptr, nullptr, nullptr, nullptr, 0, 1};
-  launchGemm<kEpiStore>(a.dz1t, N, a.xt, N, kHid, kMlpInPad, N, ks, e, s);
-  rowSumKernel<<<kHid, kBlk, 0, s>>>(a.dz1t, np, M.grad + kOffB1);
-}
-
-// Copies FP32 features [n][64] (host or device) into the BF16 workspace.
-__global__ void featCastKernel(const float* xf, uint64_t n, uint64_t np, __bf16* X, __bf16* XT) {
-  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  for (int k = 0; k < kMlpInPad; ++k) {
-    const __bf16 v = static_cast<__bf16>(i < n ? xf[i * kMlpInPad + k] : 0.f);
-    X[i * kMlpInPad + k] = v;
-    if (XT) XT[static_cast<size_t>(k) * np + i] = v;
-  }
+int checkRows(mfcl_ctx* ctx, uint64_t rows) {
+  if (rows <= ctx->mlp.ws_rows) return MFCL_OK;
+  ctx->err = "MLP workspace too small for " + std::to_string(rows) +
+             " rows: call mfcl_reserve(ctx, MFCL_WS_MLP, rows) first";
+  return MFCL_E_STATE;
 }
 
 }  // namespace
@@ -583,7 +712,11 @@ int mlpReserve(mfcl_ctx* ctx, uint64_t rows) {
     ctx->err = "MLP rows out of range (<= 2^26)";
     return MFCL_E_INVALID;
   }
-  return ensure(ctx, ctx->mlp.ws, actsBytes(pad32(rows ? rows : 1), true));
+  if (rows <= ctx->mlp.ws_rows && ctx->mlp.ws.p) return MFCL_OK;
+  const uint64_t most = std::max<uint64_t>(ctx->mlp.ws_rows, rows + rows / 4 + 32);
+  if (int rc = ensure(ctx, ctx->mlp.ws, kBlockBytes * trainBlocks(ctx, most))) return rc;
+  ctx->mlp.ws_rows = most;
+  return MFCL_OK;
 }
 
 int mlpInit(mfcl_ctx* ctx, uint64_t seed) {
@@ -617,19 +750,6 @@ int mlpSetParams(mfcl_ctx* ctx, const float* host, int n, bool reset_opt) {
     MFCL_HIP_TRY(ctx, hipMalloc(&M.v, fb));
     MFCL_HIP_TRY(ctx, hipMalloc(&M.loss, 256));
     MFCL_HIP_TRY(ctx, hipMalloc(&M.pack, kPackBytes + kPackBiasFloats * 4));
-    const size_t wb = (static_cast<size_t>(kHid) * kMlpInPad + 2 * kHid * kHid + kMlpOutPad * kHid) * 2;
-    char* w = nullptr;
-    MFCL_HIP_TRY(ctx, hipMalloc(&w, 2 * wb));
-    M.wbuf = w;
-    __bf16* q = reinterpret_cast<__bf16*>(w);
-    M.w1 = q; q += kHid * kMlpInPad;
-    M.w2 = q; q += kHid * kHid;
-    M.w3 = q; q += kHid * kHid;
-    M.w4 = q; q += kMlpOutPad * kHid;
-    M.w1t = q; q += kHid * kMlpInPad;
-    M.w2t = q; q += kHid * kHid;
-    M.w3t = q; q += kHid * kHid;
-    M.w4t = q;
   }
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(M.params, host, static_cast<size_t>(kMlpParams) * 4, hipMemcpyHostToDevice,
                                    ctx->stream));
@@ -664,7 +784,7 @@ int mlpFeatures(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, const flo
   }
   if (n == 0) return MFCL_OK;
   featureKernel<<<static_cast<unsigned>((n + kBlk - 1) / kBlk), kBlk, 0, s>>>(
-      pa, pb, posea, poseb, ctx->d_desc, ctx->n_shapes, n, n, nullptr, nullptr, xf_out);
+      pa, pb, posea, poseb, ctx->d_desc, ctx->n_shapes, n, xf_out);
   MFCL_HIP_TRY(ctx, hipGetLastError());
   return MFCL_OK;
 }
@@ -678,15 +798,20 @@ int mlpGuess(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, const float*
   }
   if (n == 0) return MFCL_OK;
   if (ctx->timing) MFCL_HIP_TRY(ctx, hipEventRecord(ctx->ev[8], s));
-  const size_t lds = kPackBytes + kPackBiasFloats * 4;
+  const size_t lds = kPackFwdBytes + kPackBiasFloats * 4;
   const uint64_t ntiles = (n + 31) / 32;
-  const int waves = ctx->tune.mlp_waves;
+  // wavefronts per block: more of them share a copy of the weights and hide
+  // each other's waits, once there is a tile for each (1,048,576 pairs: 332,
+  // 230, 205 us with 4, 8, 16; 4,000 pairs: 14, 17, 27 us)
+  const uint64_t cus = static_cast<uint64_t>(ctx->n_cu);
+  const int by_size = ntiles >= 16 * cus ? 16 : (ntiles >= 8 * cus ? 8 : 4);
+  const int waves = ctx->tune.mlp_waves ? ctx->tune.mlp_waves : by_size;
   // persistent: at most one block per CU (the weights fill most of its LDS)
   const uint64_t want = (ntiles + waves - 1) / waves;
   const uint64_t cap = static_cast<uint64_t>(ctx->n_cu);
   const unsigned grid = static_cast<unsigned>(want < cap ? want : cap);
-  const uint4* pk = static_cast<const uint4*>(ctx->mlp.pack);
-  const float* pb4 = reinterpret_cast<const float*>(static_cast<char*>(ctx->mlp.pack) + kPackBytes);
+  const uint4* pk = packOf(ctx);
+  const float* pb4 = packBias(ctx);
   const int pol = ctx->tune.guess_policy;
   if (waves == 16)
     mlpGuessFused<1024><<<grid, 1024, lds, s>>>(pa, pb, posea, poseb, ctx->d_desc, ctx->n_shapes, n, pk, pb4, pol,
@@ -704,13 +829,11 @@ int mlpGuess(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, const float*
 
 int mlpForwardFeat(mfcl_ctx* ctx, const float* xf, uint64_t n, float* y4_out, hipStream_t s) {
   if (int rc = ensureMlp(ctx)) return rc;
-  const uint64_t np = pad32(n);
-  Acts a;
-  if (int rc = carveActs(ctx, np, false, a)) return rc;
-  featCastKernel<<<static_cast<unsigned>((np + kBlk - 1) / kBlk), kBlk, 0, s>>>(xf, n, np, a.x, nullptr);
-  forward(ctx, a, np, false, s);
-  MFCL_HIP_TRY(ctx, hipMemcpy2DAsync(y4_out, 4 * sizeof(float), a.y, kMlpOutPad * sizeof(float), 4 * sizeof(float),
-                                     n, hipMemcpyDeviceToDevice, s));
+  if (int rc = checkRows(ctx, n)) return rc;
+  if (n == 0) return MFCL_OK;
+  const uint64_t want = (n + 255) / 256;  // 8 wavefronts of 32 rows
+  const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(want, static_cast<uint64_t>(ctx->n_cu)));
+  mlpForwardFused<<<grid, 512, kPackFwdBytes + kPackBiasFloats * 4, s>>>(xf, n, packOf(ctx), packBias(ctx), y4_out);
   MFCL_HIP_TRY(ctx, hipGetLastError());
   return MFCL_OK;
 }
@@ -722,26 +845,26 @@ int mlpTrainStep(mfcl_ctx* ctx, const float* xf, const float* target4, uint64_t 
     ctx->err = "training batch size out of range (1 .. 2^26)";
     return MFCL_E_INVALID;
   }
+  if (int rc = checkRows(ctx, n)) return rc;
   auto& M = ctx->mlp;
-  const uint64_t np = pad32(n);
-  Acts a;
-  if (int rc = carveActs(ctx, np, true, a)) return rc;
-  featCastKernel<<<static_cast<unsigned>((np + kBlk - 1) / kBlk), kBlk, 0, s>>>(xf, n, np, a.x, a.xt);
-  forward(ctx, a, np, true, s);
-  fillKernel<<<1, 64, 0, s>>>(M.loss, 1, 0.f);
+  const unsigned nb = trainBlocks(ctx, n);
+  float4* gelu_grad = static_cast<float4*>(M.ws.p);
+  float* part = reinterpret_cast<float*>(gelu_grad + nb * kGradFloat4);
   const float wd = hyper ? hyper[5] : 1.0f;
-  lossKernel<<<static_cast<unsigned>((np + kBlk - 1) / kBlk), kBlk, 0, s>>>(
-      a.y, target4, n, np, 1.0f / static_cast<float>(n), wd, a.dy, a.dyt, M.loss);
-  backward(ctx, a, np, s);
+  mlpTrainFused<<<nb, kBlk, sizeof(TrainLds), s>>>(xf, target4, n, reinterpret_cast<const bf16x8*>(packOf(ctx)),
+                                                   packBias(ctx), 1.0f / static_cast<float>(n), wd, part, gelu_grad);
+  AdamArgs a{M.params, M.m, M.v, 0, 0, 0, 0, 1, 1, apply_update != 0 ? 1 : 0};
   if (apply_update) {
-    const float lr = hyper ? hyper[0] : 1e-3f, b1 = hyper ? hyper[1] : 0.9f, b2 = hyper ? hyper[2] : 0.999f;
-    const float eps = hyper ? hyper[3] : 1e-8f;
+    a.lr = hyper ? hyper[0] : 1e-3f;
+    a.b1 = hyper ? hyper[1] : 0.9f;
+    a.b2 = hyper ? hyper[2] : 0.999f;
+    a.eps = hyper ? hyper[3] : 1e-8f;
     M.step += 1;
-    const float c1 = 1.f - std::pow(b1, static_cast<float>(M.step)), c2 = 1.f - std::pow(b2, static_cast<float>(M.step));
-    adamKernel<<<(kMlpParams + 255) / 256, 256, 0, s>>>(M.params, M.grad, M.m, M.v, kMlpParams, lr, b1, b2, eps, c1,
-                                                         c2);
-    castWeights(ctx, s);
+    a.c1 = 1.f - std::pow(a.b1, static_cast<float>(M.step));
+    a.c2 = 1.f - std::pow(a.b2, static_cast<float>(M.step));
   }
+  reduceAdamKernel<<<(kPartFloats + 63) / 64, kBlk, 0, s>>>(part, static_cast<int>(nb), M.grad, M.loss, a);
+  if (apply_update) castWeights(ctx, s);
   if (loss_out) MFCL_HIP_TRY(ctx, hipMemcpyAsync(loss_out, M.loss, 4, hipMemcpyDeviceToHost, s));
   MFCL_HIP_TRY(ctx, hipGetLastError());
   return MFCL_OK;
@@ -750,7 +873,7 @@ int mlpTrainStep(mfcl_ctx* ctx, const float* xf, const float* target4, uint64_t 
 void mlpFree(mfcl_ctx* ctx) {
   auto& M = ctx->mlp;
   for (void* p : {static_cast<void*>(M.params), static_cast<void*>(M.grad), static_cast<void*>(M.m),
-                  static_cast<void*>(M.v), static_cast<void*>(M.loss), static_cast<void*>(M.wbuf), M.ws.p, M.pack})
+                  static_cast<void*>(M.v), static_cast<void*>(M.loss), M.ws.p, M.pack})
     if (p) (void)hipFree(p);
   M = MlpState{};
 }
