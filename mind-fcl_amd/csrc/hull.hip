@@ -30,84 +30,116 @@ constexpr int kHullMaxHorizon = 192;
 
 enum HullStatus : int32_t { kHullOk = 0, kHullDegenerate = 1, kHullTooLarge = 2, kHullFailed = 3 };
 
-// LDS slice of one wavefront for point sets of up to cap points (faces: 2 cap).
+// A face in one word: its three vertices (10 bits each), whether this step's
+// flood fill has been at it, and whether the inserted point sees it.
+constexpr uint32_t kFaceTouched = 1u << 30, kFaceVisible = 1u << 31, kFaceVerts = kFaceTouched - 1;
+constexpr uint32_t kFaceFree = ~0u;  // vertices 1023: no point has that number
+
+struct alignas(8) HullEdge {  // border edge (a, b) of this step's cap; outer = 4 * face beyond it + edge number there
+  int16_t a, b, outer, pad;
+};
+
+// LDS slice of one wavefront for point sets of up to cap points (faces: 2
+// cap, a triangulated sphere over n vertices has 2 n - 4).  The slice decides
+// how many wavefronts a CU holds (each is one chain of dependent LDS reads,
+// so the throughput follows their number): 23,040 B at 512 points, seven a
+// CU; face state, vertices and visible list in separate words took 35,000,
+// four a CU.
 struct HullLds {
-  float *x, *y, *z;
+  float* xyz;         // [cap][3]
+  uint32_t* fv;       // [F] faces
+  HullEdge* hor;      // border of this step's cap
   int16_t* conf;      // per point: conflict face, -1 inside, -2 hull vertex
-  int16_t* fv;        // [3][F] vertices of face f: fv[k * F + f]
   int16_t* fnb;       // [3][F] neighbour across edge (v_k, v_k+1)
-  int32_t* fvis;      // per face: 0 unseen this step, 1 visible, 2 not visible, 3 being tested; -1 free
-  int32_t* start;     // per point: horizon edge starting at it (-1 none); reused as new vertex ids at the end
-  int32_t* endv;      // per point: horizon edge ending at it
-  int16_t* flist;     // faces touched by this step's flood fill (reset list)
-  int16_t* vis;       // visible faces of this step
-  int16_t* freel;     // free face slots (stack)
-  int16_t* hor;       // [4][kHullMaxHorizon] horizon edges: a, b, outer face, edge index in it
-  int32_t* cnt;       // counters: [0] visible, [1] touched, [2] horizon, [3] frontier end, [4] error
+  int16_t* start;     // per point: border edge starting at it (-1 none); reused as new vertex ids at the end
+  int16_t* endv;      // per point: border edge ending at it
+  int16_t* freel;     // stack of free face slots; this step's visible faces are listed above its top
   int F;
 };
 
+__host__ __device__ inline int hullHorizon(int cap) { return cap < kHullMaxHorizon ? cap : kHullMaxHorizon; }
 __host__ __device__ inline size_t hullLdsBytes(int cap) {
-  const size_t F = 2 * static_cast<size_t>(cap);
-  size_t b = 12 * static_cast<size_t>(cap) + 2 * cap + 6 * F + 6 * F + 4 * F + 8 * static_cast<size_t>(cap) +
-             2 * F + 2 * F + 2 * F + 8 * kHullMaxHorizon + 8 * 4 + 128;  // + alignment of 13 pieces
-  return (b + 15) & ~static_cast<size_t>(15);
+  const size_t c = (static_cast<size_t>(cap) + 3) & ~static_cast<size_t>(3);
+  return 12 * c + 8 * c + sizeof(HullEdge) * hullHorizon(static_cast<int>(c)) + 2 * c + 12 * c + 4 * c + 4 * c;
 }
 
 MFCL_D HullLds hullCarve(char* base, int cap) {
   HullLds L;
-  const int F = 2 * cap;
-  char* p = base;
-  auto take = [&](size_t bytes) {
-    char* r = p;
-    p += (bytes + 7) & ~static_cast<size_t>(7);
-    return r;
-  };
-  L.x = reinterpret_cast<float*>(take(4 * cap));
-  L.y = reinterpret_cast<float*>(take(4 * cap));
-  L.z = reinterpret_cast<float*>(take(4 * cap));
-  L.fvis = reinterpret_cast<int32_t*>(take(4 * F));
-  L.start = reinterpret_cast<int32_t*>(take(4 * cap));
-  L.endv = reinterpret_cast<int32_t*>(take(4 * cap));
-  L.cnt = reinterpret_cast<int32_t*>(take(4 * 8));
-  L.conf = reinterpret_cast<int16_t*>(take(2 * cap));
-  L.fv = reinterpret_cast<int16_t*>(take(2 * 3 * F));
-  L.fnb = reinterpret_cast<int16_t*>(take(2 * 3 * F));
-  L.flist = reinterpret_cast<int16_t*>(take(2 * F));
-  L.vis = reinterpret_cast<int16_t*>(take(2 * F));
-  L.freel = reinterpret_cast<int16_t*>(take(2 * F));
-  L.hor = reinterpret_cast<int16_t*>(take(2 * 4 * kHullMaxHorizon));
-  L.F = F;
+  const int c = (cap + 3) & ~3;
+  L.F = 2 * c;
+  L.xyz = reinterpret_cast<float*>(base);
+  L.fv = reinterpret_cast<uint32_t*>(base + 12 * c);
+  L.hor = reinterpret_cast<HullEdge*>(base + 20 * c);
+  L.conf = reinterpret_cast<int16_t*>(base + 20 * c + sizeof(HullEdge) * hullHorizon(c));
+  L.fnb = L.conf + c;
+  L.start = L.fnb + 3 * L.F;
+  L.endv = L.start + c;
+  L.freel = L.endv + c;
   return L;
 }
 
-MFCL_D d3 hp(const HullLds& L, int i) { return d3{L.x[i], L.y[i], L.z[i]}; }
+MFCL_D d3 hp(const HullLds& L, int i) { return d3{L.xyz[3 * i], L.xyz[3 * i + 1], L.xyz[3 * i + 2]}; }
 
-// Signed volume test of point p against face (a, b, c), normal (b-a)x(c-a):
-// +1 outside (beyond the relative threshold), 0 otherwise.
-MFCL_D bool sees(const HullLds& L, int a, int b, int c, int p) {
-  const d3 A = hp(L, a), B = hp(L, b), C = hp(L, c), P = hp(L, p);
+// Signed volume test of point P against face (A, B, C), normal (B-A)x(C-A),
+// in 64 bits: true outside, beyond 1e-12 of the square root of the edges'
+// square lengths.
+MFCL_D bool sees64(d3 A, d3 B, d3 C, d3 P) {
   const d3 u = B - A, v = C - A, w = P - A;
   const d3 n = cross(u, v);
   const double o = dot(n, w);
   if (!(o > 0)) return false;
-  const double scale = sqrt(sqnorm(u) * sqnorm(v) * sqnorm(w));
-  return o > 1e-12 * scale;
+  return o > 1e-12 * sqrt(sqnorm(u) * sqnorm(v) * sqnorm(w));
 }
-MFCL_D bool faceSees(const HullLds& L, int f, int p) {
-  const int F = L.F;
-  return sees(L, L.fv[f], L.fv[F + f], L.fv[2 * F + f], p);
+// The test in 32 bits decides where it is sure.  Of u, v, w, n and the
+// products each operation rounds by at most 2^-24 of its size, eight times
+// along any path to the volume, and every term is at most |u||v||w| in
+// 1-norms: the error is below 2^-20 of that product (half of it is left
+// over, which is also far above the 64-bit test's 1e-12), plus what
+// underflows.
+struct HullPlane {
+  float ax, ay, az, nx, ny, nz, err;
+};
+MFCL_D HullPlane planeOf(const HullLds& L, int a, int b, int c) {
+  const float *A = L.xyz + 3 * a, *B = L.xyz + 3 * b, *C = L.xyz + 3 * c;
+  HullPlane q;
+  q.ax = A[0];
+  q.ay = A[1];
+  q.az = A[2];
+  const float ux = B[0] - q.ax, uy = B[1] - q.ay, uz = B[2] - q.az;
+  const float vx = C[0] - q.ax, vy = C[1] - q.ay, vz = C[2] - q.az;
+  q.nx = uy * vz - uz * vy;
+  q.ny = uz * vx - ux * vz;
+  q.nz = ux * vy - uy * vx;
+  q.err = ((fabsf(ux) + fabsf(uy) + fabsf(uz)) * (fabsf(vx) + fabsf(vy) + fabsf(vz)) + 1e-30f) * 0x1p-20f;
+  return q;
+}
+// 1 sees, 0 does not, -1 not sure
+MFCL_D int sees32(const HullPlane& q, const float* P) {
+  const float wx = P[0] - q.ax, wy = P[1] - q.ay, wz = P[2] - q.az;
+  const float o = q.nx * wx + q.ny * wy + q.nz * wz;
+  const float e = q.err * (fabsf(wx) + fabsf(wy) + fabsf(wz)) + 1e-36f;
+  return o > e ? 1 : o < -e ? 0 : -1;
+}
+MFCL_D bool sees(const HullLds& L, int a, int b, int c, int p) {
+  const int s = sees32(planeOf(L, a, b, c), L.xyz + 3 * p);
+  return s >= 0 ? s != 0 : sees64(hp(L, a), hp(L, b), hp(L, c), hp(L, p));
+}
+MFCL_D bool faceSees(const HullLds& L, uint32_t v, int p) {
+  return sees(L, v & 1023, v >> 10 & 1023, v >> 20 & 1023, p);
 }
 
 MFCL_D int laneId64() { return threadIdx.x & 63; }
-MFCL_D void wsync() { __builtin_amdgcn_wave_barrier(); }
-
-MFCL_D void setFace(HullLds& L, int f, int a, int b, int c) {
-  const int F = L.F;
-  L.fv[f] = static_cast<int16_t>(a);
-  L.fv[F + f] = static_cast<int16_t>(b);
-  L.fv[2 * F + f] = static_cast<int16_t>(c);
+// What one lane writes before it, the others read after it (no instructions:
+// the LDS runs one wavefront's accesses in order).
+MFCL_D void wsync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
+
+MFCL_D uint32_t faceWord(int a, int b, int c) {
+  return static_cast<uint32_t>(a) | static_cast<uint32_t>(b) << 10 | static_cast<uint32_t>(c) << 20;
+}
+MFCL_D int below(unsigned long long m, int l) { return __popcll(m & ((1ull << l) - 1)); }
 
 // Wave argmax of val (first index on ties); all lanes get (index, value).
 MFCL_D void waveArgmax(double& val, int& idx) {
@@ -123,21 +155,34 @@ MFCL_D void waveArgmax(double& val, int& idx) {
 }
 
 // One wavefront per set (set order[b] for block b when order is given, else
-// set b), in an LDS slice for sets of up to cap points; the slots a set's
+// set b, skipped if its size is not in (lo, cap] and another launch takes
+// it), in an LDS slice for sets of up to cap points; the slots a set's
 // faces take do not depend on cap, so neither does its result.  Outputs
 // (per set i, points at pt_off[i]):
 // hull_idx[pt_off + k] = index (within the set) of the k-th hull vertex in
 // ascending order, hull_cnt[i]; tris[6 pt_off + 3 t + j] = triangle t over
 // those k-numbered vertices (outward orientation), tri_cnt[i]; status[i].
+//
+// An insertion is a chain of dependent LDS reads and FP64 tests.  Its longest
+// part was the points that lost their conflict face: each lane tried the
+// fan's faces one after another for a point of its own, so every group of 64
+// points with one such point cost a whole fan of tests.  They are gathered
+// from all groups instead and tested (point, face) pair per lane, each lane
+// with one fan face's plane in registers.  20,011 sets of 8..512 points, back
+// to back: 18.7 ms before; 5.5 with that and the smaller slices, 5.2 with a
+// frontier and a border that stay in registers, 4.8 with the test in 32 bits
+// first (a wavefront's insertion is then about 3 LDS round trips for each of
+// 3 frontiers and as many again for the rest, 10,000 cycles).
 __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_t* pt_off, const uint32_t* pt_cnt,
-                                                 const uint32_t* order, uint32_t n_sets, int cap, uint32_t* hull_cnt,
-                                                 uint32_t* hull_idx, uint32_t* tri_cnt, int32_t* tris,
-                                                 int32_t* status) {
+                                                 const uint32_t* order, uint32_t n_sets, int lo, int cap, int top,
+                                                 uint32_t* hull_cnt, uint32_t* hull_idx, uint32_t* tri_cnt,
+                                                 int32_t* tris, int32_t* status) {
   extern __shared__ __align__(16) char hull_lds[];
   if (blockIdx.x >= n_sets) return;
   const uint32_t set = order ? order[blockIdx.x] : blockIdx.x;
   const int l = laneId64();
-  const int n = static_cast<int>(pt_cnt[set]);
+  const uint32_t cnt = pt_cnt[set];
+  if (static_cast<int64_t>(cnt) <= lo || (cnt > static_cast<uint32_t>(cap) && cap < top)) return;
   const uint64_t o = pt_off[set];
   auto finish = [&](int st) {
     if (l == 0) {
@@ -146,22 +191,14 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
       tri_cnt[set] = 0;
     }
   };
-  if (n > cap || n > kHullMaxPoints) { finish(kHullTooLarge); return; }
+  if (cnt > static_cast<uint32_t>(cap)) { finish(kHullTooLarge); return; }
+  const int n = static_cast<int>(cnt);
   if (n < 4) { finish(kHullDegenerate); return; }
   HullLds L = hullCarve(hull_lds, cap);
   const int F = L.F;
-  for (int i = l; i < n; i += 64) {
-    L.x[i] = pts[3 * (o + i)];
-    L.y[i] = pts[3 * (o + i) + 1];
-    L.z[i] = pts[3 * (o + i) + 2];
-    L.conf[i] = -1;
-    L.start[i] = -1;
-    L.endv[i] = -1;
-  }
-  for (int f = l; f < F; f += 64) {
-    L.fvis[f] = -1;
-    L.fnb[f] = L.fnb[F + f] = L.fnb[2 * F + f] = 0;
-  }
+  for (int i = l; i < 3 * n; i += 64) L.xyz[i] = pts[3 * o + i];
+  for (int i = l; i < n; i += 64) L.conf[i] = L.start[i] = L.endv[i] = -1;
+  for (int f = l; f < F; f += 64) L.fv[f] = kFaceFree;
   wsync();
   // ---- initial tetrahedron: extreme x, farthest point, farthest from the
   // line, farthest from the plane (relative tolerances against the extent)
@@ -170,7 +207,7 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
     double v = -INFINITY;
     int idx = 0x7fffffff;
     for (int i = l; i < n; i += 64)
-      if (-static_cast<double>(L.x[i]) > v) { v = -static_cast<double>(L.x[i]); idx = i; }
+      if (-static_cast<double>(L.xyz[3 * i]) > v) { v = -static_cast<double>(L.xyz[3 * i]); idx = i; }
     waveArgmax(v, idx);
     i0 = idx;
   }
@@ -226,22 +263,27 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
     c = t;
   }
   if (l == 0) {
-    setFace(L, 0, a, b, c);
-    setFace(L, 1, a, d, b);
-    setFace(L, 2, b, d, c);
-    setFace(L, 3, c, d, a);
-    for (int f = 0; f < 4; ++f) L.fvis[f] = 0;
+    L.fv[0] = faceWord(a, b, c);
+    L.fv[1] = faceWord(a, d, b);
+    L.fv[2] = faceWord(b, d, c);
+    L.fv[3] = faceWord(c, d, a);
     L.conf[a] = L.conf[b] = L.conf[c] = L.conf[d] = -2;
-    for (int k = 0; k < 8; ++k) L.cnt[k] = 0;
   }
   wsync();
+  auto vertOf = [&](uint32_t w, int k) -> int { return w >> (10 * k) & 1023; };
+  // number of the edge of face word w that runs from eb to ea, -1 none
+  auto edgeOf = [&](uint32_t w, int ea, int eb) -> int {
+    int kk = -1;
+    for (int j = 0; j < 3; ++j)
+      if (vertOf(w, j) == eb && vertOf(w, j < 2 ? j + 1 : 0) == ea) kk = j;
+    return kk;
+  };
   // neighbours of the four faces by edge matching
   if (l < 12) {
     const int f = l / 3, k = l % 3;
-    const int ea = L.fv[k * F + f], eb = L.fv[((k + 1) % 3) * F + f];
+    const uint32_t w = L.fv[f];
     for (int g = 0; g < 4; ++g)
-      for (int kk = 0; kk < 3; ++kk)
-        if (L.fv[kk * F + g] == eb && L.fv[((kk + 1) % 3) * F + g] == ea) L.fnb[k * F + f] = static_cast<int16_t>(g);
+      if (edgeOf(L.fv[g], vertOf(w, k), vertOf(w, k < 2 ? k + 1 : 0)) >= 0) L.fnb[k * F + f] = static_cast<int16_t>(g);
   }
   int nf_used = 4, free_top = 0;
   wsync();
@@ -250,156 +292,251 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
     if (L.conf[i] == -2) continue;
     int cf = -1;
     for (int f = 0; f < 4 && cf < 0; ++f)
-      if (faceSees(L, f, i)) cf = f;
+      if (faceSees(L, L.fv[f], i)) cf = f;
     L.conf[i] = static_cast<int16_t>(cf);
   }
   wsync();
+  const int max_hor = hullHorizon(F / 2), list_max = max_hor < 64 ? max_hor : 64, l3 = l % 3;
   int cursor = 0;
   bool failed = false;
-  while (!failed) {
+  while (true) {
     // next outside point in index order
-    int p = -1;
+    int p = -1, f0 = 0;
     while (cursor < n) {
       const int i = cursor + l;
-      const bool out = i < n && L.conf[i] >= 0;
-      const unsigned long long m = __ballot(out);
+      const int cf = i < n ? L.conf[i] : -1;
+      const unsigned long long m = __ballot(cf >= 0);
       if (m) {
-        p = cursor + __ffsll(m) - 1;
+        const int at = __ffsll(m) - 1;
+        p = cursor + at;
+        f0 = __builtin_amdgcn_readlane(cf, at);
         break;
       }
       cursor += 64;
     }
     if (p < 0) break;
-    cursor = p;
-    const int f0 = L.conf[p];
-    // flood fill of the faces p sees, from its conflict face
+    cursor = p + 1;
+    // Flood fill of the faces p sees, from its conflict face.  A frontier of
+    // up to 21 faces stays in the lanes: lane 3 j + k has the k-th neighbour
+    // of the frontier's j-th face, and whoever finds one that p sees hands
+    // its neighbours on.
+    int16_t* vis = L.freel + free_top;
     if (l == 0) {
-      L.cnt[0] = 1;  // visible
-      L.cnt[1] = 1;  // touched
-      L.vis[0] = static_cast<int16_t>(f0);
-      L.flist[0] = static_cast<int16_t>(f0);
-      L.fvis[f0] = 1;
+      vis[0] = static_cast<int16_t>(f0);
+      L.fv[f0] |= kFaceTouched | kFaceVisible;
     }
     wsync();
-    int fr0 = 0, fr1 = 1;
-    while (fr0 < fr1) {
-      for (int e = fr0 * 3 + l; e < fr1 * 3; e += 64) {
-        const int f = L.vis[e / 3], k = e % 3;
-        const int g = L.fnb[k * F + f];
-        if (atomicCAS(&L.fvis[g], 0, 3) == 0) {
-          const bool s = faceSees(L, g, p);
-          L.fvis[g] = s ? 1 : 2;
-          L.flist[atomicAdd(&L.cnt[1], 1)] = static_cast<int16_t>(g);
-          if (s) L.vis[atomicAdd(&L.cnt[0], 1)] = static_cast<int16_t>(g);
+    int nvis = 1, last = 1;  // last: faces of the newest frontier
+    int g = L.fnb[l3 * F + f0];
+    while (last > 0 && last <= 21) {
+      bool s = false;
+      int nb[3] = {0, 0, 0};
+      if (l < 3 * last) {
+        const uint32_t w = atomicOr(&L.fv[g], kFaceTouched);
+        for (int k = 0; k < 3; ++k) nb[k] = L.fnb[k * F + g];
+        if (!(w & kFaceTouched)) {
+          s = faceSees(L, w, p);
+          if (s) L.fv[g] = w | kFaceTouched | kFaceVisible;
         }
+      }
+      const unsigned long long m = __ballot(s);
+      const int rank = below(m, l);
+      if (s) vis[nvis + rank] = static_cast<int16_t>(g);
+      last = __popcll(m);
+      nvis += last;
+      const int to = s && rank < 21 ? 3 * rank : 63;
+      const int g0 = __builtin_amdgcn_ds_permute(4 * to, nb[0]);
+      const int g1 = __builtin_amdgcn_ds_permute(to < 63 ? 4 * to + 4 : 252, nb[1]);
+      const int g2 = __builtin_amdgcn_ds_permute(to < 63 ? 4 * to + 8 : 252, nb[2]);
+      g = l3 == 0 ? g0 : l3 == 1 ? g1 : g2;
+    }
+    wsync();
+    for (int fr0 = nvis - last; fr0 < nvis;) {  // wider frontiers, from the list
+      const int fr1 = nvis;
+      for (int base = fr0 * 3; base < fr1 * 3; base += 64) {
+        const int e = base + l;
+        bool s = false;
+        int f = 0;
+        if (e < fr1 * 3) {
+          const int at = e / 3;
+          f = L.fnb[(e - 3 * at) * F + vis[at]];
+          const uint32_t w = atomicOr(&L.fv[f], kFaceTouched);
+          if (!(w & kFaceTouched)) {
+            s = faceSees(L, w, p);
+            if (s) L.fv[f] = w | kFaceTouched | kFaceVisible;
+          }
+        }
+        const unsigned long long m = __ballot(s);
+        if (s) vis[nvis + below(m, l)] = static_cast<int16_t>(f);
+        nvis += __popcll(m);
       }
       wsync();
       fr0 = fr1;
-      fr1 = L.cnt[0];
-      wsync();
     }
-    const int nvis = fr1;
-    // horizon: edges of visible faces whose neighbour is not visible
-    if (l == 0) L.cnt[2] = 0;
+    // Border: edges of visible faces whose neighbour is not visible.  What a
+    // lane found last stays in its registers: all of a border of a cap of up
+    // to 21 faces.
+    int nh = 0, h1 = 0;
+    HullEdge e1{0, 0, 0, 0};
+    bool edge1 = false;
+    for (int base = 0; base < nvis * 3; base += 63) {
+      const int at = base / 3 + l / 3;
+      bool s = false;
+      int ea = 0, eb = 0, kk = -1, out = 0;
+      if (l < 63 && at < nvis) {
+        const int f = vis[at];
+        out = L.fnb[l3 * F + f];
+        const uint32_t wf = L.fv[f], wg = L.fv[out];
+        s = !(wg & kFaceVisible);
+        ea = vertOf(wf, l3);
+        eb = vertOf(wf, l3 < 2 ? l3 + 1 : 0);
+        kk = edgeOf(wg, ea, eb);
+      }
+      const unsigned long long m = __ballot(s);
+      h1 = nh + below(m, l);
+      edge1 = s;
+      const bool fits = h1 < max_hor && kk >= 0;
+      if (s && fits) {
+        e1 = HullEdge{static_cast<int16_t>(ea), static_cast<int16_t>(eb), static_cast<int16_t>(4 * out + kk), 0};
+        L.hor[h1] = e1;
+        L.start[ea] = static_cast<int16_t>(h1);
+        L.endv[eb] = static_cast<int16_t>(h1);
+      }
+      failed |= __ballot(s && !fits) != 0;
+      nh += __popcll(m);
+    }
+    if (failed || nh < 3) {
+      failed = true;
+      break;
+    }
     wsync();
-    for (int e = l; e < nvis * 3; e += 64) {
-      const int f = L.vis[e / 3], k = e % 3;
-      const int g = L.fnb[k * F + f];
-      if (L.fvis[g] == 1) continue;
-      const int ea = L.fv[k * F + f], eb = L.fv[((k + 1) % 3) * F + f];
-      int kk = -1;
-      for (int j = 0; j < 3; ++j)
-        if (L.fv[j * F + g] == eb && L.fv[((j + 1) % 3) * F + g] == ea) kk = j;
-      const int h = atomicAdd(&L.cnt[2], 1);
-      if (h < kHullMaxHorizon && kk >= 0) {
-        L.hor[h] = static_cast<int16_t>(ea);
-        L.hor[kHullMaxHorizon + h] = static_cast<int16_t>(eb);
-        L.hor[2 * kHullMaxHorizon + h] = static_cast<int16_t>(g);
-        L.hor[3 * kHullMaxHorizon + h] = static_cast<int16_t>(kk);
-      } else {
-        atomicOr(&L.cnt[4], 1);
+    const bool small = nvis <= 21;
+    const int n_free = free_top + nvis;
+    // slot of the new face (a, b, p) at border edge h: freed visible faces
+    // first, then fresh ones
+    auto slotOf = [&](int h) -> int { return h < n_free ? L.freel[n_free - 1 - h] : nf_used + (h - n_free); };
+    // The border must be one loop: each vertex starts and ends one edge (of
+    // two edges that start at a vertex one finds the other's number).
+    bool bad = false;
+    int slot1 = 0, slot_b = 0, slot_a = 0;  // slots of the edge's own face and of the next and the one before
+    auto check = [&](const HullEdge& e, int h) {
+      const int eb = L.start[e.b], ea = L.endv[e.a];
+      bad |= L.start[e.a] != h || L.endv[e.b] != h || ea < 0 || eb < 0;
+      slot1 = slotOf(h);
+      slot_b = slotOf(eb > 0 ? eb : 0);
+      slot_a = slotOf(ea > 0 ? ea : 0);
+    };
+    if (small) {
+      if (edge1) check(e1, h1);
+    } else {
+      for (int h = l; h < nh; h += 64) check(L.hor[h], h);
+    }
+    // (the fan never needs more than the slots left: checked before any write)
+    if (__ballot(bad) || nh > n_free + (F - nf_used)) {
+      failed = true;
+      break;
+    }
+    // points that saw a removed face look for the first new face they see
+    {
+      const int lg = nh > 32 ? 6 : 32 - __clz(nh - 1);  // lanes a point: the border's length, to a power of two
+      const int G = 1 << lg, lead = l & ~(G - 1), h0 = l - lead, j0 = l >> lg, per = 64 >> lg;
+      const int hl = h0 < nh ? h0 : 0;
+      const HullEdge e0 = L.hor[hl];
+      const HullPlane plane = planeOf(L, e0.a, e0.b, p);
+      const int slot0 = slotOf(hl);
+      int n_lost = 0;  // gathered points, in the border entries' spare fields
+      auto flush = [&] {
+        wsync();
+        for (int j = 0; j < n_lost; j += per) {
+          const bool mine = j + j0 < n_lost;
+          const int i = L.hor[mine ? j + j0 : 0].pad;
+          int sure = 0;
+          if (mine && h0 < nh) {
+            sure = sees32(plane, L.xyz + 3 * i);
+            if (sure < 0) sure = sees64(hp(L, e0.a), hp(L, e0.b), hp(L, p), hp(L, i));
+          }
+          unsigned long long m = __ballot(sure != 0);
+          if (G < 64) m = m >> lead & ((1ull << G) - 1);
+          int nc = -1;
+          if (m) nc = __shfl(slot0, lead + __ffsll(m) - 1);
+          for (int hb = 64; hb < nh && nc < 0; hb += 64) {  // borders beyond 64 edges (one point at a time here)
+            const int h = hb + l;
+            const HullEdge e = L.hor[h < nh ? h : 0];
+            const unsigned long long m2 = __ballot(h < nh && sees(L, e.a, e.b, p, i));
+            if (m2) nc = slotOf(hb + __ffsll(m2) - 1);
+          }
+          if (mine && h0 == 0) L.conf[i] = static_cast<int16_t>(nc);
+        }
+        n_lost = 0;
+        wsync();
+      };
+      for (int base = p + 1; base < n; base += 256) {
+        int cf[4];
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int i = base + 64 * k + l;
+          cf[k] = i < n ? L.conf[i] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = cf[k] >= 0 ? L.fv[cf[k]] : 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const bool s = (w[k] & kFaceVisible) != 0;
+          const unsigned long long m = __ballot(s);
+          if (!m) continue;
+          const int c = __popcll(m);
+          if (n_lost + c > list_max) flush();
+          if (s) L.hor[n_lost + below(m, l)].pad = static_cast<int16_t>(base + 64 * k + l);
+          n_lost += c;
+        }
+      }
+      flush();
+    }
+    // the cap's faces go, the fan comes
+    const int taken = nh < n_free ? nh : n_free;
+    for (int j = l; j < nvis; j += 64) L.fv[vis[j]] = kFaceFree;
+    wsync();
+    auto place = [&](const HullEdge& e) {
+      const int out = e.outer >> 2, kk = e.outer & 3;
+      L.fv[slot1] = faceWord(e.a, e.b, p);
+      L.fv[out] &= kFaceVerts;
+      L.fnb[slot1] = static_cast<int16_t>(out);         // across (a, b)
+      L.fnb[F + slot1] = static_cast<int16_t>(slot_b);  // across (b, p)
+      L.fnb[2 * F + slot1] = static_cast<int16_t>(slot_a);  // across (p, a)
+      L.fnb[kk * F + out] = static_cast<int16_t>(slot1);
+    };
+    if (small) {
+      if (edge1) {
+        place(e1);
+        L.start[e1.a] = -1;
+        L.endv[e1.b] = -1;
+      }
+    } else {
+      for (int h = l; h < nh; h += 64) {
+        const HullEdge e = L.hor[h];
+        check(e, h);
+        place(e);
+      }
+      wsync();
+      for (int h = l; h < nh; h += 64) {
+        const HullEdge e = L.hor[h];
+        L.start[e.a] = -1;
+        L.endv[e.b] = -1;
       }
     }
-    wsync();
-    const int nh = L.cnt[2];
-    if (L.cnt[4] || nh < 3) {
-      failed = true;
-      break;
-    }
-    // the border must be one loop: each vertex starts and ends one edge
-    for (int h = l; h < nh; h += 64) {
-      if (atomicCAS(&L.start[L.hor[h]], -1, h) != -1) atomicOr(&L.cnt[4], 2);
-      if (atomicCAS(&L.endv[L.hor[kHullMaxHorizon + h]], -1, h) != -1) atomicOr(&L.cnt[4], 2);
-    }
-    wsync();
-    bool bad = L.cnt[4] != 0;
-    for (int h = l; h < nh && !bad; h += 64)
-      if (L.endv[L.hor[h]] < 0) bad = true;
-    if (__ballot(bad)) {
-      failed = true;
-      break;
-    }
-    // slots for the fan: freed visible faces first, then fresh ones (the
-    // fan never needs more than the slots left: checked before any write)
-    if (nh > free_top + nvis + (F - nf_used)) {
-      failed = true;
-      break;
-    }
-    for (int j = l; j < nvis; j += 64) L.freel[free_top + j] = L.vis[j];
-    free_top += nvis;
-    wsync();
-    // new face for horizon edge h: (a, b, p), slot slotOf(h)
-    auto slotOf = [&](int h) -> int { return h < free_top ? L.freel[free_top - 1 - h] : nf_used + (h - free_top); };
-    for (int h = l; h < nh; h += 64) {
-      const int s = slotOf(h);
-      const int ea = L.hor[h], eb = L.hor[kHullMaxHorizon + h];
-      setFace(L, s, ea, eb, p);
-    }
-    wsync();
-    for (int h = l; h < nh; h += 64) {
-      const int s = slotOf(h);
-      const int ea = L.hor[h], eb = L.hor[kHullMaxHorizon + h];
-      const int g = L.hor[2 * kHullMaxHorizon + h], kk = L.hor[3 * kHullMaxHorizon + h];
-      L.fnb[s] = static_cast<int16_t>(g);                       // across (a, b)
-      L.fnb[F + s] = static_cast<int16_t>(slotOf(L.start[eb]));  // across (b, p)
-      L.fnb[2 * F + s] = static_cast<int16_t>(slotOf(L.endv[ea]));  // across (p, a)
-      L.fnb[kk * F + g] = static_cast<int16_t>(s);
-    }
-    wsync();
-    // points that saw a removed face look for a new face they see
-    for (int i = l; i < n; i += 64) {
-      const int cf = L.conf[i];
-      if (cf < 0 || L.fvis[cf] != 1 || i == p) continue;
-      int nc = -1;
-      for (int h = 0; h < nh && nc < 0; ++h)
-        if (faceSees(L, slotOf(h), i)) nc = slotOf(h);
-      L.conf[i] = static_cast<int16_t>(nc);
-    }
-    wsync();
-    // bookkeeping for the next step
-    const int taken = nh < free_top ? nh : free_top;
-    const int fresh = nh - taken;
-    for (int t2 = l; t2 < L.cnt[1]; t2 += 64) {
-      const int f = L.flist[t2];
-      L.fvis[f] = L.fvis[f] == 1 ? -1 : 0;
-    }
-    wsync();
-    for (int h = l; h < nh; h += 64) {
-      L.fvis[slotOf(h)] = 0;
-      L.start[L.hor[h]] = -1;
-      L.endv[L.hor[kHullMaxHorizon + h]] = -1;
-    }
     if (l == 0) L.conf[p] = -2;
-    free_top -= taken;
-    nf_used += fresh;
-    if (nf_used > F) failed = true;
+    free_top = n_free - taken;
+    nf_used += nh - taken;
     wsync();
   }
   if (failed) { finish(kHullFailed); return; }
   // hull vertices are the points the remaining faces use (a point inserted
   // earlier is no longer one once every face around it was removed)
-  for (int f = l; f < nf_used; f += 64)
-    if (L.fvis[f] >= 0) L.start[L.fv[f]] = L.start[L.fv[F + f]] = L.start[L.fv[2 * F + f]] = -3;
+  for (int f = l; f < nf_used; f += 64) {
+    const uint32_t w = L.fv[f];
+    if (w != kFaceFree) L.start[vertOf(w, 0)] = L.start[vertOf(w, 1)] = L.start[vertOf(w, 2)] = -3;
+  }
   wsync();
   // renumber the hull vertices in ascending point order
   int nv = 0;
@@ -408,8 +545,8 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
     const bool v = i < n && L.start[i] == -3;
     const unsigned long long m = __ballot(v);
     if (v) {
-      const int id = nv + __popcll(m & ((1ull << l) - 1));
-      L.start[i] = id;
+      const int id = nv + below(m, l);
+      L.start[i] = static_cast<int16_t>(id);
       hull_idx[o + id] = static_cast<uint32_t>(i);
     }
     nv += __popcll(m);
@@ -418,14 +555,12 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
   int nt = 0;
   for (int base = 0; base < nf_used; base += 64) {
     const int f = base + l;
-    const bool alive = f < nf_used && L.fvis[f] >= 0;
+    const uint32_t w = f < nf_used ? L.fv[f] : kFaceFree;
+    const bool alive = w != kFaceFree;
     const unsigned long long m = __ballot(alive);
     if (alive) {
-      const int t = nt + __popcll(m & ((1ull << l) - 1));
-      int32_t* tp = tris + 6 * o + 3 * static_cast<uint64_t>(t);
-      tp[0] = L.start[L.fv[f]];
-      tp[1] = L.start[L.fv[F + f]];
-      tp[2] = L.start[L.fv[2 * F + f]];
+      int32_t* tp = tris + 6 * o + 3 * static_cast<uint64_t>(nt + below(m, l));
+      for (int k = 0; k < 3; ++k) tp[k] = L.start[vertOf(w, k)];
     }
     nt += __popcll(m);
   }
@@ -444,13 +579,24 @@ int hullsLaunch(mfcl_ctx* ctx, const float* pts, const uint64_t* pt_off, const u
     ctx->err = "max_points out of range [4, " + std::to_string(kHullMaxPoints) + "]";
     return MFCL_E_INVALID;
   }
-  const size_t lds = hullLdsBytes(max_points);
-  if (lds > static_cast<size_t>(ctx->max_lds_per_block)) {
+  if (hullLdsBytes(max_points) > static_cast<size_t>(ctx->max_lds_per_block)) {
     ctx->err = "hull workspace exceeds the LDS of a workgroup";
     return MFCL_E_UNSUPPORTED;
   }
-  hullKernel<<<n_sets, 64, lds, s>>>(pts, pt_off, pt_cnt, nullptr, n_sets, max_points, hull_cnt, hull_idx, tri_cnt,
-                                     tris, status);
+  // The sizes are on the device: each of two classes is a launch over all
+  // sets whose blocks leave at once if their set is of the other one, the
+  // longer sets first.  (20,011 sets of 8..512 points: one launch 6.98 ms, a
+  // line at 256 points 6.72, two at 128 and 256 6.85, three 7.00: what finer
+  // slices gain in wavefronts goes into the ends of the launches.)
+  constexpr int kClasses = 2;
+  const int caps[kClasses] = {256, kHullMaxPoints};
+  for (int c = kClasses - 1; c >= 0; --c) {
+    const int lo = c ? caps[c - 1] : -1;
+    if (c && lo >= max_points) continue;
+    const int cap = std::min(caps[c], max_points);
+    hullKernel<<<n_sets, 64, hullLdsBytes(cap), s>>>(pts, pt_off, pt_cnt, nullptr, n_sets, lo, cap, max_points,
+                                                     hull_cnt, hull_idx, tri_cnt, tris, status);
+  }
   MFCL_HIP_TRY(ctx, hipGetLastError());
   return MFCL_OK;
 }
@@ -487,8 +633,8 @@ int hullsLaunchClassed(mfcl_ctx* ctx, const float* pts, const uint64_t* pt_off, 
       ctx->err = "hull workspace exceeds the LDS of a workgroup";
       return MFCL_E_UNSUPPORTED;
     }
-    hullKernel<<<count[c], 64, lds, s>>>(pts, pt_off, pt_cnt, order_dev + start[c], count[c], caps[c], hull_cnt,
-                                         hull_idx, tri_cnt, tris, status);
+    hullKernel<<<count[c], 64, lds, s>>>(pts, pt_off, pt_cnt, order_dev + start[c], count[c], -1, caps[c],
+                                         caps[c], hull_cnt, hull_idx, tri_cnt, tris, status);
   }
   MFCL_HIP_TRY(ctx, hipGetLastError());
   // the order list is read by the kernels: keep it until they have run

@@ -189,3 +189,43 @@ def test_shared_vertices_need_shared_faces(gpu_ctx):
         gpu_ctx.upload_shapes(types, params, voff, vcnt, P,
                               faces=mfcl.faces_from_triangles(tris, np.array([0, len(t1)]),
                                                               np.array([len(t1), len(t2)])))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("apex", [0.0, 1.05, 6.0])
+def test_device_hulls_at_slice_edges(gpu_ctx, apex):
+    """Point counts at the edges of the LDS slices and of a wavefront's 64
+    lanes, counts only on the device (mfcl_convex_hulls_dev) and on the host.
+    The last point lies inside (sees nothing), just outside (a cap of a few
+    faces, kept in registers) or far out: it sees half of the faces, a
+    frontier of more than 21 of them and, over 600 points, a border of more
+    than 64 edges, with most points' conflict faces lost at once."""
+    rng = np.random.default_rng(53)
+    sets = []
+    for n in (5, 31, 64, 65, 128, 129, 255, 256, 257, 300, 512, 513, 767, 768):
+        u = rng.normal(size=(n, 3))
+        u /= np.linalg.norm(u, axis=1, keepdims=True)
+        u[n - 1] *= apex
+        if n > 64 and apex > 2:
+            u[n // 2] *= apex  # half of the points are still to come
+        sets.append(u.astype(np.float32))
+    cnt = np.array([len(s) for s in sets], np.uint32)
+    off = np.zeros(len(sets), np.uint64)
+    off[1:] = np.cumsum(cnt[:-1])
+    pts = np.concatenate(sets)
+    host = gpu_ctx.convex_hulls(pts, off, cnt)
+    up = [gpu_ctx.to_device(a) for a in (pts, off, cnt)]
+    size = (len(cnt), len(pts), len(cnt), 6 * len(pts), len(cnt))
+    out = [gpu_ctx.to_device(np.zeros(k, np.int32)) for k in size]
+    gpu_ctx._check(gpu_ctx.lib.mfcl_convex_hulls_dev(gpu_ctx.h, *(d.ptr for d in up), len(cnt), int(cnt.max()),
+                                                     *(d.ptr for d in out), None))
+    gpu_ctx.sync()
+    hc, hi, tc, tr, st = (d.download(np.zeros(k, np.int32)) for d, k in zip(out, size))
+    for k, (P, (status, hidx, tris)) in enumerate(zip(sets, host)):
+        assert status == 0 and st[k] == 0
+        o = int(off[k])
+        assert np.array_equal(hidx, hi[o:o + hc[k]])
+        assert np.array_equal(np.asarray(tris).reshape(-1), tr[6 * o:6 * o + 3 * tc[k]])
+        h = ConvexHull(P.astype(np.float64))
+        assert np.array_equal(hidx, np.unique(h.simplices))
+        assert {tuple(sorted(hidx[t].tolist())) for t in tris} == {tuple(sorted(s.tolist())) for s in h.simplices}
