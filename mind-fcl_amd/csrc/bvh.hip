@@ -546,35 +546,72 @@ MFCL_D bool project6d(d3 ax, d3 p1, d3 p2, d3 p3, d3 q1, d3 q2, d3 q3) {
   return true;
 }
 
-MFCL_D bool triTriD(const float4* P, const float4* Qm, const m33& R, d3 T) {
-  const d3 P1 = {P[0].x, P[0].y, P[0].z}, P2 = {P[1].x, P[1].y, P[1].z}, P3 = {P[2].x, P[2].y, P[2].z};
-  const d3 Q1 = mul(R, d3{Qm[0].x, Qm[0].y, Qm[0].z}) + T;
-  const d3 Q2 = mul(R, d3{Qm[1].x, Qm[1].y, Qm[1].z}) + T;
-  const d3 Q3 = mul(R, d3{Qm[2].x, Qm[2].y, Qm[2].z}) + T;
-  const d3 p1 = P1 - P1, p2 = P2 - P1, p3 = P3 - P1;
-  const d3 q1 = Q1 - P1, q2 = Q2 - P1, q3 = Q3 - P1;
-  const d3 e1 = p2 - p1, e2 = p3 - p2, e3 = p1 - p3;
-  const d3 f1 = q2 - q1, f2 = q3 - q2, f3 = q1 - q3;
-  const d3 n1 = cross(e1, e2);
-  if (!project6d(n1, p1, p2, p3, q1, q2, q3)) return false;
-  const d3 m1 = cross(f1, f2);
-  if (!project6d(m1, p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e1, f1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e1, f2), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e1, f3), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e2, f1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e2, f2), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e2, f3), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e3, f1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e3, f2), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e3, f3), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e1, n1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e2, n1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(e3, n1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(f1, m1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(f2, m1), p1, p2, p3, q1, q2, q3)) return false;
-  if (!project6d(cross(f3, m1), p1, p2, p3, q1, q2, q3)) return false;
-  return true;
+// The 17 axes of a triangle pair, each a cross product of two vectors: the
+// triangles' normals n1 = e1 x e2 and m1 = f1 x f2, the edges' pairwise
+// products, and the edges with their own triangle's normal.  One wavefront
+// tests the pairs its lanes have found, up to kTriBatch at a time: the pairs'
+// points go through LDS, then each lane takes a (pair, axis).  A query's leaf
+// step has a few pairs to some dozen a wavefront, and one lane going through
+// all 17 axes of its pair is a chain of 800 FP64 operations (7,300 cycles; a
+// whole other step takes 3,000) that holds 168 registers.
+constexpr int kTriBatch = 15;  // 255 (pair, axis) items: four rounds of 64 lanes
+struct TriLds {
+  d3 pt[kTriBatch][6];  // p1 p2 p3 q1 q2 q3, relative to the first triangle's first vertex
+  int sep[kTriBatch];   // an axis separates them
+};
+
+// triTri of the lanes in `want` (uniform over the wavefront's call): true where the triangles intersect.
+MFCL_D bool triTriWave(TriLds& L, bool want, const float4* P, const float4* Qm, const tf3& rel) {
+  const int l = threadIdx.x & 63;
+  const unsigned long long all = __ballot(want);
+  const int n = __popcll(all), rank = __popcll(all & ((1ull << l) - 1ull));
+  bool hit = false;
+  for (int b0 = 0; b0 < n; b0 += kTriBatch) {
+    const int nb = n - b0 < kTriBatch ? n - b0 : kTriBatch;
+    const bool mine = want && rank >= b0 && rank < b0 + nb;
+    if (mine) {
+      d3* pt = L.pt[rank - b0];
+      const d3 P1 = {P[0].x, P[0].y, P[0].z}, P2 = {P[1].x, P[1].y, P[1].z}, P3 = {P[2].x, P[2].y, P[2].z};
+      pt[0] = P1 - P1;
+      pt[1] = P2 - P1;
+      pt[2] = P3 - P1;
+      for (int k = 0; k < 3; ++k) pt[3 + k] = mul(rel.R, d3{Qm[k].x, Qm[k].y, Qm[k].z}) + rel.t - P1;
+      L.sep[rank - b0] = 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int it = l; it < 17 * nb; it += 64) {
+      const int pr = it / 17, ax = it - 17 * pr;
+      const d3* pt = L.pt[pr];
+      // edge k of a triangle runs from its vertex k to k + 1
+      auto edge = [&](int tri, int k) -> d3 { return pt[3 * tri + (k < 2 ? k + 1 : 0)] - pt[3 * tri + k]; };
+      int xt, xk, yt, yk;  // edges X and Y (triangle, number)
+      if (ax < 2) {
+        xt = yt = ax;
+        xk = 0;
+        yk = 1;
+      } else if (ax < 11) {
+        xt = 0;
+        yt = 1;
+        xk = (ax - 2) / 3;
+        yk = ax - 2 - 3 * xk;
+      } else {
+        xt = yt = ax < 14 ? 0 : 1;
+        xk = ax < 14 ? ax - 11 : ax - 14;
+        yk = 0;
+      }
+      const d3 X = edge(xt, xk);
+      d3 Y = edge(yt, yk);
+      if (ax >= 11) Y = cross(Y, edge(yt, 1));
+      if (!project6d(cross(X, Y), pt[0], pt[1], pt[2], pt[3], pt[4], pt[5])) L.sep[pr] = 1;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (mine) hit = L.sep[rank - b0] == 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  return hit;
 }
 
 MFCL_D void relPose(const float* pa, const float* pb, m33& R, d3& T) {
@@ -584,6 +621,9 @@ MFCL_D void relPose(const float* pa, const float* pb, m33& R, d3& T) {
 }
 
 __device__ __forceinline__ unsigned long long ballot64(bool p) { return __ballot(p); }
+__device__ __forceinline__ float uniformF(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
 __device__ __forceinline__ int laneId() { return threadIdx.x & 63; }
 __device__ __forceinline__ int prefixBelow(unsigned long long m) {
   return __popcll(m & ((1ull << laneId()) - 1ull));
@@ -675,45 +715,34 @@ MFCL_D void triContactsD(const float4* P, const float4* Qm, const m33& R, d3 T, 
 // 226-254), and a query collides when it has a contact, as a
 // CollisionResult with contacts does.
 constexpr int kMeshBlock = 256;
-constexpr int kMeshLds = 3072;  // LDS stack entries per block
-
-// Exclusive prefix of v over the block (4 wavefronts) and the total; 64-bit
-// so several 16-bit counters travel in one scan.
-MFCL_D uint64_t blockScan(uint64_t v, uint64_t& total, uint64_t* wsum) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint64_t x = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint64_t y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
-  if (lane == 63) wsum[w] = x;
-  __syncthreads();
-  uint64_t base = 0;
-  total = 0;
-#pragma unroll
-  for (int k = 0; k < kMeshBlock / 64; ++k) {
-    const uint64_t c = wsum[k];
-    if (k < w) base += c;
-    total += c;
-  }
-  __syncthreads();
-  return base + x - v;
-}
+// A step is a chain (stack entry, two gathered nodes, the box test, a barrier
+// for the sums, pushes, a barrier), about 6,000 cycles with five blocks on a
+// CU of which the wavefronts wait 60 %: what helps is more of them.  4,096
+// queries of 1e3..1e5 triangles, back to back: 273 us with a scan of the
+// lanes by shuffles and one lane for all of a pair's axes (168 registers,
+// three blocks a CU); 220 with ballots and the axes split over lanes, at four
+// blocks a CU; 194 with the pose out of the vector registers and a shorter LDS
+// stack, at five; 248 at six, where registers spill.
+constexpr int kMeshOcc = 5;
+constexpr int kMeshLds = 2048;  // LDS stack entries per block
+constexpr int kMeshStackLds = 3072;  // entries a query has besides the knob's, in LDS or in device memory
 
 template <bool PEN>
-__global__ void __launch_bounds__(kMeshBlock, 3) meshKernel(MeshArgs A) {
+__global__ void __launch_bounds__(kMeshBlock, PEN ? 3 : kMeshOcc) meshKernel(MeshArgs A) {
   __shared__ uint64_t lstk[kMeshLds];
-  __shared__ uint64_t wsum[kMeshBlock / 64];
+  __shared__ uint64_t wsum[2][kMeshBlock / 64];
+  __shared__ TriLds tri_lds[kMeshBlock / 64];
+  __shared__ tf3 s_rel;
   __shared__ uint32_t s_q;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, wave = t >> 6;
+  int turn = 0;
   uint64_t* gstk = A.stacks + static_cast<uint64_t>(blockIdx.x) * A.stack_cap;
   const float kScaleErr = 16.0f * 5.9604645e-08f;
   unsigned long long tot_bv = 0, tot_leaf = 0;
   while (true) {
     if (t == 0) s_q = atomicAdd(A.next_query, 1u);
     __syncthreads();
-    const uint32_t q = s_q;
+    const uint32_t q = __builtin_amdgcn_readfirstlane(s_q);
     __syncthreads();
     if (q >= A.n) break;
     const uint32_t ma = A.pa[q], mb = A.pb[q];
@@ -725,12 +754,22 @@ __global__ void __launch_bounds__(kMeshBlock, 3) meshKernel(MeshArgs A) {
     const uint32_t cnt1 = A.node_count[ma], cnt2 = A.node_count[mb];
     const float4* tri1 = A.tris + 3ull * A.tri_base[ma];
     const float4* tri2 = A.tris + 3ull * A.tri_base[mb];
-    m33 R;
-    d3 T;
-    relPose(A.posea + 7ull * q, A.poseb + 7ull * q, R, T);
-    const float Rq[9] = {(float)R.m00, (float)R.m01, (float)R.m02, (float)R.m10, (float)R.m11,
-                         (float)R.m12, (float)R.m20, (float)R.m21, (float)R.m22};
-    const float Tq[3] = {(float)T.x, (float)T.y, (float)T.z};
+    // the relative pose: in scalar registers for the box tests, in LDS for the triangle tests
+    float Rq[9], Tq[3];
+    {
+      m33 R;
+      d3 T;
+      relPose(A.posea + 7ull * q, A.poseb + 7ull * q, R, T);
+      const float r[9] = {(float)R.m00, (float)R.m01, (float)R.m02, (float)R.m10, (float)R.m11,
+                          (float)R.m12, (float)R.m20, (float)R.m21, (float)R.m22};
+      const float p[3] = {(float)T.x, (float)T.y, (float)T.z};
+      for (int k = 0; k < 9; ++k) Rq[k] = uniformF(r[k]);
+      for (int k = 0; k < 3; ++k) Tq[k] = uniformF(p[k]);
+      if (t == 0) {
+        s_rel.R = R;
+        s_rel.t = T;
+      }
+    }
     tf3 tf2;
     if constexpr (PEN) tf2 = poseFromQuat(A.poseb + 7ull * q);
     // block-uniform traversal state, kept identical in every thread
@@ -785,19 +824,37 @@ __global__ void __launch_bounds__(kMeshBlock, 3) meshKernel(MeshArgs A) {
       if (is_leafpair) {
         t1 = -c1 - 1;
         t2 = -c2 - 1;
-        if (triTriD(tri1 + 3 * t1, tri2 + 3 * t2, R, T)) {
-          if constexpr (PEN) triContactsD(tri1 + 3 * t1, tri2 + 3 * t2, R, T, pts, nadd, depth, nrm);
+      }
+      const unsigned long long m_leaf = ballot64(is_leafpair);
+      if (m_leaf) {
+        const bool hit = triTriWave(tri_lds[wave], is_leafpair, tri1 + 3 * t1, tri2 + 3 * t2, s_rel);
+        if (hit) {
+          if constexpr (PEN) triContactsD(tri1 + 3 * t1, tri2 + 3 * t2, s_rel.R, s_rel.t, pts, nadd, depth, nrm);
           else nadd = 1;
         }
       }
-      // one scan for four counters (16 bits each): contacts added, pushes,
-      // leaf tests, bad node ids
+      // four counters (16 bits each) of the wavefronts before this one and of
+      // all: contacts added, pushes, leaf tests, bad node ids.  A wavefront's
+      // own come from ballots (a scan of the lanes by shuffles took twelve LDS
+      // round trips); the sums alternate between two rows, so one barrier is enough.
       const bool pushes = push1 || push2;
-      const uint64_t mine = static_cast<uint64_t>(nadd) | (static_cast<uint64_t>(pushes ? 1 : 0) << 16) |
-                            (static_cast<uint64_t>(is_leafpair ? 1 : 0) << 32) |
-                            (static_cast<uint64_t>(bad ? 1 : 0) << 48);
-      uint64_t tot = 0;
-      const uint64_t pre = blockScan(mine, tot, wsum);
+      const unsigned long long m_add = ballot64(nadd > 0), m_add2 = PEN ? ballot64(nadd > 1) : 0,
+                               m_push = ballot64(pushes), m_bad = ballot64(bad);
+      if (laneId() == 0)
+        wsum[turn][wave] = static_cast<uint64_t>(__popcll(m_add) + __popcll(m_add2)) |
+                           static_cast<uint64_t>(__popcll(m_push)) << 16 |
+                           static_cast<uint64_t>(__popcll(m_leaf)) << 32 | static_cast<uint64_t>(__popcll(m_bad)) << 48;
+      __syncthreads();
+      uint64_t tot = 0, pre = 0;
+#pragma unroll
+      for (int w = 0; w < kMeshBlock / 64; ++w) {
+        const uint64_t c = wsum[turn][w];
+        if (w < wave) pre += c;
+        tot += c;
+      }
+      turn ^= 1;
+      pre += static_cast<uint64_t>(prefixBelow(m_add) + prefixBelow(m_add2)) |
+             static_cast<uint64_t>(prefixBelow(m_push)) << 16;
       const int n_add = static_cast<int>(tot & 0xFFFF), n_push = static_cast<int>((tot >> 16) & 0xFFFF);
       leaf += static_cast<int>((tot >> 32) & 0xFFFF);
       if ((tot >> 48) & 0xFFFF) {
@@ -887,7 +944,7 @@ __global__ void zeroU32(uint32_t* p, int n) {
 // 4 wavefronts per CU).
 int reserveMesh(mfcl_ctx* ctx) {
   const uint32_t waves = static_cast<uint32_t>(ctx->n_cu * ctx->tune.mesh_blocks_per_cu * 4);
-  const uint32_t cap = static_cast<uint32_t>(ctx->tune.mesh_stack);
+  const uint32_t cap = static_cast<uint32_t>(ctx->tune.mesh_stack + kMeshStackLds - kMeshLds);
   if (ctx->ws_arena.p && ctx->mesh_ws_waves == waves && ctx->mesh_ws_cap == cap) return MFCL_OK;
   ctx->mesh_ws_waves = ctx->mesh_ws_cap = 0;
   // one device-memory stack per block (4 wavefronts)
@@ -906,7 +963,7 @@ int meshCollideLaunch(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, con
     return MFCL_E_STATE;
   }
   const uint32_t waves = ctx->mesh_ws_waves, cap = ctx->mesh_ws_cap;
-  if (!ctx->ws_arena.p || waves == 0 || cap != static_cast<uint32_t>(ctx->tune.mesh_stack) ||
+  if (!ctx->ws_arena.p || waves == 0 || cap != static_cast<uint32_t>(ctx->tune.mesh_stack + kMeshStackLds - kMeshLds) ||
       waves != static_cast<uint32_t>(ctx->n_cu * ctx->tune.mesh_blocks_per_cu * 4)) {
     ctx->err = "mesh traversal stacks not sized for the current knobs";
     return MFCL_E_STATE;

@@ -142,3 +142,34 @@ def test_mesh_penetration_contacts(oracle, gpu_ctx, cap):
     print(f"\n[mesh penetration cap={cap}] hits={int(out['hit'].sum())} equal sets {n_eq} subsets {n_sub} "
           f"contacts {int(out['n_contacts'].sum())}")
     assert n_eq + n_sub > 20
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [1, 2, 15, 16, 17, 32])
+def test_mesh_dense_leaf_pairs(oracle, gpu_ctx, k):
+    """Two fans of k triangles, most of each fan crossing most of the other:
+    the triangle pairs of one traversal step are a wavefront's batch of 15
+    (pair, axis) tests, one less, one more and several, with separated and
+    intersecting pairs in one batch."""
+    rng = np.random.default_rng(60 + k)
+    verts, tris = [], []
+    for axis in (0, 1):
+        c = rng.uniform(-0.02, 0.02, (k, 1, 3))
+        u = rng.normal(size=(k, 3, 3))
+        u[:, :, axis] *= 0.2
+        verts.append((c + 0.3 * u).reshape(-1, 3).astype(np.float32))
+        tris.append(np.arange(3 * k, dtype=np.uint32).reshape(k, 3))
+    vo, vc = np.array([0, 3 * k], np.uint64), np.full(2, 3 * k, np.uint32)
+    to, tc = np.array([0, k], np.uint64), np.full(2, k, np.uint32)
+    arrays = (np.concatenate(verts), vo, vc, np.concatenate(tris), to, tc)
+    M = oracle.MeshSet(*arrays)
+    gpu_ctx.upload_meshes(*arrays)
+    n = 40
+    a, b = np.zeros(n, np.uint32), np.ones(n, np.uint32)
+    qa, qb = W.poses(rng, n, 0.0, 0.1), W.poses(rng, n, 0.0, 0.6)
+    ta, tb = oracle.pose12(qa), oracle.pose12(qb)
+    out, cont = gpu_ctx.mesh_collide(a, b, qa, qb, 1024)
+    for i in range(n):
+        full, nfull = M.collide_all(0, 1, ta[i], tb[i])
+        assert out["n_contacts"][i] == nfull
+        assert set(map(tuple, cont[i, :nfull].tolist())) == set(map(tuple, full.tolist()))
