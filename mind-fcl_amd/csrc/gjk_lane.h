@@ -23,14 +23,18 @@ namespace mfcl {
 // A simplex holds at most 4 vertices, so freeSlot() returns at most 4.
 constexpr int kLaneSlots = 5;
 
-// Per-wavefront LDS block ([field][lane], 8.5 KB): the relative transform
-// of each lane's pair and the hull
+// Per-wavefront LDS block ([field][lane], 10.5 KB): the relative transform
+// of each lane's pair, the hull
 // vertex indices of the support points recorded in each direction slot
-// (-1 for a primitive).
+// (-1 for a primitive), and for each of its two shapes that has walk blocks
+// where they start and the walk's six seeds.
 struct LaneWs {
   double tf[12][64];  // R row-major (9), t (3)
   int i0[kLaneSlots][64], i1[kLaneSlots][64];
+  uint32_t blk[2][64];      // first vertex of the hull in the block table, kNoBlk without
+  uint32_t seed[2][3][64];  // seeds of the hull's walk, two a word
 };
+constexpr uint32_t kNoBlk = ~0u;
 // The directions themselves live in device memory, [slot][xyz][lane] per
 // wavefront: they are written once per support point and read only for
 // primitive witnesses and for the EPA queue.
@@ -66,6 +70,40 @@ struct MinkLane {
     w->tf[3][lane] = t.R.m10; w->tf[4][lane] = t.R.m11; w->tf[5][lane] = t.R.m12;
     w->tf[6][lane] = t.R.m20; w->tf[7][lane] = t.R.m21; w->tf[8][lane] = t.R.m22;
     w->tf[9][lane] = t.t.x; w->tf[10][lane] = t.t.y; w->tf[11][lane] = t.t.z;
+  }
+  // The walks' starts: read once a pair, for every support call of the pair.
+  // (A vertex's block is 128 bytes, so the table has fewer than 2^32 vertices.)
+  MFCL_D void setWalks() const {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t si = k ? ib : ia;
+      uint32_t b = kNoBlk;
+      if ((k ? type1 : type0) == kConvex && T.wblk && T.nbr_off && T.nbr_off[si] >= 0 && T.vert_cnt[si] <= 65535u) {
+        b = static_cast<uint32_t>(T.vert_off[si]);
+        const int* sd = T.seed + 8 * static_cast<uint64_t>(si);
+        for (int j = 0; j < 3; ++j)
+          w->seed[k][j][lane] = static_cast<uint32_t>(sd[2 * j]) | static_cast<uint32_t>(sd[2 * j + 1]) << 16;
+      }
+      w->blk[k][lane] = b;
+    }
+  }
+  // blkInit's start: the seed of the axis direction with the largest product
+  MFCL_D int walkSeed(int k, d3 d) const {
+    int at = 0;
+    double best = 0;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const double sg = (i & 1) ? -1.0 : 1.0;
+      const double ax = (i >> 1) == 0 ? sg : sg * 0.0;
+      const double ay = (i >> 1) == 1 ? sg : sg * 0.0;
+      const double az = (i >> 1) == 2 ? sg : sg * 0.0;
+      const double dv = ax * d.x + ay * d.y + az * d.z;
+      if (i == 0 || dv > best) {
+        at = i;
+        best = dv;
+      }
+    }
+    return static_cast<int>(w->seed[k][at >> 1][lane] >> (16 * (at & 1)) & 0xFFFFu);
   }
   MFCL_D DevShape prim(int k) const {
     reloadFence();
@@ -237,6 +275,93 @@ MFCL_D void coopScanBatch(uint64_t& m, uint64_t vp, int nv, float rb, d3 d, int 
   }
 }
 
+// The walks over blocks of a lane's two hulls (blkInit, blkStep: the same
+// seeds, comparisons, order and parent rule), one after the other in one
+// loop: the wavefront makes as many steps as its lane with the most steps in
+// both walks together, not the most in the first plus the most in the
+// second, and there is one copy of the step's code.  A step is one gathered
+// block of memory latency; a support call used to add five more around the
+// walks (the shape's table entries, the seed, the vertex found), which are
+// now in LDS or in the last block.  The extreme vertices' indices go to idx0
+// and idx1, their coordinates to q0 and q1.
+MFCL_D void laneWalks(const MinkLane& md, bool w0, bool w1, d3 d0, d3 d1, int& idx0, int& idx1, float3& q0,
+                      float3& q1, int& walked) {
+  bool on = w0 || w1, first = true;
+  int k = w0 ? 0 : 1, ext = 0, parent0 = 0, parent1 = 0;
+  d3 d = w0 ? d0 : d1;
+  double ext_v = 0;
+  const float4* blk = nullptr;
+  if (on) {
+    ext = md.walkSeed(k, d);
+    blk = md.T.wblk + 8 * static_cast<uint64_t>(md.w->blk[k][md.lane]);
+  }
+  while (on) {
+    BlkWalk B;
+    const float3 q = blkLoad(blk, ext, B);
+    if (first) {
+      ext_v = d.x * static_cast<double>(q.x) + d.y * static_cast<double>(q.y) + d.z * static_cast<double>(q.z);
+      parent0 = parent1 = ext;
+      first = false;
+      ++walked;
+    }
+    bool keep = false;
+    const int old = ext;
+#pragma unroll
+    for (int j = 0; j < kWalkChunk; ++j) {
+      const int id = static_cast<int>((B.ids[j >> 1] >> (16 * (j & 1))) & 0xFFFFu);
+      if (j >= B.cnt || id == parent0 || id == parent1) continue;
+      const double v = d.x * static_cast<double>(B.nx[j][0]) + d.y * static_cast<double>(B.nx[j][1]) +
+                       d.z * static_cast<double>(B.nx[j][2]);
+      ++walked;
+      if (v > ext_v) {
+        parent1 = ext;
+        keep = true;
+        ext = id;
+        ext_v = v;
+      }
+    }
+    if (B.cnt > kWalkChunk) {
+      // neighbours beyond the eighth come from the adjacency table
+      const uint32_t si = k ? md.ib : md.ia;
+      const int* nbr = md.T.nbr + md.T.nbr_off[si];
+      const float4* verts = md.T.verts + md.T.vert_off[si];
+      const int start = __float_as_int(verts[old].w);
+      for (int c = kWalkChunk; c < B.cnt; ++c) {
+        const int id = nbr[start + 1 + c];
+        if (id == parent0 || id == parent1) continue;
+        const float4 t = verts[id];
+        const double v = d.x * static_cast<double>(t.x) + d.y * static_cast<double>(t.y) +
+                         d.z * static_cast<double>(t.z);
+        ++walked;
+        if (v > ext_v) {
+          parent1 = ext;
+          keep = true;
+          ext = id;
+          ext_v = v;
+        }
+      }
+    }
+    parent0 = old;
+    if (!keep) {
+      if (k == 0) {
+        idx0 = ext;
+        q0 = q;
+      } else {
+        idx1 = ext;
+        q1 = q;
+      }
+      on = k == 0 && w1;
+      if (on) {
+        k = 1;
+        first = true;
+        d = d1;
+        ext = md.walkSeed(1, d);
+        blk = md.T.wblk + 8 * static_cast<uint64_t>(md.w->blk[1][md.lane]);
+      }
+    }
+  }
+}
+
 // Support stage: every lane with `need` gets support(d) of its Minkowski
 // difference, recorded in its slot `id` (direction and vertex indices).
 // Wavefront-cooperative: all 64 lanes must call this together.  `scanned`
@@ -246,11 +371,19 @@ constexpr int kScanBatch = 8;
 MFCL_D void laneSupport(bool need, const MinkLane& md, d3 d, int id, MV& out, uint64_t& scanned, int& walked) {
   const d3 d1 = tmul(md.tf0().R, -d);
   int idx0 = -1, idx1 = -1;
+  const bool b0 = need && md.w->blk[0][md.lane] != kNoBlk, b1 = need && md.w->blk[1][md.lane] != kNoBlk;
 #pragma nounroll
   for (int k = 0; k < 2; ++k) {
-    const bool hull = need && (k ? md.type1 : md.type0) == kConvex;
+    // hulls without walk blocks: each lane walks its own over the adjacency
+    // table, hulls without adjacency are scanned by the wavefront together
+    const bool hull = need && !(k ? b1 : b0) && (k ? md.type1 : md.type0) == kConvex;
+    if (__ballot(hull) == 0ull) continue;
     const uint32_t si = k ? md.ib : md.ia;
-    const bool want = hull && !(md.T.nbr_off && md.T.nbr_off[si] >= 0);
+    const bool tab = hull && md.T.nbr_off && md.T.nbr_off[si] >= 0;
+    const bool want = hull && !tab;
+    const d3 dd = k ? d1 : d;
+    int res = -1;
+    if (tab) res = hullWalkTab(loadShape(md.T, si), dd, &walked);
     uint64_t vp = 0;
     int nv = 0;
     float rb = 0;
@@ -260,35 +393,26 @@ MFCL_D void laneSupport(bool need, const MinkLane& md, d3 d, int id, MV& out, ui
       nv = static_cast<int>(md.T.vert_cnt[si]);
       rb = md.T.param[si].w;
     }
-    const d3 dd = k ? d1 : d;
-    // naive hulls: cooperative scans; walking hulls: each lane walks its
-    // own (below)
     uint64_t m = __ballot(want);
-    int res = -1;
     while (m) coopScanBatch<kScanBatch>(m, vp, nv, rb, dd, md.lane, res, scanned);
     if (k) idx1 = res;
     else idx0 = res;
   }
-  {
-    const bool w0 = need && md.type0 == kConvex && md.T.nbr_off && md.T.nbr_off[md.ia] >= 0;
-    const bool w1 = need && md.type1 == kConvex && md.T.nbr_off && md.T.nbr_off[md.ib] >= 0;
-    if (w0 || w1) {
-      const DevShape s0 = loadShape(md.T, md.ia), s1 = loadShape(md.T, md.ib);
-      // one walk after the other: the lanes' independent walks already keep
-      // enough memory requests in flight, and lock-step pairs cost registers
-      if (w0) idx0 = hullWalk(s0, d, &walked);
-      if (w1) idx1 = hullWalk(s1, d1, &walked);
-    }
-  }
+  float3 q0 = make_float3(0, 0, 0), q1 = q0;
+  laneWalks(md, b0, b1, d, d1, idx0, idx1, q0, q1, walked);
   if (need) {
     d3 a, x;
-    if (idx0 >= 0) {
+    if (b0) {
+      a = d3{q0.x, q0.y, q0.z};
+    } else if (idx0 >= 0) {
       const float4 q = md.verts(0)[idx0];
       a = d3{q.x, q.y, q.z};
     } else {
       a = primSupport(md.prim(0), d);
     }
-    if (idx1 >= 0) {
+    if (b1) {
+      x = d3{q1.x, q1.y, q1.z};
+    } else if (idx1 >= 0) {
       const float4 q = md.verts(1)[idx1];
       x = d3{q.x, q.y, q.z};
     } else {

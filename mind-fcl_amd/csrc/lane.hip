@@ -43,6 +43,7 @@ MFCL_D bool laneSetup(const ShapeTables& T, const PairIO& io, const Params& P, u
       md.type1 = tb_;
       md.setTf0(relTf(poseFromQuat(io.posea + 7 * static_cast<uint64_t>(i)),
                       poseFromQuat(io.poseb + 7 * static_cast<uint64_t>(i))));
+      md.setWalks();
       if (P.use_guess) guess = d3{io.guess[3 * i], io.guess[3 * i + 1], io.guess[3 * i + 2]};
       return true;
     }

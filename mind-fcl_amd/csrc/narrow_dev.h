@@ -352,8 +352,8 @@ struct BlkWalk {
   uint32_t ids[4];
   float nx[8][3];
 };
-MFCL_D float3 blkLoad(const DevShape& s, int v, BlkWalk& B) {
-  const float4* p = s.wblk + 8 * static_cast<uint64_t>(v);
+MFCL_D float3 blkLoad(const float4* wblk, int v, BlkWalk& B) {
+  const float4* p = wblk + 8 * static_cast<uint64_t>(v);
   const float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3], q4 = p[4], q5 = p[5], q6 = p[6], q7 = p[7];
   B.cnt = __float_as_int(q0.w);
   B.ids[0] = __float_as_uint(q1.x); B.ids[1] = __float_as_uint(q1.y);
@@ -401,7 +401,7 @@ MFCL_D void blkInit(BlkState& W, const DevShape& s, d3 d, bool active, int start
       max_dot = dv;
     }
   }
-  const float3 q = blkLoad(s, init, W.B);
+  const float3 q = blkLoad(s.wblk, init, W.B);
   W.ext_v = d.x * static_cast<double>(q.x) + d.y * static_cast<double>(q.y) + d.z * static_cast<double>(q.z);
   W.ext = W.parent0 = W.parent1 = init;
   W.visited = 1;
@@ -455,7 +455,7 @@ MFCL_D void blkStep(BlkState& W, const DevShape& s) {
     }
   }
   W.parent0 = old;
-  if (W.keep) blkLoad(s, W.ext, W.B);
+  if (W.keep) blkLoad(s.wblk, W.ext, W.B);
 }
 
 MFCL_D int hullWalkBlk(const DevShape& s, d3 d, int* scanned, int start = -1) {
@@ -466,10 +466,8 @@ MFCL_D int hullWalkBlk(const DevShape& s, d3 d, int* scanned, int start = -1) {
   return W.ext;
 }
 
-// The walk over blocks when the hull has them and is not staged in LDS,
-// else over the adjacency table.
-MFCL_D int hullWalk(const DevShape& s, d3 d, int* scanned, int start = -1) {
-  if (s.wblk && !s.lv) return hullWalkBlk(s, d, scanned, start);
+// The walk over the adjacency table.
+MFCL_D int hullWalkTab(const DevShape& s, d3 d, int* scanned, int start = -1) {
   Walk W;
   walkInit(W, s, d, true, start);
   while (W.keep) {
@@ -479,6 +477,13 @@ MFCL_D int hullWalk(const DevShape& s, d3 d, int* scanned, int start = -1) {
   }
   *scanned += W.visited;
   return W.ext;
+}
+
+// The walk over blocks when the hull has them and is not staged in LDS,
+// else over the adjacency table.
+MFCL_D int hullWalk(const DevShape& s, d3 d, int* scanned, int start = -1) {
+  if (s.wblk && !s.lv) return hullWalkBlk(s, d, scanned, start);
+  return hullWalkTab(s, d, scanned, start);
 }
 
 // Two walks (either may be inactive) advanced together; ia / ib receive
