@@ -275,9 +275,16 @@ uint64_t staticScratchMaxPairs() {
 }
 
 
-// Batches of at most this many pairs run one pair per wavefront
-// (wave.hip); larger ones fill the chip with one pair per lane.
-constexpr uint64_t kWavePairs = 16384;
+// Batches of at most this many pairs run one pair per wavefront (wave.hip);
+// larger ones fill the chip with one pair per lane.  A lane's pair takes
+// 1.1-1.5 ms however few there are, a wavefront's 40-100 us.  The lines lie
+// where the wavefronts win both alone and with two other batches beside them
+// (us per batch, lane / wave; hulls of 8..512 vertices, contacts 8..256):
+//   distance    24,576 pairs: alone 1413 / 868, beside others 560 / 500
+//               32,768 pairs: alone 1550 / 1120, beside others 574 / 677
+//   penetration  8,192 pairs: alone 1663 / 1298, beside others 747 / 699
+//               16,384 pairs: alone 1668 / 1494, beside others 773 / 892
+constexpr uint64_t kWavePairsSd = 24576, kWavePairsPen = 8192;
 
 int convexQueryLaunch(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, const float* posea,
                       const float* poseb, const float* guess, uint64_t n, const mfcl_request* req,
@@ -315,6 +322,14 @@ int convexQueryLaunch(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, con
     ctx->err = "a contact array needs a collide request with penetration";
     return MFCL_E_INVALID;
   }
+  // the line of the error is part of the interface: 674 faces of 241 bytes
+  // each (1.51 vertices and edges a face), also where records take less
+  constexpr int kMaxFaces = 674;
+  if (req->epa_max_faces > kMaxFaces) {
+    ctx->err = "epa_max_faces = " + std::to_string(req->epa_max_faces) + ": the LDS of a wavefront holds at most " +
+               std::to_string(kMaxFaces);
+    return MFCL_E_UNSUPPORTED;
+  }
   const size_t full_slice = epaFullBytes(req->epa_max_faces);
   if (full_slice > static_cast<size_t>(ctx->max_lds_per_block)) {
     ctx->err = "epa_max_faces = " + std::to_string(req->epa_max_faces) + " needs " + std::to_string(full_slice) +
@@ -343,7 +358,8 @@ int convexQueryLaunch(mfcl_ctx* ctx, const uint32_t* pa, const uint32_t* pb, con
   // the boolean mode (MPR first) always takes a wavefront per pair; knob
   // values above 1 force it, 1 forces one lane per pair
   const int group = ctx->tune.gjk_group;
-  const bool waves = j.mode == kModeBool || group > 1 || (group == 0 && n <= kWavePairs);
+  const bool waves = j.mode == kModeBool || group > 1 || 
+                     (group == 0 && n <= (j.mode == kModeSd ? kWavePairsSd : kWavePairsPen));
   const unsigned nb = static_cast<unsigned>((n + kBlock - 1) / kBlock);
   if (ctx->timing) MFCL_HIP_TRY(ctx, hipEventRecord(ctx->ev[0], s));
   zeroKernel<<<1, 512, 0, s>>>(hist, 512);
