@@ -106,7 +106,7 @@ struct mfcl_ctx {
     int epa_spill{1};           // overflow continues in a device-memory polytope (1) or reruns (0)
     int epa_overflow_waves{512};   // persistent wavefronts (one per block) for overflow pairs
     int mesh_blocks_per_cu{5};  // persistent mesh-traversal blocks (4 waves, one query each) per CU
-    int mesh_stack{16384};      // node-pair stack entries per wavefront
+    int mesh_stack{16384};      // node-pair stack entries per block
     int mlp_waves{0};           // wavefronts per block of the fused warm-start inference (0: by batch size)
     int lane_refill{48};        // lane kernel: 0 one pair per lane; k > 0 refill lanes when <= k run
   } tune;

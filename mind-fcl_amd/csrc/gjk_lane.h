@@ -9,8 +9,8 @@
 // part; they are served cooperatively -- whenever lanes need a support
 // point, the wavefront scans each requesting lane's hull in turn with all
 // 64 lanes (coalesced loads, a butterfly argmax, the same FP32 scan with a
-// rounding bound and FP64 rescan as the group kernel), so every support
-// point is the same vertex.  The GJK loop is a state machine so that all
+// rounding bound and FP64 rescan), so every support point is the vertex that
+// an FP64 scan in index order finds.  The GJK loop is a state machine so that all
 // lanes meet at the one support stage:
 //   support stage (converged) -> advance every lane by one step -> ...
 // Primitive supports are closed forms evaluated by the requesting lane.
@@ -87,7 +87,8 @@ struct MinkLane {
       w->blk[k][lane] = b;
     }
   }
-  // blkInit's start: the seed of the axis direction with the largest product
+  // the walk's start: the seed of the axis direction with the largest product
+  // (convex-inl.h:151-199: +-UnitX, +-UnitY, +-UnitZ)
   MFCL_D int walkSeed(int k, d3 d) const {
     int at = 0;
     double best = 0;
@@ -112,7 +113,6 @@ struct MinkLane {
     s.type = k ? type1 : type0;
     s.p0 = p.x; s.p1 = p.y; s.p2 = p.z;
     s.verts = nullptr; s.nv = 0; s.rbound = p.w;
-    s.lv = nullptr; s.ls = 0;
     s.nbr = nullptr; s.seed = nullptr; s.wblk = nullptr;
     return s;
   }
@@ -158,7 +158,7 @@ MFCL_D double readLaneD(double v, int src) {
   return __longlong_as_double(static_cast<long long>(readLaneU64(static_cast<uint64_t>(__double_as_longlong(v)), src)));
 }
 
-// FP64 pass of hullArgmaxOOL<64> (first index attaining the FP64 maximum of
+// FP64 pass of the scan (first index attaining the FP64 maximum of
 // dot(d, v)), inline: a call inside the lane machine's loop would make every
 // value live across it occupy callee-saved registers.
 MFCL_D int waveRescan64(const float4* verts, int nv, double dx, double dy, double dz, int lane) {
@@ -187,9 +187,8 @@ MFCL_D int waveRescan64(const float4* verts, int nv, double dx, double dy, doubl
 // Argmax of dot(d_j, v) over the hulls of up to K requesting lanes at once
 // (wave-uniform parameters): lane l visits vertices l, l + 64, ... of every
 // hull, with the K hulls' loads issued together so their latencies overlap;
-// then one butterfly per hull.  The visiting order, the merge and the FP32
-// bound / FP64 rescan rule are those of hullArgmaxOOL<64>, so the indices
-// are the same.  Takes requests from `m` (lowest lanes first); the lane that
+// then one butterfly per hull.  Where the best two FP32 products are closer
+// than their rounding bound, an FP64 rescan decides.  Takes requests from `m` (lowest lanes first); the lane that
 // made request j receives its index in `res`.
 template <int K>
 MFCL_D void coopScanBatch(uint64_t& m, uint64_t vp, int nv, float rb, d3 d, int lane, int& res,
@@ -275,8 +274,8 @@ MFCL_D void coopScanBatch(uint64_t& m, uint64_t vp, int nv, float rb, d3 d, int 
   }
 }
 
-// The walks over blocks of a lane's two hulls (blkInit, blkStep: the same
-// seeds, comparisons, order and parent rule), one after the other in one
+// The walks over blocks of a lane's two hulls (the
+// reference's seeds, comparisons, order and parent rule, convex-inl.h:133-199), one after the other in one
 // loop: the wavefront makes as many steps as its lane with the most steps in
 // both walks together, not the most in the first plus the most in the
 // second, and there is one copy of the step's code.  A step is one gathered

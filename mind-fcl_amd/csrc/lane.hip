@@ -99,7 +99,7 @@ MFCL_D void laneStore(const PairIO& io, uint32_t i, const MinkLane& md, const La
 
 // One lane per pair (penetration and signed-distance modes): closed forms
 // per lane, GJK through the lane machine of gjk_lane.h.  Results, EPA queue
-// entries and scan counts equal those of narrowKernel.  dir_ws holds
+// entries and scan counts equal those of the wavefront kernel (wave.hip).  dir_ws holds
 // kLaneDirDoubles per wavefront of the grid.
 template <int MODE>
 __global__ void __launch_bounds__(kBlock) laneKernel(ShapeTables T, PairIO io, const uint32_t* order, uint64_t n,

@@ -309,8 +309,6 @@ MFCL_D void msCfg(const MeshShapeArgs& A, const MsItem& m, MFCL_LDS WaveCfg* cfg
   B.verts = m.tri;
   B.nv = 3;
   B.rbound = 0.f;
-  B.lv = nullptr;
-  B.ls = 0;
   B.nbr = nullptr;
   B.seed = nullptr;
   B.wblk = nullptr;

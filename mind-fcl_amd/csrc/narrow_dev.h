@@ -26,10 +26,6 @@ struct DevShape {
   const float4* verts;  // convex: vertices (x, y, z, unused)
   int nv;
   float rbound;         // convex: max |coordinate| over the vertices
-  // convex: optional copy of the vertices in LDS (x at lv[i], y at lv[i + ls],
-  // z at lv[i + 2 ls]); nullptr when the hull is read from device memory
-  const MFCL_LDS float* lv;
-  int ls;
   // convex with faces and more than 32 vertices: adjacency table in the
   // reference's encoding and the six axis seed vertices (support by the
   // vertex walk); nullptr: support by the naive scan
@@ -40,38 +36,14 @@ struct DevShape {
   const float4* wblk;
 };
 
-// Vertex i of a hull, from the LDS copy when there is one (same values).
-MFCL_D float3 hullVert(const DevShape& s, int i) {
-  if (s.lv) return make_float3(s.lv[i], s.lv[i + s.ls], s.lv[i + 2 * s.ls]);
-  const float4 q = s.verts[i];
-  return make_float3(q.x, q.y, q.z);
-}
-
 // Vertex i of a walking hull and the offset of its neighbour record: the
 // record offset rides in the vertex's fourth (otherwise unused) word in
 // device memory, written when the faces are uploaded, so one 16-byte load
-// serves both; the LDS copy has no fourth row and reads the table instead.
+// serves both.
 MFCL_D float3 hullVertRec(const DevShape& s, int i, int& rec) {
-  if (s.lv) {
-    rec = s.nbr[i];
-    return make_float3(s.lv[i], s.lv[i + s.ls], s.lv[i + 2 * s.ls]);
-  }
   const float4 q = s.verts[i];
   rec = __float_as_int(q.w);
   return make_float3(q.x, q.y, q.z);
-}
-
-// Copies a hull's vertices into LDS (SoA rows of stride ls), lanes lg, lg+G, ...
-template <int G>
-MFCL_D void stageHull(DevShape& s, MFCL_LDS float* dst, int ls, int lg) {
-  for (int i = lg; i < s.nv; i += G) {
-    const float4 q = s.verts[i];
-    dst[i] = q.x;
-    dst[i + ls] = q.y;
-    dst[i + 2 * ls] = q.z;
-  }
-  s.lv = dst;
-  s.ls = ls;
 }
 
 struct ShapeTables {
@@ -112,96 +84,7 @@ MFCL_D DevShape loadShape(const ShapeTables& T, uint32_t i) {
     s.verts = nullptr;
     s.nv = 0;
   }
-  s.lv = nullptr;
-  s.ls = 0;
   return s;
-}
-
-// Support-point search over a hull, shared by the G lanes that own a pair
-// (G = 1: one lane per pair).  Lane lg scans vertices lg, lg + G, ... in
-// FP32 keeping the best and runner-up scores; a butterfly over the group
-// merges them (ties resolve to the lower index).  When the FP32 gap is
-// inside the rounding bound the group rescans in FP64, so the result is the
-// first vertex attaining the FP64 maximum of dot(d, v) -- the reference's
-// naive scan result (convex-inl.h:133-149), which the reference's adjacency
-// walk also returns whenever that maximum is unique.
-// Out of line: the scan is the largest piece of code on the support path
-// and is reached from every support call site; one copy keeps the kernels'
-// instruction footprint small.  Returns the index, with bit 30 set when the
-// FP64 rescan ran.
-template <int G>
-__device__ __attribute__((noinline)) int hullArgmaxOOL(const float4* verts, const MFCL_LDS float* lv, int ls, int nv,
-                                                      float rbound, double dx, double dy, double dz, int lg) {
-  int bi = 0x7fffffff;
-  float best = -INFINITY, second = -INFINITY;
-  {
-#pragma clang fp contract(fast)
-    const float fx = static_cast<float>(dx), fy = static_cast<float>(dy), fz = static_cast<float>(dz);
-    auto visit = [&](int i, float x, float y, float z) {
-      const float val = fx * x + fy * y + fz * z;
-      if (val > best) {
-        second = best;
-        best = val;
-        bi = i;
-      } else if (val > second) {
-        second = val;
-      }
-    };
-    if (lv) {
-      for (int i = lg; i < nv; i += G) visit(i, lv[i], lv[i + ls], lv[i + 2 * ls]);
-    } else {
-      for (int i = lg; i < nv; i += G) {
-        const float4 q = verts[i];
-        visit(i, q.x, q.y, q.z);
-      }
-    }
-  }
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) {
-    const float ob = __shfl_xor(best, off, G);
-    const float os = __shfl_xor(second, off, G);
-    const int oi = __shfl_xor(bi, off, G);
-    if (ob > best || (ob == best && oi < bi)) {
-      second = fmaxf(fmaxf(second, os), best);
-      best = ob;
-      bi = oi;
-    } else {
-      second = fmaxf(fmaxf(second, os), ob);
-    }
-  }
-  // |fl32(d.v) - d.v| <= (rounding of d + 3 roundings of the dot) * |d|_1 max|v|
-  // <= 8 * 2^-24 * |d|_1 * rbound; the gap test uses twice that.
-  const float bound = 2.0f * 8.0f * 5.9604645e-08f * rbound *
-                      (fabsf(static_cast<float>(dx)) + fabsf(static_cast<float>(dy)) + fabsf(static_cast<float>(dz)));
-  // a NaN direction or vertex leaves no candidate: vertex 0 keeps every
-  // read in bounds
-  if (best - second > bound) return bi < nv ? bi : 0;
-  double bd = -INFINITY;
-  bi = 0x7fffffff;
-  for (int i = lg; i < nv; i += G) {
-    float x, y, z;
-    if (lv) {
-      x = lv[i]; y = lv[i + ls]; z = lv[i + 2 * ls];
-    } else {
-      const float4 q = verts[i];
-      x = q.x; y = q.y; z = q.z;
-    }
-    const double val = dx * static_cast<double>(x) + dy * static_cast<double>(y) + dz * static_cast<double>(z);
-    if (val > bd) {
-      bd = val;
-      bi = i;
-    }
-  }
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) {
-    const double ob = __shfl_xor(bd, off, G);
-    const int oi = __shfl_xor(bi, off, G);
-    if (ob > bd || (ob == bd && oi < bi)) {
-      bd = ob;
-      bi = oi;
-    }
-  }
-  return (bi < nv ? bi : 0) | (1 << 30);
 }
 
 // convex-inl.h:202-290: the walk starts from the seed vertex of the axis
@@ -369,103 +252,6 @@ MFCL_D float3 blkLoad(const float4* wblk, int v, BlkWalk& B) {
   return make_float3(q0.x, q0.y, q0.z);
 }
 
-struct BlkState {
-  BlkWalk B;
-  d3 d;
-  double ext_v;
-  int ext, parent0, parent1, visited;
-  bool keep;
-};
-
-MFCL_D void blkInit(BlkState& W, const DevShape& s, d3 d, bool active, int start = -1) {
-  W.d = d;
-  W.keep = active;
-  W.visited = 0;
-  W.ext = 0;
-  W.ext_v = 0;
-  W.B.cnt = 0;
-  if (!active) return;
-  int init = start;
-  double max_dot = 0;
-  if (init < 0)
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    // the seed directions of convex-inl.h:151-199: +-UnitX, +-UnitY, +-UnitZ
-    const double sg = (i & 1) ? -1.0 : 1.0;
-    const double ax = (i >> 1) == 0 ? sg : sg * 0.0;
-    const double ay = (i >> 1) == 1 ? sg : sg * 0.0;
-    const double az = (i >> 1) == 2 ? sg : sg * 0.0;
-    const double dv = ax * d.x + ay * d.y + az * d.z;
-    if (init < 0 || dv > max_dot) {
-      init = s.seed[i];
-      max_dot = dv;
-    }
-  }
-  const float3 q = blkLoad(s.wblk, init, W.B);
-  W.ext_v = d.x * static_cast<double>(q.x) + d.y * static_cast<double>(q.y) + d.z * static_cast<double>(q.z);
-  W.ext = W.parent0 = W.parent1 = init;
-  W.visited = 1;
-}
-
-MFCL_D void blkStep(BlkState& W, const DevShape& s) {
-  if (!W.keep) return;
-  W.keep = false;
-  const int old = W.ext;
-  const int count = W.B.cnt;
-  const d3 d = W.d;
-#pragma unroll
-  for (int j = 0; j < kWalkChunk; ++j) {
-    const int id = static_cast<int>((W.B.ids[j >> 1] >> (16 * (j & 1))) & 0xFFFFu);
-    if (j >= count || id == W.parent0 || id == W.parent1) continue;
-    const double v = d.x * static_cast<double>(W.B.nx[j][0]) + d.y * static_cast<double>(W.B.nx[j][1]) +
-                     d.z * static_cast<double>(W.B.nx[j][2]);
-    ++W.visited;
-    if (v > W.ext_v) {
-      W.parent1 = W.ext;
-      W.keep = true;
-      W.ext = id;
-      W.ext_v = v;
-    }
-  }
-  if (count > kWalkChunk) {
-    const int start = __float_as_int(s.verts[old].w);
-    for (int c0 = kWalkChunk; c0 < count; c0 += kWalkChunk) {
-      int id[kWalkChunk];
-      float3 w[kWalkChunk];
-#pragma unroll
-      for (int j = 0; j < kWalkChunk; ++j) {
-        const int nb = s.nbr[start + 1 + c0 + j];
-        id[j] = c0 + j < count ? nb : old;
-        const float4 t = s.verts[id[j]];
-        w[j] = make_float3(t.x, t.y, t.z);
-      }
-#pragma unroll
-      for (int j = 0; j < kWalkChunk; ++j) {
-        if (c0 + j >= count || id[j] == W.parent0 || id[j] == W.parent1) continue;
-        const double v = d.x * static_cast<double>(w[j].x) + d.y * static_cast<double>(w[j].y) +
-                         d.z * static_cast<double>(w[j].z);
-        ++W.visited;
-        if (v > W.ext_v) {
-          W.parent1 = W.ext;
-          W.keep = true;
-          W.ext = id[j];
-          W.ext_v = v;
-        }
-      }
-    }
-  }
-  W.parent0 = old;
-  if (W.keep) blkLoad(s.wblk, W.ext, W.B);
-}
-
-MFCL_D int hullWalkBlk(const DevShape& s, d3 d, int* scanned, int start = -1) {
-  BlkState W;
-  blkInit(W, s, d, true, start);
-  while (W.keep) blkStep(W, s);
-  *scanned += W.visited;
-  return W.ext;
-}
-
 // The walk over the adjacency table.
 MFCL_D int hullWalkTab(const DevShape& s, d3 d, int* scanned, int start = -1) {
   Walk W;
@@ -477,54 +263,6 @@ MFCL_D int hullWalkTab(const DevShape& s, d3 d, int* scanned, int start = -1) {
   }
   *scanned += W.visited;
   return W.ext;
-}
-
-// The walk over blocks when the hull has them and is not staged in LDS,
-// else over the adjacency table.
-MFCL_D int hullWalk(const DevShape& s, d3 d, int* scanned, int start = -1) {
-  if (s.wblk && !s.lv) return hullWalkBlk(s, d, scanned, start);
-  return hullWalkTab(s, d, scanned, start);
-}
-
-// Two walks (either may be inactive) advanced together; ia / ib receive
-// the extreme vertices of the active ones.
-MFCL_D void hullWalk2(const DevShape& sa, d3 da, bool act_a, int& ia, const DevShape& sb, d3 db, bool act_b,
-                      int& ib, int* scanned, int start_a = -1, int start_b = -1) {
-  if (sa.wblk && !sa.lv && sb.wblk && !sb.lv) {
-    BlkState A, B;
-    blkInit(A, sa, da, act_a, start_a);
-    blkInit(B, sb, db, act_b, start_b);
-    while (A.keep || B.keep) {
-      blkStep(A, sa);
-      blkStep(B, sb);
-    }
-    if (act_a) ia = A.ext;
-    if (act_b) ib = B.ext;
-    *scanned += A.visited + B.visited;
-    return;
-  }
-  Walk A, B;
-  walkInit(A, sa, da, act_a, start_a);
-  walkInit(B, sb, db, act_b, start_b);
-  while (A.keep || B.keep) {
-    walkFetchRecord(A, sa);
-    walkFetchRecord(B, sb);
-    walkFetchNeighbours(A, sa);
-    walkFetchNeighbours(B, sb);
-    walkCompare(A, sa);
-    walkCompare(B, sb);
-  }
-  if (act_a) ia = A.ext;
-  if (act_b) ib = B.ext;
-  *scanned += A.visited + B.visited;
-}
-
-template <int G>
-MFCL_D int hullArgmax(const DevShape& s, d3 d, int lg, int* scanned, int start = -1) {
-  if (s.nbr) return hullWalk(s, d, scanned, start);
-  const int r = hullArgmaxOOL<G>(s.verts, s.lv, s.ls, s.nv, s.rbound, d.x, d.y, d.z, lg);
-  *scanned += (r >> 30) ? 2 * s.nv : s.nv;
-  return r & ((1 << 30) - 1);
 }
 
 // Closed-form support points of the primitives
@@ -562,94 +300,9 @@ MFCL_D d3 primSupport(const DevShape& s, d3 dir) {
   }
 }
 
-// include/fcl/cvx_collide/gjk_shape.hpp:41-180; shape_gjk_interface-inl.h:87-92.
-template <int G>
-MFCL_D d3 shapeSupport(const DevShape& s, d3 dir, int lg, int* scanned) {
-  if (s.type == kConvex) {
-    const float3 q = hullVert(s, hullArgmax<G>(s, dir, lg, scanned));
-    return {q.x, q.y, q.z};
-  }
-  return primSupport(s, dir);
-}
-
-// shapeSupport plus the index of the hull vertex returned (-1 for primitives).
-template <int G>
-MFCL_D d3 shapeSupportI(const DevShape& s, d3 dir, int lg, int* scanned, int& idx, int start = -1) {
-  if (s.type == kConvex) {
-    idx = hullArgmax<G>(s, dir, lg, scanned, start);
-    const float3 q = hullVert(s, idx);
-    return {q.x, q.y, q.z};
-  }
-  idx = -1;
-  return shapeSupport<G>(s, dir, lg, scanned);
-}
-
-MFCL_D d3 shapeInterior(const DevShape& s, const float4* interior_tab, uint32_t id) {
-  if (s.type == kConvex) {
-    const float4 c = interior_tab[id];
-    return {c.x, c.y, c.z};
-  }
-  return {0, 0, 0};
-}
-
-// ---------------------------------------------------------------------------
-// The same Minkowski difference with its configuration (both shapes, the two
-// relative transforms, interior points) held in LDS instead of VGPRs.  The
-// lanes that own a pair all write the same values to their slot and re-read
-// them at every support call (a compiler-only memory fence stops the loads
-// being hoisted into registers), which keeps ~80 FP64 registers out of the
-// long-lived state of the GJK and EPA loops.
-#define MFCL_LDS __attribute__((address_space(3)))
-
-// Direction that produced a simplex vertex, and the hull vertex indices its
-// support points came from (-1 for a primitive shape: recomputed from the
-// direction when needed).
-struct DirSlot {
-  double d[3];
-  int i0, i1;
-};
-constexpr int kDirSlots = 8;
-
-struct MinkCfg {
-  DirSlot slot[kDirSlots];
-  double r1[9];  // frame 0 -> frame 1 rotation (toshape1)
-  double r0[9];  // frame 1 -> frame 0 rotation (toshape0)
-  double t0[3];  // frame 1 -> frame 0 translation
-  double q0[3], q1[3];  // primitive parameters of shape 0 / 1
-  double int0[3], int1[3];
-  const float4* v0;
-  const float4* v1;
-  const MFCL_LDS float* lv0;
-  const MFCL_LDS float* lv1;
-  const int* nbr0;
-  const int* nbr1;
-  const int* seed0;
-  const int* seed1;
-  const float4* wblk0;
-  const float4* wblk1;
-  int ls0, ls1;
-  int type0, type1, nv0, nv1;
-  float rb0, rb1;
-};
-
+// A compiler-only fence: values read from LDS or the tables are read again
+// after it instead of being held in registers across the GJK loop.
 MFCL_D void reloadFence() { asm volatile("" ::: "memory"); }
-
-// Wavefront-uniform copies of values that every lane holds identically.
-template <class T>
-MFCL_D T* uptr(T* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  return reinterpret_cast<T*>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-MFCL_D void uniformShape(DevShape& s) {
-  s.type = __builtin_amdgcn_readfirstlane(s.type);
-  s.nv = __builtin_amdgcn_readfirstlane(s.nv);
-  s.verts = uptr(s.verts);
-  s.nbr = uptr(s.nbr);
-  s.seed = uptr(s.seed);
-  s.wblk = uptr(s.wblk);
-}
 
 MFCL_D void storeM33(MFCL_LDS double* o, const m33& A) {
   o[0] = A.m00; o[1] = A.m01; o[2] = A.m02;
@@ -663,166 +316,6 @@ MFCL_D m33 loadM33(const MFCL_LDS double* o) {
   A.m20 = o[6]; A.m21 = o[7]; A.m22 = o[8];
   return A;
 }
-
-MFCL_D void writeCfg(MFCL_LDS MinkCfg* c, const DevShape& a, const tf3& ta, const DevShape& b, const tf3& tb,
-                     d3 int0, d3 int1) {
-  const m33 r1 = tmulm(tb.R, ta.R);
-  const tf3 t0 = relTf(ta, tb);
-  storeM33(c->r1, r1);
-  storeM33(c->r0, t0.R);
-  c->t0[0] = t0.t.x; c->t0[1] = t0.t.y; c->t0[2] = t0.t.z;
-  c->q0[0] = a.p0; c->q0[1] = a.p1; c->q0[2] = a.p2;
-  c->q1[0] = b.p0; c->q1[1] = b.p1; c->q1[2] = b.p2;
-  c->int0[0] = int0.x; c->int0[1] = int0.y; c->int0[2] = int0.z;
-  c->int1[0] = int1.x; c->int1[1] = int1.y; c->int1[2] = int1.z;
-  c->v0 = a.verts; c->v1 = b.verts;
-  c->lv0 = a.lv; c->lv1 = b.lv;
-  c->nbr0 = a.nbr; c->nbr1 = b.nbr;
-  c->seed0 = a.seed; c->seed1 = b.seed;
-  c->wblk0 = a.wblk; c->wblk1 = b.wblk;
-  c->ls0 = a.ls; c->ls1 = b.ls;
-  c->type0 = a.type; c->type1 = b.type;
-  c->nv0 = a.nv; c->nv1 = b.nv;
-  c->rb0 = a.rbound; c->rb1 = b.rbound;
-}
-
-MFCL_D d3 slotDir(const MFCL_LDS MinkCfg* c, int id) {
-  reloadFence();
-  const MFCL_LDS DirSlot& sl = c->slot[id & (kDirSlots - 1)];
-  return d3{sl.d[0], sl.d[1], sl.d[2]};
-}
-
-template <int G>
-struct MinkL {
-  MFCL_LDS MinkCfg* c;
-  int lg;
-  int scanned;
-  MFCL_D DevShape sh0() const {
-    DevShape s;
-    s.type = c->type0; s.p0 = c->q0[0]; s.p1 = c->q0[1]; s.p2 = c->q0[2];
-    s.verts = c->v0; s.nv = c->nv0; s.rbound = c->rb0;
-    s.lv = c->lv0; s.ls = c->ls0;
-    s.nbr = c->nbr0; s.seed = c->seed0; s.wblk = c->wblk0;
-    if constexpr (G == 64) uniformShape(s);  // one pair per wavefront
-    return s;
-  }
-  MFCL_D DevShape sh1() const {
-    DevShape s;
-    s.type = c->type1; s.p0 = c->q1[0]; s.p1 = c->q1[1]; s.p2 = c->q1[2];
-    s.verts = c->v1; s.nv = c->nv1; s.rbound = c->rb1;
-    s.lv = c->lv1; s.ls = c->ls1;
-    s.nbr = c->nbr1; s.seed = c->seed1; s.wblk = c->wblk1;
-    if constexpr (G == 64) uniformShape(s);  // one pair per wavefront
-    return s;
-  }
-  MFCL_D m33 rot1() const { return loadM33(c->r1); }
-  MFCL_D tf3 tf0() const {
-    tf3 t;
-    t.R = loadM33(c->r0);
-    t.t = d3{c->t0[0], c->t0[1], c->t0[2]};
-    return t;
-  }
-  MFCL_D d3 support0(d3 d) {
-    reloadFence();
-    return shapeSupport<G>(sh0(), d, lg, &scanned);
-  }
-  MFCL_D d3 support1(d3 d) {
-    reloadFence();
-    const d3 x = shapeSupport<G>(sh1(), mul(rot1(), d), lg, &scanned);
-    reloadFence();
-    return apply(tf0(), x);
-  }
-  // support points of both shapes (vertex indices, -1 for a primitive);
-  // two walking hulls walk together
-  // st0 / st1: walk starts (-1: the reference's seed)
-  MFCL_D void supportPair(d3 d, d3& a, d3& x, int& i0, int& i1, int st0 = -1, int st1 = -1) {
-    reloadFence();
-    const DevShape s0 = sh0(), s1 = sh1();
-    const d3 d1 = mul(rot1(), -d);
-    if (s0.nbr && s1.nbr) {
-      hullWalk2(s0, d, true, i0, s1, d1, true, i1, &scanned, st0, st1);
-      const float3 q0 = hullVert(s0, i0), q1 = hullVert(s1, i1);
-      a = d3{q0.x, q0.y, q0.z};
-      x = d3{q1.x, q1.y, q1.z};
-      return;
-    }
-    a = shapeSupportI<G>(s0, d, lg, &scanned, i0, st0);
-    reloadFence();
-    x = shapeSupportI<G>(sh1(), d1, lg, &scanned, i1, st1);
-  }
-  // support(d) with walk starts; i0 / i1 receive the support vertices
-  // (-1 for a primitive)
-  MFCL_D d3 supportFrom(d3 d, int st0, int st1, int& i0, int& i1) {
-    d3 a, x;
-    supportPair(d, a, x, i0, i1, st0, st1);
-    reloadFence();
-    return a - apply(tf0(), x);
-  }
-  // support0(d) / support1(-d) from a known support vertex when there is one
-  MFCL_D d3 point0At(int i0, d3 d) {
-    if (i0 >= 0) {
-      const float3 q = hullVert(sh0(), i0);
-      return d3{q.x, q.y, q.z};
-    }
-    return support0(d);
-  }
-  MFCL_D d3 point1At(int i1, d3 d) {
-    if (i1 >= 0) {
-      const float3 q = hullVert(sh1(), i1);
-      return apply(tf0(), d3{q.x, q.y, q.z});
-    }
-    return support1(-d);
-  }
-  MFCL_D d3 support(d3 d) {
-    d3 a, x;
-    int i0, i1;
-    supportPair(d, a, x, i0, i1);
-    reloadFence();
-    return a - apply(tf0(), x);
-  }
-  // support(d), recording d and the support vertex indices in slot id.
-  MFCL_D d3 supportNew(d3 d, int id) {
-    int i0, i1;
-    d3 a, x;
-    supportPair(d, a, x, i0, i1);
-    reloadFence();
-    const d3 b = apply(tf0(), x);
-    MFCL_LDS DirSlot& sl = c->slot[id & (kDirSlots - 1)];
-    sl.d[0] = d.x; sl.d[1] = d.y; sl.d[2] = d.z;
-    sl.i0 = i0; sl.i1 = i1;
-    return a - b;
-  }
-  MFCL_D d3 dirOf(int id) {
-    reloadFence();
-    const MFCL_LDS DirSlot& sl = c->slot[id & (kDirSlots - 1)];
-    return d3{sl.d[0], sl.d[1], sl.d[2]};
-  }
-  // support0(dir of slot id), from the recorded hull vertex when there is one
-  MFCL_D d3 point0(int id) {
-    reloadFence();
-    const int i0 = c->slot[id & (kDirSlots - 1)].i0;
-    if (i0 >= 0) {
-      const float3 q = hullVert(sh0(), i0);
-      return d3{q.x, q.y, q.z};
-    }
-    return support0(dirOf(id));
-  }
-  // support1(-dir of slot id), likewise
-  MFCL_D d3 point1(int id) {
-    reloadFence();
-    const int i1 = c->slot[id & (kDirSlots - 1)].i1;
-    if (i1 >= 0) {
-      const float3 q = hullVert(sh1(), i1);
-      return apply(tf0(), d3{q.x, q.y, q.z});
-    }
-    return support1(-dirOf(id));
-  }
-  MFCL_D d3 interior() {
-    reloadFence();
-    const d3 i1 = d3{c->int1[0], c->int1[1], c->int1[2]};
-    return d3{c->int0[0], c->int0[1], c->int0[2]} - apply(tf0(), i1);
-  }
-};
 
 // A simplex vertex during GJK: the Minkowski-difference point plus the id
 // of the LDS slot holding the direction that produced it and the support

@@ -22,6 +22,15 @@ namespace mfcl {
 
 enum WaveKind : int { kWavePrim = 0, kWaveScan = 1, kWaveBlk = 2, kWaveTab = 3 };
 
+// Direction that produced a simplex vertex, and the hull vertex indices its
+// support points came from (-1 for a primitive shape: recomputed from the
+// direction when needed).
+struct DirSlot {
+  double d[3];
+  int i0, i1;
+};
+constexpr int kDirSlots = 8;
+
 struct WaveShape {
   double q[3];          // primitive parameters
   const float4* verts;
@@ -141,12 +150,12 @@ struct WaveSup {
 };
 
 // All 64 lanes call this with the same arguments and get the same result.
-// Walks take the neighbour that hullWalk's sequential comparisons end on
+// Walks take the neighbour that the reference's sequential comparisons end on
 // (the first of the largest values, when it exceeds the current vertex's),
 // so they visit the same vertices; the two vertices a walk has just left are
 // compared again here, which cannot change a step (their values are below
 // the current one).  Scans return the first vertex attaining the FP64
-// maximum, as hullArgmaxOOL does, without its FP32 pre-scan: the 32 lanes'
+// maximum, without an FP32 pre-scan: the 32 lanes'
 // loads, not the FP64 products, take the time.
 __device__ __attribute__((noinline)) static WaveSup waveSupport(const MFCL_LDS WaveCfg* c, double dx, double dy, double dz) {
   const int lane = __lane_id(), sub = lane & 31, j = lane & 7;
@@ -290,7 +299,7 @@ __device__ __attribute__((noinline)) static WaveSup waveSupport(const MFCL_LDS W
 }
 
 // The Minkowski difference of the wavefront's pair, with the interface of
-// the group kernels' MinkL.
+// the lanes' MinkLane.
 struct MinkW {
   MFCL_LDS WaveCfg* c;
   int scanned;
