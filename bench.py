@@ -178,8 +178,8 @@ def main():
             ctx.convex_query_dev(dpa, dpb, dqa, dqb, n, req, dout)
 
         t_group = autotune.tune(ctx, autotune.GJK_GROUP, [1, 32], run, reps=2, log=log)
-        t_epa = autotune.tune(ctx, autotune.EPA_THREADS, [32768, 131072], run, reps=2, log=log)
-        t_lds = autotune.tune(ctx, autotune.EPA_LDS_FACES, [48, 64], run, reps=3, log=log)
+        t_epa = autotune.tune(ctx, autotune.EPA_THREADS, [131072, 196608], run, reps=2, log=log)
+        t_lds = autotune.tune(ctx, autotune.EPA_LDS_FACES, [42, 64], run, reps=3, log=log)
         tuned = {"gjk_group": min(t_group, key=t_group.get), "epa_threads": min(t_epa, key=t_epa.get),
                  "epa_lds_faces": min(t_lds, key=t_lds.get)}
         if tuned["gjk_group"] == 1:
@@ -443,7 +443,7 @@ def bench_mesh(ctx, args, threads):
         def run():
             ctx.mesh_collide_dev(dpa, dpb, dqa, dqb, n, 16, dres, dcon)
 
-        t_bpc = autotune.tune(ctx, autotune.MESH_BLOCKS_PER_CU, [2, 3], run, reps=5, log=log)
+        t_bpc = autotune.tune(ctx, autotune.MESH_BLOCKS_PER_CU, [3, 5], run, reps=5, log=log)
         tuned = {"mesh_blocks_per_cu": min(t_bpc, key=t_bpc.get)}
     for _ in range(2):
         ctx.mesh_collide_dev(dpa, dpb, dqa, dqb, n, 16, dres, dcon)

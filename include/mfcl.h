@@ -139,29 +139,31 @@ int mfcl_set_timing(mfcl_ctx* ctx, int enabled);
  * stage, ms[3] mesh traversal, ms[4] broadphase, ms[5] MLP. */
 int mfcl_last_timing(mfcl_ctx* ctx, float* ms6);
 /* Work counters of the last convex query: [0] pairs, [1] hull vertices
- * scanned by support mapping, [2] EPA pairs, [3] EPA pairs rerun at full
- * polytope capacity after exhausting the on-chip polytope. */
+ * scanned by support mapping, [2] EPA pairs, [3] EPA pairs restarted at full
+ * polytope capacity after exhausting the first LDS polytope. */
 int mfcl_last_counters(mfcl_ctx* ctx, uint64_t* c4);
 /* The same counters and more, the first n of: [0..3] as above, [4] hull
  * vertices read by the EPA stage alone, [5] EPA pairs that outgrew the
- * on-chip polytope and continued in a device-memory polytope of full
+ * first LDS polytope and continued, from a dump, in one of full
  * capacity (entries beyond 5 read 0). */
 int mfcl_last_counters_n(mfcl_ctx* ctx, uint64_t* c, int32_t n);
 
 /* Launch-shape knobs (no counterpart in the reference: GPU scheduling
  * parameters, chosen by the autotuner in mind-fcl_amd/mfcl/autotune.py). */
-#define MFCL_TUNE_GJK_GROUP 1         /* lanes per pair in the GJK stage: 1 (penetration and signed-distance
-                                         modes; cooperative hull scans), 16, 32, 64 */
+#define MFCL_TUNE_GJK_GROUP 1         /* lanes per pair in the GJK stage: 0 (default) by batch size; 1
+                                         (penetration and signed-distance modes; cooperative hull scans);
+                                         16, 32, 64: one wavefront per pair */
 #define MFCL_TUNE_EPA_THREADS 2       /* persistent EPA lanes (64 per pair), multiple of 256 */
 #define MFCL_TUNE_MESH_BLOCKS_PER_CU 3 /* persistent traversal blocks (4 wavefronts) per CU, 1..16 */
-#define MFCL_TUNE_MESH_STACK 4        /* node-pair stack entries per wavefront, 1024..262144 */
-#define MFCL_TUNE_EPA_LDS_FACES 5     /* face capacity of the LDS polytope, 16..128 */
+#define MFCL_TUNE_MESH_STACK 4        /* node-pair stack entries per block, 1024..262144 */
+#define MFCL_TUNE_EPA_LDS_FACES 5     /* face capacity of the first LDS polytope, 16..128 (64 from there on) */
 #define MFCL_TUNE_GUESS_POLICY 6      /* mfcl_mlp_guess_dev: 0 the MLP direction for every pair; 1 (default)
                                          the default guess where the MLP predicts penetration */
-#define MFCL_TUNE_EPA_SPILL 7         /* 1 (default): a pair that outgrows the LDS polytope continues in a
-                                         device-memory polytope of full capacity; 0: it reruns afterwards */
-#define MFCL_TUNE_MLP_WAVES 8         /* wavefronts per block of the fused warm-start inference (4, 8 or 16),
-                                         sharing one LDS copy of the weights; one block per CU */
+#define MFCL_TUNE_EPA_SPILL 7         /* 1 (default): a pair that outgrows the first LDS polytope is dumped and
+                                         continues at full capacity; 0: it restarts there */
+#define MFCL_TUNE_MLP_WAVES 8         /* wavefronts per block of the fused warm-start inference (4, 8 or 16; 0,
+                                         the default, by batch size), sharing one LDS copy of the weights;
+                                         one block per CU */
 #define MFCL_TUNE_LANE_REFILL 9       /* GJK lane kernel (signed distance and penetration): 0 one pair per
                                          lane over a grid of all pairs; k in 1..63 (default 48) a persistent
                                          grid whose finished lanes take new pairs once at most k lanes of
