@@ -11,7 +11,8 @@
 // connected cap found by a flood fill from its conflict face, the cap's
 // border becomes a fan of new triangles to the point, and the points that
 // saw the removed faces look for a new face they see among the fan.
-// Orientation tests run in FP64 on the FP32 coordinates; a point within a
+// Orientation tests run in FP64 on the FP32 coordinates, after an FP32 test
+// that leaves to them what it is not sure of (hull_orient.h); a point within a
 // relative 1e-12 of a face's plane does not see it, so (near-)coplanar
 // points are left out of the hull as qhull leaves out coplanar points.
 #include <hip/hip_runtime.h>
@@ -22,6 +23,7 @@
 
 #include "ctx.h"
 #include "dmath.h"
+#include "hull_orient.h"
 
 namespace mfcl {
 
@@ -90,38 +92,8 @@ MFCL_D bool sees64(d3 A, d3 B, d3 C, d3 P) {
   if (!(o > 0)) return false;
   return o > 1e-12 * sqrt(sqnorm(u) * sqnorm(v) * sqnorm(w));
 }
-// The test in 32 bits decides where it is sure.  Of u, v, w, n and the
-// products each operation rounds by at most 2^-24 of its size, eight times
-// along any path to the volume, and every term is at most |u||v||w| in
-// 1-norms: the error is below 2^-20 of that product (half of it is left
-// over, which is also far above the 64-bit test's 1e-12), plus what
-// underflows.
-struct HullPlane {
-  float ax, ay, az, nx, ny, nz, err;
-};
-MFCL_D HullPlane planeOf(const HullLds& L, int a, int b, int c) {
-  const float *A = L.xyz + 3 * a, *B = L.xyz + 3 * b, *C = L.xyz + 3 * c;
-  HullPlane q;
-  q.ax = A[0];
-  q.ay = A[1];
-  q.az = A[2];
-  const float ux = B[0] - q.ax, uy = B[1] - q.ay, uz = B[2] - q.az;
-  const float vx = C[0] - q.ax, vy = C[1] - q.ay, vz = C[2] - q.az;
-  q.nx = uy * vz - uz * vy;
-  q.ny = uz * vx - ux * vz;
-  q.nz = ux * vy - uy * vx;
-  q.err = ((fabsf(ux) + fabsf(uy) + fabsf(uz)) * (fabsf(vx) + fabsf(vy) + fabsf(vz)) + 1e-30f) * 0x1p-20f;
-  return q;
-}
-// 1 sees, 0 does not, -1 not sure
-MFCL_D int sees32(const HullPlane& q, const float* P) {
-  const float wx = P[0] - q.ax, wy = P[1] - q.ay, wz = P[2] - q.az;
-  const float o = q.nx * wx + q.ny * wy + q.nz * wz;
-  const float e = q.err * (fabsf(wx) + fabsf(wy) + fabsf(wz)) + 1e-36f;
-  return o > e ? 1 : o < -e ? 0 : -1;
-}
 MFCL_D bool sees(const HullLds& L, int a, int b, int c, int p) {
-  const int s = sees32(planeOf(L, a, b, c), L.xyz + 3 * p);
+  const int s = sees32(planeOf(L.xyz + 3 * a, L.xyz + 3 * b, L.xyz + 3 * c), L.xyz + 3 * p);
   return s >= 0 ? s != 0 : sees64(hp(L, a), hp(L, b), hp(L, c), hp(L, p));
 }
 MFCL_D bool faceSees(const HullLds& L, uint32_t v, int p) {
@@ -442,7 +414,7 @@ __global__ void __launch_bounds__(64) hullKernel(const float* pts, const uint64_
       const int G = 1 << lg, lead = l & ~(G - 1), h0 = l - lead, j0 = l >> lg, per = 64 >> lg;
       const int hl = h0 < nh ? h0 : 0;
       const HullEdge e0 = L.hor[hl];
-      const HullPlane plane = planeOf(L, e0.a, e0.b, p);
+      const HullPlane plane = planeOf(L.xyz + 3 * e0.a, L.xyz + 3 * e0.b, L.xyz + 3 * p);
       const int slot0 = slotOf(hl);
       int n_lost = 0;  // gathered points, in the border entries' spare fields
       auto flush = [&] {

@@ -229,3 +229,22 @@ def test_device_hulls_at_slice_edges(gpu_ctx, apex):
         h = ConvexHull(P.astype(np.float64))
         assert np.array_equal(hidx, np.unique(h.simplices))
         assert {tuple(sorted(hidx[t].tolist())) for t in tris} == {tuple(sorted(s.tolist())) for s in h.simplices}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exp2", [-47, 41, 42, 43, 44, 46, 80])
+def test_device_hulls_scale_with_their_points(gpu_ctx, exp2):
+    """Scaling by a power of two changes no 64-bit orientation decision, so the
+    hulls are those of the unscaled points to the last index -- also where the
+    32-bit test's volumes overflow (from about 2^42 on) or underflow."""
+    rng = np.random.default_rng(54)
+    sets = [s for s in _sets(rng) if len(s) >= 33]
+    cnt = np.array([len(s) for s in sets], np.uint32)
+    off = np.zeros(len(sets), np.uint64)
+    off[1:] = np.cumsum(cnt[:-1])
+    pts = np.concatenate(sets)
+    ref = gpu_ctx.convex_hulls(pts, off, cnt)
+    got = gpu_ctx.convex_hulls(pts * np.float32(2.0 ** exp2), off, cnt)
+    for (st0, hidx0, tris0), (st, hidx, tris) in zip(ref, got):
+        assert st0 == 0 and st == 0
+        assert np.array_equal(hidx, hidx0) and np.array_equal(tris, tris0)
