@@ -209,8 +209,9 @@ def main():
     pair_verts = float(nv[h["pair_a"]].sum() + nv[h["pair_b"]].sum())
     alg_bytes = 12.0 * pair_verts + 120.0 * n
     # secondary: the bytes of the vertex records the support searches
-    # actually request (16 B per vertex read, counted by the library, EPA's
-    # share excluded, plus a 4 B neighbour id) and 184 B of pair I/O
+    # evaluate (16 B per vertex, counted by the library -- vertices that a
+    # rounding tie has read again are not counted twice --, EPA's share
+    # excluded, plus a 4 B neighbour id) and 184 B of pair I/O
     gjk_vertices = float(counters[1]) - float(counters[4])
     support_bytes = 20.0 * gjk_vertices + 184.0 * n
     t_gjk = float(kern[:, 1].mean()) * 1e-3

@@ -139,11 +139,15 @@ int mfcl_set_timing(mfcl_ctx* ctx, int enabled);
  * stage, ms[3] mesh traversal, ms[4] broadphase, ms[5] MLP. */
 int mfcl_last_timing(mfcl_ctx* ctx, float* ms6);
 /* Work counters of the last convex query: [0] pairs, [1] hull vertices
- * scanned by support mapping, [2] EPA pairs, [3] EPA pairs restarted at full
- * polytope capacity after exhausting the first LDS polytope. */
+ * evaluated by support mapping, [2] EPA pairs, [3] EPA pairs restarted at full
+ * polytope capacity after exhausting the first LDS polytope.  A support search
+ * evaluates every vertex of a hull that it scans (counted once, also where a
+ * rounding tie has it read them again in FP64) and, of a hull that it walks,
+ * the start and all neighbours of each vertex it stood on (all are read, also
+ * the two it has just left).  The counts do not depend on the launch shape. */
 int mfcl_last_counters(mfcl_ctx* ctx, uint64_t* c4);
 /* The same counters and more, the first n of: [0..3] as above, [4] hull
- * vertices read by the EPA stage alone, [5] EPA pairs that outgrew the
+ * vertices evaluated by the EPA stage alone, [5] EPA pairs that outgrew the
  * first LDS polytope and continued, from a dump, in one of full
  * capacity (entries beyond 5 read 0). */
 int mfcl_last_counters_n(mfcl_ctx* ctx, uint64_t* c, int32_t n);

@@ -303,6 +303,7 @@ MFCL_D void laneWalks(const MinkLane& md, bool w0, bool w1, d3 d0, d3 d1, int& i
       first = false;
       ++walked;
     }
+    walked += B.cnt;
     bool keep = false;
     const int old = ext;
 #pragma unroll
@@ -311,7 +312,6 @@ MFCL_D void laneWalks(const MinkLane& md, bool w0, bool w1, d3 d0, d3 d1, int& i
       if (j >= B.cnt || id == parent0 || id == parent1) continue;
       const double v = d.x * static_cast<double>(B.nx[j][0]) + d.y * static_cast<double>(B.nx[j][1]) +
                        d.z * static_cast<double>(B.nx[j][2]);
-      ++walked;
       if (v > ext_v) {
         parent1 = ext;
         keep = true;
@@ -331,7 +331,6 @@ MFCL_D void laneWalks(const MinkLane& md, bool w0, bool w1, d3 d0, d3 d1, int& i
         const float4 t = verts[id];
         const double v = d.x * static_cast<double>(t.x) + d.y * static_cast<double>(t.y) +
                          d.z * static_cast<double>(t.z);
-        ++walked;
         if (v > ext_v) {
           parent1 = ext;
           keep = true;
@@ -364,8 +363,8 @@ MFCL_D void laneWalks(const MinkLane& md, bool w0, bool w1, d3 d0, d3 d1, int& i
 // Support stage: every lane with `need` gets support(d) of its Minkowski
 // difference, recorded in its slot `id` (direction and vertex indices).
 // Wavefront-cooperative: all 64 lanes must call this together.  `scanned`
-// (wave-uniform) counts the hull vertices read by the cooperative scans,
-// `walked` (per lane) those read by the lane's vertex walks.
+// (wave-uniform) counts the vertices of the hulls scanned cooperatively,
+// `walked` (per lane) those the lane's walks stood on or next to.
 constexpr int kScanBatch = 8;
 MFCL_D void laneSupport(bool need, const MinkLane& md, d3 d, int id, MV& out, uint64_t& scanned, int& walked) {
   const d3 d1 = tmul(md.tf0().R, -d);

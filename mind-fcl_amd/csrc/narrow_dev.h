@@ -193,6 +193,7 @@ MFCL_D void walkFetchNeighbours(Walk& W, const DevShape& s) {
 MFCL_D void walkCompare(Walk& W, const DevShape& s) {
   if (!W.keep) return;
   W.keep = false;
+  W.visited += W.count;
   const int old = W.ext;
   int next_start = W.start;
   for (int c0 = 0; c0 < W.count; c0 += kWalkChunk) {
@@ -210,7 +211,6 @@ MFCL_D void walkCompare(Walk& W, const DevShape& s) {
       if (c0 + j >= W.count || W.id[j] == W.parent0 || W.id[j] == W.parent1) continue;
       const double v = W.d.x * static_cast<double>(W.w[j].x) + W.d.y * static_cast<double>(W.w[j].y) +
                        W.d.z * static_cast<double>(W.w[j].z);
-      ++W.visited;
       if (v > W.ext_v) {
         W.parent1 = W.ext;
         W.keep = true;

@@ -143,7 +143,8 @@ MFCL_D int waveSeedAxis(d3 d) {
 
 // Support points of both shapes for direction d (frame 0): p0 = support0(d),
 // p1 = support1(-d) in frame 0; i0 / i1 the hull vertices they are (-1 for a
-// primitive); scanned the hull vertices evaluated.
+// primitive); scanned the hull vertices evaluated: all of a scanned hull's,
+// of a walked one the start and the neighbours of each vertex it stood on.
 struct WaveSup {
   d3 p0, p1;
   int i0, i1, scanned;

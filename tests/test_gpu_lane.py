@@ -76,13 +76,8 @@ def test_lane_kernel_equals_group_kernel(gpu_ctx, mode, pen, guess):
           f"gjk statuses {np.bincount(out['gjk_status'].astype(np.int64) + 1).tolist()} "
           f"epa queued {int((out['epa_status'] >= 0).sum())} counters lane {cout[:3].tolist()} group {cref[:3].tolist()}")
     assert len(bad) == 0, (bad[:10], out[bad[:3]], ref[bad[:3]])
-    # pairs, EPA pairs, EPA reruns and EPA vertices equal; the count of
-    # vertices read may
-    # differ by the rare FP64 rescan that one kernel's FP32 pre-scan needs
-    # and the other's does not (the compilers contract the FP32 dot product
-    # differently at the two call sites; the chosen vertex is the same)
-    assert cout[0] == cref[0] and cout[2] == cref[2] and cout[3] == cref[3] and cout[4] == cref[4]
-    assert abs(int(cout[1]) - int(cref[1])) <= 1e-4 * int(cref[1])
+    # pairs, vertices evaluated, EPA pairs, EPA restarts and EPA vertices
+    assert np.array_equal(cout[:5], cref[:5])
     assert (out["ok"] == -1).sum() == len(out[::97])
 
 
@@ -145,5 +140,4 @@ def test_lane_refill_thresholds_identical(gpu_ctx, walking, guess, pen):
           f"EPA queued {int((ref['epa_status'] >= 0).sum())} counters {cref[:5].tolist()}")
     for out, cnt in runs[1:]:
         assert out.tobytes() == ref.tobytes()
-        assert cnt[0] == cref[0] and cnt[2] == cref[2] and cnt[3] == cref[3] and cnt[4] == cref[4]
-        assert abs(int(cnt[1]) - int(cref[1])) <= 1e-4 * int(cref[1])
+        assert np.array_equal(cnt[:5], cref[:5])

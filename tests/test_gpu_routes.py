@@ -129,3 +129,23 @@ def test_guess_block_sizes_by_batch(gpu_ctx, n):
     assert np.all(np.isfinite(out[0][0]))
     for g, d in out[1:]:
         assert np.array_equal(g, out[0][0]) and np.array_equal(d, out[0][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("faces", [True, False])
+@pytest.mark.parametrize("pen", [0, 1])
+def test_work_counters_do_not_depend_on_the_route(gpu_ctx, pen, faces):
+    """Pairs, hull vertices evaluated (GJK's and EPA's), EPA pairs: the same for
+    one lane and one wavefront per pair, on hulls that walk and hulls that are
+    scanned."""
+    h = W.hull_pairs(3000, 33, nmin=8, nmax=512, faces=True)
+    tri = mfcl.faces_from_triangles(h["tris"], h["tri_off"], h["tri_cnt"]) if faces else None
+    gpu_ctx.upload_shapes(h["types"], h["params"], h["vert_off"], h["vert_cnt"], h["verts"], faces=tri)
+    w = dict(h, guess=np.zeros((len(h["pair_a"]), 3), np.float32))
+    req = mfcl.request(mfcl.MODE_COLLIDE, max_contacts=1, penetration=1) if pen else mfcl.request(
+        mfcl.MODE_SIGNED_DISTANCE)
+    (lane, cl), (wave, cw) = _run(gpu_ctx, w, req, 1, False), _run(gpu_ctx, w, req, 64, False)
+    assert np.array_equal(_bytes(lane), _bytes(wave))
+    print(f"\n[counters pen={pen} faces={faces}] lane {cl.tolist()} wavefront {cw.tolist()}")
+    assert cl[1] > cl[4] > 0 and cl[2] > 100
+    assert np.array_equal(cl[[0, 1, 2, 4]], cw[[0, 1, 2, 4]])
