@@ -180,8 +180,8 @@ int mfcl_tune(mfcl_ctx* ctx, int32_t knob, int32_t value);
  * shrinks it.  Synchronises the device when it grows.
  *   MFCL_WS_CONVEX: pairs per mfcl_convex_query_dev /
  *                   mfcl_convex_collide_contacts_dev call;
- *   MFCL_WS_MLP:    rows per mfcl_mlp_forward_dev / mfcl_mlp_train_step_dev
- *                   call (mfcl_mlp_guess_dev needs none).
+ *   MFCL_WS_MLP:    rows per mfcl_mlp_train_step_dev call
+ *                   (mfcl_mlp_forward_dev and mfcl_mlp_guess_dev need none).
  * The mesh traversal's stacks are sized at mfcl_upload_meshes and by
  * mfcl_tune's mesh knobs; the broadphase query needs no workspace. */
 #define MFCL_WS_CONVEX 1

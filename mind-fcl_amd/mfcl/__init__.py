@@ -699,7 +699,6 @@ class Context:
                                                 None if dist is None else dist.ptr, None))
 
     def mlp_forward_dev(self, feat: DeviceArray, n: int, out4: DeviceArray):
-        self.reserve(WS_MLP, n)
         self._check(self.lib.mfcl_mlp_forward_dev(self.h, feat.ptr, n, out4.ptr, None))
 
     def mlp_train_step_dev(self, feat: DeviceArray, target: DeviceArray, n: int, hyper=None,

@@ -57,6 +57,26 @@ def test_mlp_forward_matches_reference(gpu_ctx):
 
 
 @pytest.mark.gpu
+def test_mlp_forward_needs_no_reservation():
+    """Activations stay in registers: any number of rows, whatever was reserved."""
+    import mfcl
+
+    p, X, _ = _problem(6, 5000)
+    with mfcl.Context(0) as ctx:
+        ctx.mlp_set_params(p)
+        dX, dY = ctx.to_device(X), ctx.alloc(len(X) * 16)
+        y = []
+        for rows in (0, 1, len(X)):  # none, one, all
+            if rows:
+                ctx.reserve(mfcl.WS_MLP, rows)
+            dY.upload(np.full((len(X), 4), np.nan, np.float32))
+            ctx._check(ctx.lib.mfcl_mlp_forward_dev(ctx.h, dX.ptr, len(X), dY.ptr, None))
+            y.append(dY.download(np.zeros((len(X), 4), np.float32)))
+    assert np.all(np.isfinite(y[0]))
+    assert np.array_equal(y[0], y[1]) and np.array_equal(y[0], y[2])
+
+
+@pytest.mark.gpu
 def test_mlp_gradients_match_reference(gpu_ctx):
     p, X, T = _problem(2, 4096)
     gpu_ctx.mlp_set_params(p)
