@@ -29,6 +29,8 @@ namespace mfcl {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+// four floats of a caller's array, which is aligned to one (a 16-byte load all the same)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kBlk = 256;
 
@@ -240,9 +242,9 @@ __device__ __forceinline__ void loadWeights(uint4* lds, const uint4* pack, const
 __device__ __forceinline__ void featureOperands(const float* xf, uint64_t i, uint64_t n, int h, bf16x8* x0) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float4 u = make_float4(0, 0, 0, 0), w = u;
+    f32x4u u = {0, 0, 0, 0}, w = u;
     if (i < n) {
-      const float4* f = reinterpret_cast<const float4*>(xf + i * kMlpInPad + 16 * j + 8 * h);
+      const f32x4u* f = reinterpret_cast<const f32x4u*>(xf + i * kMlpInPad + 16 * j + 8 * h);
       u = f[0];
       w = f[1];
     }

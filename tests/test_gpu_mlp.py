@@ -18,6 +18,7 @@ Bars:
 import numpy as np
 import pytest
 
+import mfcl
 import mlp_ref as R
 
 BLOCKS = [("W1", R.OFF_W1, R.OFF_B1), ("b1", R.OFF_B1, R.OFF_W2), ("W2", R.OFF_W2, R.OFF_B2), ("b2", R.OFF_B2, R.OFF_W3),
@@ -59,8 +60,6 @@ def test_mlp_forward_matches_reference(gpu_ctx):
 @pytest.mark.gpu
 def test_mlp_forward_needs_no_reservation():
     """Activations stay in registers: any number of rows, whatever was reserved."""
-    import mfcl
-
     p, X, _ = _problem(6, 5000)
     with mfcl.Context(0) as ctx:
         ctx.mlp_set_params(p)
@@ -74,6 +73,34 @@ def test_mlp_forward_needs_no_reservation():
             y.append(dY.download(np.zeros((len(X), 4), np.float32)))
     assert np.all(np.isfinite(y[0]))
     assert np.array_equal(y[0], y[1]) and np.array_equal(y[0], y[2])
+
+
+@pytest.mark.gpu
+def test_mlp_rows_aligned_to_a_float(gpu_ctx):
+    """Feature rows, targets and outputs at 4, 8 and 12 bytes past a 16-byte
+    boundary: the same outputs, loss and gradients."""
+    import ctypes as C
+
+    p, X, T = _problem(7, 300)
+    n = len(X)
+    gpu_ctx.mlp_set_params(p)
+    got = []
+    for k in range(4):
+        pad = np.zeros(k, np.float32)
+        dX, dT = (gpu_ctx.to_device(np.concatenate([pad, a.reshape(-1)])) for a in (X, T))
+        dY = gpu_ctx.to_device(np.full(k + 4 * n, np.nan, np.float32))
+        x, t, y = (C.c_void_p(d.ptr.value + 4 * k) for d in (dX, dT, dY))
+        gpu_ctx._check(gpu_ctx.lib.mfcl_mlp_forward_dev(gpu_ctx.h, x, n, y, None))
+        out = dY.download(np.zeros(k + 4 * n, np.float32))[k:]
+        gpu_ctx.reserve(mfcl.WS_MLP, n)
+        loss = np.zeros(1, np.float32)
+        gpu_ctx._check(gpu_ctx.lib.mfcl_mlp_train_step_dev(gpu_ctx.h, x, t, n, None, 0,
+                                                           loss.ctypes.data_as(C.c_void_p), None))
+        got.append((out, loss.copy(), gpu_ctx.mlp_get_params(grads=True)[1]))
+    assert np.all(np.isfinite(got[0][0]))
+    for g in got[1:]:
+        for a, b in zip(g, got[0]):
+            assert np.array_equal(a, b)
 
 
 @pytest.mark.gpu
