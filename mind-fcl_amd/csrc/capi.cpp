@@ -22,9 +22,15 @@ int ensure(mfcl_ctx* ctx, DevBuf& b, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
   }
-  const size_t grown = bytes + bytes / 4;
+  size_t grown = bytes + bytes / 4;
   hipError_t e = hipMalloc(&b.p, grown);
+  if (e != hipSuccess) {  // no room for what later calls might need
+    (void)hipGetLastError();
+    grown = bytes;
+    e = hipMalloc(&b.p, grown);
+  }
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     ctx->err = std::string("workspace allocation failed: ") + hipGetErrorString(e);
     b.p = nullptr;
     return MFCL_E_NOMEM;
@@ -85,7 +91,8 @@ void freeAll(mfcl_ctx* c) {
   freePtr(c->ws_io.p);
   freePtr(c->ws_arm.p);
   freePtr(c->ws_cand.p);
-  c->ws_convex = c->ws_arena = c->ws_io = c->ws_arm = c->ws_cand = DevBuf();
+  freePtr(c->ws_dump.p);
+  c->ws_convex = c->ws_arena = c->ws_io = c->ws_arm = c->ws_cand = c->ws_dump = DevBuf();
   c->ws_convex_pairs = c->ws_arm_configs = 0;
   c->mesh_ws_waves = c->mesh_ws_cap = 0;
   c->d_counters = nullptr;

@@ -160,7 +160,7 @@ struct mfcl_ctx {
   // upload (query entry points never grow them) and, for the host-pointer
   // wrappers, ws_io
   mfcl::DevBuf ws_convex, ws_arena, ws_io, ws_arm;
-  mfcl::DevBuf ws_cand;         // mesh-shape candidates
+  mfcl::DevBuf ws_cand, ws_dump;  // mesh-shape candidates, pairs that continue at full capacity
   uint64_t ws_convex_pairs{0};  // pairs ws_convex holds
   uint64_t ws_arm_configs{0};   // configurations ws_arm holds (for ws_arm_key's arm)
   uint64_t ws_arm_key[4]{};     // links, broadphase cap, max pairs per config, pair capacity

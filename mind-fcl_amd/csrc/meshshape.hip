@@ -54,8 +54,7 @@ struct MeshShapeArgs {
   uint32_t* bv_tests;  // per query: OBB tests
   uint32_t* overflow;  // per query: 1 when the LDS stack would overflow
   int max_contacts;
-  int32_t* tri_tmp;    // colliding triangles in the order of arrival
-  int32_t* tri_out;
+  int32_t* tri_out;    // colliding triangles: in the order of arrival, then ascending
   int gjk_max_it;
   double gjk_tol;
 };
@@ -321,7 +320,7 @@ MFCL_D void msCfg(const MeshShapeArgs& A, const MsItem& m, MFCL_LDS WaveCfg* cfg
 MFCL_D void msHit(const MeshShapeArgs& A, uint64_t q, uint32_t t) {
   const uint32_t slot = atomicAdd(&A.counts[q], 1u);
   if (static_cast<int>(slot) < A.max_contacts)
-    A.tri_tmp[q * static_cast<uint64_t>(A.max_contacts) + slot] = static_cast<int32_t>(t);
+    A.tri_out[q * static_cast<uint64_t>(A.max_contacts) + slot] = static_cast<int32_t>(t);
 }
 __global__ void __launch_bounds__(256) msLeafKernel(MeshShapeArgs A, uint64_t ncand, int chunk) {
   __shared__ WaveCfg cfgs[4];
@@ -364,7 +363,7 @@ __global__ void __launch_bounds__(256) msLeafKernel(MeshShapeArgs A, uint64_t nc
 // reversal (bvh_solver-inl.h:55-65, shape_pair_intersect-inl.h:19-26): b1 =
 // the triangle, b2 = -1.
 struct MsPen {
-  mfcl_mesh_contact* tmp;  // n * max_contacts, in the order of arrival
+  mfcl_mesh_contact* out;  // n * max_contacts: in the order of arrival, then by triangle
   int cap_faces;           // LDS polytope capacity
   size_t slice_bytes;      // LDS bytes per wavefront
   char* dumps;             // pairs to continue
@@ -382,7 +381,7 @@ enum MsCount : int { kMsNext = 0, kMsDumps = 1, kMsRedo = 2, kMsFullNext = 3, kM
 MFCL_D void msContact(const MeshShapeArgs& A, const MsPen& E, uint64_t q, uint32_t t, d3 pos, d3 nrm, double depth) {
   const uint32_t slot = atomicAdd(&A.counts[q], 1u);
   if (static_cast<int>(slot) >= A.max_contacts) return;
-  mfcl_mesh_contact& o = E.tmp[q * static_cast<uint64_t>(A.max_contacts) + slot];
+  mfcl_mesh_contact& o = E.out[q * static_cast<uint64_t>(A.max_contacts) + slot];
   o.b1 = static_cast<int32_t>(t);
   o.b2 = -1;
   o.pos[0] = pos.x; o.pos[1] = pos.y; o.pos[2] = pos.z;
@@ -474,8 +473,8 @@ __global__ void __launch_bounds__(64) msPenFullKernel(MeshShapeArgs A, MsPen E) 
 }
 
 // Result headers, one wavefront per query.  Kept triangles (contacts) move
-// from the order of arrival to ascending triangle ids: a triangle's place is
-// the number of smaller ids (each triangle is a candidate once).
+// from the order of arrival to ascending triangle ids, in place: a triangle's
+// place is the number of smaller ids (each triangle is a candidate once).
 MFCL_D int msHeader(const MeshShapeArgs& A, uint64_t q, mfcl_mesh_result* out) {
   const uint32_t cnt = A.counts[q];
   const int kept = static_cast<int>(cnt) < A.max_contacts ? static_cast<int>(cnt) : A.max_contacts;
@@ -490,34 +489,43 @@ MFCL_D int msHeader(const MeshShapeArgs& A, uint64_t q, mfcl_mesh_result* out) {
   return kept;
 }
 constexpr int kMsMaxContacts = 1024;
-MFCL_D int msPlace(const int32_t* ids, int kept, int32_t id) {
+MFCL_D int msPlace(const MFCL_LDS int32_t* ids, int kept, int32_t id) {
   int r = 0;
   for (int j = 0; j < kept; ++j) r += ids[j] < id;
   return r;
 }
-__global__ void __launch_bounds__(64) msFinishPenKernel(MeshShapeArgs A, const mfcl_mesh_contact* tmp,
-                                                        mfcl_mesh_contact* contacts, mfcl_mesh_result* out) {
-  __shared__ int32_t ids[kMsMaxContacts];
+// LDS: the kept records (eight 8-byte words each), their triangles, their places.
+constexpr size_t kMsFinishBytes = sizeof(mfcl_mesh_contact) + 2 * sizeof(int32_t);  // a record
+__global__ void __launch_bounds__(64) msFinishPenKernel(MeshShapeArgs A, mfcl_mesh_contact* contacts,
+                                                        mfcl_mesh_result* out) {
+  extern __shared__ __align__(16) char ms_lds[];
+  static_assert(sizeof(mfcl_mesh_contact) == 64, "eight words");
+  MFCL_LDS uint64_t* rec = (MFCL_LDS uint64_t*)(ms_lds);
+  MFCL_LDS int32_t* ids = (MFCL_LDS int32_t*)(rec + 8 * A.max_contacts);
+  MFCL_LDS int32_t* place = ids + A.max_contacts;
   const uint64_t q = blockIdx.x;
   const int kept = msHeader(A, q, out), l = threadIdx.x;
-  const mfcl_mesh_contact* in = tmp + q * static_cast<uint64_t>(A.max_contacts);
-  mfcl_mesh_contact* o = contacts + q * static_cast<uint64_t>(A.max_contacts);
-  for (int i = l; i < kept; i += 64) ids[i] = in[i].b1;
+  uint64_t* w = reinterpret_cast<uint64_t*>(contacts + q * static_cast<uint64_t>(A.max_contacts));
+  for (int i = l; i < 8 * kept; i += 64) {
+    const uint64_t v = w[i];
+    rec[i] = v;
+    if (i % 8 == 0) ids[i / 8] = static_cast<int32_t>(v);  // b1
+  }
   __syncthreads();
-  for (int i = l; i < kept; i += 64) o[msPlace(ids, kept, ids[i])] = in[i];
-  // the others: b1 = b2 = -1, zeros (eight 8-byte words a record)
-  uint64_t* w = reinterpret_cast<uint64_t*>(o);
-  static_assert(sizeof(mfcl_mesh_contact) == 64, "eight words");
+  for (int i = l; i < kept; i += 64) place[i] = msPlace(ids, kept, ids[i]);
+  __syncthreads();
+  for (int i = l; i < 8 * kept; i += 64) w[8 * place[i / 8] + i % 8] = rec[i];
+  // the others: b1 = b2 = -1, zeros
   for (int i = 8 * kept + l; i < 8 * A.max_contacts; i += 64) w[i] = i % 8 == 0 ? ~0ull : 0ull;
 }
 
 __global__ void __launch_bounds__(64) msFinishKernel(MeshShapeArgs A, mfcl_mesh_result* out) {
-  __shared__ int32_t ids[kMsMaxContacts];
+  __shared__ int32_t lds_ids[kMsMaxContacts];
+  MFCL_LDS int32_t* ids = (MFCL_LDS int32_t*)(lds_ids);
   const uint64_t q = blockIdx.x;
   const int kept = msHeader(A, q, out), l = threadIdx.x;
-  const int32_t* in = A.tri_tmp + q * static_cast<uint64_t>(A.max_contacts);
   int32_t* o = A.tri_out + q * static_cast<uint64_t>(A.max_contacts);
-  for (int i = l; i < kept; i += 64) ids[i] = in[i];
+  for (int i = l; i < kept; i += 64) ids[i] = o[i];
   __syncthreads();
   for (int i = l; i < kept; i += 64) o[msPlace(ids, kept, ids[i])] = ids[i];
   for (int i = kept + l; i < A.max_contacts; i += 64) o[i] = -1;
@@ -530,6 +538,29 @@ __global__ void msZeroKernel(uint32_t* p, uint64_t n) {
 
 // Dump slots and blocks of the full-capacity pass.
 constexpr uint32_t kMsDumpSlots = 2048, kMsFullBlocks = 512;
+
+namespace {
+// Device memory of one call.
+struct DevTemp {
+  void* p{nullptr};
+  ~DevTemp() {
+    if (p) (void)hipFree(p);
+  }
+};
+// A call's workspaces stay with the context for the next call, up to this
+// much each; what a call grew beyond it is given back at its end.
+constexpr size_t kMsKeepBytes = 256ull << 20;
+struct GiveBack {
+  DevBuf& b;
+  const size_t before;
+  explicit GiveBack(DevBuf& buf) : b(buf), before(buf.bytes) {}
+  ~GiveBack() {
+    if (b.bytes <= kMsKeepBytes || b.bytes <= before) return;
+    (void)hipFree(b.p);
+    b = DevBuf();
+  }
+};
+}  // namespace
 
 int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* shape_ids, const float* pose_m7,
                      const float* pose_s7, uint64_t n, const mfcl_request* req, mfcl_mesh_result* out,
@@ -562,7 +593,9 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
   const hipStream_t s = ctx->stream;
   // the call's buffers, carved from the context's host-call workspace; the
   // candidates, whose number is known only after the tree walk, from a
-  // workspace of their own (64 per query, grown to the exact count and rerun)
+  // workspace of their own (64 per query, grown to the exact count and
+  // rerun); what only some candidates need is sized by their number
+  const GiveBack keep_io(ctx->ws_io), keep_cand(ctx->ws_cand);
   const uint64_t slots = n * static_cast<uint64_t>(maxc);
   int lds_faces = std::min(std::min(req->epa_max_faces, 42), kSmallFaces);
   while (lds_faces > 4 && 4 * epaSliceBytes<SmallMem>(lds_faces) > static_cast<size_t>(ctx->max_lds_per_block))
@@ -574,8 +607,7 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
   const bool full_lds = full_slice <= static_cast<size_t>(ctx->max_lds_per_block);
   const size_t arena_slice = full_lds ? 0 : arenaBytes<GlobalMem>(req->epa_max_faces);
   const size_t b_out = pen ? sizeof(mfcl_mesh_contact) * slots : 4 * slots;
-  const size_t sizes[] = {4 * n, 4 * n, 28 * n, 28 * n, 16 * n, 64, sizeof(mfcl_mesh_result) * n, b_out, b_out,
-                          spills ? kMsDumpSlots * epaDumpBytes(lds_faces) : 0, spills ? arena_slice * kMsFullBlocks : 0};
+  const size_t sizes[] = {4 * n, 4 * n, 28 * n, 28 * n, 16 * n, 64, sizeof(mfcl_mesh_result) * n, b_out};
   constexpr int kPieces = sizeof(sizes) / sizeof(sizes[0]);
   size_t total = 0;
   for (size_t b : sizes) total += (b + 255) & ~static_cast<size_t>(255);
@@ -618,8 +650,7 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
   A.overflow = dcnt + 3 * n;
   A.cand_count = dcc;
   A.max_contacts = maxc;
-  A.tri_tmp = reinterpret_cast<int32_t*>(piece[7]);
-  A.tri_out = reinterpret_cast<int32_t*>(piece[8]);
+  A.tri_out = reinterpret_cast<int32_t*>(piece[7]);
   A.gjk_max_it = req->gjk_max_iterations;
   A.gjk_tol = req->gjk_tolerance;
   uint64_t cap = std::max<uint64_t>(64 * n, 1 << 16);
@@ -666,26 +697,33 @@ int meshShapeCollide(mfcl_ctx* ctx, const uint32_t* mesh_ids, const uint32_t* sh
   E.epa_tol = req->epa_tolerance;
   E.cap_faces = lds_faces;
   E.slice_bytes = epaSliceBytes<SmallMem>(lds_faces);
-  E.tmp = reinterpret_cast<mfcl_mesh_contact*>(piece[7]);
-  auto* dcon = reinterpret_cast<mfcl_mesh_contact*>(piece[8]);
-  E.dumps = piece[9];
-  E.n_dumps = spills ? kMsDumpSlots : 0;
+  E.out = reinterpret_cast<mfcl_mesh_contact*>(piece[7]);
+  E.n_dumps = spills ? static_cast<uint32_t>(std::min<uint64_t>(kMsDumpSlots, ncand)) : 0;
   E.dump_bytes = epaDumpBytes(lds_faces);
+  if (E.n_dumps)
+    if (int rc = ensure(ctx, ctx->ws_dump, E.n_dumps * E.dump_bytes)) return rc;
+  E.dumps = static_cast<char*>(ctx->ws_dump.p);
+  const unsigned fb = static_cast<unsigned>(std::min<uint64_t>(kMsFullBlocks, ncand));
+  DevTemp arena;
+  if (spills && !full_lds && fb && hipMalloc(&arena.p, arena_slice * fb) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->err = "out of device memory for the mesh-shape EPA polytopes";
+    return MFCL_E_NOMEM;
+  }
   E.redo = reinterpret_cast<uint32_t*>(A.cand + cap);
   E.cnt = reinterpret_cast<uint32_t*>(dcc) + 2;
-  E.arena = piece[10];
+  E.arena = static_cast<char*>(arena.p);
   E.arena_slice = arena_slice;
   if (ncand) {
     msPenKernel<<<blocks, 256, 4 * E.slice_bytes, s>>>(A, E, ncand, chunk);
-    const unsigned fb = static_cast<unsigned>(std::min<uint64_t>(kMsFullBlocks, ncand));
     if (spills && full_lds && mid) msPenFullKernel<MidMem><<<fb, 64, full_slice, s>>>(A, E);
     else if (spills && full_lds) msPenFullKernel<LargeMem><<<fb, 64, full_slice, s>>>(A, E);
     else if (spills) msPenFullKernel<GlobalMem><<<fb, 64, kEpaHeadBytes, s>>>(A, E);
   }
-  msFinishPenKernel<<<static_cast<unsigned>(n), 64, 0, s>>>(A, E.tmp, dcon, dout);
+  msFinishPenKernel<<<static_cast<unsigned>(n), 64, kMsFinishBytes * maxc, s>>>(A, E.out, dout);
   MFCL_HIP_TRY(ctx, hipGetLastError());
   MFCL_HIP_TRY(ctx, hipMemcpyAsync(out, dout, sizeof(mfcl_mesh_result) * n, hipMemcpyDeviceToHost, s));
-  MFCL_HIP_TRY(ctx, hipMemcpyAsync(contacts, dcon, sizeof(mfcl_mesh_contact) * slots, hipMemcpyDeviceToHost, s));
+  MFCL_HIP_TRY(ctx, hipMemcpyAsync(contacts, E.out, sizeof(mfcl_mesh_contact) * slots, hipMemcpyDeviceToHost, s));
   MFCL_HIP_TRY(ctx, hipStreamSynchronize(s));
   return MFCL_OK;
 }

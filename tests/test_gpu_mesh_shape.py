@@ -152,3 +152,66 @@ def test_mesh_shape_contacts_bit_exact(oracle, gpu_ctx):
           f"contacts bit-identical on {n_eq}")
     assert all(per_type.get(t, 0) > 10 for t in (BOX, SPHERE, CAPSULE, CYLINDER, CONVEX))
     assert n_eq > 300
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pen", [0, 1])
+@pytest.mark.parametrize("cap", [1, 63, 65, 1023])
+def test_mesh_shape_contact_caps(oracle, gpu_ctx, cap, pen):
+    """The kept triangles are sorted where they lie, in LDS of the cap's size:
+    ascending, each once, among the colliding ones and (where they fit the cap)
+    all of them, with the contact's record along."""
+    n = 96
+    _, _, _, mesh_ids, shape_ids, pm, ps = _setup(oracle, gpu_ctx, 97, n)
+    run = gpu_ctx.mesh_shape_collide_contacts if pen else gpu_ctx.mesh_shape_collide
+    ref_out, ref = run(mesh_ids, shape_ids, pm, ps, mfcl.request(mfcl.MODE_COLLIDE, max_contacts=1024, penetration=pen))
+    out, got = run(mesh_ids, shape_ids, pm, ps, mfcl.request(mfcl.MODE_COLLIDE, max_contacts=cap, penetration=pen))
+    assert ref_out["n_contacts"].max() > 65 and (ref_out["n_contacts"] < 1024).all()
+    assert np.array_equal(out["hit"], ref_out["hit"])
+    assert np.array_equal(out["n_contacts"], np.minimum(ref_out["n_contacts"], cap))
+    for i in range(n):
+        k, full = out["n_contacts"][i], ref[i, :ref_out["n_contacts"][i]]
+        g = got[i, :k]
+        tri, all_tri = (g["b1"], full["b1"]) if pen else (g, full)
+        assert (np.diff(all_tri) > 0).all() and (np.diff(tri) > 0).all()
+        assert g.tobytes() == full[np.isin(all_tri, tri)].tobytes()
+        rest = got[i, k:]
+        assert (rest["b1"] == -1).all() and not rest["depth"].any() if pen else (rest == -1).all()
+
+
+def _free_bytes(ctx):
+    import ctypes as C
+
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert ctx.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.gpu
+def test_mesh_shape_call_memory():
+    """What a call of a few queries keeps does not depend on the polytope
+    capacity it asks for, and a large call's buffers are given back (each
+    context keeps at most 256 MiB of each of them)."""
+    pool = W.mesh_pool(1, 98, 300, 400)
+    with mfcl.Context(0) as ctx:
+        ctx.upload_meshes(pool["verts"], pool["vert_off"], pool["vert_cnt"], pool["tris"], pool["tri_off"],
+                          pool["tri_cnt"])
+        ctx.upload_shapes(np.array([BOX, CAPSULE], np.int32), np.array([[0.1, 0.2, 0.3, 0], [0.1, 0.2, 0, 0]], np.float32))
+        rng = np.random.default_rng(99)
+
+        def call(n, faces, cap, far=0.0):
+            pm, ps = W.poses(rng, n, 0.0, 0.0), W.poses(rng, n, far, far)
+            return ctx.mesh_shape_collide_contacts(np.zeros(n, np.uint32), np.arange(n, dtype=np.uint32) % 2, pm, ps,
+                                                   mfcl.request(mfcl.MODE_COLLIDE, max_contacts=cap, penetration=1,
+                                                                epa_max_faces=faces))[0]
+
+        for faces in (8, 256, 600):
+            call(2, faces, 8)
+        before = _free_bytes(ctx)
+        call(2, 8192, 8)
+        kept = before - _free_bytes(ctx)
+        assert not call(8192, 256, 1024, far=50.0)["hit"].any()  # 512 MiB of contacts
+        kept_large = before - _free_bytes(ctx)
+    print(f"\n[mesh-shape memory] a call at 8,192 faces keeps {kept >> 20} MiB more, a call of 512 MiB {kept_large >> 20}")
+    assert kept < 128 << 20
+    assert kept_large < 320 << 20
