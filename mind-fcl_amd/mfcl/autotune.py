@@ -25,6 +25,10 @@ EPA_SPILL = 7
 MLP_WAVES = 8
 LANE_REFILL = 9
 
+# What a context starts with (csrc/ctx.h).
+DEFAULTS = {GJK_GROUP: 0, EPA_THREADS: 196608, MESH_BLOCKS_PER_CU: 5, MESH_STACK: 16384, EPA_LDS_FACES: 42,
+            GUESS_POLICY: 1, EPA_SPILL: 1, MLP_WAVES: 0, LANE_REFILL: 48}
+
 
 def set_knob(ctx, knob: int, value: int) -> None:
     ctx._check(load_library().mfcl_tune(ctx.h, C.c_int32(knob), C.c_int32(value)))

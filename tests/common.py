@@ -1,7 +1,23 @@
 """Shared helpers for the parity tests (workload setup for oracle and device)."""
+from contextlib import contextmanager
+
 import numpy as np
 
+from mfcl import autotune
 from mfcl import workloads as W
+
+
+@contextmanager
+def knobs(ctx, values):
+    """Launch knobs {knob: value} for a block of a test; back to the defaults
+    after it (the suites share one context)."""
+    try:
+        for k, v in values.items():
+            autotune.set_knob(ctx, k, v)
+        yield
+    finally:
+        for k in values:
+            autotune.set_knob(ctx, k, autotune.DEFAULTS[k])
 
 
 def hull_shapes_for_oracle(h, idx_hulls):

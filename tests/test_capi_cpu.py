@@ -135,3 +135,19 @@ def test_dtype_views_roundtrip():
     a["distance"] = [1.0, -2.0, 3.5]
     b = np.frombuffer(a.tobytes(), mfcl.CONVEX_RESULT_DTYPE)
     assert np.array_equal(b["distance"], a["distance"])
+
+
+def test_knob_defaults_are_the_contexts():
+    """The defaults that the autotuner's users (and the tests) go back to are
+    those a context is created with."""
+    import re
+
+    from mfcl import autotune
+
+    text = open(os.path.join(ROOT, "mind-fcl_amd", "csrc", "ctx.h")).read()
+    tune = dict(re.findall(r"^    int (\w+)\{(\d+)\};", text[text.index("launch-shape knobs"):text.index("} tune;")], re.M))
+    names = {n.lower(): getattr(autotune, n) for n in ("GJK_GROUP", "EPA_THREADS", "MESH_BLOCKS_PER_CU", "MESH_STACK",
+                                                       "EPA_LDS_FACES", "GUESS_POLICY", "EPA_SPILL", "MLP_WAVES",
+                                                       "LANE_REFILL")}
+    assert set(autotune.DEFAULTS) == set(names.values())
+    assert {k: int(tune[n]) for n, k in names.items()} == autotune.DEFAULTS

@@ -5,14 +5,15 @@
   1124-1127): GJK iteration caps of 0, 1 and 2 (IterLimit paths and GJK
   giving up before separation is proven), EPA iteration caps of 1 and 3
   (IterationLimit), and EPA face capacities of 8 (MallocFailed inside the
-  on-chip polytope) and 96 (pairs that outgrow the on-chip polytope rerun at
-  full capacity);
+  first LDS polytope) and 96 (pairs that outgrow it continue at full
+  capacity);
 * an empty batch.
-Both GJK kernels, hulls with faces (vertex walk) and without.
+One lane and one wavefront per pair, the default choice, hulls with faces (vertex walk) and without.
 """
 import numpy as np
 import pytest
 
+from common import knobs
 from mfcl import autotune
 from mfcl import workloads as W
 import mfcl
@@ -35,15 +36,12 @@ def _compare(out, ref):
 
 
 def _run(ctx, h, sel, req, group):
-    autotune.set_knob(ctx, autotune.GJK_GROUP, group)
-    try:
+    with knobs(ctx, {autotune.GJK_GROUP: group}):
         return ctx.convex_query(h["pair_a"][sel], h["pair_b"][sel], h["pose_a"][sel], h["pose_b"][sel], req)
-    finally:
-        autotune.set_knob(ctx, autotune.GJK_GROUP, 1)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("group", [1, 32])
+@pytest.mark.parametrize("group", [0, 1, 32])
 @pytest.mark.parametrize("n", [1, 63, 65, 257])
 def test_ragged_sizes(oracle, gpu_ctx, setup, n, group):
     h, S, _, faces = setup
@@ -66,7 +64,7 @@ LIMITS = [  # gjk_max_iterations, epa_max_faces, epa_max_iterations
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("walk", [True, False])
-@pytest.mark.parametrize("group", [1, 32])
+@pytest.mark.parametrize("group", [0, 1, 32])
 @pytest.mark.parametrize("gjk_it,epa_faces,epa_it", LIMITS)
 def test_solver_limits(oracle, gpu_ctx, setup, gjk_it, epa_faces, epa_it, group, walk):
     h, S_walk, S_naive, faces = setup
@@ -88,28 +86,24 @@ def test_solver_limits(oracle, gpu_ctx, setup, gjk_it, epa_faces, epa_it, group,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("group", [0, 1])
 @pytest.mark.parametrize("lds_faces,epa_threads", [(16, 131072), (24, 524288), (48, 131072)])
-def test_epa_continuation_and_rerun(oracle, gpu_ctx, setup, lds_faces, epa_threads):
-    """Pairs that outgrow the LDS polytope continue in a device-memory
-    polytope of full capacity (the first 2048 wavefronts of the EPA grid) or
-    rerun at full capacity (the others): results equal the oracle's at the
-    request's capacity, field for field."""
+def test_epa_continuation_and_rerun(oracle, gpu_ctx, setup, lds_faces, epa_threads, group):
+    """Pairs that outgrow the first LDS polytope continue from a dump in one of
+    full capacity, or restart there when no dump is free: results equal the
+    oracle's at the request's capacity, field for field."""
     h, S, _, faces = setup
     gpu_ctx.upload_shapes(h["types"], h["params"], h["vert_off"], h["vert_cnt"], h["verts"], faces=faces)
     ta, tb = oracle.pose12(h["pose_a"]), oracle.pose12(h["pose_b"])
     ref, _ = S.signed_distance(h["pair_a"], h["pair_b"], ta, tb, threads=8)
-    autotune.set_knob(gpu_ctx, autotune.EPA_LDS_FACES, lds_faces)
-    autotune.set_knob(gpu_ctx, autotune.EPA_THREADS, epa_threads)
-    try:
+    with knobs(gpu_ctx, {autotune.GJK_GROUP: group, autotune.EPA_LDS_FACES: lds_faces,
+                         autotune.EPA_THREADS: epa_threads}):
         out = gpu_ctx.convex_query(h["pair_a"], h["pair_b"], h["pose_a"], h["pose_b"],
                                    mfcl.request(mfcl.MODE_SIGNED_DISTANCE))
         c = gpu_ctx.last_counters()
-    finally:
-        autotune.set_knob(gpu_ctx, autotune.EPA_LDS_FACES, 64)
-        autotune.set_knob(gpu_ctx, autotune.EPA_THREADS, 131072)
     diff = _compare(out, ref)
-    print(f"\n[epa lds_faces={lds_faces} threads={epa_threads}] EPA pairs {int(c[2])} continued in device memory "
-          f"{int(c[5])} rerun {int(c[3])} differing {diff}")
+    print(f"\n[epa lds_faces={lds_faces} threads={epa_threads}] EPA pairs {int(c[2])} continued "
+          f"{int(c[5])} restarted {int(c[3])} differing {diff}")
     assert all(v == 0 for v in diff.values())
     if lds_faces < 48:
         assert c[5] + c[3] > 0

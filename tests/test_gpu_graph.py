@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 
 import mfcl
+from common import knobs
+from mfcl import autotune
 from mfcl import workloads as W
 
 
@@ -14,9 +16,16 @@ def _records(a):
 
 
 @pytest.mark.gpu
-def test_graph_convex_warm_start_sequence(gpu_ctx):
+@pytest.mark.parametrize("group", [0, 1])
+def test_graph_convex_warm_start_sequence(gpu_ctx, group):
     """MLP guesses + the warm-started signed-distance query + a boolean
-    collide query, recorded once, replayed three times."""
+    collide query, recorded once, replayed three times: distances by the
+    batch's own route (a wavefront per pair) and by lanes."""
+    with knobs(gpu_ctx, {autotune.GJK_GROUP: group}):
+        _convex_warm_start_sequence(gpu_ctx)
+
+
+def _convex_warm_start_sequence(gpu_ctx):
     h = W.hull_pairs(20000, 13, faces=True)
     gpu_ctx.upload_shapes(h["types"], h["params"], h["vert_off"], h["vert_cnt"], h["verts"],
                           faces=mfcl.faces_from_triangles(h["tris"], h["tri_off"], h["tri_cnt"]))

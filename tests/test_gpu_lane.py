@@ -1,7 +1,7 @@
 """GPU: the one-lane-per-pair GJK kernel (cooperative hull scans) against the
-group kernel and the oracle.
+one-wavefront-per-pair kernel and the oracle.
 
-The lane kernel runs the same FP64 operations in the same order as the group
+The lane kernel runs the same FP64 operations in the same order as the wavefront
 kernel, only scheduled differently, so the bar between them is bit equality
 of every result record (and equal work counters), on a mixed
 workload (hull-hull, hull-primitive and primitive-primitive pairs, hulls of
@@ -12,6 +12,7 @@ kernels also equal the oracle bit for bit on hulls given as vertex sets.
 import numpy as np
 import pytest
 
+from common import knobs
 from mfcl import autotune
 from mfcl import workloads as W
 import mfcl
@@ -44,13 +45,10 @@ def _run(ctx, w, req, group, guess):
     n = len(w["pair_a"])
     dev = [ctx.to_device(np.ascontiguousarray(w[k])) for k in ("pair_a", "pair_b", "pose_a", "pose_b", "guess")]
     dout = ctx.alloc(n * mfcl.CONVEX_RESULT_DTYPE.itemsize)
-    autotune.set_knob(ctx, autotune.GJK_GROUP, group)
-    try:
+    with knobs(ctx, {autotune.GJK_GROUP: group}):
         ctx.convex_query_dev(dev[0], dev[1], dev[2], dev[3], n, req, dout, guess=dev[4] if guess else None)
         ctx.sync()
         cnt = ctx.last_counters().copy()
-    finally:
-        autotune.set_knob(ctx, autotune.GJK_GROUP, 1)
     out = np.zeros(n, mfcl.CONVEX_RESULT_DTYPE)
     dout.download(out)
     for d in dev + [dout]:
@@ -72,9 +70,9 @@ def test_lane_kernel_equals_group_kernel(gpu_ctx, mode, pen, guess):
     out, cout = _run(gpu_ctx, w, req, 1, guess)
     diff = out.view(np.uint8).reshape(len(out), -1) != ref.view(np.uint8).reshape(len(ref), -1)
     bad = np.nonzero(diff.any(1))[0]
-    print(f"\n[lane vs group {mode} guess={guess}] pairs={len(out)} differing={len(bad)} "
+    print(f"\n[lane vs wavefront {mode} guess={guess}] pairs={len(out)} differing={len(bad)} "
           f"gjk statuses {np.bincount(out['gjk_status'].astype(np.int64) + 1).tolist()} "
-          f"epa queued {int((out['epa_status'] >= 0).sum())} counters lane {cout[:3].tolist()} group {cref[:3].tolist()}")
+          f"epa queued {int((out['epa_status'] >= 0).sum())} counters lane {cout[:3].tolist()} wavefront {cref[:3].tolist()}")
     assert len(bad) == 0, (bad[:10], out[bad[:3]], ref[bad[:3]])
     # pairs, vertices evaluated, EPA pairs, EPA restarts and EPA vertices
     assert np.array_equal(cout[:5], cref[:5])
@@ -82,7 +80,7 @@ def test_lane_kernel_equals_group_kernel(gpu_ctx, mode, pen, guess):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("group", [1, 32])
+@pytest.mark.parametrize("group", [0, 1, 32])
 def test_hull_signed_distance_bit_exact_vs_naive_oracle(oracle, gpu_ctx, group):
     """Hulls given as bare vertex sets use the naive support scan
     (convex-inl.h:133-149) in the reference, the oracle and both GPU kernels;
@@ -94,11 +92,8 @@ def test_hull_signed_distance_bit_exact_vs_naive_oracle(oracle, gpu_ctx, group):
     ref, _ = S.signed_distance(h["pair_a"], h["pair_b"], ta, tb, threads=8)
     gpu_ctx.upload_shapes(h["types"], h["params"], h["vert_off"], h["vert_cnt"], h["verts"])
     req = mfcl.request(mfcl.MODE_SIGNED_DISTANCE)
-    autotune.set_knob(gpu_ctx, autotune.GJK_GROUP, group)
-    try:
+    with knobs(gpu_ctx, {autotune.GJK_GROUP: group}):
         out = gpu_ctx.convex_query(h["pair_a"], h["pair_b"], h["pose_a"], h["pose_b"], req)
-    finally:
-        autotune.set_knob(gpu_ctx, autotune.GJK_GROUP, 1)
     fields = ("ok", "gjk_status", "epa_status", "gjk_iters", "epa_iters", "distance", "pa", "pb")
     diff = {f: int((out[f] != ref[f]).reshape(len(out), -1).any(1).sum()) for f in fields}
     print(f"\n[naive oracle, group {group}] pairs={len(out)} intersecting={int((ref['distance'] < 0).sum())} "
@@ -129,12 +124,9 @@ def test_lane_refill_thresholds_identical(gpu_ctx, walking, guess, pen):
     else:
         req = mfcl.request(mfcl.MODE_SIGNED_DISTANCE, use_guess=int(guess))
     runs = []
-    try:
-        for k in (0, 1, 48, 63):
-            autotune.set_knob(gpu_ctx, autotune.LANE_REFILL, k)
+    for k in (0, 1, 48, 63):
+        with knobs(gpu_ctx, {autotune.LANE_REFILL: k}):
             runs.append(_run(gpu_ctx, w, req, 1, guess))
-    finally:
-        autotune.set_knob(gpu_ctx, autotune.LANE_REFILL, 48)
     ref, cref = runs[0]
     print(f"\n[lane refill walking={walking} guess={guess} pen={pen}] pairs={len(ref)} "
           f"EPA queued {int((ref['epa_status'] >= 0).sum())} counters {cref[:5].tolist()}")

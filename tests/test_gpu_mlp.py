@@ -20,6 +20,7 @@ import pytest
 
 import mfcl
 import mlp_ref as R
+from common import knobs
 
 BLOCKS = [("W1", R.OFF_W1, R.OFF_B1), ("b1", R.OFF_B1, R.OFF_W2), ("W2", R.OFF_W2, R.OFF_B2), ("b2", R.OFF_B2, R.OFF_W3),
           ("W3", R.OFF_W3, R.OFF_B3), ("b3", R.OFF_B3, R.OFF_W4), ("W4", R.OFF_W4, R.OFF_B4), ("b4", R.OFF_B4, R.N_PARAMS)]
@@ -179,9 +180,8 @@ def test_fused_guess_matches_layered_forward(gpu_ctx):
     dg, dd = gpu_ctx.alloc(n * 12), gpu_ctx.alloc(n * 4)
     gpu_ctx.mlp_features_dev(dpa, dpb, dqa, dqb, n, dfeat)
     gpu_ctx.mlp_forward_dev(dfeat, n, dy)
-    autotune.set_knob(gpu_ctx, autotune.GUESS_POLICY, 0)
-    gpu_ctx.mlp_guess_dev(dpa, dpb, dqa, dqb, n, dg, dd)
-    autotune.set_knob(gpu_ctx, autotune.GUESS_POLICY, 1)
+    with knobs(gpu_ctx, {autotune.GUESS_POLICY: 0}):
+        gpu_ctx.mlp_guess_dev(dpa, dpb, dqa, dqb, n, dg, dd)
     feat = np.zeros((n, 64), np.float32)
     y = np.zeros((n, 4), np.float32)
     g = np.zeros((n, 3), np.float32)
@@ -218,16 +218,13 @@ def test_fused_guess_same_for_every_block_shape(gpu_ctx):
     dqa, dqb = gpu_ctx.to_device(h["pose_a"]), gpu_ctx.to_device(h["pose_b"])
     dg, dd = gpu_ctx.alloc(n * 12), gpu_ctx.alloc(n * 4)
     outs = []
-    try:
-        for waves in (4, 8, 16):
-            autotune.set_knob(gpu_ctx, autotune.MLP_WAVES, waves)
+    for waves in (4, 8, 16):
+        with knobs(gpu_ctx, {autotune.MLP_WAVES: waves}):
             gpu_ctx.mlp_guess_dev(dpa, dpb, dqa, dqb, n, dg, dd)
-            g, d = np.zeros((n, 3), np.float32), np.zeros(n, np.float32)
-            dg.download(g)
-            dd.download(d)
-            outs.append((g, d))
-    finally:
-        autotune.set_knob(gpu_ctx, autotune.MLP_WAVES, 8)
+        g, d = np.zeros((n, 3), np.float32), np.zeros(n, np.float32)
+        dg.download(g)
+        dd.download(d)
+        outs.append((g, d))
     for g, d in outs[1:]:
         assert np.array_equal(g, outs[0][0]) and np.array_equal(d, outs[0][1])
     assert np.all(np.isfinite(outs[0][0]))

@@ -15,6 +15,7 @@ import pytest
 
 import mlp_ref as R
 import mfcl
+from common import knobs
 from mfcl import autotune
 from mfcl import workloads as W
 from test_gpu_edge import _compare, setup  # noqa: F401  (fixture)
@@ -48,16 +49,10 @@ def test_epa_capacities(oracle, gpu_ctx, setup, faces, lds_faces, spill, group):
     ta, tb = oracle.pose12(h["pose_a"]), oracle.pose12(h["pose_b"])
     sp = np.array([128, 1e-6, faces, 255, 1e-6, 0], np.float64)
     ref, _ = S.signed_distance(h["pair_a"], h["pair_b"], ta, tb, solver=sp, threads=8)
-    knobs = ((autotune.GJK_GROUP, group, 1), (autotune.EPA_LDS_FACES, lds_faces, 64), (autotune.EPA_SPILL, spill, 1))
-    for k, v, _ in knobs:
-        autotune.set_knob(gpu_ctx, k, v)
-    try:
+    with knobs(gpu_ctx, {autotune.GJK_GROUP: group, autotune.EPA_LDS_FACES: lds_faces, autotune.EPA_SPILL: spill}):
         out = gpu_ctx.convex_query(h["pair_a"], h["pair_b"], h["pose_a"], h["pose_b"],
                                    mfcl.request(mfcl.MODE_SIGNED_DISTANCE, epa_max_faces=faces))
         c = gpu_ctx.last_counters()
-    finally:
-        for k, _, v in knobs:
-            autotune.set_knob(gpu_ctx, k, v)
     assert all(v == 0 for v in _compare(out, ref).values())
     with pytest.raises(RuntimeError, match="675"):
         gpu_ctx.convex_query(h["pair_a"], h["pair_b"], h["pose_a"], h["pose_b"],
@@ -118,14 +113,11 @@ def test_guess_block_sizes_by_batch(gpu_ctx, n):
                                           rng.integers(0, len(h["types"]), n).astype(np.uint32),
                                           W.poses(rng, n, 0.0, 1.0), W.poses(rng, n, 0.0, 1.0))]
     out = []
-    try:
-        for waves in (0, 4, 16):
-            autotune.set_knob(gpu_ctx, autotune.MLP_WAVES, waves)
+    for waves in (0, 4, 16):
+        with knobs(gpu_ctx, {autotune.MLP_WAVES: waves}):
             dg, dd = gpu_ctx.to_device(np.full((n, 3), np.nan, np.float32)), gpu_ctx.alloc(n * 4)
             gpu_ctx.mlp_guess_dev(*dev, n, dg, dd)
             out.append((dg.download(np.zeros((n, 3), np.float32)), dd.download(np.zeros(n, np.float32))))
-    finally:
-        autotune.set_knob(gpu_ctx, autotune.MLP_WAVES, 0)
     assert np.all(np.isfinite(out[0][0]))
     for g, d in out[1:]:
         assert np.array_equal(g, out[0][0]) and np.array_equal(d, out[0][1])

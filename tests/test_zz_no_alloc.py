@@ -9,6 +9,8 @@ import numpy as np
 import pytest
 
 import mfcl
+from common import knobs
+from mfcl import autotune
 from mfcl import workloads as W
 
 
@@ -34,7 +36,13 @@ def _run(ctx, fn, dev, n, req):
 
 
 @pytest.mark.gpu
-def test_static_workspace_query_matches_reserved(gpu_ctx):
+@pytest.mark.parametrize("group", [0, 1])
+def test_static_workspace_query_matches_reserved(gpu_ctx, group):
+    with knobs(gpu_ctx, {autotune.GJK_GROUP: group}):
+        _static_workspace_query_matches_reserved(gpu_ctx)
+
+
+def _static_workspace_query_matches_reserved(gpu_ctx):
     lib = gpu_ctx.lib
     cap = C.c_uint64(0)
     assert lib.mfcl_convex_query_static_dev_max_pairs(C.byref(cap)) == 0
