@@ -92,7 +92,7 @@ def cpu_baseline(h, geom, n_sample, threads, target_cpu_s=10.0):
 def measured_traffic(tuned):
     """HBM bytes per launch of the lane GJK kernel on this workload, from the
     rocprofv3 passes summarised in profiles/ (read bytes from the L2's read
-    requests by size, written bytes from WRITE_SIZE); None when the group
+    requests by size, written bytes from WRITE_SIZE); None when the wavefront
     kernel was chosen (not profiled)."""
     if tuned.get("gjk_group", 1) != 1:
         return None
@@ -217,8 +217,8 @@ def main():
     t_gjk = float(kern[:, 1].mean()) * 1e-3
     achieved = alg_bytes / t_gjk / 1e9
     log(f"[gpu] {ms_step:.3f} ms/step; kernels ms (order, gjk, epa) = {kern.mean(0)}; "
-        f"epa pairs {int(counters[2])} (rerun at full capacity {int(counters[3])}); "
-        f"vertices scanned {int(counters[1])}")
+        f"epa pairs {int(counters[2])} (restarted at full capacity {int(counters[3])}); "
+        f"vertices evaluated {int(counters[1])}")
     ep = out["epa_status"] >= 0
     if ep.any():
         it = out["epa_iters"][ep].astype(np.int64)
@@ -252,7 +252,7 @@ def main():
         },
         "roofline": {
             "kernel": "laneKernelRSd (GJK stage, lanes refilled)" if tuned.get("gjk_group", 1) == 1
-                      else "narrowKernel (GJK stage)",
+                      else "waveKernel (whole pairs)",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,

@@ -136,7 +136,9 @@ int mfcl_sync(mfcl_ctx* ctx);
  * durations of the last query are read back with mfcl_last_timing(). */
 int mfcl_set_timing(mfcl_ctx* ctx, int enabled);
 /* ms[0] order/bucketing kernels, ms[1] GJK/closed-form stage, ms[2] EPA
- * stage, ms[3] mesh traversal, ms[4] broadphase, ms[5] MLP. */
+ * stage, ms[3] mesh traversal, ms[4] broadphase, ms[5] MLP.  Where a
+ * wavefront takes a whole pair (small batches, boolean queries) ms[1] holds
+ * its EPA too and ms[2] only the pairs that continue at full capacity. */
 int mfcl_last_timing(mfcl_ctx* ctx, float* ms6);
 /* Work counters of the last convex query: [0] pairs, [1] hull vertices
  * evaluated by support mapping, [2] EPA pairs, [3] EPA pairs restarted at full

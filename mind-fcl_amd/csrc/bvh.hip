@@ -5,10 +5,10 @@
 // breadth-first (siblings adjacent) as 64-byte FP32 nodes; node boxes are
 // inflated when rounded to FP32 so they still contain their triangles.
 //
-// Device: a persistent grid of wavefronts; each wavefront takes one query at
-// a time from an atomic counter and runs the bounding-volume test tree
+// Device: a persistent grid of blocks; each block takes one query at a time
+// from an atomic counter and runs the bounding-volume test tree
 // (reference: narrowphase/detail/traversal/collision/bvh_solver-inl.h:75-164)
-// 64 node pairs per step off a wave-private stack in device memory:
+// 256 node pairs per step off its stack in LDS and device memory:
 // FP32 OBB separating-axis tests with a rounding margin (never prunes a pair
 // the FP64 test keeps), ballot/prefix compaction of children and contacts,
 // and the 17-axis triangle test in FP64 with contraction off, so a leaf
@@ -708,9 +708,10 @@ MFCL_D void triContactsD(const float4* P, const float4* Qm, const m33& R, d3 T, 
 // pushes children and contacts with block-wide prefix sums.  A whole block
 // per query cuts the number of dependent steps of the costliest queries,
 // which set the launch's duration.  Descent rule as the reference (the
-// larger inner node first); the pop order differs, so with a contact cap the
-// kept contacts are a subset of the full set rather than the reference's
-// first ones.  PEN: contacts with position, normal and depth (each
+// larger inner node first); the pop order differs (and follows how much of
+// the stack is in LDS), so with a contact cap the kept contacts are a subset
+// of the full set rather than the reference's first ones, and the counts of
+// tests of a query that reaches the cap depend on it.  PEN: contacts with position, normal and depth (each
 // colliding triangle pair adds 0-2 of them, shape_pair_intersect-inl.h:
 // 226-254), and a query collides when it has a contact, as a
 // CollisionResult with contacts does.
@@ -718,11 +719,13 @@ constexpr int kMeshBlock = 256;
 // A step is a chain (stack entry, two gathered nodes, the box test, a barrier
 // for the sums, pushes, a barrier), about 6,000 cycles with five blocks on a
 // CU of which the wavefronts wait 60 %: what helps is more of them.  4,096
-// queries of 1e3..1e5 triangles, back to back: 273 us with a scan of the
-// lanes by shuffles and one lane for all of a pair's axes (168 registers,
-// three blocks a CU); 220 with ballots and the axes split over lanes, at four
-// blocks a CU; 194 with the pose out of the vector registers and a shorter LDS
-// stack, at five; 248 at six, where registers spill.
+// queries of 1e3..1e5 triangles, a launch alone (ends on its longest query) /
+// back to back (which differs from run to run as much as given): 0.43 ms /
+// 252..273 us with a scan of the lanes by shuffles and one lane for all of a
+// pair's axes (168 registers, three blocks a CU); 220 us with ballots and the
+// axes split over lanes, at four blocks a CU; 0.38 ms / 165..194 us with the
+// pose out of the vector registers and a shorter LDS stack, at five; 248 us at
+// six, where registers spill.
 constexpr int kMeshOcc = 5;
 constexpr int kMeshLds = 2048;  // LDS stack entries per block
 constexpr int kMeshStackLds = 3072;  // entries a query has besides the knob's, in LDS or in device memory

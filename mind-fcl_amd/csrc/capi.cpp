@@ -239,7 +239,7 @@ static int refreshCounters(mfcl_ctx* ctx) {
   if (ctx->d_counters && ctx->d_qcounts) {
     MFCL_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     uint64_t dev[2] = {0, 0};
-    uint32_t q[5] = {0, 0, 0, 0, 0};  // EPA queue count, overflow count, 2 cursors, continued in device memory
+    uint32_t q[5] = {0, 0, 0, 0, 0};  // EpaCounts: queued, restarted, 2 cursors, continued
     MFCL_HIP_TRY(ctx, hipMemcpy(dev, ctx->d_counters, sizeof(dev), hipMemcpyDeviceToHost));
     MFCL_HIP_TRY(ctx, hipMemcpy(q, ctx->d_qcounts, sizeof(q), hipMemcpyDeviceToHost));
     ctx->counters[5] = q[4];

@@ -102,9 +102,9 @@ struct mfcl_ctx {
     int gjk_group{0};           // 0 by batch size; 1 a lane per pair; 16, 32, 64 a wavefront per pair
     int epa_threads{196608};    // persistent EPA lanes (multiple of 256): 64 per wavefront
     int guess_policy{1};        // warm start: 0 MLP direction for every pair, 1 not for predicted penetration
-    int epa_lds_faces{42};      // face capacity of the LDS polytope (overflow continues or reruns at full size)
-    int epa_spill{1};           // overflow continues in a device-memory polytope (1) or reruns (0)
-    int epa_overflow_waves{512};   // persistent wavefronts (one per block) for overflow pairs
+    int epa_lds_faces{42};      // face capacity of the first LDS polytope (pairs that outgrow it: epa_spill)
+    int epa_spill{1};           // 1: they continue from a dump at full capacity, 0: they restart there
+    int epa_overflow_waves{512};   // persistent wavefronts (one per block) of the full-capacity pass
     int mesh_blocks_per_cu{5};  // persistent mesh-traversal blocks (4 waves, one query each) per CU
     int mesh_stack{16384};      // node-pair stack entries per block
     int mlp_waves{0};           // wavefronts per block of the fused warm-start inference (0: by batch size)

@@ -6,9 +6,14 @@
 // indices, FP64 geometry), visited by the 64 lanes in parallel; creation
 // stamps stand in for the reference's newest-first element lists.
 //
-// The loop is bound by the latency of one pair's chain of dependent steps.
-// What a step keeps between its phases lives in LDS, the support search is
-// one out-of-line function (wave_dev.h), and nothing spills.
+// The loop is a chain of one pair's dependent steps; three wavefronts a SIMD
+// (epaQueueKernel) keep the vector units 66 % busy, the few long pairs of the
+// full-capacity pass 5 %.  What a step keeps between its phases lives in LDS
+// and the support search is one out-of-line function (wave_dev.h), so that no
+// value of the loop spills: the kernels' scratch (208 bytes a lane in
+// epaQueueKernel, 64 in the full-capacity pass) holds the registers that the
+// out-of-line functions save at their entry.  GJK in waveKernel, in front of
+// it, has 54 spills (400 bytes a lane) to stay at three wavefronts a SIMD.
 #pragma once
 
 #include <type_traits>
@@ -1008,7 +1013,7 @@ template <class M>
 __host__ __device__ inline size_t epaSliceBytes(int cap_faces) {
   return kEpaHeadBytes + arenaBytes<M>(cap_faces);
 }
-// A spilled pair in device memory: RawF, EpaResume and the slot arrays.
+// A dumped pair in device memory: RawF, EpaResume and the slot arrays.
 constexpr size_t kEpaDumpHead = sizeof(RawF) + sizeof(EpaResume);
 __host__ __device__ inline size_t epaDumpBytes(int cap_faces) {
   return (kEpaDumpHead + polyBytes<SmallMem>(cap_faces) + 255) & ~static_cast<size_t>(255);
@@ -1433,7 +1438,7 @@ __device__ __attribute__((noinline)) int epaRun(MFCL_LDS EpaLds* L, typename M::
   return status;
 }
 
-// A spilled pair to / from device memory: the records keep their slot
+// A dumped pair to / from device memory: the records keep their slot
 // numbers, the larger polytope's extra slots are free.  Slot numbers never
 // influence a result, so continuing there equals a run at the larger
 // capacity from the start.

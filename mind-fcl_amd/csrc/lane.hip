@@ -137,15 +137,16 @@ __global__ void __launch_bounds__(kBlock) laneKernel(ShapeTables T, PairIO io, c
   if (md.lane == 0 && v) atomicAdd(scanned_total, v);
 }
 
-// The same with refill: a persistent grid (two wavefronts per SIMD) whose
-// lanes take pairs from a shared cursor (the costly end of the bucketed
-// order first).  When at most refill_at lanes of a wavefront are still
+// The same with refill: a persistent grid (three wavefronts per SIMD for
+// distances, two for penetration) whose lanes take pairs from a shared cursor
+// (the costly end of the bucketed order first).  When at most refill_at lanes of a wavefront are still
 // running, the finished lanes write their results and take new pairs, so a
 // wavefront does not wait on its slowest pair.  Each pair's result and EPA
 // queue entry equal laneKernel's (a pair's computation does not depend on
-// its lane or wavefront).  The penetration-mode kernel is bounded to two
-// wavefronts per SIMD (it spills a little to fit); the signed-distance one
-// fits without the bound.
+// its lane or wavefront).  Both kernels are bounded to those wavefronts and
+// spill to fit: distances 864 spills (360 bytes of scratch a lane) at 168
+// registers, penetration 53 beside the closed forms' contact arrays (960
+// bytes).
 template <int MODE>
 __device__ __attribute__((always_inline)) inline void laneRefillBody(
     ShapeTables T, PairIO io, const uint32_t* order, uint64_t n, Params P, QEntry* queue, uint32_t* qcount,
@@ -203,8 +204,9 @@ __device__ __attribute__((always_inline)) inline void laneRefillBody(
   if (md.lane == 0 && v) atomicAdd(scanned_total, v);
 }
 
-// three wavefronts per SIMD: the spills this costs (168 VGPRs) are cheaper
-// than the latency left exposed at two; four spill too much
+// three wavefronts per SIMD: the spills this costs are cheaper than the
+// latency left exposed at two (524,288 pairs: 2.44 ms against 2.50 without
+// spills); four spill too much
 __global__ void __launch_bounds__(kBlock, 3) laneKernelRSd(ShapeTables T, PairIO io, const uint32_t* order, uint64_t n,
                                                         Params P, QEntry* queue, uint32_t* qcount,
                                                         unsigned long long* scanned_total, double* dir_ws,

@@ -1,5 +1,5 @@
-// Mesh-shape collision (fcl::collide(BVHModel<OBBRSS>, shape) with
-// penetration disabled): OrientedNodeBVHSolver::MeshShapeIntersect
+// Mesh-shape collision (fcl::collide(BVHModel<OBBRSS>, shape), penetration
+// disabled, and enabled below): OrientedNodeBVHSolver::MeshShapeIntersect
 // (include/fcl/narrowphase/detail/traversal/collision/bvh_solver-inl.h:6-72)
 // tests the mesh's tree against the shape's volume and every reached leaf
 // triangle against the shape (ShapeSimplexIntersect, shape_pair_intersect-

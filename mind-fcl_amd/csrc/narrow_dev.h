@@ -100,8 +100,7 @@ MFCL_D DevShape loadShape(const ShapeTables& T, uint32_t i) {
 // padding, so the fixed-size read stays in bounds), then the neighbours'
 // vertices -- each 16-byte vertex also carrying its own record offset -- in a
 // second batch, and only then runs the reference's sequential comparisons in
-// registers: two dependent memory round trips per step.  The two walks of one support query (one per
-// shape) advance in lock step so their round trips overlap.
+// registers: two dependent memory round trips per step.
 constexpr int kWalkChunk = 8;
 
 struct Walk {
@@ -113,47 +112,16 @@ struct Walk {
   float3 w[kWalkChunk];
 };
 
-// Walk starts: the reference seeds every walk from the best of six axis-
-// direction caches (convex-inl.h:151-199); a start >= 0 replaces that seed
-// with a given vertex (the caller's earlier support point for a nearby
-// direction).  On a convex hull a walk ends where no neighbour improves the
-// support value, which is the unique maximiser whatever the start; only
-// exact ties between support values (a face orthogonal to the direction)
-// can make the end depend on the start.
-MFCL_D int walkSeed(const DevShape& s, d3 d) {
+// The walk's start: the best of the six axis directions' seeds
+// (convex-inl.h:151-199: +-UnitX, +-UnitY, +-UnitZ), first on ties.
+MFCL_D void walkInit(Walk& W, const DevShape& s, d3 d) {
+  W.d = d;
+  W.keep = true;
+  W.count = 0;
   int init = -1;
   double max_dot = 0;
 #pragma unroll
   for (int i = 0; i < 6; ++i) {
-    // the seed directions of convex-inl.h:151-199: +-UnitX, +-UnitY, +-UnitZ
-    const double sg = (i & 1) ? -1.0 : 1.0;
-    const double ax = (i >> 1) == 0 ? sg : sg * 0.0;
-    const double ay = (i >> 1) == 1 ? sg : sg * 0.0;
-    const double az = (i >> 1) == 2 ? sg : sg * 0.0;
-    const double dv = ax * d.x + ay * d.y + az * d.z;
-    if (init < 0 || dv > max_dot) {
-      init = s.seed[i];
-      max_dot = dv;
-    }
-  }
-  return init;
-}
-
-MFCL_D void walkInit(Walk& W, const DevShape& s, d3 d, bool active, int start = -1) {
-  W.d = d;
-  W.keep = active;
-  W.visited = 0;
-  W.ext = 0;
-  W.ext_v = 0;
-  W.start = 0;
-  W.count = 0;
-  if (!active) return;
-  int init = start;
-  double max_dot = 0;
-  if (init < 0)
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    // the seed directions of convex-inl.h:151-199: +-UnitX, +-UnitY, +-UnitZ
     const double sg = (i & 1) ? -1.0 : 1.0;
     const double ax = (i >> 1) == 0 ? sg : sg * 0.0;
     const double ay = (i >> 1) == 1 ? sg : sg * 0.0;
@@ -253,9 +221,9 @@ MFCL_D float3 blkLoad(const float4* wblk, int v, BlkWalk& B) {
 }
 
 // The walk over the adjacency table.
-MFCL_D int hullWalkTab(const DevShape& s, d3 d, int* scanned, int start = -1) {
+MFCL_D int hullWalkTab(const DevShape& s, d3 d, int* scanned) {
   Walk W;
-  walkInit(W, s, d, true, start);
+  walkInit(W, s, d);
   while (W.keep) {
     walkFetchRecord(W, s);
     walkFetchNeighbours(W, s);

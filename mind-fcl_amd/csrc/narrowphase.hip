@@ -279,7 +279,8 @@ uint64_t staticScratchMaxPairs() {
 // larger ones fill the chip with one pair per lane.  A lane's pair takes
 // 1.1-1.5 ms however few there are, a wavefront's 40-100 us.  The lines lie
 // where the wavefronts win both alone and with two other batches beside them
-// (us per batch, lane / wave; hulls of 8..512 vertices, contacts 8..256):
+// (us per batch on 256 CUs, lane / wave; hulls of 8..512 vertices, contacts
+// 8..256); alone they win to beyond them:
 //   distance    24,576 pairs: alone 1413 / 868, beside others 560 / 500
 //               32,768 pairs: alone 1550 / 1120, beside others 574 / 677
 //   penetration  8,192 pairs: alone 1663 / 1298, beside others 747 / 699

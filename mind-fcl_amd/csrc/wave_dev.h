@@ -110,7 +110,7 @@ MFCL_D double readLaneF64(double v, int src) {
   return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
 }
 
-// The seed of a walk (walkSeed's rule): the axis of the largest support
+// The seed of a walk (walkInit's rule): the axis of the largest support
 // value, first on ties.  A finite direction's six products with the signed
 // unit axes are its signed components; with a non-finite one the sums
 // mostly turn NaN, so they are formed in full.

@@ -349,9 +349,9 @@ class Context:
         return ms
 
     def last_counters(self) -> np.ndarray:
-        """[pairs, hull vertices read (GJK + EPA stages), EPA pairs, EPA
-        reruns at full capacity, hull vertices read by the EPA stage, EPA
-        pairs continued in a device-memory polytope of full capacity]"""
+        """[pairs, hull vertices evaluated (GJK + EPA stages), EPA pairs, EPA
+        pairs restarted at full capacity, hull vertices evaluated by the EPA
+        stage, EPA pairs continued at full capacity] (mfcl_last_counters_n)"""
         c = np.zeros(6, np.uint64)
         self._check(self.lib.mfcl_last_counters_n(self.h, _ptr(c), 6))
         return c
