@@ -55,7 +55,8 @@ __device__ __forceinline__ float normalTail(float x) {
   p = __builtin_fmaf(p, t, -1.0f);
   return __builtin_amdgcn_exp2f(p);
 }
-// x Phi(x) = max(x, 0) - |x| q
+// x Phi(x) = max(x, 0) - |x| q; NaN for an infinite x (with erff for -inf alone:
+// the next layer's sums of mixed signs are NaN from either)
 __device__ __forceinline__ float geluF(float x, float q) { return __builtin_fmaf(-fabsf(x), q, fmaxf(x, 0.f)); }
 __device__ __forceinline__ float geluF(float x) { return geluF(x, normalTail(x)); }
 // GELU's derivative Phi(x) + x phi(x)
